@@ -147,6 +147,98 @@ __global__ void __launch_bounds__(256) colsum_kernel(const void *x, int x_dt, lo
     if (dt_bits(out_dt) == 32) ((uint32_t *)out)[c] = bits;
     else ((uint16_t *)out)[c] = (uint16_t)bits;
 }
+
+// The same sums in the same order with the loads taken out of the chain.  The additions of a column are serial (a
+// handful of cycles each), but in colsum_kernel every one of them also waits for its own load: 0.3 us a row.  Here a
+// workgroup owns 64 columns (a whole 128-byte line of a 16-bit row); all four wavefronts fetch chunks of 16 KB, two
+// chunks ahead in registers, and park them in LDS with the rows of a column side by side; wavefront 0 adds them, 16
+// bytes of a column's rows per LDS read.  2048 x 14336 bf16: 689 -> 21 us.
+template <int DT>
+__global__ void __launch_bounds__(256) colsum_chunks_kernel(const char *x, long rows, long cols, long ld, void *out,
+        int out_dt) {
+    constexpr int EB = DT == MI355_DT_F32 ? 4 : 2; // bytes per element
+    constexpr int CR = EB == 2 ? 128 : 64;         // rows of a chunk
+    constexpr int PITCH = CR * EB / 4 + 4;         // dwords per column in LDS: 16-byte aligned, columns 4 banks apart
+    constexpr int TPR = 64 * EB / 16;              // threads that fetch a row's 64 columns, 16 bytes each
+    constexpr int RPP = 256 / TPR;                 // rows per pass of the workgroup
+    constexpr int NP = CR / RPP;                   // passes (loads of a thread) per chunk: 4
+    static_assert(NP == 4, "four 16-byte loads per thread and chunk");
+    __shared__ __attribute__((aligned(16))) uint32_t tile[2][64 * PITCH];
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    const int t = threadIdx.x, lane = t & 63;
+    const long c0 = (long)blockIdx.x * 64;
+    const int cc = t % TPR * (16 / EB);            // first of the thread's columns inside the 64
+    const long cg = c0 + cc < cols ? c0 + cc : c0; // (a group beyond the last column fetches the first one's)
+    // 16-bit: a thread fetches pairs of rows, so that a dword of LDS is two rows of a column
+    auto row_of = [&](int p) { return EB == 2 ? 2 * (t / TPR) + (p & 1) + 2 * RPP * (p >> 1) : t / TPR + RPP * p; };
+    auto fetch = [&](long r0, u4v (&q)[NP]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            long r = r0 + row_of(p);
+            r = r < rows ? r : rows - 1;           // rows beyond the last are fetched from it and not added
+            q[p] = *(const u4v *)(x + (r * ld + cg) * EB);
+        }
+    };
+    auto park = [&](uint32_t *buf, const u4v (&q)[NP]) __attribute__((always_inline)) {
+        if constexpr (EB == 2) {
+#pragma unroll
+            for (int p = 0; p < NP; p += 2)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    uint32_t *d = buf + (cc + 2 * e) * PITCH + row_of(p) / 2;
+                    d[0] = __builtin_amdgcn_perm(q[p + 1][e], q[p][e], 0x05040100u);
+                    d[PITCH] = __builtin_amdgcn_perm(q[p + 1][e], q[p][e], 0x07060302u);
+                }
+        } else {
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) buf[(cc + e) * PITCH + row_of(p)] = q[p][e];
+        }
+    };
+    float acc = 0.f;
+    auto add = [&](const uint32_t *buf, long left) __attribute__((always_inline)) {
+        const u4v *col = (const u4v *)(buf + lane * PITCH);
+        constexpr int PER = 16 / EB;               // rows per 16-byte read
+        auto value = [&](const u4v &v, int i) -> float {
+            if (EB == 4) return u2f(v[i]);
+            const uint32_t w = v[i / 2], h = (i & 1) ? w >> 16 : w & 0xffffu;
+            return DT == MI355_DT_BF16 ? u2f((i & 1) ? w & 0xffff0000u : w << 16) : (float)__builtin_bit_cast(_Float16, (unsigned short)h);
+        };
+        if (left >= CR) {
+#pragma unroll 4
+            for (int r = 0; r < CR / PER; ++r) {
+                const u4v v = col[r];
+#pragma unroll
+                for (int i = 0; i < PER; ++i) acc += value(v, i);
+            }
+        } else {
+            for (int r = 0; r < CR / PER; ++r) {
+                const u4v v = col[r];
+#pragma unroll
+                for (int i = 0; i < PER; ++i)
+                    if (r * PER + i < left) acc += value(v, i);
+            }
+        }
+    };
+    u4v qa[NP], qb[NP];
+    fetch(0, qa);
+    fetch(CR, qb);
+    for (long r0 = 0; r0 < rows; r0 += 2 * CR) {
+        park(tile[0], qa);
+        fetch(r0 + 2 * CR, qa);
+        __syncthreads();   // (also: wavefront 0 is done with tile[1])
+        if (t < 64) add(tile[0], rows - r0);
+        park(tile[1], qb);
+        fetch(r0 + 3 * CR, qb);
+        __syncthreads();
+        if (t < 64 && rows - r0 > CR) add(tile[1], rows - r0 - CR);
+    }
+    if (t >= 64 || c0 + lane >= cols) return;
+    const uint32_t bits = cvt_store_bits(out_dt, acc);
+    if (dt_bits(out_dt) == 32) ((uint32_t *)out)[c0 + lane] = bits;
+    else ((uint16_t *)out)[c0 + lane] = (uint16_t)bits;
+}
 } // namespace mi355
 
 extern "C" int mi355_colsum_launch(const void *x, int x_dt, int64_t rows, int64_t cols, int64_t ld, void *out, int out_dt,
@@ -157,6 +249,19 @@ extern "C" int mi355_colsum_launch(const void *x, int x_dt, int64_t rows, int64_
         return MI355_INVALID_ARGUMENTS;
     }
     if (cols == 0) return MI355_SUCCESS;
+    // 16-byte loads of whole column groups; a single row or an odd pitch stays with the plain kernel
+    const int eb = dt_bits(x_dt) / 8, per = 16 / eb;
+    if (rows > 1 && cols % per == 0 && ld % per == 0 && (uintptr_t)x % 16 == 0) {
+        const dim3 grid((unsigned)((cols + 63) / 64));
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, (const char *)x, (long)rows, (long)cols,
+                    (long)ld, out, out_dt);
+        };
+        if (x_dt == MI355_DT_BF16) go(colsum_chunks_kernel<MI355_DT_BF16>);
+        else if (x_dt == MI355_DT_F16) go(colsum_chunks_kernel<MI355_DT_F16>);
+        else go(colsum_chunks_kernel<MI355_DT_F32>);
+        return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
+    }
     hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, (hipStream_t)stream, x, x_dt,
             (long)rows, (long)cols, (long)ld, out, out_dt);
     return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
