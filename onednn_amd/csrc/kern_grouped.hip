@@ -245,16 +245,19 @@ __device__ __forceinline__ void gk_store(const grouped_k_dev_t &P, const gk_f4 (
     // dst is written once and not read again by the launch: non-temporal stores, which do not take lines of the
     // L2s (a quarter faster on a launch that writes 1.3 GB: 0.325 -> 0.25 ms)
     // bf16: v_cvt_pk_bf16_f32 unless the wavefront holds a NaN or an f32 subnormal, which the software conversion
-    // (the reference's: subnormals flush, NaNs are quieted its way) treats differently
+    // (the reference's: subnormals flush, NaNs are quieted its way) treats differently; f16: v_cvt_f16_f32 unless it
+    // holds a NaN (the 64 software roundings a lane were the kernel's bound: 64 groups of 435 rows, 3712 x 8064, f16,
+    // 2179 -> 732 us)
     bool hw = false;
-    if (DT == MI355_DT_BF16) {
+    if (DT == MI355_DT_BF16 || DT == MI355_DT_F16) {
+        constexpr int SPECIAL = DT == MI355_DT_BF16 ? 0x93 : 0x03;
         bool special = false;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int c = 0; c < 4; ++c)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) special |= __builtin_amdgcn_classf(acc[r][c][e], 0x93);
+                for (int e = 0; e < 4; ++e) special |= __builtin_amdgcn_classf(acc[r][c][e], SPECIAL);
         hw = __builtin_amdgcn_ballot_w64(special) == 0;
     }
     if (col >= P.NB) return;
@@ -274,6 +277,12 @@ __device__ __forceinline__ void gk_store(const grouped_k_dev_t &P, const gk_f4 (
                 gk_u2 o;
                 o.x = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2_t {v0, v1}, bf16x2_t));
                 o.y = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2_t {v2, v3}, bf16x2_t));
+                __builtin_nontemporal_store(o, (gk_u2 *)((uint16_t *)P.dst + off));
+            } else if (DT == MI355_DT_F16 && hw) {
+                typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+                gk_u2 o;
+                o.x = __builtin_bit_cast(unsigned, f16x2_t {(_Float16)v0, (_Float16)v1});
+                o.y = __builtin_bit_cast(unsigned, f16x2_t {(_Float16)v2, (_Float16)v3});
                 __builtin_nontemporal_store(o, (gk_u2 *)((uint16_t *)P.dst + off));
             } else {
                 gk_u2 o;
