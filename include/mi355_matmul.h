@@ -550,6 +550,20 @@ typedef struct {
 int mi355_sdpa_softmax_launch(const mi355_softmax_desc_t *desc, const void *scores, void *probs, const void *scale,
         const void *mask, void *stream);
 
+/* Scaled dot-product attention as one kernel: bf16 / f16 tensors with rows of d = 64 or 128 contiguous elements,
+ * hk = h or 1 key / value heads.  Strides in elements: batch, head, row; those of q, k, v multiples of 8, those of dst
+ * of 4; buffers 16-byte aligned.  mask_type, scale and inf_as_zero as above; mask strides are 0 along a dimension the
+ * mask is broadcast over.  mi355_sdpa_query: MI355_UNIMPLEMENTED for anything else, otherwise the scratch a launch
+ * needs (the keys may be split over workgroups). */
+typedef struct {
+    int64_t b, h, hk, sq, sk, d;
+    int64_t q_stride[3], k_stride[3], v_stride[3], dst_stride[3], mask_stride[4];
+    int32_t dt, dst_dt, scale_dt, invert_scale, mask_type, mask_dt, inf_as_zero, reserved;
+} mi355_sdpa_desc_t;
+int mi355_sdpa_query(const mi355_sdpa_desc_t *desc, size_t *scratch_bytes);
+int mi355_sdpa_launch(const mi355_sdpa_desc_t *desc, const void *q, const void *k, const void *v, void *dst,
+        const void *scale, const void *mask, void *scratch, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -255,6 +255,9 @@ struct dnnl_primitive_desc {
         bool invert_scale = false, inf_as_zero = false;
         int mask_type = 0;
         std::shared_ptr<dnnl_primitive_desc> kq, vs;
+        bool fused = false;             // one kernel over the keys (mi355_sdpa_launch) instead of the composition
+        mi355_sdpa_desc_t fused_desc;
+        size_t fused_scratch = 0, composed_scratch = 0;
     };
     std::shared_ptr<sdpa_t> sdpa;
     mi355_grouped_desc_t gdesc;
@@ -284,8 +287,9 @@ struct dnnl_primitive_desc {
 
 struct dnnl_primitive {
     dnnl_primitive_desc pd;
-    dnnl_primitive *sdpa_kq = nullptr, *sdpa_vs = nullptr; // the two matmuls of an attention primitive
+    dnnl_primitive *sdpa_kq = nullptr, *sdpa_vs = nullptr; // the two matmuls of a composed attention primitive
     void *scratch = nullptr; // library-mode scratchpad (device)
+    void *composed = nullptr; // the composition's scores and probabilities: `scratch`, or on demand behind the fused kernel
     std::mutex scratch_mutex;
     // runtime dims: the lowering of the last executed shapes, and the scratch
     // buffers allocated for executions so far (kept until the primitive is
@@ -305,6 +309,7 @@ struct dnnl_primitive {
     ~dnnl_primitive() {
         delete sdpa_kq;
         delete sdpa_vs;
+        if (composed && composed != scratch) mi355_mem_free(composed);
         if (scratch) mi355_mem_free(scratch);
         for (void *q : rt_scratch) mi355_mem_free(q);
         if (host_scalars) mi355_mem_free(host_scalars);
@@ -2286,7 +2291,33 @@ DNNL_EXPORT dnnl_status_t dnnl_amd_sdpa_primitive_desc_create(dnnl_primitive_des
     if (st) return st;
     S->vs.reset(vs);
     pd->src = q; pd->wei = k; pd->dst = d;
-    pd->scratch_bytes = ((S->scores.size_bytes() + 255) & ~(size_t)255) + S->probs.size_bytes();
+    // One kernel over the keys where it takes the problem (mi355_sdpa_query): rows of one head contiguous, the same
+    // key / value heads for both.  The composition stays for everything else and for unaligned buffers.
+    if (k.dims[1] == v.dims[1] && q.dims[3] == v.dims[3]) {
+        mi355_sdpa_desc_t &F = S->fused_desc;
+        memset(&F, 0, sizeof(F));
+        F.b = B; F.h = H; F.hk = k.dims[1]; F.sq = Sq; F.sk = Sk; F.d = q.dims[3];
+        F.dt = (int)q.dt; F.dst_dt = (int)d.dt;
+        F.scale_dt = with_scale ? (int)scale_desc->dt : (int)MI355_DT_UNDEF;
+        F.invert_scale = S->invert_scale;
+        F.mask_type = mask_type;
+        F.inf_as_zero = S->inf_as_zero;
+        auto take = [](const dnnl_memory_desc &md, int row_dim, int64_t *st3) {
+            for (int i = 0; i < 3; ++i) {
+                const int dim = i < 2 ? i : row_dim;
+                st3[i] = md.dims[dim] == 1 ? 0 : md.strides[dim];
+            }
+            return md.strides[5 - row_dim] == 1; // the other one of the last two dims
+        };
+        bool ok = take(q, 2, F.q_stride) && take(k, 3, F.k_stride) && take(v, 2, F.v_stride) && take(d, 2, F.dst_stride);
+        if (mask_type == 1) {
+            F.mask_dt = (int)mask_desc->dt;
+            for (int i = 0; i < 4; ++i) F.mask_stride[i] = mask_desc->dims[i] == 1 ? 0 : mask_desc->strides[i];
+        }
+        S->fused = ok && mi355_sdpa_query(&F, &S->fused_scratch) == MI355_SUCCESS;
+    }
+    S->composed_scratch = ((S->scores.size_bytes() + 255) & ~(size_t)255) + S->probs.size_bytes();
+    pd->scratch_bytes = S->fused ? S->fused_scratch : S->composed_scratch;
     pd->scratchpad = dnnl_memory_desc(); // library mode only: nothing for the caller to provide
     pd->impl_name = "hip:sdpa(" + kq->impl_name + "," + vs->impl_name + ")";
     pd->sdpa = S;
@@ -2523,6 +2554,24 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_desc_query(const_dnnl_primitive_desc_t 
 }
 
 // ---- primitive
+// The matmuls of an attention primitive and the memory between them: at creation, or -- where the fused kernel takes the
+// problem -- at the first execution on buffers it does not take.
+static dnnl_status_t sdpa_compose(dnnl_primitive &p) {
+    const dnnl_primitive_desc::sdpa_t &S = *p.pd.sdpa;
+    if (!p.composed && S.composed_scratch > 0) {
+        const int st = mi355_mem_alloc(&p.composed, S.composed_scratch);
+        if (st != MI355_SUCCESS) return from_mi355(st);
+    }
+    for (int i = 0; i < 2; ++i) {
+        dnnl_primitive *&slot = i ? p.sdpa_vs : p.sdpa_kq;
+        if (slot) continue;
+        dnnl_primitive_t made = nullptr;
+        const dnnl_status_t st = dnnl_primitive_create(&made, i ? S.vs.get() : S.kq.get());
+        if (st != dnnl_success) return st;
+        slot = made;
+    }
+    return dnnl_success;
+}
 DNNL_EXPORT dnnl_status_t dnnl_primitive_create(dnnl_primitive_t *primitive, const_dnnl_primitive_desc_t pd) {
     CHECK_ARG(primitive && pd);
     std::unique_ptr<dnnl_primitive> p(new dnnl_primitive);
@@ -2532,12 +2581,9 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_create(dnnl_primitive_t *primitive, con
         const int st = mi355_mem_alloc(&p->scratch, p->pd.scratch_bytes);
         if (st != MI355_SUCCESS) return from_mi355(st);
     }
-    if (p->pd.sdpa) {
-        dnnl_primitive_t kq = nullptr, vs = nullptr;
-        dnnl_status_t st = dnnl_primitive_create(&kq, p->pd.sdpa->kq.get());
-        if (st == dnnl_success) st = dnnl_primitive_create(&vs, p->pd.sdpa->vs.get());
-        p->sdpa_kq = kq;
-        p->sdpa_vs = vs;
+    if (p->pd.sdpa && !p->pd.sdpa->fused) {
+        p->composed = p->scratch;
+        const dnnl_status_t st = sdpa_compose(*p);
         if (st != dnnl_success) return st;
     }
     bool any_on_host = false;
@@ -2636,13 +2682,32 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
         CHECK_ARG(IMPLICATION(S.mask_type == 1, mask && mask->handle));
         CHECK_ARG(IMPLICATION(!S.scale.is_zero(), scale && scale->handle));
         if (S.dst.nelems() == 0) return dnnl_success;
-        CHECK_ARG(q->handle && k->handle && v->handle && d->handle && prim->scratch);
+        CHECK_ARG(q->handle && k->handle && v->handle && d->handle);
         if (mi355_device_set((int)pd0.engine->index) != MI355_SUCCESS) return dnnl_runtime_error;
+        auto record = [&]() {
+            if (prim->order_event && mi355_event_record(prim->order_event, stream->hip_stream) == MI355_SUCCESS) {
+                prim->event_recorded = true;
+                prim->last_stream = stream->hip_stream;
+            }
+        };
+        const uintptr_t low = (uintptr_t)q->handle | (uintptr_t)k->handle | (uintptr_t)v->handle | (uintptr_t)d->handle;
+        if (S.fused && low % 16 == 0) {
+            if (prim->scratch) order_on_device(); // the parts of a split launch belong to the primitive
+            const int rc = mi355_sdpa_launch(&S.fused_desc, q->handle, k->handle, v->handle, d->handle,
+                    scale ? scale->handle : nullptr, mask ? mask->handle : nullptr, prim->scratch, stream->hip_stream);
+            if (ordered) record();
+            return from_mi355(rc);
+        }
         order_on_device(); // the scores and probabilities belong to the primitive
+        if (S.fused) {
+            const dnnl_status_t cs = sdpa_compose(*prim);
+            if (cs != dnnl_success) return cs;
+        }
+        CHECK_ARG(prim->composed);
         dnnl_memory sc_mem, pr_mem;
-        sc_mem.md = S.scores; sc_mem.engine = pd0.engine; sc_mem.handle = prim->scratch;
+        sc_mem.md = S.scores; sc_mem.engine = pd0.engine; sc_mem.handle = prim->composed;
         pr_mem.md = S.probs; pr_mem.engine = pd0.engine;
-        pr_mem.handle = (char *)prim->scratch + ((S.scores.size_bytes() + 255) & ~(size_t)255);
+        pr_mem.handle = (char *)prim->composed + ((S.scores.size_bytes() + 255) & ~(size_t)255);
         const dnnl_exec_arg_t a1[3] = {{DNNL_ARG_SRC, q}, {DNNL_ARG_WEIGHTS, k}, {DNNL_ARG_DST, &sc_mem}};
         dnnl_status_t st = dnnl_primitive_execute(prim->sdpa_kq, stream, 3, a1);
         if (st != dnnl_success) return st;
@@ -2666,10 +2731,7 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
         if (rc != MI355_SUCCESS) return from_mi355(rc);
         const dnnl_exec_arg_t a2[3] = {{DNNL_ARG_SRC, &pr_mem}, {DNNL_ARG_WEIGHTS, v}, {DNNL_ARG_DST, d}};
         st = dnnl_primitive_execute(prim->sdpa_vs, stream, 3, a2);
-        if (prim->order_event && mi355_event_record(prim->order_event, stream->hip_stream) == MI355_SUCCESS) {
-            prim->event_recorded = true;
-            prim->last_stream = stream->hip_stream;
-        }
+        record();
         return st;
     }
     void *rt_scratch = nullptr;

@@ -1,0 +1,74 @@
+"""The one-kernel attention path (bf16 / f16, head size 64 or 128) at the sizes where it can go wrong: ends of the tiles
+of 32 / 64 keys and 32 / 128 query rows, both forms around 64 rows, keys split over workgroups, masks whose rows start at
+any element or whose keys do not lie side by side, and buffers it does not take (the composition runs then)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from onednn_amd import cabi, dnnl
+from tests.test_sdpa import DT, ideal, make, md4, run, storage, tolerance, values
+from onednn_amd.problem import storage_dtype
+
+SHAPES = [  # b, h, hk, sq, sk
+    (1, 2, 2, 1, 1), (2, 3, 3, 1, 31), (1, 2, 2, 3, 33), (1, 4, 1, 16, 64), (1, 4, 1, 17, 65),   # few rows, 64 and 68
+    (1, 2, 2, 64, 63), (1, 2, 2, 65, 64), (1, 1, 1, 128, 65), (1, 3, 1, 129, 191), (2, 2, 2, 257, 40),
+    (1, 2, 1, 1, 3000), (1, 1, 1, 200, 2500),                                                        # split keys
+]
+
+
+def check(dt, d, shape, **kw):
+    b, h, hk, sq, sk = shape
+    q, k, v = make(21, b, h, hk, sq, sk, d, d, dt)
+    sc = np.array([kw.pop("sc", 1.0 / np.sqrt(d))], np.float32)
+    mask = kw.pop("mask", None)
+    got, impl = run(q, k, v, dt, dt, True, scale=sc, mask=mask, mask_type=kw.get("mask_type", 0))
+    want, pabs = ideal(q, k, v, dt, scale=float(sc[0]), mask=None if mask is None else mask.astype(np.float64),
+                       mask_type=kw.get("mask_type", 0))
+    err = np.abs(values(dt, got) - want)
+    tol = tolerance(dt, dt, sk, pabs, want)
+    assert (err <= tol).all(), f"{impl}: worst {np.nanmax(err / tol):.2f} of the bound"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_edges_of_the_tiles(gpu, dt, d, shape):
+    check(dt, d, shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 2, 2, 200, 200), (1, 4, 1, 40, 150), (1, 2, 2, 150, 333)])
+@pytest.mark.parametrize("mask_type", [1, 2, 3])
+def test_masks_and_a_negative_scale(gpu, shape, mask_type):
+    b, h, hk, sq, sk = shape
+    mask = (np.random.default_rng(5).standard_normal((1, 1, sq, sk)) * 2).astype(np.float32) if mask_type == 1 else None
+    check("bf16", 64, shape, mask=mask, mask_type=mask_type, sc=-0.11)
+
+
+@pytest.mark.gpu
+def test_unaligned_buffers_run_the_composition(gpu):
+    """q one element off a 16-byte boundary: the same result within the same bound."""
+    b, h, sq, sk, d = 1, 2, 40, 72, 64
+    q, k, v = make(22, b, h, h, sq, sk, d, d, "bf16")
+    eng = dnnl.engine(dnnl.gpu, 0)
+    strm = dnnl.stream(eng)
+    mds = [md4(q.shape, "bf16"), md4(k.shape, "bf16", transposed=True), md4(v.shape, "bf16"), md4((b, h, sq, d), "bf16")]
+    pd = dnnl.sdpa_primitive_desc(eng, *mds)
+    prim = dnnl.sdpa(pd)
+    flat = np.zeros(q.size + 1, storage_dtype(DT["bf16"]))
+    flat[1:] = storage(q).reshape(-1)
+    raw = cabi.DeviceBuffer.from_numpy(flat)
+    qm = dnnl.memory.__new__(dnnl.memory)
+    qm.md, qm.engine, qm.h = mds[0], eng, C.c_void_p()
+    assert dnnl.lib().dnnl_memory_create(C.byref(qm.h), mds[0].h, eng.h, C.c_void_p(raw.ptr + 2)) == dnnl.success
+    dst = dnnl.memory(mds[3], eng)
+    args = {dnnl.ARG_QUERIES: qm, dnnl.ARG_KEYS: dnnl.memory(mds[1], eng, storage(k)),
+            dnnl.ARG_VALUES: dnnl.memory(mds[2], eng, storage(v)), dnnl.ARG_DST: dst}
+    want, pabs = ideal(q, k, v, "bf16")
+    for _ in range(2):
+        prim.execute(strm, args)
+        strm.wait()
+        got = values("bf16", dst.read(storage_dtype(DT["bf16"])).reshape(b, h, sq, d))
+        assert (np.abs(got - want) <= tolerance("bf16", "bf16", sk, pabs, want)).all()
