@@ -41,6 +41,7 @@ typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 struct __attribute__((packed, aligned(2))) mask2_t { i2v v; };
 struct __attribute__((packed, aligned(4))) mask4_t { f4v v; };
 typedef const i4v __attribute__((address_space(3))) *lds_i4_t;
+typedef i4v __attribute__((address_space(3))) *lds_w4_t;
 typedef s4v __attribute__((address_space(3))) *lds_s4_t;
 typedef float __attribute__((address_space(3))) *lds_f_t;
 
@@ -155,8 +156,10 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
     const bool neg = c < 0.f; // folded into Q, so that a larger score stays a larger exponent
     c = neg ? -c : c;
     const float sc = c;
-    if (MASK) c = LOG2E;
-    else c = c * LOG2E;
+    // (with a buffer the scores stay in units of e until the maximum is taken off: a mask of the type's lowest value
+    // times log2(e) would be -inf, and a row of nothing else has to weigh its keys alike)
+    constexpr float UNIT = MASK ? LOG2E : 1.f;
+    c = MASK ? 1.f : c * LOG2E;
     c = c < 1e-30f ? 1e-30f : c; // (a scale of zero must not meet the infinities of masked keys)
 
     i4v qf[QT];
@@ -230,12 +233,20 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
         }
     }
 
+    // Rows beyond the last key hold that key's values again, and meet probabilities of 0: zeros instead, since an
+    // infinity there would make NaN of a result that is infinite.  (A row of V fills its ROWB bytes of the tile.)
+    auto clear_tail = [&](int t, int buf, int first, int step) __attribute__((always_inline)) {
+        const unsigned v0 = lds0 + ring + (unsigned)buf * 2 * TILE + TILE;
+        for (int at = (sk - t * KT) * ROWB + 16 * first; at < TILE; at += 16 * step)
+            *(lds_w4_t)(size_t)(v0 + (unsigned)at) = i4v {0, 0, 0, 0};
+    };
+
     f16v o[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[n][r] = 0.f;
-    float m = -INFINITY, l = 0.f; // running maximum (in units of log2), this lane half's sum of p
+    float m = -INFINITY, l = 0.f; // running maximum (in units of 1 / UNIT of log2), this lane half's sum of p
 
     auto tile = [&](int t, int buf) __attribute__((always_inline)) {
         const unsigned kl = lds0 + ring + (unsigned)buf * 2 * TILE, vl = kl + TILE;
@@ -313,9 +324,9 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[x][r]);
         mx = halves_max(mx) * c;
-        if (__builtin_amdgcn_ballot_w64(mx > m + 8.f) != 0) {
+        if (__builtin_amdgcn_ballot_w64(mx > m + 8.f / UNIT) != 0) {
             const float mn = fmaxf(m, mx);
-            const float f = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+            const float f = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m - mn) * UNIT);
             m = mn;
             l *= f;
 #pragma unroll
@@ -330,8 +341,8 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
         for (int x = 0; x < ST; ++x)
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
-                const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[x][r], c, -shift));
-                const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[x][r + 1], c, -shift));
+                const float p0 = __builtin_amdgcn_exp2f(MASK ? (s[x][r] - shift) * UNIT : __builtin_fmaf(s[x][r], c, -shift));
+                const float p1 = __builtin_amdgcn_exp2f(MASK ? (s[x][r + 1] - shift) * UNIT : __builtin_fmaf(s[x][r + 1], c, -shift));
                 sum += p0 + p1;
                 p[2 * x + r / 8][(r % 8) / 2] = sdpa_pack<DT>(p0, p1);
             }
@@ -354,6 +365,10 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads(); // the tile is in LDS, and everybody is done with the other buffer
             if (t + 1 < t_end) issue(t + 1, buf ^ 1);
+            if (t * KT + KT > sk) { // the last tile, partly filled
+                clear_tail(t, buf, (int)threadIdx.x, 256);
+                __syncthreads();
+            }
             if (t * KT < w_hi) tile(t, buf); // (a tile beyond this wavefront's diagonal holds nothing for it)
         }
     } else {
@@ -369,6 +384,7 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
             } else {
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             }
+            if (t * KT + KT > sk) clear_tail(t, buf, lane, 64); // (a wavefront's own tile: its LDS accesses keep their order)
             tile(t, buf);
             buf ^= 1;
         }
@@ -398,7 +414,7 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
         l = 0.f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-            f[w] = mm == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(mw[w] - mm);
+            f[w] = mm == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((mw[w] - mm) * UNIT);
             l += f[w] * *(lds_f_t)(size_t)(ml + (unsigned)(w * 128 + 64 + lane) * 4);
         }
         m = mm;
@@ -462,13 +478,14 @@ __global__ void __launch_bounds__(256) sdpa_combine_kernel(const sdpa_dev_t P) {
     if (id >= nbh * P.rows) return;
     const int col = 4 * (threadIdx.x % tpr);
     const long total = nbh * P.rows;
+    const float unit = Dd.mask_type == 1 ? 1.44269504088896340736f : 1.f; // as in sdpa_kernel
     float mm = -INFINITY;
     for (int s = 0; s < P.splits; ++s) mm = fmaxf(mm, P.part_ml[2 * (s * total + id)]);
     float l = 0.f;
     f4v acc = {0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < P.splits; ++s) {
         const long at = s * total + id;
-        const float f = mm == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(P.part_ml[2 * at] - mm);
+        const float f = mm == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((P.part_ml[2 * at] - mm) * unit);
         l += f * P.part_ml[2 * at + 1];
         const f4v v = *(const f4v *)(P.part_o + at * Dd.d + col);
 #pragma unroll

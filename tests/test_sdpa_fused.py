@@ -72,3 +72,38 @@ def test_unaligned_buffers_run_the_composition(gpu):
         strm.wait()
         got = values("bf16", dst.read(storage_dtype(DT["bf16"])).reshape(b, h, sq, d))
         assert (np.abs(got - want) <= tolerance("bf16", "bf16", sk, pabs, want)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mdt,lowest", [("f32", np.finfo(np.float32).min), ("bf16", -3.3895313892515355e38), ("f16", -65504.0)])
+@pytest.mark.parametrize("shape", [(1, 2, 2, 150, 333), (1, 2, 2, 3, 1200)])
+def test_mask_of_the_types_lowest_value(gpu, shape, mdt, lowest):
+    """Not -inf: a query all of whose keys are masked so weighs them alike in f32 (the scores vanish beside the mask;
+    65504 in f16 leaves them), the others see what is left."""
+    b, h, hk, sq, sk = shape
+    q, k, v = make(23, b, h, hk, sq, sk, 64, 64, "bf16")
+    mask = np.zeros((1, 1, sq, sk), np.float32)
+    mask[..., : sk // 2] = lowest
+    mask[:, :, 1, :] = lowest
+    stored = {"f32": mask, "bf16": (mask.view(np.uint32) >> 16).astype(np.uint16), "f16": mask.astype(np.float16).view(np.uint16)}[mdt]
+    sc = np.array([0.125], np.float32)
+    got, _ = run(q, k, v, "bf16", "bf16", True, scale=sc, mask=stored, mdt=mdt, mask_type=1)
+    want, pabs = ideal(q, k, v, "bf16", scale=0.125, mask=mask.astype(np.float64))
+    if mdt != "f16":
+        want[:, :, 1, :] = values("bf16", v).astype(np.float64).mean(axis=2)
+        pabs[:, :, 1, :] = np.abs(values("bf16", v)).astype(np.float64).mean(axis=2)
+    else:   # a score beside 65504 is rounded to 2^-8, so a weight and their sum move by 2^-9 each: twice bf16's 2^-8
+        pabs = 2 * pabs
+    assert (np.abs(values("bf16", got) - want) <= tolerance("bf16", "bf16", sk, pabs, want)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 2, 2, 129, 65), (1, 2, 2, 3, 33)])
+def test_an_infinite_last_value_stays_infinite(gpu, shape):
+    """The tile's rows beyond the last key must not turn it into NaN."""
+    b, h, hk, sq, sk = shape
+    q, k, v = make(24, b, h, hk, sq, sk, 64, 64, "bf16")
+    v[:, :, sk - 1, 5] = 0x7f80
+    got = values("bf16", run(q, k, v, "bf16", "bf16", True)[0])
+    assert np.isposinf(got[..., 5]).all()
+    assert np.isfinite(np.delete(got, 5, axis=3)).all()
