@@ -488,6 +488,40 @@ __global__ void __launch_bounds__(256) reorder_direct_kernel(const reorder_t R_)
     }
 }
 
+// Four values to four bytes of an 8-bit dst, convert()'s arithmetic: x = src_scale * x; x = x / dst_scale + dst_zp;
+// saturate, round to nearest even.  `fast`: integer dst and every |s1| within 2^-20 .. 2^20, the division is then
+// div_by_fma where the values are in its range (the IEEE quotient bit for bit where the rounding to an integer can
+// see it).
+template <int DDT>
+__device__ __forceinline__ uint32_t quantize4(float (&x)[4], const float (&s0)[4], const float (&s1)[4],
+        const float (&y1)[4], bool with_s0, bool with_div, bool fast, float dzp) {
+    unsigned mag = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (with_s0) x[e] = s0[e] * x[e];
+        mag = max(mag, gemm::mag_bits(x[e]));
+    }
+    if (with_div) {
+        if (fast && mag < gemm::DIV_BY_FMA_LIMIT) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = gemm::div_by_fma(x[e], s1[e], y1[e]) + dzp;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = x[e] / s1[e] + dzp;
+        }
+    }
+    uint32_t w = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t b;
+        if constexpr (DDT == MI355_DT_S8) b = (uint32_t)(int)__builtin_rintf(sat(x[e], -128.f, 127.f)) & 0xffu;
+        else if constexpr (DDT == MI355_DT_U8) b = (uint32_t)(int)__builtin_rintf(sat(x[e], 0.f, 255.f)) & 0xffu;
+        else b = cvt_store_bits(DDT, x[e]) & 0xffu;
+        w |= b << (8 * e);
+    }
+    return w;
+}
+
 // Row quantization: float src (f32 / bf16 / f16) to an 8-bit dst (s8 / u8 /
 // e4m3 / e5m2), both unit-stride along `a`, at most one outer dim (rows), no
 // sum, no src zero point, f32 scales per tensor or per column.  This is what
@@ -497,10 +531,7 @@ __global__ void __launch_bounds__(256) reorder_direct_kernel(const reorder_t R_)
 // consecutive ones -- for a block of rows: the scales and, for integer dst, the
 // reciprocals of the dst scales are fetched once per lane, the data types are
 // template parameters, four rows are in flight per lane, and every load or
-// store instruction moves whole 128-byte lines.  The arithmetic is convert()'s:
-// x = src_scale * x; x = x / dst_scale + dst_zp; saturate, round to nearest
-// even.  For integer dst the division is div_by_fma where its conditions hold
-// (the IEEE quotient bit for bit where the rounding to an integer can see it).
+// store instruction moves whole 128-byte lines.
 template <int SDT, int DDT>
 __global__ void __launch_bounds__(256) reorder_rows_kernel(const reorder_t R_, unsigned rows_per_wg) {
     const auto &R = *(const __attribute__((address_space(4))) reorder_t *)__builtin_amdgcn_kernarg_segment_ptr();
@@ -546,31 +577,9 @@ __global__ void __launch_bounds__(256) reorder_rows_kernel(const reorder_t R_, u
         for (int u = 0; u < U; ++u) {
             if (r + u >= r1) break;
             float x[4];
-            unsigned mag = 0;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                x[e] = raw_to_float(SDT, raw[u][e]);
-                if (with_s0) x[e] = s0[e] * x[e];
-                mag = max(mag, gemm::mag_bits(x[e]));
-            }
-            if (with_div) {
-                if (fast && mag < gemm::DIV_BY_FMA_LIMIT) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x[e] = gemm::div_by_fma(x[e], s1[e], y1[e]) + dzp;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x[e] = x[e] / s1[e] + dzp;
-                }
-            }
-            uint32_t w = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                uint32_t b;
-                if constexpr (DDT == MI355_DT_S8) b = (uint32_t)(int)__builtin_rintf(sat(x[e], -128.f, 127.f)) & 0xffu;
-                else if constexpr (DDT == MI355_DT_U8) b = (uint32_t)(int)__builtin_rintf(sat(x[e], 0.f, 255.f)) & 0xffu;
-                else b = cvt_store_bits(DDT, x[e]) & 0xffu;
-                w |= b << (8 * e);
-            }
+            for (int e = 0; e < 4; ++e) x[e] = raw_to_float(SDT, raw[u][e]);
+            const uint32_t w = quantize4<DDT>(x, s0, s1, y1, with_s0, with_div, fast, dzp);
             __builtin_nontemporal_store(w, (uint32_t *)(dst + (long)(r + u) * rd));
         }
     }
@@ -656,72 +665,43 @@ __global__ void __launch_bounds__(256) reorder_tiled_kernel(const reorder_t R_) 
     }
 }
 
-// Transposition of 8-bit elements without attributes (the layout change of
-// int8 / fp8 weights that format_tag::any asks for): 64 x 64 tile over (a, b),
-// b has src stride 1, a has dst stride 1, both extents multiples of 64.  A
-// thread loads a 4 x 4 block as four dwords, transposes it in registers with
-// eight byte permutes and parks the four result dwords in LDS; the tile then
-// leaves as 16-byte stores along a.
-__global__ void __launch_bounds__(256) transpose8_kernel(const reorder_t R_) {
-    const auto &R = *(const __attribute__((address_space(4))) reorder_t *)__builtin_amdgcn_kernarg_segment_ptr();
-    constexpr int PITCH = 17; // dwords per LDS row (16 + 1: spreads the banks)
-    __shared__ uint32_t tile[64 * PITCH];
-    const unsigned ntiles = R.tiles_a * R.tiles_b;
-    const int bi = threadIdx.x & 15, ai = threadIdx.x >> 4; // read: block (4 ai .. +3, 4 bi .. +3)
-    const int wb = threadIdx.x >> 2, wq = threadIdx.x & 3;  // write: row b, 16 bytes of a
-    const uint8_t *src = (const uint8_t *)R.src;
-    uint8_t *dst = (uint8_t *)R.dst;
-    for (unsigned o = blockIdx.y; o < R.outer_total; o += gridDim.y) {
-        long so = 0, dof = 0;
-        {
-            unsigned oo = o;
-            for (int i = 0; i < R.n_outer; ++i) {
-                const unsigned n = R.outer[i].n;
-                const unsigned q = oo / n, r = oo - q * n;
-                oo = q;
-                so += (long)r * R.outer[i].ss;
-                dof += (long)r * R.outer[i].ds;
-            }
-        }
-        for (unsigned t = blockIdx.x; t < ntiles; t += gridDim.x) {
-            const unsigned tb = t % R.tiles_b, ta = t / R.tiles_b;
-            const long a0 = (long)ta * 64, b0 = (long)tb * 64;
-            const uint8_t *p = src + so + (a0 + 4 * ai) * R.a.ss + b0 + 4 * bi;
-            const uint32_t r0 = *(const uint32_t *)p, r1 = *(const uint32_t *)(p + R.a.ss),
-                           r2 = *(const uint32_t *)(p + 2 * R.a.ss), r3 = *(const uint32_t *)(p + 3 * R.a.ss);
-            // byte k of r_i is element (a + i, b + k); T_k collects byte k of the four rows
-            const uint32_t x0 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), x1 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
-            const uint32_t y0 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), y1 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
-            tile[(4 * bi + 0) * PITCH + ai] = __builtin_amdgcn_perm(y0, x0, 0x05040100u);
-            tile[(4 * bi + 1) * PITCH + ai] = __builtin_amdgcn_perm(y0, x0, 0x07060302u);
-            tile[(4 * bi + 2) * PITCH + ai] = __builtin_amdgcn_perm(y1, x1, 0x05040100u);
-            tile[(4 * bi + 3) * PITCH + ai] = __builtin_amdgcn_perm(y1, x1, 0x07060302u);
-            __syncthreads();
-            uint4 v;
-            v.x = tile[wb * PITCH + 4 * wq]; v.y = tile[wb * PITCH + 4 * wq + 1];
-            v.z = tile[wb * PITCH + 4 * wq + 2]; v.w = tile[wb * PITCH + 4 * wq + 3];
-            *(uint4 *)(dst + dof + (b0 + wb) * R.b.ds + a0 + 16 * wq) = v;
-            __syncthreads();
-        }
-    }
-}
+// Transposition into 8-bit elements: 128 (a) x TB (b) tiles, b has src stride 1, a has dst stride 1.  SDT is a float
+// type (quantization into a transposed layout: f32 scales per tensor or along b, a dst zero point) or BITS8 (8-bit
+// elements moved unconverted: the layout change of int8 / fp8 weights that format_tag::any asks for).  Bound by HBM:
+// a load instruction fetches whole 128-byte lines of src rows (16 bytes a lane), a store instruction whole lines of
+// dst rows, so with aligned rows no line is touched by two workgroups (64-byte tile rows fetched every src line
+// twice, by workgroups on different L2s).  A thread takes four rows x 16 bytes at a time, which makes one dword of
+// four consecutive `a` per column -- packed by the conversion itself, or by eight v_perm_b32 per 4 x 4 bytes -- and
+// parks it in LDS; dword column c of tile row b sits at (c + SHIFT * (b / EL)) % 32, which spreads a store
+// instruction over all banks and keeps the 16-byte reads aligned.  Extents along `a` and dst pitches may be anything
+// (rows past the end are loaded from the last one, a ragged chunk leaves byte by byte, an unaligned one as an
+// unaligned 16-byte store); rows of src are 16-byte aligned and an extent of b is a multiple of EL.
+// Measured, against the 64 x 64 tiled kernel that took these before: f32 -> s8 8192 x 8192 with a scale per column 147 ->
+// 69 us (4.9 TB/s), bf16 -> s8 1622 x 10752 56 -> 17 us, s8 1621 x 10752 (odd pitch) 41 -> 13 us; s8 8192 x 8192 in
+// 29 us, as the aligned-only kernel it replaces.
+constexpr int BITS8 = -1;
 
-// The same transposition on 128 x 128 tiles, for extents that are multiples of
-// 128 and 16-byte aligned rows: every load instruction fetches the whole
-// 128-byte lines of eight src rows and every store instruction writes the
-// whole lines of eight dst rows, so no line is touched by two workgroups
-// (with 64-byte tile rows every src line was fetched twice, by workgroups on
-// different L2s).  A thread loads 4 rows x 16 bytes, transposes the four
-// 4 x 4 blocks in registers and parks 16 dwords in LDS; dword column c of
-// tile row b sits at (c + 8 (b / 16)) % 32, which spreads a store instruction
-// over all banks and keeps the 16-byte reads aligned.
-__global__ void __launch_bounds__(256) transpose8w_kernel(const reorder_t R_) {
+template <int SDT>
+struct t8_shape {
+    static constexpr int EL = SDT == BITS8 ? 16 : SDT == MI355_DT_F32 ? 4 : 8; // elements in 16 bytes of src
+    static constexpr int LN = SDT == MI355_DT_F32 ? 16 : 8;                    // lanes along b
+    static constexpr int TB = EL * LN;
+};
+
+template <int SDT, int DDT>
+__global__ void __launch_bounds__(256) reorder_transpose8_kernel(const reorder_t R_) {
     const auto &R = *(const __attribute__((address_space(4))) reorder_t *)__builtin_amdgcn_kernarg_segment_ptr();
-    __shared__ __attribute__((aligned(16))) uint32_t tile[128 * 32];
-    const unsigned tiles_b = R.b.n / 128, ntiles = (R.a.n / 128) * tiles_b;
-    const int bi = threadIdx.x & 7, ag = threadIdx.x >> 3; // read: rows 4 ag .. +3, bytes 16 bi .. +15
-    const int wq = threadIdx.x & 7, wr = threadIdx.x >> 3; // write: row wr + 32 pass, bytes 16 wq .. +15
-    const uint8_t *src = (const uint8_t *)R.src;
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    typedef uint32_t u4un __attribute__((ext_vector_type(4), aligned(1)));
+    constexpr int EL = t8_shape<SDT>::EL, LN = t8_shape<SDT>::LN, TB = t8_shape<SDT>::TB;
+    constexpr int PASSES = 128 / (256 / LN * 4), SHIFT = 256 / LN / 4;
+    constexpr int SBYTES = 16 / EL;
+    constexpr bool INT_DST = DDT == MI355_DT_S8 || DDT == MI355_DT_U8;
+    __shared__ __attribute__((aligned(16))) uint32_t tile[TB * 32];
+    const unsigned tiles_b = (R.b.n + TB - 1) / TB, ntiles = ((R.a.n + 127) / 128) * tiles_b;
+    const unsigned bi = threadIdx.x % LN, ag0 = threadIdx.x / LN; // read: rows 4 (ag0 + 256 / LN * pass) .. +3
+    const unsigned wq = threadIdx.x & 7, wr = threadIdx.x >> 3;   // write: row wr + 32 pass, bytes 16 wq .. +15
+    const char *src = (const char *)R.src;
     uint8_t *dst = (uint8_t *)R.dst;
     for (unsigned o = blockIdx.y; o < R.outer_total; o += gridDim.y) {
         long so = 0, dof = 0;
@@ -737,34 +717,79 @@ __global__ void __launch_bounds__(256) transpose8w_kernel(const reorder_t R_) {
         }
         for (unsigned t = blockIdx.x; t < ntiles; t += gridDim.x) {
             const unsigned tb = t % tiles_b, ta = t / tiles_b;
-            const long a0 = (long)ta * 128, b0 = (long)tb * 128;
-            const uint8_t *p = src + so + (a0 + 4 * ag) * R.a.ss + b0 + 16 * bi;
-            typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-            u4v r[4];
+            const unsigned a0 = ta * 128, b0 = tb * TB, b_lane = b0 + EL * bi;
+            if (b_lane < R.b.n) {
+                u4v v[PASSES][4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) r[i] = __builtin_nontemporal_load((const u4v *)(p + i * R.a.ss));
-            const int col = (ag + 8 * (bi & 3)) & 31;
+                for (int p = 0; p < PASSES; ++p)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint32_t r0 = k == 0 ? r[0].x : k == 1 ? r[0].y : k == 2 ? r[0].z : r[0].w;
-                const uint32_t r1 = k == 0 ? r[1].x : k == 1 ? r[1].y : k == 2 ? r[1].z : r[1].w;
-                const uint32_t r2 = k == 0 ? r[2].x : k == 1 ? r[2].y : k == 2 ? r[2].z : r[2].w;
-                const uint32_t r3 = k == 0 ? r[3].x : k == 1 ? r[3].y : k == 2 ? r[3].z : r[3].w;
-                // byte j of r_i is element (a + i, b + 4 k + j); T_j collects byte j of the four rows
-                const uint32_t x0 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), x1 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
-                const uint32_t y0 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), y1 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
-                const int row = 16 * bi + 4 * k;
-                tile[(row + 0) * 32 + col] = __builtin_amdgcn_perm(y0, x0, 0x05040100u);
-                tile[(row + 1) * 32 + col] = __builtin_amdgcn_perm(y0, x0, 0x07060302u);
-                tile[(row + 2) * 32 + col] = __builtin_amdgcn_perm(y1, x1, 0x05040100u);
-                tile[(row + 3) * 32 + col] = __builtin_amdgcn_perm(y1, x1, 0x07060302u);
+                    for (int i = 0; i < 4; ++i) {
+                        const unsigned a = min(a0 + 4 * (ag0 + 256 / LN * p) + i, R.a.n - 1);
+                        v[p][i] = __builtin_nontemporal_load((const u4v *)(src + (so + (long)a * R.a.ss + b_lane) * SBYTES));
+                    }
+                float s0[EL], s1[EL], y1[EL];
+                bool fast = INT_DST;
+                if constexpr (SDT != BITS8) {
+#pragma unroll
+                    for (int e = 0; e < EL; ++e) {
+                        s0[e] = R.qp[0] ? ((const float *)R.qp[0])[R.b.qs[0] ? b_lane + e : 0] : 1.f;
+                        s1[e] = R.qp[1] ? ((const float *)R.qp[1])[R.b.qs[1] ? b_lane + e : 0] : 1.f;
+                        y1[e] = 1.f / s1[e];
+                        const float m = __builtin_fabsf(s1[e]);
+                        fast = fast && m >= 0x1p-20f && m <= 0x1p20f;
+                    }
+                }
+                const bool with_s0 = R.qp[0] != nullptr, with_div = R.qp[1] != nullptr || R.dst_zp != nullptr;
+                const float dzp = R.dst_zp ? (float)*(const int *)R.dst_zp : 0.f;
+#pragma unroll
+                for (int p = 0; p < PASSES; ++p) {
+                    const unsigned col = (ag0 + 256 / LN * p + SHIFT * bi) & 31;
+                    if constexpr (SDT == BITS8) {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const uint32_t r0 = v[p][0][k], r1 = v[p][1][k], r2 = v[p][2][k], r3 = v[p][3][k];
+                            // byte j of r_i is element (a + i, b + 4 k + j); T_j collects byte j of the four rows
+                            const uint32_t x0 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), x1 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
+                            const uint32_t z0 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), z1 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
+                            const unsigned row = EL * bi + 4 * k;
+                            tile[(row + 0) * 32 + col] = __builtin_amdgcn_perm(z0, x0, 0x05040100u);
+                            tile[(row + 1) * 32 + col] = __builtin_amdgcn_perm(z0, x0, 0x07060302u);
+                            tile[(row + 2) * 32 + col] = __builtin_amdgcn_perm(z1, x1, 0x05040100u);
+                            tile[(row + 3) * 32 + col] = __builtin_amdgcn_perm(z1, x1, 0x07060302u);
+                        }
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < EL; ++e) {
+                            float x[4], c0[4], c1[4], cy[4];
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const uint32_t raw = EL == 4 ? v[p][i][e] : (v[p][i][e / 2] >> (16 * (e & 1))) & 0xffffu;
+                                x[i] = raw_to_float(SDT, raw);
+                                c0[i] = s0[e]; c1[i] = s1[e]; cy[i] = y1[e];
+                            }
+                            tile[(EL * bi + e) * 32 + col] = quantize4<DDT>(x, c0, c1, cy, with_s0, with_div, fast, dzp);
+                        }
+                    }
+                }
             }
             __syncthreads();
 #pragma unroll
-            for (int pass = 0; pass < 4; ++pass) {
-                const int b = wr + 32 * pass;
-                const u4v v = *(const u4v *)&tile[b * 32 + ((4 * wq + 8 * ((b >> 4) & 3)) & 31)];
-                __builtin_nontemporal_store(v, (u4v *)(dst + dof + (b0 + b) * R.b.ds + a0 + 16 * wq));
+            for (int p = 0; p < TB / 32; ++p) {
+                const unsigned row = wr + 32 * p, b = b0 + row, a = a0 + 16 * wq;
+                if (b < R.b.n && a < R.a.n) {
+                    const u4v w = *(const u4v *)&tile[row * 32 + ((4 * wq + SHIFT * (row / EL)) & 31)];
+                    uint8_t *q = dst + dof + (long)b * R.b.ds + a;
+                    if (a + 16 > R.a.n) {
+                        const unsigned left = R.a.n - a;
+#pragma unroll
+                        for (unsigned e = 0; e < 15; ++e)
+                            if (e < left) q[e] = (uint8_t)(w[e / 4] >> (8 * (e & 3)));
+                    } else if (R.packed) {
+                        __builtin_nontemporal_store(w, (u4v *)q);
+                    } else {
+                        *(u4un *)q = w;
+                    }
+                }
             }
             __syncthreads();
         }
@@ -1062,7 +1087,7 @@ extern "C" int mi355_reorder_launch(const mi355_reorder_desc_t *desc, const mi35
     if (outer >= (1L << 31)) return MI355_UNIMPLEMENTED;
     R.outer_total = (unsigned)outer;
 
-    // MI355_REORDER_GENERIC=1 keeps the dedicated kernels (row quantization, whole-line transposition) out: for
+    // MI355_REORDER_GENERIC=1 keeps the dedicated kernels (row quantization, transposition into 8 bits) out: for
     // measurements and tests of the kernels behind them
     static const bool generic_only = getenv("MI355_REORDER_GENERIC") != nullptr;
     const int dbits = dt_bits(d.dst_dt), sbits = dt_bits(d.src_dt);
@@ -1103,11 +1128,6 @@ extern "C" int mi355_reorder_launch(const mi355_reorder_desc_t *desc, const mi35
         R.elems = 4;
         long gx = (long)R.tiles_a * R.tiles_b;
         if (gx > (1 << 20)) gx = 1 << 20;
-        // 8-bit transposition without attributes: whole tiles, dword loads along b, 16-byte stores along a
-        bool t8 = R.plain_copy && dbits == 8 && R.a.n % 64 == 0 && R.b.n % 64 == 0 && R.a.ss % 4 == 0
-                && R.b.ds % 16 == 0 && (uintptr_t)R.src % 4 == 0 && (uintptr_t)R.dst % 16 == 0;
-        for (int i = 0; i < R.n_outer && t8; ++i)
-            if (R.outer[i].ss % 4 || R.outer[i].ds % 16) t8 = false;
         const bool simple = d.beta == 0.f && d.src_scale.dt == MI355_DT_UNDEF && d.dst_scale.dt == MI355_DT_UNDEF
                 && d.src_zp.dt == MI355_DT_UNDEF && d.dst_zp.dt == MI355_DT_UNDEF;
         // a lane converts four consecutive a at one b: every parameter tensor constant
@@ -1120,17 +1140,42 @@ extern "C" int mi355_reorder_launch(const mi355_reorder_desc_t *desc, const mi35
             for (int i = 0; i < R.n_outer && qvec; ++i)
                 if (R.outer[i].qs[k] % 4) qvec = false;
         }
-        // ... and whole 128-byte lines on both sides where the extents and the row pitches allow
-        bool t8w = t8 && R.a.n % 128 == 0 && R.b.n % 128 == 0 && R.a.ss % 16 == 0 && (uintptr_t)R.src % 16 == 0
-                && !generic_only;
-        for (int i = 0; i < R.n_outer && t8w; ++i)
-            if (R.outer[i].ss % 16) t8w = false;
+        // transposition into 8-bit elements, from 8-bit ones without attributes or from floats with f32 scales per
+        // tensor or along b: the dedicated kernel wherever src can be read in aligned 16-byte pieces.  The tiled
+        // kernel reads element by element, a dispatch and a set of offsets per four
+        const bool dst8 = d.dst_dt == MI355_DT_S8 || d.dst_dt == MI355_DT_U8 || d.dst_dt == MI355_DT_F8_E4M3
+                || d.dst_dt == MI355_DT_F8_E5M2;
+        const bool src_f = d.src_dt == MI355_DT_F32 || d.src_dt == MI355_DT_BF16 || d.src_dt == MI355_DT_F16;
+        const long el = 128 / sbits;
+        bool t8 = ((R.plain_copy && dbits == 8) || (src_f && dst8 && d.beta == 0.f && !R.qp[2])) && R.b.n % el == 0
+                && R.a.ss % el == 0 && (uintptr_t)R.src % 16 == 0 && !generic_only;
+        for (int i = 0; i < R.n_outer && t8; ++i) t8 = R.outer[i].ss % el == 0;
+        for (int k = 0; k < 2 && t8; ++k) {
+            if (!R.qp[k]) continue;
+            t8 = R.qdt[k] == MI355_DT_F32 && R.a.qs[k] == 0 && (R.b.qs[k] == 0 || (R.b.qs[k] == 1 && R.b.qg[k] == 1));
+            for (int i = 0; i < R.n_outer && t8; ++i) t8 = R.outer[i].qs[k] == 0;
+        }
         const dim3 grid((unsigned)gx, gy), block(256);
-        if (t8w) {
-            long gw = (long)(R.a.n / 128) * (R.b.n / 128);
+        if (t8) {
+            R.packed = (uintptr_t)R.dst % 16 == 0 && R.b.ds % 16 == 0;
+            for (int i = 0; i < R.n_outer; ++i) R.packed = R.packed && R.outer[i].ds % 16 == 0;
+            const unsigned tb = sbits == 8 ? t8_shape<BITS8>::TB : t8_shape<MI355_DT_BF16>::TB;
+            static_assert(t8_shape<MI355_DT_F32>::TB == t8_shape<MI355_DT_BF16>::TB, "one tile width for the float types");
+            long gw = (long)((R.a.n + 127) / 128) * ((R.b.n + tb - 1) / tb);
             if (gw > (1 << 20)) gw = 1 << 20;
-            hipLaunchKernelGGL(transpose8w_kernel, dim3((unsigned)gw, gy), block, 0, hs, R);
-        } else if (t8) hipLaunchKernelGGL(transpose8_kernel, grid, block, 0, hs, R);
+            const dim3 tgrid((unsigned)gw, gy);
+            if (R.plain_copy) hipLaunchKernelGGL((reorder_transpose8_kernel<BITS8, MI355_DT_U8>), tgrid, block, 0, hs, R);
+#define MI355_T8_CASE(S_, D_) \
+    else if (d.src_dt == S_ && d.dst_dt == D_) hipLaunchKernelGGL((reorder_transpose8_kernel<S_, D_>), tgrid, block, 0, hs, R);
+#define MI355_T8_SRC(S_) \
+    MI355_T8_CASE(S_, MI355_DT_S8) MI355_T8_CASE(S_, MI355_DT_U8) MI355_T8_CASE(S_, MI355_DT_F8_E4M3) \
+    MI355_T8_CASE(S_, MI355_DT_F8_E5M2)
+            MI355_T8_SRC(MI355_DT_F32)
+            MI355_T8_SRC(MI355_DT_BF16)
+            MI355_T8_SRC(MI355_DT_F16)
+#undef MI355_T8_SRC
+#undef MI355_T8_CASE
+        }
         else if (R.a.n % 4 == 0 && simple) hipLaunchKernelGGL(reorder_tiled_kernel<MODE_SIMPLE>, grid, block, 0, hs, R);
         else if (R.a.n % 4 == 0 && qvec) hipLaunchKernelGGL(reorder_tiled_kernel<MODE_QVEC>, grid, block, 0, hs, R);
         else hipLaunchKernelGGL(reorder_tiled_kernel<MODE_GENERIC>, grid, block, 0, hs, R);

@@ -323,6 +323,42 @@ ROW_CASES = [
 ]
 
 
+# Transposition into 8-bit elements (16-byte pieces of src rows, 128 dst-contiguous elements a tile): tiles that end
+# inside on either side, dst rows at odd addresses, a last chunk of 1 .. 15 bytes, batches, every type pair, and extents
+# that have to stay with the tiled kernel (no whole 16-byte pieces)
+TRANSPOSE8_CASES = [
+    lambda: _case("s8 odd dst pitch, last chunk of 13", (269, 272), cabi.DT_S8, cabi.DT_S8, 110, dst_perm=(1, 0)),
+    lambda: _case("s8 last chunk of 1, one column piece", (129, 16), cabi.DT_S8, cabi.DT_S8, 111, dst_perm=(1, 0)),
+    lambda: _case("e4m3 smallest", (16, 16), cabi.DT_F8_E4M3, cabi.DT_F8_E4M3, 112, dst_perm=(1, 0)),
+    lambda: _case("u8 batched, odd extent", (3, 31, 144), cabi.DT_U8, cabi.DT_U8, 113, dst_perm=(0, 2, 1)),
+    lambda: _case("s8 src rows of 24 bytes (tiled)", (40, 24), cabi.DT_S8, cabi.DT_S8, 114, dst_perm=(1, 0)),
+    lambda: _case("f32->s8 per column, dst zp, two tiles each way", (150, 68), cabi.DT_F32, cabi.DT_S8, 115, dst_perm=(1, 0),
+                  quant={"src_scale": _qp(116, cabi.DT_F32, 0, (1,)), "dst_scale": _qp(117, cabi.DT_F32, 2, (68,)),
+                         "dst_zp": _qp(118, cabi.DT_S32, 0, (1,))}),
+    lambda: _case("bf16->s8 per column, odd rows", (257, 136), cabi.DT_BF16, cabi.DT_S8, 119, dst_perm=(1, 0),
+                  quant={"dst_scale": _qp(120, cabi.DT_F32, 2, (136,))}),
+    lambda: _case("f16->u8 per-column src scale", (128, 64), cabi.DT_F16, cabi.DT_U8, 121, dst_perm=(1, 0),
+                  quant={"src_scale": _qp(122, cabi.DT_F32, 2, (64,))}),
+    lambda: _case("f32->e5m2 common scale, batched", (2, 143, 20), cabi.DT_F32, cabi.DT_F8_E5M2, 123, dst_perm=(0, 2, 1),
+                  quant={"dst_scale": _qp(124, cabi.DT_F32, 0, (1,))}),
+    lambda: _case("bf16->e4m3 attribute-free", (19, 520), cabi.DT_BF16, cabi.DT_F8_E4M3, 125, dst_perm=(1, 0)),
+    lambda: _case("f32->s8 scale per dst-contiguous dim (tiled)", (132, 64), cabi.DT_F32, cabi.DT_S8, 126, dst_perm=(1, 0),
+                  quant={"dst_scale": _qp(127, cabi.DT_F32, 1, (132,))}),
+    lambda: _case("bf16->s8 scale per batch (tiled)", (2, 32, 64), cabi.DT_BF16, cabi.DT_S8, 128, dst_perm=(0, 2, 1),
+                  quant={"dst_scale": _qp(129, cabi.DT_F32, 1, (2,))}),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("make", TRANSPOSE8_CASES, ids=[f"t8_{i}" for i in range(len(TRANSPOSE8_CASES))])
+def test_gpu_transposition_to_8_bit_is_bit_exact(make):
+    p = make()
+    assert query(p) == cabi.SUCCESS, p.name
+    got, want = run_gpu(p), oracle.reorder(p)
+    bad = np.flatnonzero(got != want)
+    assert bad.size == 0, f"{p.name}: {bad.size} of {got.size} storage elements differ, first at {bad[:5]}"
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("make", ROW_CASES, ids=[f"rows{i}" for i in range(len(ROW_CASES))])
 def test_gpu_row_quantization_is_bit_exact(make):
