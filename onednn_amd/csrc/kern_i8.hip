@@ -491,15 +491,16 @@ i8_plan_t make_plan(const mi355_matmul_desc_t &d) {
     p.Bw = d.wei_stride[0] ? d.batch : 1;
     p.Bs = d.src_stride[0] ? d.batch : 1;
     p.need_transpose = !(d.wei_stride[1] == 1);
-    // the small tiles when the LDS tiles would occupy too little of the device
-    // (measured with K = 1024 / 4096 against the 256 x 128 tiles, which take 16.7 /
-    // 35 us for anything up to 128 large tiles: the small tiles take 14.5 / 30.3 us
-    // at 12 large tiles, 17.2 / 37.5 at 16, 22.4 / 53.5 at 20), or when the LDS
-    // tiles cannot step through K (the small tiles compute their own sums and have
-    // no dynamic dst quantization)
-    const long big_tiles = ((d.M + BM - 1) / BM) * ((d.N + i8_geo_t::BN - 1) / i8_geo_t::BN) * d.batch;
-    const long crossover = 16;
-    p.small = !d.dst_scale_dynamic && (big_tiles < crossover || d.K % BK != 0);
+    // the small tiles when the LDS tiles would occupy too little of the device, or
+    // when the LDS tiles cannot step through K (the small tiles compute their own
+    // sums and have no dynamic dst quantization).  Up to 128 large tiles the LDS
+    // tiles' time depends on K alone; the small tiles' grows with their number:
+    // K = 1024 / 4096, 16.7 / 35 us on the LDS tiles against 14.5 / 30.3 us on 768
+    // small ones, 17.2 / 37.5 on 1024, 22.4 / 53.5 on 1280.  Counted in small tiles
+    // and not in large ones, because a short M fills few rows of a large tile.
+    const long small_tiles = ((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch;
+    const long crossover = 1024;
+    p.small = !d.dst_scale_dynamic && (small_tiles < crossover || d.K % BK != 0);
     // the MI355_I8_TILES switch overrides the choice where both can run (tests and
     // tuning): large = the LDS tiles, 256 x 128 or 256 x 256 by the number of
     // tiles; wide = the 256 x 256 ones

@@ -131,3 +131,13 @@ def test_mid_size_problems_on_the_dispatchers_own_choice(gpu, oracle, src_dt):
     with cabi.tuning("MI355_I8_TILES", "wide"):
         wide, name = run_gpu(p, cabi.IMPL_I8_MFMA)
     assert np.array_equal(np.asarray(got), np.asarray(wide))
+
+
+@pytest.mark.parametrize("M,N", [(1, 8160), (32, 32736), (32, 32768), (100, 8160), (200, 4096)])
+def test_a_short_m_stays_on_the_small_tiles(gpu, oracle, M, N):
+    """Up to 1023 small tiles need no scratch (they make their own sums); 1024 are the large tiles' again."""
+    p = int8_problem(M, N, 64, cabi.DT_U8, cabi.DT_S8, cabi.DT_S8, src_zp=7, dst_scale=0.5)
+    tiles = -(-M // 32) * -(-N // 32)
+    assert (cabi.scratch_bytes(p.desc()) == 0) == (tiles < 1024)
+    got, name = run_gpu(p)
+    assert_bit_exact(p, got, oracle.run_oracle(p), name)
