@@ -317,6 +317,10 @@ int mi355_graph_capture_begin(void *stream);
 int mi355_graph_capture_end(void *stream, void **graph);
 int mi355_graph_launch(void *graph, void *stream);
 int mi355_graph_destroy(void *graph);
+/* Swaps the calling thread's rule for calls that a capture in progress forbids
+ * (hipMalloc among them) with *mode: 2 allows them.  For setup that an
+ * execution does on its first call; swap back afterwards. */
+int mi355_capture_mode_exchange(int *mode);
 /* writes the low `nbytes` (1, 2, 4 or 8) of `bits` to device memory in stream
  * order, without a host copy: the value travels as a kernel argument, so the
  * call never waits for the stream (a host-side scalar of the attributes) */

@@ -150,6 +150,7 @@ KERNEL_SYMBOLS = [
     "mi355_event_destroy", "mi355_event_record", "mi355_event_sync", "mi355_event_elapsed_ms",
     "mi355_stream_wait_event", "mi355_mem_store_scalar",
     "mi355_graph_capture_begin", "mi355_graph_capture_end", "mi355_graph_launch", "mi355_graph_destroy",
+    "mi355_capture_mode_exchange",
     "mi355_last_error", "mi355_matmul_query", "mi355_matmul_impl_name",
     "mi355_matmul_scratch_bytes", "mi355_matmul_launch", "mi355_matmul_launch_noalloc", "mi355_reorder_query",
     "mi355_reorder_launch", "mi355_wei_pack_reorder_dims", "mi355_tuning_set", "mi355_colsum_launch", "mi355_sdpa_softmax_launch",

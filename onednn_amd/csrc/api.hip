@@ -454,6 +454,14 @@ int mi355_graph_destroy(void *graph) {
     if (!graph) return MI355_SUCCESS;
     return hip_status(hipGraphExecDestroy((hipGraphExec_t)graph), "hipGraphExecDestroy");
 }
+int mi355_capture_mode_exchange(int *mode) {
+    static_assert((int)hipStreamCaptureModeRelaxed == 2, "the value that mi355_matmul.h states");
+    if (!mode || *mode < 0 || *mode > 2) return MI355_INVALID_ARGUMENTS;
+    hipStreamCaptureMode m = (hipStreamCaptureMode)*mode;
+    const int st = hip_status(hipThreadExchangeStreamCaptureMode(&m), "hipThreadExchangeStreamCaptureMode");
+    *mode = (int)m;
+    return st;
+}
 int mi355_stream_sync(void *stream) {
     return hip_status(hipStreamSynchronize((hipStream_t)stream), "hipStreamSynchronize");
 }

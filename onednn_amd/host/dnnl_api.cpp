@@ -2700,7 +2700,10 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
         }
         order_on_device(); // the scores and probabilities belong to the primitive
         if (S.fused) {
+            int mode = 2; // the stream may be under capture, which forbids the allocation otherwise
+            if (mi355_capture_mode_exchange(&mode) != MI355_SUCCESS) return dnnl_runtime_error;
             const dnnl_status_t cs = sdpa_compose(*prim);
+            mi355_capture_mode_exchange(&mode);
             if (cs != dnnl_success) return cs;
         }
         CHECK_ARG(prim->composed);
