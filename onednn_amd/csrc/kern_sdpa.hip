@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
     // times log2(e) would be -inf, and a row of nothing else has to weigh its keys alike)
     constexpr float UNIT = MASK ? LOG2E : 1.f;
     c = MASK ? 1.f : c * LOG2E;
-    c = c < 1e-30f ? 1e-30f : c; // (a scale of zero must not meet the infinities of masked keys)
+    c = c == 0.f ? 0x1p-149f : c; // (zero must not meet the infinities of masked keys; finite scores times this are 0 to exp2)
 
     i4v qf[QT];
     {

@@ -19,7 +19,7 @@ SHAPES = [  # b, h, hk, sq, sk
 
 def check(dt, d, shape, **kw):
     b, h, hk, sq, sk = shape
-    q, k, v = make(21, b, h, hk, sq, sk, d, d, dt)
+    q, k, v = make(21, b, h, hk, sq, sk, d, d, dt, mag=kw.pop("mag", 1.0))
     sc = np.array([kw.pop("sc", 1.0 / np.sqrt(d))], np.float32)
     mask = kw.pop("mask", None)
     got, impl = run(q, k, v, dt, dt, True, scale=sc, mask=mask, mask_type=kw.get("mask_type", 0))
@@ -45,6 +45,16 @@ def test_masks_and_a_negative_scale(gpu, shape, mask_type):
     b, h, hk, sq, sk = shape
     mask = (np.random.default_rng(5).standard_normal((1, 1, sq, sk)) * 2).astype(np.float32) if mask_type == 1 else None
     check("bf16", 64, shape, mask=mask, mask_type=mask_type, sc=-0.11)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 2, 2, 3, 33), (1, 2, 2, 90, 100), (1, 1, 1, 3, 600)])
+@pytest.mark.parametrize("sc,mag", [(0.0, 1.0), (-0.0, 1.0), (1e-35, 1e17), (-1e-38, 2e18)])
+@pytest.mark.parametrize("mask_type", [0, 3])
+def test_scales_at_and_near_zero(gpu, shape, sc, mag, mask_type):
+    """Small scales of large scores are used as they are (a subnormal one too); with a scale of zero every key that is
+    seen weighs the same and masked ones weigh nothing."""
+    check("bf16", 64, shape, sc=sc, mag=mag, mask_type=mask_type)
 
 
 @pytest.mark.gpu
