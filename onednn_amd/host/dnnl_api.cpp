@@ -2690,8 +2690,18 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
                 prim->last_stream = stream->hip_stream;
             }
         };
+        // The fused kernel takes aligned buffers, and a dst of its own: it stores rows while others are still reading.
+        // (The composition has read q, k, the mask and the scale before it stores; q itself is safe as dst where every
+        // element stays in its place, since a wavefront holds its queries before it stores their rows.)
         const uintptr_t low = (uintptr_t)q->handle | (uintptr_t)k->handle | (uintptr_t)v->handle | (uintptr_t)d->handle;
-        if (S.fused && low % 16 == 0) {
+        auto meets_dst = [&](dnnl_memory_t x, const dnnl_memory_desc &md) {
+            if (!x || md.is_zero()) return false;
+            const uintptr_t x0 = (uintptr_t)x->handle, d0 = (uintptr_t)d->handle;
+            return x0 < d0 + S.dst.size_bytes() && d0 < x0 + md.size_bytes();
+        };
+        const bool in_place = q->handle == d->handle && S.q.dt == S.dst.dt && std::equal(S.q.strides, S.q.strides + 4, S.dst.strides);
+        if (S.fused && low % 16 == 0 && (in_place || !meets_dst(q, S.q)) && !meets_dst(k, S.k) && !meets_dst(v, S.v)
+                && !meets_dst(mask, S.mask) && !meets_dst(scale, S.scale)) {
             if (prim->scratch) order_on_device(); // the parts of a split launch belong to the primitive
             const int rc = mi355_sdpa_launch(&S.fused_desc, q->handle, k->handle, v->handle, d->handle,
                     scale ? scale->handle : nullptr, mask ? mask->handle : nullptr, prim->scratch, stream->hip_stream);

@@ -105,6 +105,43 @@ def test_unaligned_buffers_run_the_composition(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("what,shape", [("k", (1, 64, 64, 2048, 2048)), ("q", (1, 2, 2, 200, 200)), ("q", (1, 4, 1, 9, 1100)),
+                                        ("mask", (1, 1, 1, 300, 400))])
+def test_dst_in_the_memory_of_an_input(gpu, what, shape):
+    """The keys, the queries and a mask are read before dst is stored, wherever dst lies: what a dst of its own holds."""
+    b, h, hk, sq, sk = shape
+    d = 64
+    eng = dnnl.engine(dnnl.gpu, 0)
+    strm = dnnl.stream(eng)
+    q, k, v = make(25, b, h, hk, sq, sk, d, d, "bf16")
+    mds = [md4(q.shape, "bf16"), md4(k.shape, "bf16", transposed=True), md4(v.shape, "bf16"), md4((b, h, sq, d), "bf16")]
+    mask = (np.random.default_rng(6).standard_normal((1, 1, sq, sk)) * 2).astype(np.float32) if what == "mask" else None
+    m_md = md4(mask.shape, "f32") if what == "mask" else None
+    prim = dnnl.sdpa(dnnl.sdpa_primitive_desc(eng, *mds, mask_md=m_md, kv_head_number=hk, attn_mask_type=int(what == "mask")))
+
+    def result(shared):
+        args = {dnnl.ARG_QUERIES: dnnl.memory(mds[0], eng, storage(q)), dnnl.ARG_KEYS: dnnl.memory(mds[1], eng, storage(k)),
+                dnnl.ARG_VALUES: dnnl.memory(mds[2], eng, storage(v)), dnnl.ARG_DST: dnnl.memory(mds[3], eng)}
+        if what == "mask":
+            args[dnnl.ARG_ATTN_MASK] = dnnl.memory(m_md, eng, mask)
+        if shared:
+            dst = dnnl.memory.__new__(dnnl.memory)
+            dst.md, dst.engine, dst.h = mds[3], eng, C.c_void_p()
+            at = args[{"k": dnnl.ARG_KEYS, "q": dnnl.ARG_QUERIES, "mask": dnnl.ARG_ATTN_MASK}[what]].get_data_handle()
+            assert dnnl.lib().dnnl_memory_create(C.byref(dst.h), mds[3].h, eng.h, C.c_void_p(at)) == dnnl.success
+            args[dnnl.ARG_DST] = dst
+        prim.execute(strm, args)
+        strm.wait()
+        return values("bf16", args[dnnl.ARG_DST].read(storage_dtype(DT["bf16"])))
+
+    own, inside = result(False), result(True)
+    if what == "q":   # in place, element for element: the same kernel
+        assert np.array_equal(own, inside)
+    else:             # both paths round the probabilities and dst once, 2^-8 of a value each
+        assert np.linalg.norm(own - inside) <= 2 * 2.0 ** -8 * np.linalg.norm(own)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mdt,lowest", [("f32", np.finfo(np.float32).min), ("bf16", -3.3895313892515355e38), ("f16", -65504.0)])
 @pytest.mark.parametrize("shape", [(1, 2, 2, 150, 333), (1, 2, 2, 3, 1200)])
 def test_mask_of_the_types_lowest_value(gpu, shape, mdt, lowest):
