@@ -152,7 +152,8 @@ __global__ void __launch_bounds__(256) colsum_kernel(const void *x, int x_dt, lo
 // handful of cycles each), but in colsum_kernel every one of them also waits for its own load: 0.3 us a row.  Here a
 // workgroup owns 64 columns (a whole 128-byte line of a 16-bit row); all four wavefronts fetch chunks of 16 KB, two
 // chunks ahead in registers, and park them in LDS with the rows of a column side by side; wavefront 0 adds them, 16
-// bytes of a column's rows per LDS read.  2048 x 14336 bf16: 689 -> 21 us.
+// bytes of a column's rows per LDS read.  2048 x 14336 bf16: 689 -> 21 us.  A last chunk that is not full adds its own
+// rows only.
 template <int DT>
 __global__ void __launch_bounds__(256) colsum_chunks_kernel(const char *x, long rows, long cols, long ld, void *out,
         int out_dt) {
@@ -213,11 +214,12 @@ __global__ void __launch_bounds__(256) colsum_chunks_kernel(const char *x, long 
                 for (int i = 0; i < PER; ++i) acc += value(v, i);
             }
         } else {
-            for (int r = 0; r < CR / PER; ++r) {
+            const int n = (int)left;
+            for (int r = 0; r * PER < n; ++r) {
                 const u4v v = col[r];
 #pragma unroll
                 for (int i = 0; i < PER; ++i)
-                    if (r * PER + i < left) acc += value(v, i);
+                    if (r * PER + i < n) acc += value(v, i);
             }
         }
     };
@@ -249,10 +251,14 @@ extern "C" int mi355_colsum_launch(const void *x, int x_dt, int64_t rows, int64_
         return MI355_INVALID_ARGUMENTS;
     }
     if (cols == 0) return MI355_SUCCESS;
-    // 16-byte loads of whole column groups; a single row or an odd pitch stays with the plain kernel
+    // 16-byte loads of whole column groups; an odd pitch stays with the plain kernel, and so do few rows: that one costs
+    // 1.9 us and 0.15 a row, the chunks 3 us and more for each round of workgroups (LDS for four a CU).  bf16, plain /
+    // chunks: 8 x 512 2.9 / 3.0 us, 12 x 512 3.7 / 3.0, 24 x 50000 6.1 / 5.8 (f32 5.2 / 5.8), 32 x 50000 7.6 / 5.9,
+    // 32 x 200000 8.4 / 14.1, 64 x 200000 20.3 / 15.4
     const int eb = dt_bits(x_dt) / 8, per = 16 / eb;
-    if (rows > 1 && cols % per == 0 && ld % per == 0 && (uintptr_t)x % 16 == 0) {
-        const dim3 grid((unsigned)((cols + 63) / 64));
+    const long wgs = (cols + 63) / 64, least = wgs < 39 * 48 ? 9 + wgs / 48 : 48;
+    if (rows >= least && cols % per == 0 && ld % per == 0 && (uintptr_t)x % 16 == 0) {
+        const dim3 grid((unsigned)wgs);
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, (const char *)x, (long)rows, (long)cols,
                     (long)ld, out, out_dt);

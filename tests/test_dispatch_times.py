@@ -1,0 +1,56 @@
+"""Calls that a dispatch rule sends to one of several kernels take no longer than the kernel the rule should have found.
+Both sides run on one GPU in turn, as graphs of many launches; the least of several turns counts."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from onednn_amd import cabi
+
+pytestmark = pytest.mark.gpu
+
+
+def in_turn(*launches, n=20, turns=12):
+    """The least microseconds a launch of each; a launch takes the stream's handle."""
+    lib, s = cabi.load_kernels(), cabi.Stream()
+    ev = [C.c_void_p(), C.c_void_p()]
+    for e in ev:
+        cabi.check(lib.mi355_event_create(C.byref(e)))
+    graphs, best = [], [np.inf] * len(launches)
+    for launch in launches:
+        launch(s.ptr)
+        s.sync()
+        with cabi.Graph(s) as g:
+            for _ in range(n):
+                launch(s.ptr)
+        g.launch()
+        s.sync()
+        graphs.append(g)
+    for _ in range(turns):
+        for i, g in enumerate(graphs):
+            cabi.check(lib.mi355_event_record(ev[0], s.ptr))
+            g.launch()
+            cabi.check(lib.mi355_event_record(ev[1], s.ptr))
+            s.sync()
+            ms = C.c_float()
+            cabi.check(lib.mi355_event_elapsed_ms(C.byref(ms), ev[0], ev[1]))
+            best[i] = min(best[i], ms.value * 1e3 / n)
+    for g in graphs:
+        g.destroy()
+    for e in ev:
+        lib.mi355_event_destroy(e)
+    s.destroy()
+    return best
+
+
+@pytest.mark.parametrize("rows,cols", [(2, 512), (8, 14336), (16, 50000), (32, 200000)])
+def test_column_sums_of_few_rows(gpu, rows, cols):
+    """x off a 16-byte boundary is the plain kernel's, a load per row and column; aligned x is no slower."""
+    x, out = cabi.DeviceBuffer(4 * (rows * cols + 1)), cabi.DeviceBuffer(4 * cols)
+    lib = cabi.load_kernels()
+
+    def launch(at):
+        return lambda s: cabi.check(lib.mi355_colsum_launch(x.ptr + at, cabi.DT_F32, rows, cols, cols, out.ptr, cabi.DT_F32, s))
+
+    aligned, plain = in_turn(launch(0), launch(4))
+    assert aligned <= 1.2 * plain, (aligned, plain)
