@@ -254,10 +254,10 @@ extern "C" int mi355_colsum_launch(const void *x, int x_dt, int64_t rows, int64_
     // 16-byte loads of whole column groups; an odd pitch stays with the plain kernel, and so do few rows: that one costs
     // 1.9 us and 0.15 a row, the chunks 3 us and more for each round of workgroups (LDS for four a CU).  bf16, plain /
     // chunks: 8 x 512 2.9 / 3.0 us, 12 x 512 3.7 / 3.0, 24 x 50000 6.1 / 5.8 (f32 5.2 / 5.8), 32 x 50000 7.6 / 5.9,
-    // 32 x 200000 8.4 / 14.1, 64 x 200000 20.3 / 15.4
+    // 32 x 200000 8.4 / 14.1, 64 x 200000 20.3 / 15.4.  (A grid holds 2^32 threads: 2^24 workgroups of 256.)
     const int eb = dt_bits(x_dt) / 8, per = 16 / eb;
     const long wgs = (cols + 63) / 64, least = wgs < 39 * 48 ? 9 + wgs / 48 : 48;
-    if (rows >= least && cols % per == 0 && ld % per == 0 && (uintptr_t)x % 16 == 0) {
+    if (rows >= least && wgs < (1L << 24) && cols % per == 0 && ld % per == 0 && (uintptr_t)x % 16 == 0) {
         const dim3 grid((unsigned)wgs);
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, (const char *)x, (long)rows, (long)cols,
