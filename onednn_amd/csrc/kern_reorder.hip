@@ -24,10 +24,13 @@
 //   rows          quantization of activations / weights (float src, 8-bit dst,
 //                 scales per tensor or per column), data types as template
 //                 parameters, parameters fetched once per lane
-//   transpose8(w) 8-bit transposition in registers (the layout change of
-//                 int8 / fp8 weights), 64 x 64 or 128 x 128 tiles
+//   transpose8    transposition into 8-bit elements in registers (the layout
+//                 change of int8 / fp8 weights, quantization into a transposed
+//                 layout), on 128 x 128 or 128 x 64 tiles; 64 x 64 ones for
+//                 short launches and rows that are only 4-byte aligned
 //   pack_woq64    4-bit weights into the packed decode layout
-// MI355_REORDER_GENERIC=1 in the environment keeps rows and transpose8w out.
+// MI355_REORDER_GENERIC=1 in the environment keeps rows and transpose8 out
+// (64 x 64 tiles excepted).
 #include "kernels.hpp"
 #include "tile_epilogue.hpp" // div_by_fma
 
@@ -665,6 +668,56 @@ __global__ void __launch_bounds__(256) reorder_tiled_kernel(const reorder_t R_) 
     }
 }
 
+// Transposition of 8-bit elements without attributes on 64 x 64 tiles over (a, b): both extents multiples of 64, rows of
+// src 4-byte aligned, rows of dst 16-byte aligned.  A thread loads a 4 x 4 block as four dwords, transposes it in
+// registers with eight byte permutes and parks the four result dwords in LDS; the tile then leaves as 16-byte stores
+// along a.  What the kernel behind it does not take or is slower at: rows of src off a 16-byte boundary (8192 x 8192
+// with a pitch of 8196 in 39 us, 84 in the tiled kernel), and extents that are no multiples of 128 while the launch is
+// short (576 x 1088 in 2.1 us, 3.1 on 128 x 128 tiles; 2112 x 2112 in 2.9, 4.1; 8256 x 8256 in 38.2, 35.4).
+__global__ void __launch_bounds__(256) transpose8_kernel(const reorder_t R_) {
+    const auto &R = *(const __attribute__((address_space(4))) reorder_t *)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int PITCH = 17; // dwords per LDS row (16 + 1: spreads the banks)
+    __shared__ uint32_t tile[64 * PITCH];
+    const unsigned ntiles = R.tiles_a * R.tiles_b;
+    const int bi = threadIdx.x & 15, ai = threadIdx.x >> 4; // read: block (4 ai .. +3, 4 bi .. +3)
+    const int wb = threadIdx.x >> 2, wq = threadIdx.x & 3;  // write: row b, 16 bytes of a
+    const uint8_t *src = (const uint8_t *)R.src;
+    uint8_t *dst = (uint8_t *)R.dst;
+    for (unsigned o = blockIdx.y; o < R.outer_total; o += gridDim.y) {
+        long so = 0, dof = 0;
+        {
+            unsigned oo = o;
+            for (int i = 0; i < R.n_outer; ++i) {
+                const unsigned n = R.outer[i].n;
+                const unsigned q = oo / n, r = oo - q * n;
+                oo = q;
+                so += (long)r * R.outer[i].ss;
+                dof += (long)r * R.outer[i].ds;
+            }
+        }
+        for (unsigned t = blockIdx.x; t < ntiles; t += gridDim.x) {
+            const unsigned tb = t % R.tiles_b, ta = t / R.tiles_b;
+            const long a0 = (long)ta * 64, b0 = (long)tb * 64;
+            const uint8_t *p = src + so + (a0 + 4 * ai) * R.a.ss + b0 + 4 * bi;
+            const uint32_t r0 = *(const uint32_t *)p, r1 = *(const uint32_t *)(p + R.a.ss),
+                           r2 = *(const uint32_t *)(p + 2 * R.a.ss), r3 = *(const uint32_t *)(p + 3 * R.a.ss);
+            // byte k of r_i is element (a + i, b + k); T_k collects byte k of the four rows
+            const uint32_t x0 = __builtin_amdgcn_perm(r1, r0, 0x05010400u), x1 = __builtin_amdgcn_perm(r1, r0, 0x07030602u);
+            const uint32_t y0 = __builtin_amdgcn_perm(r3, r2, 0x05010400u), y1 = __builtin_amdgcn_perm(r3, r2, 0x07030602u);
+            tile[(4 * bi + 0) * PITCH + ai] = __builtin_amdgcn_perm(y0, x0, 0x05040100u);
+            tile[(4 * bi + 1) * PITCH + ai] = __builtin_amdgcn_perm(y0, x0, 0x07060302u);
+            tile[(4 * bi + 2) * PITCH + ai] = __builtin_amdgcn_perm(y1, x1, 0x05040100u);
+            tile[(4 * bi + 3) * PITCH + ai] = __builtin_amdgcn_perm(y1, x1, 0x07060302u);
+            __syncthreads();
+            uint4 v;
+            v.x = tile[wb * PITCH + 4 * wq]; v.y = tile[wb * PITCH + 4 * wq + 1];
+            v.z = tile[wb * PITCH + 4 * wq + 2]; v.w = tile[wb * PITCH + 4 * wq + 3];
+            *(uint4 *)(dst + dof + (b0 + wb) * R.b.ds + a0 + 16 * wq) = v;
+            __syncthreads();
+        }
+    }
+}
+
 // Transposition into 8-bit elements: 128 (a) x TB (b) tiles, b has src stride 1, a has dst stride 1.  SDT is a float
 // type (quantization into a transposed layout: f32 scales per tensor or along b, a dst zero point) or BITS8 (8-bit
 // elements moved unconverted: the layout change of int8 / fp8 weights that format_tag::any asks for).  Bound by HBM:
@@ -677,8 +730,8 @@ __global__ void __launch_bounds__(256) reorder_tiled_kernel(const reorder_t R_) 
 // (rows past the end are loaded from the last one, a ragged chunk leaves byte by byte, an unaligned one as an
 // unaligned 16-byte store); rows of src are 16-byte aligned and an extent of b is a multiple of EL.
 // Measured, against the 64 x 64 tiled kernel that took these before: f32 -> s8 8192 x 8192 with a scale per column 147 ->
-// 69 us (4.9 TB/s), bf16 -> s8 1622 x 10752 56 -> 17 us, s8 1621 x 10752 (odd pitch) 41 -> 13 us; s8 8192 x 8192 in
-// 29 us, as the aligned-only kernel it replaces.
+// 69 us (4.9 TB/s), bf16 -> s8 1622 x 10752 56 -> 17 us, s8 1621 x 10752 (odd pitch) 41 -> 13 us.  WHOLE: extents of whole
+// tiles and aligned rows on both sides, without the checks (s8 8192 x 8192 27.8 us, 28.7 with them; 4096 x 4096 7.3, 7.6).
 constexpr int BITS8 = -1;
 
 template <int SDT>
@@ -688,7 +741,7 @@ struct t8_shape {
     static constexpr int TB = EL * LN;
 };
 
-template <int SDT, int DDT>
+template <int SDT, int DDT, bool WHOLE = false>
 __global__ void __launch_bounds__(256) reorder_transpose8_kernel(const reorder_t R_) {
     const auto &R = *(const __attribute__((address_space(4))) reorder_t *)__builtin_amdgcn_kernarg_segment_ptr();
     typedef uint32_t u4v __attribute__((ext_vector_type(4)));
@@ -718,13 +771,14 @@ __global__ void __launch_bounds__(256) reorder_transpose8_kernel(const reorder_t
         for (unsigned t = blockIdx.x; t < ntiles; t += gridDim.x) {
             const unsigned tb = t % tiles_b, ta = t / tiles_b;
             const unsigned a0 = ta * 128, b0 = tb * TB, b_lane = b0 + EL * bi;
-            if (b_lane < R.b.n) {
+            if (WHOLE || b_lane < R.b.n) {
                 u4v v[PASSES][4];
 #pragma unroll
                 for (int p = 0; p < PASSES; ++p)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const unsigned a = min(a0 + 4 * (ag0 + 256 / LN * p) + i, R.a.n - 1);
+                        unsigned a = a0 + 4 * (ag0 + 256 / LN * p) + i;
+                        if (!WHOLE) a = min(a, R.a.n - 1);
                         v[p][i] = __builtin_nontemporal_load((const u4v *)(src + (so + (long)a * R.a.ss + b_lane) * SBYTES));
                     }
                 float s0[EL], s1[EL], y1[EL];
@@ -776,15 +830,15 @@ __global__ void __launch_bounds__(256) reorder_transpose8_kernel(const reorder_t
 #pragma unroll
             for (int p = 0; p < TB / 32; ++p) {
                 const unsigned row = wr + 32 * p, b = b0 + row, a = a0 + 16 * wq;
-                if (b < R.b.n && a < R.a.n) {
+                if (WHOLE || (b < R.b.n && a < R.a.n)) {
                     const u4v w = *(const u4v *)&tile[row * 32 + ((4 * wq + SHIFT * (row / EL)) & 31)];
                     uint8_t *q = dst + dof + (long)b * R.b.ds + a;
-                    if (a + 16 > R.a.n) {
+                    if (!WHOLE && a + 16 > R.a.n) {
                         const unsigned left = R.a.n - a;
 #pragma unroll
                         for (unsigned e = 0; e < 15; ++e)
                             if (e < left) q[e] = (uint8_t)(w[e / 4] >> (8 * (e & 3)));
-                    } else if (R.packed) {
+                    } else if (WHOLE || R.packed) {
                         __builtin_nontemporal_store(w, (u4v *)q);
                     } else {
                         *(u4un *)q = w;
@@ -1155,8 +1209,17 @@ extern "C" int mi355_reorder_launch(const mi355_reorder_desc_t *desc, const mi35
             t8 = R.qdt[k] == MI355_DT_F32 && R.a.qs[k] == 0 && (R.b.qs[k] == 0 || (R.b.qs[k] == 1 && R.b.qg[k] == 1));
             for (int i = 0; i < R.n_outer && t8; ++i) t8 = R.outer[i].qs[k] == 0;
         }
+        // 8-bit copies of whole 64 x 64 tiles whose src rows are 4-byte aligned
+        bool whole64 = R.plain_copy && dbits == 8 && R.a.n % 64 == 0 && R.b.n % 64 == 0 && R.a.ss % 4 == 0
+                && R.b.ds % 16 == 0 && (uintptr_t)R.src % 4 == 0 && (uintptr_t)R.dst % 16 == 0;
+        for (int i = 0; i < R.n_outer && whole64; ++i) whole64 = R.outer[i].ss % 4 == 0 && R.outer[i].ds % 16 == 0;
+        const bool whole128 = t8 && whole64 && R.a.n % 128 == 0 && R.b.n % 128 == 0;
+        // where 128 divides both extents, 64 x 64 / 128 x 128 tiles: 512 x 512 in 2.04 / 2.22 us, 1024 x 1024 in 2.15 /
+        // 2.32, about 2048 x 2048 in 2.9 either way, about 4096 x 4096 in 9.4 / 7.3 (elsewhere: at transpose8_kernel)
+        const long few = whole128 ? 4L << 20 : 32L << 20;
         const dim3 grid((unsigned)gx, gy), block(256);
-        if (t8) {
+        if (whole64 && (!t8 || (long)R.a.n * R.b.n * outer < few)) hipLaunchKernelGGL(transpose8_kernel, grid, block, 0, hs, R);
+        else if (t8) {
             R.packed = (uintptr_t)R.dst % 16 == 0 && R.b.ds % 16 == 0;
             for (int i = 0; i < R.n_outer; ++i) R.packed = R.packed && R.outer[i].ds % 16 == 0;
             const unsigned tb = sbits == 8 ? t8_shape<BITS8>::TB : t8_shape<MI355_DT_BF16>::TB;
@@ -1164,7 +1227,8 @@ extern "C" int mi355_reorder_launch(const mi355_reorder_desc_t *desc, const mi35
             long gw = (long)((R.a.n + 127) / 128) * ((R.b.n + tb - 1) / tb);
             if (gw > (1 << 20)) gw = 1 << 20;
             const dim3 tgrid((unsigned)gw, gy);
-            if (R.plain_copy) hipLaunchKernelGGL((reorder_transpose8_kernel<BITS8, MI355_DT_U8>), tgrid, block, 0, hs, R);
+            if (whole128) hipLaunchKernelGGL((reorder_transpose8_kernel<BITS8, MI355_DT_U8, true>), tgrid, block, 0, hs, R);
+            else if (R.plain_copy) hipLaunchKernelGGL((reorder_transpose8_kernel<BITS8, MI355_DT_U8>), tgrid, block, 0, hs, R);
 #define MI355_T8_CASE(S_, D_) \
     else if (d.src_dt == S_ && d.dst_dt == D_) hipLaunchKernelGGL((reorder_transpose8_kernel<S_, D_>), tgrid, block, 0, hs, R);
 #define MI355_T8_SRC(S_) \

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from onednn_amd import cabi
+from onednn_amd.reorder import GpuReorder, ReorderProblem
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +55,19 @@ def test_column_sums_of_few_rows(gpu, rows, cols):
 
     aligned, plain = in_turn(launch(0), launch(4))
     assert aligned <= 1.2 * plain, (aligned, plain)
+
+
+@pytest.mark.parametrize("pitch,offset", [(8196, 0), (8192, 4), (8200, 8)])
+def test_transposition_out_of_rows_that_are_4_byte_aligned(gpu, pitch, offset):
+    """Four elements a load: about half of what rows off a 4-byte boundary, an element a load, take."""
+    n = 8192
+    raw = np.zeros(offset + n * pitch + 1, np.int8)
+
+    def launch(pitch, offset):
+        g = GpuReorder(ReorderProblem(dims=(n, n), src_dt=cabi.DT_S8, dst_dt=cabi.DT_S8, src=raw, src_stride=(pitch, 1),
+                                      dst_stride=(1, n), name="transposition"))
+        g.args.src += offset
+        return g.launch
+
+    by_4, by_1 = in_turn(launch(pitch, offset), launch(n, 1))
+    assert by_4 <= 0.75 * by_1, (by_4, by_1)

@@ -23,7 +23,7 @@ import pytest
 from onednn_amd import cabi
 from onednn_amd import dtypes as dtp
 from onednn_amd.problem import QuantParam, decode
-from onednn_amd.reorder import ReorderProblem, dense_strides, query, run_gpu
+from onednn_amd.reorder import GpuReorder, ReorderProblem, dense_strides, query, run_gpu
 from oracle import binding as oracle
 
 
@@ -357,6 +357,27 @@ def test_gpu_transposition_to_8_bit_is_bit_exact(make):
     got, want = run_gpu(p), oracle.reorder(p)
     bad = np.flatnonzero(got != want)
     assert bad.size == 0, f"{p.name}: {bad.size} of {got.size} storage elements differ, first at {bad[:5]}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,rows,cols,pitch,offset", [
+    (1, 64, 64, 68, 4), (1, 192, 128, 132, 0), (2, 128, 64, 72, 8),       # 64 x 64 tiles: rows of src 4-byte aligned
+    (1, 128, 128, 144, 16), (2, 384, 256, 256, 0), (1, 2176, 2048, 2064, 32),   # whole tiles, 64 x 64 and 128 x 128
+    (1, 2176, 2048, 2052, 0), (1, 2048, 2112, 2112, 0),                   # only the alignment, only an extent misses the latter
+    (1, 64, 64, 66, 0), (1, 64, 64, 64, 2), (1, 128, 80, 84, 4),          # neither kernel's: every element by itself
+])
+def test_gpu_transposition_out_of_padded_or_offset_rows(gpu, batch, rows, cols, pitch, offset):
+    raw = rng(130).integers(-128, 128, size=offset + batch * rows * pitch, dtype=np.int8)
+    p = ReorderProblem(dims=(batch, rows, cols), src_dt=cabi.DT_S8, dst_dt=cabi.DT_S8, src=raw,
+                       src_stride=(rows * pitch, pitch, 1), dst_stride=(rows * cols, 1, rows), name="padded")
+    g = GpuReorder(p)
+    dst = cabi.DeviceBuffer.from_numpy(np.full(batch * rows * cols + 16, 77, np.int8))
+    g.args.src, g.args.dst = g.bufs["src"].ptr + offset, dst.ptr
+    g.launch()
+    cabi.check(g.lib.mi355_stream_sync(None))
+    got = dst.to_numpy(np.int8, (batch * rows * cols + 16,))
+    want = raw[offset:].reshape(batch, rows, pitch)[:, :, :cols].transpose(0, 2, 1)
+    assert np.array_equal(got[:-16].reshape(want.shape), want) and (got[-16:] == 77).all()
 
 
 @pytest.mark.gpu
