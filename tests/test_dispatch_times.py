@@ -6,7 +6,9 @@ import numpy as np
 import pytest
 
 from onednn_amd import cabi
+from onednn_amd.problem import GpuRun, PostOp
 from onednn_amd.reorder import GpuReorder, ReorderProblem
+from tests.test_gpu_i8_small import int8_problem
 
 pytestmark = pytest.mark.gpu
 
@@ -55,6 +57,25 @@ def test_column_sums_of_few_rows(gpu, rows, cols):
 
     aligned, plain = in_turn(launch(0), launch(4))
     assert aligned <= 1.2 * plain, (aligned, plain)
+
+
+@pytest.mark.parametrize("M,N,K", [(32, 25600, 1024), (32, 20480, 256), (256, 3712, 1024)])
+def test_int8_layers_with_a_short_m(gpu, M, N, K):
+    """s8 x s8 -> s8 without zero points on whole columns: the LDS tiles from three small tiles a compute unit on."""
+    p = int8_problem(M, N, K, cabi.DT_S8, cabi.DT_S8, cabi.DT_S8, dst_scale=20.0,
+                     post_ops=[PostOp(kind=cabi.PO_ELTWISE, alg=cabi.ELTWISE["relu"])])
+
+    def launch(tiles):
+        g = GpuRun(p)
+
+        def go(s):
+            g.stream = s
+            with cabi.tuning("MI355_I8_TILES", tiles):
+                g.launch()
+        return go
+
+    chosen, lds = in_turn(launch(None), launch("large"))
+    assert chosen <= 1.06 * lds, (chosen, lds)
 
 
 @pytest.mark.parametrize("pitch,offset", [(8196, 0), (8192, 4), (8200, 8)])
