@@ -2319,7 +2319,7 @@ DNNL_EXPORT dnnl_status_t dnnl_amd_sdpa_primitive_desc_create(dnnl_primitive_des
     S->composed_scratch = ((S->scores.size_bytes() + 255) & ~(size_t)255) + S->probs.size_bytes();
     pd->scratch_bytes = S->fused ? S->fused_scratch : S->composed_scratch;
     pd->scratchpad = dnnl_memory_desc(); // library mode only: nothing for the caller to provide
-    pd->impl_name = "hip:sdpa(" + kq->impl_name + "," + vs->impl_name + ")";
+    pd->impl_name = S->fused ? "hip:sdpa(hip:mfma_sdpa:gfx950)" : "hip:sdpa(" + kq->impl_name + "," + vs->impl_name + ")";
     pd->sdpa = S;
     if (verbose_level() >= 1)
         fprintf(stderr, "onednn_verbose,v1,primitive,create:dispatch,gpu,sdpa,%s\n", pd->impl_name.c_str());

@@ -171,8 +171,17 @@ def test_descriptor_rules(eng):
 
 
 def test_the_two_matmuls_run_on_the_matrix_cores(eng):
-    pd = sdpa_pd(eng, b=1, h=16, hk=16, sq=512, sk=512, d=128, dv=128)
+    pd = sdpa_pd(eng, b=1, h=16, hk=16, sq=512, sk=512, d=96, dv=96)
     assert pd.impl_info_str() == "hip:sdpa(hip:mfma_h16:gfx950,hip:mfma_h16:gfx950)"
+
+
+def test_the_implementation_name_tells_one_kernel_from_the_composition(eng):
+    one = "hip:sdpa(hip:mfma_sdpa:gfx950)"
+    name = lambda **kw: sdpa_pd(eng, **{"sq": 40, "sk": 72, "d": 64, "dv": 64, **kw}).impl_info_str()  # noqa: E731
+    assert all(name(dt=dt, d=d, dv=d, hk=hk, ddt=ddt) == one
+               for dt in ("bf16", "f16") for d in (64, 128) for hk in (4, 1) for ddt in (None, "f32"))
+    for kw in (dict(dt="f32"), dict(d=32, dv=32), dict(d=80, dv=80), dict(dv=32), dict(d=128)):
+        assert name(**kw).startswith("hip:sdpa(") and name(**kw) != one, kw
 
 
 # ------------------------------------------------------------------ execution on the device

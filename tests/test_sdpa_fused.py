@@ -17,6 +17,9 @@ SHAPES = [  # b, h, hk, sq, sk
 ]
 
 
+ONE_KERNEL = "hip:sdpa(hip:mfma_sdpa:gfx950)"
+
+
 def check(dt, d, shape, **kw):
     b, h, hk, sq, sk = shape
     q, k, v = make(21, b, h, hk, sq, sk, d, d, dt, mag=kw.pop("mag", 1.0))
@@ -25,6 +28,7 @@ def check(dt, d, shape, **kw):
     got, impl = run(q, k, v, dt, dt, True, scale=sc, mask=mask, mask_type=kw.get("mask_type", 0))
     want, pabs = ideal(q, k, v, dt, scale=float(sc[0]), mask=None if mask is None else mask.astype(np.float64),
                        mask_type=kw.get("mask_type", 0))
+    assert impl == ONE_KERNEL
     err = np.abs(values(dt, got) - want)
     tol = tolerance(dt, dt, sk, pabs, want)
     assert (err <= tol).all(), f"{impl}: worst {np.nanmax(err / tol):.2f} of the bound"
@@ -154,7 +158,8 @@ def test_mask_of_the_types_lowest_value(gpu, shape, mdt, lowest):
     mask[:, :, 1, :] = lowest
     stored = {"f32": mask, "bf16": (mask.view(np.uint32) >> 16).astype(np.uint16), "f16": mask.astype(np.float16).view(np.uint16)}[mdt]
     sc = np.array([0.125], np.float32)
-    got, _ = run(q, k, v, "bf16", "bf16", True, scale=sc, mask=stored, mdt=mdt, mask_type=1)
+    got, impl = run(q, k, v, "bf16", "bf16", True, scale=sc, mask=stored, mdt=mdt, mask_type=1)
+    assert impl == ONE_KERNEL
     want, pabs = ideal(q, k, v, "bf16", scale=0.125, mask=mask.astype(np.float64))
     if mdt != "f16":
         want[:, :, 1, :] = values("bf16", v).astype(np.float64).mean(axis=2)
@@ -171,6 +176,7 @@ def test_an_infinite_last_value_stays_infinite(gpu, shape):
     b, h, hk, sq, sk = shape
     q, k, v = make(24, b, h, hk, sq, sk, 64, 64, "bf16")
     v[:, :, sk - 1, 5] = 0x7f80
-    got = values("bf16", run(q, k, v, "bf16", "bf16", True)[0])
-    assert np.isposinf(got[..., 5]).all()
+    got, impl = run(q, k, v, "bf16", "bf16", True)
+    got = values("bf16", got)
+    assert impl == ONE_KERNEL and np.isposinf(got[..., 5]).all()
     assert np.isfinite(np.delete(got, 5, axis=3)).all()
