@@ -391,7 +391,7 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
     }
     l = halves_sum(l);
 
-    int n0 = 0, n1 = NT; // the 32-column blocks of dst that this wavefront finishes
+    int n0 = 0; // the first 32-column block of dst that this wavefront finishes (NWQ = 1: the only one)
     if constexpr (NWQ == 1) {
         // four partial results of the same rows: [wave][block][register][lane], then m and l
         __syncthreads();
@@ -420,7 +420,6 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
         m = mm;
         // wavefront w takes block w (the upper two have none when there are two)
         n0 = wave < NT ? wave : NT;
-        n1 = n0 < NT ? n0 + 1 : NT;
         if (n0 < NT) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -467,7 +466,6 @@ __global__ void __launch_bounds__(256, 2) sdpa_kernel(const sdpa_dev_t P) {
             else *(i2v *)((uint16_t *)P.dst + at) = i2v {sdpa_pack<MI355_DT_F16>(v0, v1), sdpa_pack<MI355_DT_F16>(v2, v3)};
         }
     }
-    (void)n1;
 }
 
 // The parts of the keys added up: D / 4 lanes a row, four columns each.

@@ -141,3 +141,26 @@ def test_weights_gradient_shape_at_full_size_against_the_reference_order_kernel(
     assert np.all(np.abs(ref - want) <= tol)
     assert np.all(np.abs(got - want) <= tol)
     assert np.all(np.abs(got - ref) <= 2 * tol)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtag", ["abc", "acb"])
+def test_f16_results_beyond_its_normal_range(gpu, oracle, variant, dtag):
+    """Groups of one k: every dst element is one product, from 2^-34 to 2^17 and halfway cases on the way (flushed to
+    zero, subnormal, normal, rounded up to infinity), through the hardware conversion; the same with a NaN and an
+    infinity among them, whose wavefronts take the software conversion."""
+    from onednn_amd import grouped
+    M, N = 264, 136
+    p, _ = gc.case_2dx2d([1, 1], M, N, dt=F16, dtag=dtag)
+    r = np.random.default_rng(33)
+    spread = lambda n: np.ldexp(r.integers(1024, 2048, n) / 1024.0, r.integers(-17, 9, n)) * r.choice([-1, 1], n)  # noqa: E731
+    S, W = np.stack([spread(M), spread(M)]), np.stack([spread(N), spread(N)])
+    S[:, :6], W[:, :4] = [2.0 ** -12, 2.0 ** -13, 1.5, 256.0, 2.0 ** -14, 3.0], [2.0 ** -12, 2.0 ** -11, 65504 / 256, 65520 / 256]
+    S[1, [7, 200]], W[1, 100] = [np.nan, np.inf], -np.inf
+    p.src, p.wei = encode(F16, S), encode(F16, W)
+    assert impl_of(p) == "hip:mfma_grouped_k"
+    st, ref = oracle.run_oracle_grouped(p)
+    assert st == cabi.SUCCESS
+    got, ref = gc.logical_dst(p, grouped.run_gpu(p)), gc.logical_dst(p, ref)
+    assert np.isnan(ref[1]).any() and np.isinf(ref[0]).any() and ((ref[0] != 0) & (np.abs(ref[0]) < 2.0 ** -14)).any()
+    assert np.array_equal(got, ref, equal_nan=True) and np.array_equal(np.signbit(got[0]), np.signbit(ref[0]))

@@ -1,6 +1,7 @@
 """The one-kernel attention path (bf16 / f16, head size 64 or 128) at the sizes where it can go wrong: ends of the tiles
 of 32 / 64 keys and 32 / 128 query rows, both forms around 64 rows, keys split over workgroups, masks whose rows start at
-any element or whose keys do not lie side by side, and buffers it does not take (the composition runs then)."""
+any element or whose keys do not lie side by side, rows without a key, strided and broadcast tensors, and buffers it does
+not take (the composition runs then)."""
 import ctypes as C
 
 import numpy as np
@@ -9,6 +10,7 @@ import pytest
 from onednn_amd import cabi, dnnl
 from tests.test_sdpa import DT, ideal, make, md4, run, storage, tolerance, values
 from onednn_amd.problem import storage_dtype
+from tests.test_inner_product import encode
 
 SHAPES = [  # b, h, hk, sq, sk
     (1, 2, 2, 1, 1), (2, 3, 3, 1, 31), (1, 2, 2, 3, 33), (1, 4, 1, 16, 64), (1, 4, 1, 17, 65),   # few rows, 64 and 68
@@ -49,6 +51,99 @@ def test_masks_and_a_negative_scale(gpu, shape, mask_type):
     b, h, hk, sq, sk = shape
     mask = (np.random.default_rng(5).standard_normal((1, 1, sq, sk)) * 2).astype(np.float32) if mask_type == 1 else None
     check("bf16", 64, shape, mask=mask, mask_type=mask_type, sc=-0.11)
+
+
+def run_views(q, k, v, dt, mask=None, mdt=None, mask_type=0, alg=dnnl.softmax_accurate, dst_bshd=False):
+    """As `run`, every tensor with the strides of its numpy view; dst stored [b][h][s][d] or [b][s][h][d]."""
+    eng = dnnl.engine(dnnl.gpu, 0)
+    strm = dnnl.stream(eng)
+    (b, h, sq, d), hk = q.shape, k.shape[1]
+    view_md = lambda x, t: dnnl.memory_desc(list(x.shape), DT[t], strides=[n // x.itemsize for n in x.strides])  # noqa: E731
+    d_md = dnnl.memory_desc([b, h, sq, d], DT[dt], strides=[sq * h * d, d, h * d, 1] if dst_bshd else [h * sq * d, sq * d, d, 1])
+    m_md = None if mask is None else view_md(mask, mdt)
+    pd = dnnl.sdpa_primitive_desc(eng, view_md(q, dt), view_md(k, dt), view_md(v, dt), d_md, mask_md=m_md, kv_head_number=hk,
+                                  attn_mask_type=mask_type, softmax_alg=alg)
+    assert pd.impl_info_str() == ONE_KERNEL
+    dst = dnnl.memory(d_md, eng)
+    args = {arg: dnnl.memory(view_md(x, dt), eng, storage(x)) for arg, x in
+            ((dnnl.ARG_QUERIES, q), (dnnl.ARG_KEYS, k), (dnnl.ARG_VALUES, v))}
+    args[dnnl.ARG_DST] = dst
+    if mask is not None:
+        args[dnnl.ARG_ATTN_MASK] = dnnl.memory(m_md, eng, storage(mask))
+    dnnl.sdpa(pd).execute(strm, args)
+    strm.wait()
+    got = dst.read(storage_dtype(DT[dt]))
+    got = got.reshape(b, sq, h, d).transpose(0, 2, 1, 3) if dst_bshd else got.reshape(b, h, sq, d)
+    return values(dt, got)
+
+
+def within(dt, got, want, pabs, v, rows=slice(None)):
+    """`tolerance`, and for f16 half a step of its subnormals (2^-25) for dst and for every probability, which meets |v| and
+    a division by a sum of at least 1: without a scale the scores spread over dozens of units of e."""
+    tol = tolerance(dt, dt, v.shape[2], pabs, want)
+    if dt == "f16":
+        tol = tol + 2.0 ** -25 * (1 + np.abs(values(dt, v)).sum(axis=2, keepdims=True))
+    return (np.abs(got - want) <= tol)[:, :, rows].all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("alg", [dnnl.softmax_accurate, dnnl.softmax_accurate_inf_as_zero])
+@pytest.mark.parametrize("dt,d", [("bf16", 64), ("f16", 128)])
+@pytest.mark.parametrize("mask_type,shape", [(1, (1, 2, 2, 6, 40)), (1, (1, 2, 2, 130, 200)), (1, (1, 1, 1, 130, 2500)),
+                                             (1, (1, 2, 1, 3, 3000)), (3, (1, 2, 2, 200, 70)), (3, (1, 1, 1, 600, 500)),
+                                             (3, (1, 2, 1, 20, 9))])
+def test_rows_without_a_key(gpu, mask_type, shape, dt, d, alg):
+    """0 / 0, or zeros if asked for, in both forms and with the keys of one and of several parts; the rows beside them."""
+    b, h, hk, sq, sk = shape
+    q, k, v = make(26, b, h, hk, sq, sk, d, d, dt)
+    mask = None
+    if mask_type == 1:
+        mask = (np.random.default_rng(7).standard_normal((1, 1, sq, sk)) * 2).astype(np.float32)
+        mask[0, 0, [1, sq - 1]] = -np.inf
+    got = run_views(q, k, v, dt, mask, "f32", mask_type, alg)
+    want, pabs = ideal(q, k, v, dt, mask=None if mask is None else mask.astype(np.float64), mask_type=mask_type)
+    none = np.isnan(want).all(axis=(0, 1, 3))
+    assert none.sum() == (2 if mask_type == 1 else sq - sk)
+    empty = got[:, :, none]
+    assert np.isnan(empty).all() if alg == dnnl.softmax_accurate else not empty.any()
+    assert within(dt, got, want, pabs, v, ~none)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt,d", [("bf16", 128), ("f16", 64)])
+@pytest.mark.parametrize("mask_type", [2, 3])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 200, 2500), (1, 2, 1, 16, 3000), (1, 1, 1, 1500, 1500), (2, 1, 1, 33, 1000)])
+def test_causal_masks_with_split_keys(gpu, shape, mask_type, dt, d):
+    check(dt, d, shape, mask_type=mask_type)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(2, 2, 2, 150, 200), (2, 2, 2, 3, 200), (1, 4, 1, 40, 131)])
+@pytest.mark.parametrize("mdt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("layout", ["shared", "per head", "per batch", "keys apart", "one key", "one query"])
+def test_mask_layouts(gpu, layout, mdt, shape):
+    b, h, hk, sq, sk = shape
+    dims = {"per head": (1, h, sq, sk), "per batch": (b, 1, sq, sk), "one key": (b, h, sq, 1), "one query": (1, h, 1, sk)}
+    dims = dims.get(layout, (1, 1, sq, sk))
+    raw = encode((np.random.default_rng(8).standard_normal(dims) * 2).astype(np.float32), mdt)
+    if layout == "keys apart":   # [..][keys][queries] in memory
+        raw = np.ascontiguousarray(raw.transpose(0, 1, 3, 2)).transpose(0, 1, 3, 2)
+    q, k, v = make(27, b, h, hk, sq, sk, 128, 128, "bf16")
+    want, pabs = ideal(q, k, v, "bf16", mask=values(mdt, raw))
+    assert within("bf16", run_views(q, k, v, "bf16", raw, mdt, 1), want, pabs, v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(2, 4, 4, 150, 200), (2, 4, 1, 33, 70), (2, 4, 1, 5, 1200)])
+def test_heads_inside_the_rows_and_keys_of_one_batch(gpu, shape):
+    """q, k, v and dst stored [b][s][h][d]; then keys and values of one batch under two."""
+    b, h, hk, sq, sk = shape
+    r = np.random.default_rng(28)
+    bshd = lambda n, s, heads: encode(r.standard_normal((n, s, heads, 64)).astype(np.float32), "f16").transpose(0, 2, 1, 3)  # noqa: E731
+    for kb in (b, 1):
+        q, k, v = bshd(b, sq, h), bshd(kb, sk, hk).transpose(0, 1, 3, 2), bshd(kb, sk, hk)
+        want, pabs = ideal(q, k, v, "f16")
+        assert within("f16", run_views(q, k, v, "f16", dst_bshd=True), want, pabs, v)
 
 
 @pytest.mark.gpu
