@@ -246,7 +246,7 @@ __device__ __forceinline__ void gk_store(const grouped_k_dev_t &P, const gk_f4 (
     // L2s (a quarter faster on a launch that writes 1.3 GB: 0.325 -> 0.25 ms)
     // bf16: v_cvt_pk_bf16_f32 unless the wavefront holds a NaN or an f32 subnormal, which the software conversion
     // (the reference's: subnormals flush, NaNs are quieted its way) treats differently; f16: v_cvt_f16_f32 unless it
-    // holds a NaN (the 64 software roundings a lane were the kernel's bound: 64 groups of 435 rows, 3712 x 8064, f16,
+    // holds a NaN (the 64 software roundings a lane were the kernel's bound: 435 rows over 64 groups, 3712 x 8064, f16,
     // 2179 -> 732 us)
     bool hw = false;
     if (DT == MI355_DT_BF16 || DT == MI355_DT_F16) {

@@ -23,9 +23,11 @@
 // and sdpa_combine_kernel adds the parts.
 //
 // Bound: vector arithmetic next to the matrix instructions for long queries (16 heads, 4096 x 4096, d 128, causal, bf16:
-// the composition 1221 us, of which 729 were the softmax over scores in memory, this 95 us = 725 TFLOP/s; 8 x 8 heads,
-// 1918 x 2942, d 64: 4024 -> 119 us); memory for few (8 x 16 heads, one query, 8192 keys: 653 -> 103 us, 5.2 TB/s).
-// 64 rows is where the forms cross: at 64 rows half of the large form's wavefronts have none.
+// the composition 1221 us, of which 729 were the softmax over scores in memory, this 95 us = 725 TFLOP/s, the matrix
+// cores and the vector units busy 43 % of the time each, a wavefront waiting 24 %; 8 x 8 heads, 1918 x 2942, d 64:
+// 4024 -> 119 us); memory for few (8 x 16 heads, one query, 8192 keys: 653 -> 103 us, 5.2 TB/s; a wavefront waits 55 %).
+// 64 rows is where the forms cross: at 64 rows half of the large form's wavefronts have none.  The form for few rows
+// reads every mask buffer element by element (the decode above: 172 us with one).
 #include "kernels.hpp"
 
 namespace mi355 {
