@@ -59,7 +59,7 @@ def test_column_sums_of_few_rows(gpu, rows, cols):
     assert aligned <= 1.2 * plain, (aligned, plain)
 
 
-@pytest.mark.parametrize("M,N,K", [(32, 25600, 1024), (32, 20480, 256), (256, 3712, 1024)])
+@pytest.mark.parametrize("M,N,K", [(32, 25600, 1024), (32, 20480, 256), (256, 3712, 1024), (22, 28672, 1024)])
 def test_int8_layers_with_a_short_m(gpu, M, N, K):
     """s8 x s8 -> s8 without zero points on whole columns: the LDS tiles from three small tiles a compute unit on."""
     p = int8_problem(M, N, K, cabi.DT_S8, cabi.DT_S8, cabi.DT_S8, dst_scale=20.0,
