@@ -556,9 +556,9 @@ int mi355_sdpa_softmax_launch(const mi355_softmax_desc_t *desc, const void *scor
 
 /* Scaled dot-product attention as one kernel: bf16 / f16 tensors with rows of d = 64 or 128 contiguous elements,
  * hk = h or 1 key / value heads.  Strides in elements: batch, head, row; those of q, k, v multiples of 8, those of dst
- * of 4; buffers 16-byte aligned.  mask_type, scale and inf_as_zero as above; mask strides are 0 along a dimension the
- * mask is broadcast over.  mi355_sdpa_query: MI355_UNIMPLEMENTED for anything else, otherwise the scratch a launch
- * needs (the keys may be split over workgroups). */
+ * of 4; buffers 16-byte aligned, dst apart from the others (or q itself, with the same strides and type).  mask_type,
+ * scale and inf_as_zero as above; mask strides are 0 along a dimension the mask is broadcast over.  mi355_sdpa_query:
+ * MI355_UNIMPLEMENTED for anything else, otherwise the scratch a launch needs (the keys may be split over workgroups). */
 typedef struct {
     int64_t b, h, hk, sq, sk, d;
     int64_t q_stride[3], k_stride[3], v_stride[3], dst_stride[3], mask_stride[4];

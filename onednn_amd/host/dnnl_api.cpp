@@ -2292,7 +2292,7 @@ DNNL_EXPORT dnnl_status_t dnnl_amd_sdpa_primitive_desc_create(dnnl_primitive_des
     S->vs.reset(vs);
     pd->src = q; pd->wei = k; pd->dst = d;
     // One kernel over the keys where it takes the problem (mi355_sdpa_query): rows of one head contiguous, the same
-    // key / value heads for both.  The composition stays for everything else and for unaligned buffers.
+    // key / value heads for both.  The composition stays for everything else, for unaligned buffers and for a dst inside an input.
     if (k.dims[1] == v.dims[1] && q.dims[3] == v.dims[3]) {
         mi355_sdpa_desc_t &F = S->fused_desc;
         memset(&F, 0, sizeof(F));
