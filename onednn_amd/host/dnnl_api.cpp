@@ -258,6 +258,8 @@ struct dnnl_primitive_desc {
         bool fused = false;             // one kernel over the keys (mi355_sdpa_launch) instead of the composition
         mi355_sdpa_desc_t fused_desc;
         size_t fused_scratch = 0, composed_scratch = 0;
+        size_t q_bytes = 0, k_bytes = 0, v_bytes = 0, mask_bytes = 0, scale_bytes = 0, dst_bytes = 0; // from first to last element
+        bool q_in_place = false;        // dst may be q's memory: same type and strides
     };
     std::shared_ptr<sdpa_t> sdpa;
     mi355_grouped_desc_t gdesc;
@@ -2315,6 +2317,10 @@ DNNL_EXPORT dnnl_status_t dnnl_amd_sdpa_primitive_desc_create(dnnl_primitive_des
             for (int i = 0; i < 4; ++i) F.mask_stride[i] = mask_desc->dims[i] == 1 ? 0 : mask_desc->strides[i];
         }
         S->fused = ok && mi355_sdpa_query(&F, &S->fused_scratch) == MI355_SUCCESS;
+        S->q_bytes = q.size_bytes(); S->k_bytes = k.size_bytes(); S->v_bytes = v.size_bytes(); S->dst_bytes = d.size_bytes();
+        if (with_mask) S->mask_bytes = mask_desc->size_bytes();
+        if (with_scale) S->scale_bytes = scale_desc->size_bytes();
+        S->q_in_place = q.dt == d.dt && std::equal(q.strides, q.strides + 4, d.strides);
     }
     S->composed_scratch = ((S->scores.size_bytes() + 255) & ~(size_t)255) + S->probs.size_bytes();
     pd->scratch_bytes = S->fused ? S->fused_scratch : S->composed_scratch;
@@ -2694,14 +2700,13 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
         // (The composition has read q, k, the mask and the scale before it stores; q itself is safe as dst where every
         // element stays in its place, since a wavefront holds its queries before it stores their rows.)
         const uintptr_t low = (uintptr_t)q->handle | (uintptr_t)k->handle | (uintptr_t)v->handle | (uintptr_t)d->handle;
-        auto meets_dst = [&](dnnl_memory_t x, const dnnl_memory_desc &md) {
-            if (!x || md.is_zero()) return false;
-            const uintptr_t x0 = (uintptr_t)x->handle, d0 = (uintptr_t)d->handle;
-            return x0 < d0 + S.dst.size_bytes() && d0 < x0 + md.size_bytes();
+        auto meets_dst = [&](dnnl_memory_t x, size_t bytes) {
+            const uintptr_t x0 = bytes ? (uintptr_t)x->handle : 0, d0 = (uintptr_t)d->handle;
+            return x0 < d0 + S.dst_bytes && d0 < x0 + bytes;
         };
-        const bool in_place = q->handle == d->handle && S.q.dt == S.dst.dt && std::equal(S.q.strides, S.q.strides + 4, S.dst.strides);
-        if (S.fused && low % 16 == 0 && (in_place || !meets_dst(q, S.q)) && !meets_dst(k, S.k) && !meets_dst(v, S.v)
-                && !meets_dst(mask, S.mask) && !meets_dst(scale, S.scale)) {
+        const bool q_apart = (S.q_in_place && q->handle == d->handle) || !meets_dst(q, S.q_bytes);
+        if (S.fused && low % 16 == 0 && q_apart && !meets_dst(k, S.k_bytes) && !meets_dst(v, S.v_bytes)
+                && !meets_dst(mask, S.mask_bytes) && !meets_dst(scale, S.scale_bytes)) {
             if (prim->scratch) order_on_device(); // the parts of a split launch belong to the primitive
             const int rc = mi355_sdpa_launch(&S.fused_desc, q->handle, k->handle, v->handle, d->handle,
                     scale ? scale->handle : nullptr, mask ? mask->handle : nullptr, prim->scratch, stream->hip_stream);
