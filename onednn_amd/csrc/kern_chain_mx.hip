@@ -1,0 +1,20 @@
+// The block-scaled types (MXFP8 e4m3 x e4m3 of hip:mfma_f8, hip:mfma_mxf4) on the chain kernels (chain_gemm.hpp).
+#define MI355_CHAIN_KERNELS
+#include "chain_gemm.hpp"
+#include "line_policies.hpp"
+
+namespace mi355 {
+
+int chain_launch_mx(bool fp4, int dst_dt, chain_t &C, unsigned batch, hipStream_t stream) {
+    using wide_t = geo_t<8, 256>;
+    auto go = [&](auto dst) -> int {
+        constexpr int D = decltype(dst)::value;
+        return fp4 ? chain_go<mxf4_mma_t<wide_t>, D>(C, batch, stream, "mfma_mxf4")
+                   : chain_go<mxf8_mma_t<0, 0, wide_t>, D>(C, batch, stream, "mfma_f8");
+    };
+    if (dst_dt == MI355_DT_BF16) return go(std::integral_constant<int, CHAIN_BF16> {});
+    if (dst_dt == MI355_DT_F32) return go(std::integral_constant<int, CHAIN_F32> {});
+    return MI355_UNIMPLEMENTED;
+}
+
+} // namespace mi355

@@ -1,69 +1,15 @@
 // "hip:mfma_h16" -- the same tiles for bf16 x bf16, f16 x f16 and f32 x f32 operands
-// (ref_matmul_t's f32 sum of exact products): a 64-byte stage is 32 elements of
-// K, one v_mfma_f32_16x16x32_{bf16,f16} per pair of 16-row fragments, in the
-// matrix cycles of the fp8 family's instruction per stage, so the data path
-// (DMA, LDS ring, epilogue) is shared unchanged.
+// (ref_matmul_t's f32 sum of exact products): the 16-bit types on the whole-line
+// loops with v_mfma_f32_16x16x32_{bf16,f16}, f32 on the 64-byte stages of the
+// plain loop, whose matrix instructions take eight times the cycles per byte.
 #include <cstdlib>
 #include <cstring>
 #include "f8_family.hpp"
+#include "chain_gemm.hpp"
+#include "line_policies.hpp"
 
 namespace mi355 {
 namespace {
-
-typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
-typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
-
-// bf16 (BF16) or f16 operands on the 16 x 16 x 32 instruction: a lane's one
-// 16-byte chunk of a stage (row lane % 16, chunk lane / 16) is the whole
-// operand.  The 32 x 32 x 16 shape (two instructions per fragment pair of the
-// fp8 policy's layout) costs the same matrix cycles and LDS bytes per stage, but
-// sustains 1.53 instead of 1.85 PFLOP/s on random operand bits (the clock the
-// power manager allows, `bench.py --calib-mfma`): 0.90 against 0.84 ms on
-// 8192^3, the fp8 family's whole-row bf16 epilogue included.
-template <bool BF16, class G_>
-struct h16x16_mma_t {
-    using G = G_;
-    static constexpr bool TILE16 = true;
-    static constexpr int ELEM_BYTES = 2;
-    static constexpr bool HOT = false;
-    static constexpr int EXTRA_DMAS = 0;
-    __device__ static __forceinline__ void issue_extra(const f8_ctx_t &, int, int, int, int) {}
-    static constexpr int ROWS = 8, COLS = G::WCOLS / 16, A_READS = 1, B_READS = 1;
-    struct frag_t {
-        v4i a[ROWS], b[COLS];
-    };
-    __device__ static __forceinline__ frag_t zero_frag() { return frag_t {}; }
-    struct addr_t {
-        unsigned a, b;
-    };
-    __device__ static __forceinline__ addr_t lane_addr(int wm, int wn, int lane) {
-        const int frow = lane & 15, q = lane >> 4;
-        const int ra = wm * 128 + frow, rb = wn * G::WCOLS + frow;
-        return addr_t {(unsigned)swz(ra, q), (unsigned)(B_OFF + swz(rb, q))};
-    }
-    __device__ static __forceinline__ void load_b(frag_t &f, const unsigned (&S)[1], const addr_t &ad,
-            const f8_ctx_t &, int) {
-#pragma unroll
-        for (int j = 0; j < COLS; ++j) f.b[j] = lds_read16(S[0] + ad.b + j * 1024);
-    }
-    __device__ static __forceinline__ void load_a(frag_t &f, int i, const unsigned (&S)[1], const addr_t &ad,
-            const f8_ctx_t &, int) {
-        f.a[i] = lds_read16(S[0] + ad.a + i * 1024);
-    }
-    __device__ static __forceinline__ void mma_row(v4f (&acc)[ROWS][COLS], const frag_t &f, int i,
-            const f8_ctx_t &, int) {
-#pragma unroll
-        for (int j = 0; j < COLS; ++j) {
-            // operands exchanged: the tile comes out transposed (a lane holds four consecutive n of one row)
-            if constexpr (BF16)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf_t, f.b[j]),
-                        __builtin_bit_cast(v8bf_t, f.a[i]), acc[i][j], 0, 0, 0);
-            else
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h_t, f.b[j]),
-                        __builtin_bit_cast(v8h_t, f.a[i]), acc[i][j], 0, 0, 0);
-        }
-    }
-};
 
 // f32 x f32: a 64-byte stage is 16 elements of K, eight v_mfma_f32_32x32x2_f32 per
 // fragment pair (instruction t takes dword t of the lane's eight: k = t from the
@@ -74,28 +20,34 @@ template <class G_>
 struct f32_mma_t {
     using G = G_;
     static constexpr int ELEM_BYTES = 4;
-    static constexpr bool HOT = false;
-    static constexpr int EXTRA_DMAS = 0;
-    __device__ static __forceinline__ void issue_extra(const f8_ctx_t &, int, int, int, int) {}
-    static constexpr int ROWS = 4, COLS = G::WCOLS / 32, A_READS = 2, B_READS = 2;
+    static constexpr int ROWS = 4, COLS = G::WCOLS / 32;
     struct frag_t {
         v8i a[ROWS], b[COLS];
     };
     __device__ static __forceinline__ frag_t zero_frag() { return frag_t {}; }
-    using base_t = f8_mma_t<0, 0, G_>;
-    using addr_t = typename base_t::addr_t;
-    __device__ static __forceinline__ addr_t lane_addr(int wm, int wn, int lane) { return base_t::lane_addr(wm, wn, lane); }
-    __device__ static __forceinline__ void load_b(frag_t &f, const unsigned (&S)[1], const addr_t &ad,
-            const f8_ctx_t &, int) {
+    // lane l supplies row l % 32 and bytes 32 (l / 32) .. + 32 of the stage: two 16-byte chunks.  Per-lane LDS offsets
+    // of fragment 0; fragment i is 32 rows (2 KB) further with the same swizzle.
+    struct addr_t {
+        unsigned a0, a1, b0, b1;
+    };
+    __device__ static __forceinline__ addr_t lane_addr(int wm, int wn, int lane) {
+        const int frow = lane & 31, c0 = (lane >> 5) * 2;
+        const int ra = wm * 128 + frow, rb = wn * G::WCOLS + frow;
+        return addr_t {(unsigned)swz(ra, c0), (unsigned)swz(ra, c0 + 1), (unsigned)(B_OFF + swz(rb, c0)),
+                (unsigned)(B_OFF + swz(rb, c0 + 1))};
+    }
+    __device__ static __forceinline__ v8i read32(unsigned lo_addr, unsigned hi_addr) {
+        const v4i lo = lds_read16(lo_addr), hi = lds_read16(hi_addr);
+        return v8i {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+    __device__ static __forceinline__ void load_b(frag_t &f, unsigned S, const addr_t &ad) {
 #pragma unroll
-        for (int j = 0; j < COLS; ++j) f.b[j] = base_t::read32(S[0] + ad.b0 + j * 2048, S[0] + ad.b1 + j * 2048);
+        for (int j = 0; j < COLS; ++j) f.b[j] = read32(S + ad.b0 + j * 2048, S + ad.b1 + j * 2048);
     }
-    __device__ static __forceinline__ void load_a(frag_t &f, int i, const unsigned (&S)[1], const addr_t &ad,
-            const f8_ctx_t &, int) {
-        f.a[i] = base_t::read32(S[0] + ad.a0 + i * 2048, S[0] + ad.a1 + i * 2048);
+    __device__ static __forceinline__ void load_a(frag_t &f, int i, unsigned S, const addr_t &ad) {
+        f.a[i] = read32(S + ad.a0 + i * 2048, S + ad.a1 + i * 2048);
     }
-    __device__ static __forceinline__ void mma_row(v16f (&acc)[ROWS][COLS], const frag_t &f, int i,
-            const f8_ctx_t &, int) {
+    __device__ static __forceinline__ void mma_row(v16f (&acc)[ROWS][COLS], const frag_t &f, int i) {
 #pragma unroll
         for (int t = 0; t < 8; ++t)
 #pragma unroll
@@ -264,14 +216,14 @@ static int h16_down_dt(const mi355_matmul_desc_t &d) {
 }
 
 // How a problem reaches the tiles.  An operand is read where it lies when it is K-contiguous with 16-byte aligned
-// rows and K fills whole 64-byte stages; otherwise a reorder launch copies it into scratch as dense K-contiguous
-// rows of Kp = K rounded up to whole stages (converted on the way under fpmath, transposed on the way for
-// N-contiguous weights), the padding zeroed -- so any K and any plain layout with a unit stride runs here, at the
-// price of the copy.
+// rows and K is whole 16-byte chunks (f32: whole 64-byte stages); otherwise a reorder launch copies it into scratch
+// as K-contiguous rows (converted on the way under fpmath, transposed on the way for N-contiguous weights), zeroed from
+// K to Kp, K rounded up to whole chunks -- so any K and any plain layout with a unit stride runs here, at the price of
+// the copy.  pitch: elements between the rows of a copy, whole 64 bytes.
 struct h16_plan_t {
     bool ok, woq;
     int op_dt;
-    long EB, Kp, Bs, Bw;
+    long EB, Kp, pitch, Bs, Bw;
     bool copy_src, copy_wei;
     size_t off_wei, total;
 };
@@ -285,8 +237,9 @@ static h16_plan_t h16_plan(const mi355_matmul_desc_t &d) {
     p.woq = d.src_dt != d.wei_dt; // 8- or 4-bit integer weights under a 16-bit src (checked by h16_supported)
     p.op_dt = down ? down : d.src_dt;
     p.EB = dt_bits(p.op_dt) / 8;
-    const long KE = BKB * KSTEP / p.EB, AL = 16 / p.EB;
+    const long ST = BKB / p.EB, AL = 16 / p.EB, KE = p.op_dt == MI355_DT_F32 ? ST : AL;
     p.Kp = (d.K + KE - 1) / KE * KE;
+    p.pitch = (d.K + ST - 1) / ST * ST;
     const bool pad = p.Kp != d.K;
     const bool src_direct = !down && !pad && d.src_stride[2] == 1 && d.src_stride[1] % AL == 0 && d.src_stride[0] % AL == 0;
     const bool wei_direct = !down && !pad && !p.woq && d.wei_stride[1] == 1 && d.wei_stride[2] % AL == 0
@@ -297,12 +250,15 @@ static h16_plan_t h16_plan(const mi355_matmul_desc_t &d) {
     if (p.copy_src && d.src_stride[2] != 1 && d.src_stride[1] != 1) return p;
     if (p.copy_wei && d.wei_stride[2] != 1 && d.wei_stride[1] != 1) return p;
     // byte offsets inside a tile are 32-bit
-    const long lda = p.copy_src ? p.Kp : d.src_stride[1], ldb = p.copy_wei ? p.Kp : d.wei_stride[2];
+    const long lda = p.copy_src ? p.pitch : d.src_stride[1], ldb = p.copy_wei ? p.pitch : d.wei_stride[2];
     if (lda * p.EB * BM >= (1L << 31) || ldb * p.EB * f8_geo_t::BN >= (1L << 31)) return p;
+    // (a K that ends inside 64 bytes is read where it lies as well; the scratch such a problem asks for, room for the
+    // copies, stays what callers that allocate by it have been told)
+    const bool inside = p.pitch != d.K;
     size_t off = 0;
-    if (p.copy_src) off += align_up((size_t)p.Bs * d.M * p.Kp * p.EB, 256);
+    if (p.copy_src || inside) off += align_up((size_t)p.Bs * d.M * p.pitch * p.EB, 256);
     p.off_wei = off;
-    if (p.copy_wei) off += align_up((size_t)p.Bw * d.N * p.Kp * p.EB, 256);
+    if (p.copy_wei || inside) off += align_up((size_t)p.Bw * d.N * p.pitch * p.EB, 256);
     p.total = off;
     p.ok = true;
     return p;
@@ -418,7 +374,7 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
         set_error("mfma_h16: the problem is not one this family takes");
         return MI355_UNIMPLEMENTED;
     }
-    if (plan.total > 0 && !scratch) {
+    if ((plan.copy_src || plan.copy_wei) && !scratch) {
         set_error("mfma_h16: %zu bytes of scratch required", plan.total);
         return MI355_INVALID_ARGUMENTS;
     }
@@ -427,11 +383,11 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
     const long EB = plan.EB;
     char *a_copy = (char *)scratch, *b_copy = (char *)scratch + plan.off_wei;
     if (plan.copy_src) {
-        if (const int st = h16_convert(P.src, d.src_dt, plan.Bs, d.M, d.K, d.src_stride, false, plan.op_dt, a_copy, plan.Kp,
+        if (const int st = h16_convert(P.src, d.src_dt, plan.Bs, d.M, d.K, d.src_stride, false, plan.op_dt, a_copy, plan.pitch,
                     stream))
             return st;
         P.src = a_copy;
-        P.ss[0] = plan.Bs > 1 ? d.M * plan.Kp : 0; P.ss[1] = plan.Kp; P.ss[2] = 1;
+        P.ss[0] = plan.Bs > 1 ? d.M * plan.pitch : 0; P.ss[1] = plan.pitch; P.ss[2] = 1;
     }
     const int fast = plan.copy_wei ? h16_woq_fast(d, plan) : 0;
     const uintptr_t align = fast == 1 ? ((uintptr_t)P.wei | (uintptr_t)P.wei_scale.p | (uintptr_t)P.wei_zp.p) & 15
@@ -441,7 +397,7 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
         A.wei = (const uint8_t *)P.wei;
         A.out = (uint16_t *)b_copy;
         A.ldw = fast == 1 ? d.wei_stride[1] : d.wei_stride[2];
-        A.ldo = plan.Kp;
+        A.ldo = plan.pitch;
         A.K = (int)d.K; A.N = (int)d.N;
         auto param = [&](const mi355_quant_t &q, const void *ptr, const void *&p_, int &dt, int &gk, int &per_n) {
             p_ = q.dt != MI355_DT_UNDEF ? ptr : nullptr;
@@ -460,15 +416,15 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
                     0, stream, A);
         if (hipGetLastError() != hipSuccess) return MI355_RUNTIME_ERROR;
     } else if (plan.copy_wei) {
-        if (const int st = h16_convert(P.wei, d.wei_dt, plan.Bw, d.K, d.N, d.wei_stride, true, plan.op_dt, b_copy, plan.Kp,
+        if (const int st = h16_convert(P.wei, d.wei_dt, plan.Bw, d.K, d.N, d.wei_stride, true, plan.op_dt, b_copy, plan.pitch,
                     stream, plan.woq ? &d.wei_scale : nullptr, P.wei_scale.p, plan.woq ? &d.wei_zp : nullptr, P.wei_zp.p))
             return st;
     }
     if (plan.copy_wei) {
         if (plan.woq) P.wei_scale.dt = P.wei_zp.dt = MI355_DT_UNDEF; // applied by the copy
         X.bt = b_copy;
-        X.ldb = plan.Kp * EB;
-        X.bt_bstride = plan.Bw > 1 ? d.N * plan.Kp * EB : 0;
+        X.ldb = plan.pitch * EB;
+        X.bt_bstride = plan.Bw > 1 ? d.N * plan.pitch * EB : 0;
     } else {
         X.bt = (const char *)P.wei;
         X.ldb = d.wei_stride[2] * EB;
@@ -477,34 +433,35 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
     P.src_dt = P.wei_dt = plan.op_dt;
     P.K = plan.Kp; // the padding multiplies zeros by zeros
     X.tiles_m = (int)((d.M + BM - 1) / BM);
-    X.tiles_n = (int)((d.N + f8_geo_t::BN - 1) / f8_geo_t::BN);
-    // Few tiles (prefill at a few hundred rows): 256 x 128 tiles of four wavefronts, two workgroups a CU, put twice
-    // the CUs to work; a wavefront's part, 128 x 64, and with it the fragments and the epilogue are the same.
-    using narrow_t = geo_t<4, 128>;
-    // (the MI355_H16_TILES switch keeps the 256 x 256 tiles: tests, tuning)
-    if (plan.op_dt != MI355_DT_F32 && (long)X.tiles_m * X.tiles_n * d.batch <= 128 && d.N > 128
-            && tuning(TUNE_H16_TILES) != TUNE_WIDE) {
-        X.tiles_n = (int)((d.N + narrow_t::BN - 1) / narrow_t::BN);
-        dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);
-        constexpr int smem_bytes = narrow_t::NSTAGE * narrow_t::STAGE_BYTES + NTAB_BYTES;
-        auto go = [&](auto kern) -> int {
-            if (const int st = ensure_dynamic_lds((const void *)kern, smem_bytes, "mfma_h16")) return st;
-            hipLaunchKernelGGL(kern, grid, dim3(narrow_t::NT), smem_bytes, stream, P, X);
-            return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
-        };
-        if (plan.op_dt == MI355_DT_BF16) return go(f8_gemm_kernel<h16x16_mma_t<true, narrow_t>>);
-        return go(f8_gemm_kernel<h16x16_mma_t<false, narrow_t>>);
-    }
-    dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);
-    constexpr int smem_bytes = NSTAGE * f8_geo_t::STAGE_BYTES + NTAB_BYTES;
-    auto go = [&](auto kern) -> int {
+    auto go = [&](auto mma, auto kern) -> int {
+        using Mma = decltype(mma);
+        constexpr int smem_bytes = ring_of<Mma>::BYTES + NTAB_BYTES;
+        X.tiles_n = (int)((d.N + Mma::G::BN - 1) / Mma::G::BN);
+        const dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);
         if (const int st = ensure_dynamic_lds((const void *)kern, smem_bytes, "mfma_h16")) return st;
-        hipLaunchKernelGGL(kern, grid, dim3(f8_geo_t::NT), smem_bytes, stream, P, X);
+        hipLaunchKernelGGL(kern, grid, dim3(Mma::G::NT), smem_bytes, stream, P, X);
         return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
     };
-    if (plan.op_dt == MI355_DT_BF16) return go(f8_gemm_kernel<h16x16_mma_t<true, f8_geo_t>>);
-    if (plan.op_dt == MI355_DT_F32) return go(f8_gemm_kernel<f32_mma_t<f8_geo_t>>);
-    return go(f8_gemm_kernel<h16x16_mma_t<false, f8_geo_t>>);
+    using narrow_t = narrow_geo_t;
+    using f32_t = f32_mma_t<f8_geo_t>;
+    if (plan.op_dt == MI355_DT_F32) return go(f32_t {}, f8_gemm_kernel<f32_t>);
+    // (the MI355_H16_TILES switch keeps the 256 x 256 tiles: tests, tuning)
+    const bool narrow = line_tiles_narrow(d.batch, d.M, d.N) && tuning(TUNE_H16_TILES) != TUNE_WIDE;
+    chain_t C {};
+    if (chain_from(P, false, true, C)) {
+        C.a = (const char *)P.src; C.lda = P.ss[1] * EB; C.a_bs = P.ss[0] * EB;
+        C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
+        C.kbytes = P.K * EB;
+        const int st = chain_launch_h16(plan.op_dt == MI355_DT_BF16, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
+        if (st != MI355_UNIMPLEMENTED) return st;
+    }
+    using bf16_t = h16x16_mma_t<true, f8_geo_t>;
+    using bf16_narrow_t = h16x16_mma_t<true, narrow_t>;
+    using f16_t = h16x16_mma_t<false, f8_geo_t>;
+    using f16_narrow_t = h16x16_mma_t<false, narrow_t>;
+    if (plan.op_dt == MI355_DT_BF16)
+        return narrow ? go(bf16_narrow_t {}, f8_gemm_kernel<bf16_narrow_t>) : go(bf16_t {}, f8_gemm_kernel<bf16_t>);
+    return narrow ? go(f16_narrow_t {}, f8_gemm_kernel<f16_narrow_t>) : go(f16_t {}, f8_gemm_kernel<f16_t>);
 }
 
 } // namespace mi355

@@ -1,5 +1,5 @@
 // "hip:mfma_i8" -- LDS-tiled int8 GEMM on the gfx950 matrix cores
-// (v_mfma_i32_16x16x64_i8) with the zero-point compensation folded into an
+// (v_mfma_i32_16x16x64_i8, line_loops.hpp) with the zero-point compensation folded into an
 // s32 row/column-sum correction and the reference's epilogue fused in.
 //
 // Replaces, for integer src and weights, the reference's brgemm int8 path
@@ -12,7 +12,8 @@
 //     with s' = src - off_s, w' = wei - off_w the bytes re-biased to s8
 //     (off = 128 for u8, 0 for s8), a = off_s - zs, c[n] = off_w - zw[n];
 //   d = (float)acc * src_scale * wei_scale[n]  -> shared epilogue.
-#include "gemm_core.hpp"
+#include "chain_gemm.hpp"
+#include "line_policies.hpp"
 
 #include <cstdlib>
 #include <cstring>
@@ -22,15 +23,8 @@ namespace mi355 {
 namespace {
 
 using namespace gemm;
-// 1: the loop that reads a stage ahead instead of the two-group loop.  Both pass the parity tests and measured the
-// same on the 8192^3 configuration (0.4560 against 0.4566 ms, same box): the kernel's time is set by the energy of
-// its data movement, not by how the wavefronts take turns.
-#ifndef MI355_I8_AHEAD
-#define MI355_I8_AHEAD 0
-#endif
 constexpr int BK = BKB;       // int8: one byte per K element
 using i8_geo_t = geo_t<8, 256>;
-constexpr int NSTAGE = i8_geo_t::NSTAGE;
 
 struct i8_extra_t {
     const int8_t *bt; // weights as [N][K] bytes, K contiguous
@@ -39,92 +33,6 @@ struct i8_extra_t {
     const int *colsum; // [Bw][N] sum_k w'  (null when a == 0)
     const int *rowsum; // [Bs][M] sum_k s'  (null when c == 0)
     int tiles_m, tiles_n;
-};
-
-struct i8_ctx_t {};
-
-// v_mfma_i32_16x16x64_i8: lane l supplies row l%16, K bytes 16*(l/16)..+16, so
-// one instruction consumes the whole 64-byte K extent of a stage for a 16x16
-// tile.  (Measured on MI355X: this shape sustains ~4.0 POPS, the 32x32x32
-// shape ~3.0 POPS.)
-template <bool SRC_U8, bool WEI_U8, class G_>
-struct i8_mma_t {
-    using G = G_;
-    static constexpr int EXTRA_DMAS = 0;
-    __device__ static __forceinline__ void issue_extra(const i8_ctx_t &, int, int, int, int) {}
-    static constexpr int ROWS = 8, COLS = G::WCOLS / 16, A_READS = 1, B_READS = 1;
-    struct frag_t {
-        v4i a[ROWS], b[COLS];
-    };
-    // fragments whose products are zero: a u8 operand is re-biased by 128 where
-    // it is used, so its zero is the byte 0x80
-    __device__ static __forceinline__ frag_t zero_frag() {
-        frag_t f;
-        const int za = SRC_U8 ? (int)0x80808080 : 0, zb = WEI_U8 ? (int)0x80808080 : 0;
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i) f.a[i] = v4i {za, za, za, za};
-#pragma unroll
-        for (int j = 0; j < COLS; ++j) f.b[j] = v4i {zb, zb, zb, zb};
-        return f;
-    }
-    // Per-lane LDS offsets of fragment 0 of both operands.  Fragment i is 16 rows
-    // further: the swizzle depends on the row modulo 16 only, so it is the same
-    // address plus i KB, which goes into the offset field of the read.
-    struct addr_t {
-        unsigned a, b;
-    };
-    __device__ static __forceinline__ addr_t lane_addr(int wm, int wn, int lane) {
-        const int frow = lane & 15, fch = lane >> 4;
-        return addr_t {(unsigned)swz(wm * 128 + frow, fch), (unsigned)(B_OFF + swz(wn * G::WCOLS + frow, fch))};
-    }
-    __device__ static __forceinline__ void load_b(frag_t &f, const unsigned (&S)[1], const addr_t &ad,
-            const i8_ctx_t &, int) {
-#pragma unroll
-        for (int j = 0; j < COLS; ++j) f.b[j] = lds_read16(S[0] + ad.b + j * 1024);
-    }
-    __device__ static __forceinline__ void load_a(frag_t &f, int i, const unsigned (&S)[1], const addr_t &ad,
-            const i8_ctx_t &, int) {
-        f.a[i] = lds_read16(S[0] + ad.a + i * 1024);
-    }
-    // The loop that reads a stage ahead (gemm_core.hpp): a u8 operand is
-    // re-biased in place when its stage's turn comes, and the instruction is
-    // written out with the accumulator tied to one operand -- left to itself the
-    // compiler accumulates out of place in a loop that alternates between two
-    // fragment sets and then copies accumulators around in every iteration.  (No
-    // wait states are owed inside the loop: an accumulator is next touched 31
-    // instructions later, and a VALU result may feed the following MFMA.)
-    static constexpr bool READS_AHEAD = MI355_I8_AHEAD && G::NSTAGE >= 4;
-    __device__ static __forceinline__ void load_b_one(frag_t &f, int j, const unsigned (&S)[1], const addr_t &ad,
-            const i8_ctx_t &, int) {
-        f.b[j] = lds_read16(S[0] + ad.b + j * 1024);
-    }
-    __device__ static __forceinline__ void prepare(frag_t &f) {
-        if (SRC_U8) {
-#pragma unroll
-            for (int i = 0; i < ROWS; ++i) f.a[i] ^= (int)0x80808080;
-        }
-        if (WEI_U8) {
-#pragma unroll
-            for (int j = 0; j < COLS; ++j) f.b[j] ^= (int)0x80808080;
-        }
-    }
-    __device__ static __forceinline__ void mma_row(v4i (&acc)[ROWS][COLS], const frag_t &f, int i,
-            const i8_ctx_t &, int) {
-        if constexpr (READS_AHEAD) {
-#pragma unroll
-            for (int j = 0; j < COLS; ++j)
-                asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(f.b[j]), "v"(f.a[i]));
-        } else {
-            const v4i a = SRC_U8 ? (f.a[i] ^ (int)0x80808080) : f.a[i];
-#pragma unroll
-            for (int j = 0; j < COLS; ++j) {
-                const v4i b = WEI_U8 ? (f.b[j] ^ (int)0x80808080) : f.b[j];
-                // operands exchanged: the tile comes out transposed, a lane holds four
-                // consecutive n of one row (tile_epilogue.hpp)
-                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(b, a, acc[i][j], 0, 0, 0);
-            }
-        }
-    }
 };
 
 // raw s32 accumulator -> f32 entering the shared epilogue
@@ -148,79 +56,11 @@ struct i8_conv_t {
     }
     __device__ __forceinline__ int row_data(long m) const { return rowsum ? rowsum[m] : 0; }
 
-    // The chain of the compute-bound int8 configuration and its neighbours, fully
-    // unrolled over the wavefront's 8 x 4 accumulator tiles with every choice a
-    // template parameter:
-    //   f32(acc) * src_scale * wei_scale[n]  [-> max(., 0)]  [-> / dst_scale]  -> s8 / u8
-    // (no compensation terms, no bias, no zero points).  Per element: convert, two
-    // multiplications, maximum, five operations of the fma-corrected division,
-    // round, convert, clamp, 3/4 of a byte permute.
-    template <bool RELU, int DS, class PT>
-    __device__ __forceinline__ void hot_store(const PT &P, const epi_uniform_t &H, unsigned ntab,
-            const v4i (&acc)[8][4], long b, long m_base, long n_base, int col0) const {
-        const int lane = threadIdx.x & 63, lrow = lane & 15, cq = 4 * (lane >> 4);
-        v4f_t w[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) w[k] = nt4f(ntab, NT_WSC, col0 + 16 * k + cq);
-        const int lo = H.dst_dt == MI355_DT_S8 ? -128 : 0, hi = H.dst_dt == MI355_DT_S8 ? 127 : 255;
-        uint8_t *dcol = (uint8_t *)P.dst + b * P.ds[0] + n_base + cq;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const long m = m_base + 16 * i + lrow;
-            float x[4][4];
-            unsigned mx = 0;
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float t = (float)acc[i][k][e] * ssc;
-                    t *= w[k][e];
-                    if (RELU) t = fmaxf(t, 0.f); // an integer dst turns NaN and -0 into 0 either way
-                    if (DS == 2) t *= H.ds_inv;
-                    if (DS == 3) mx = max(mx, mag_bits(t));
-                    x[k][e] = t;
-                }
-            if (DS == 3) {
-                if (__builtin_amdgcn_ballot_w64(mx >= DIV_BY_FMA_LIMIT) == 0) {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) x[k][e] = div_by_fma(x[k][e], H.ds, H.ds_inv);
-                } else {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) x[k][e] /= H.ds;
-                }
-            }
-            unsigned word[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) word[k] = pack4_i8(x[k], lo, hi);
-            if (m < P.M) {
-                uint8_t *d = dcol + m * P.ds[1];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) *(uint32_t *)(d + 16 * k) = word[k];
-            }
-        }
-    }
-    template <class PT>
-    __device__ __forceinline__ bool hot_chain(const PT &P, const epi_uniform_t &H, unsigned ntab, unsigned,
-            const v4i (&acc)[8][4], long b, long m_base, long n_base, int col0) const {
-        const bool relu0 = H.n_po == 1 && H.pf0.kind == MI355_PO_ELTWISE && H.pf0.alg == MI355_ELTWISE_RELU
-                && H.pf0.alpha == 0.f && H.pf0.scale == 1.f;
-        if (has_comp || !with_src_sc || !with_wei_sc || H.bias_mode != 0 || H.dzp_mode != 0 || H.dynamic
-                || (H.n_po != 0 && !relu0) || H.ds_mode == 1 || (H.dst_dt != MI355_DT_S8 && H.dst_dt != MI355_DT_U8))
-            return false;
-        if (relu0) {
-            if (H.ds_mode == 0) hot_store<true, 0>(P, H, ntab, acc, b, m_base, n_base, col0);
-            else if (H.ds_mode == 2) hot_store<true, 2>(P, H, ntab, acc, b, m_base, n_base, col0);
-            else hot_store<true, 3>(P, H, ntab, acc, b, m_base, n_base, col0);
-        } else {
-            if (H.ds_mode == 0) hot_store<false, 0>(P, H, ntab, acc, b, m_base, n_base, col0);
-            else if (H.ds_mode == 2) hot_store<false, 2>(P, H, ntab, acc, b, m_base, n_base, col0);
-            else hot_store<false, 3>(P, H, ntab, acc, b, m_base, n_base, col0);
-        }
-        return true;
+    // (the chains that layers are made of run on the kernels of chain_gemm.hpp)
+    template <class PT, class Acc>
+    __device__ __forceinline__ bool hot_chain(const PT &, const epi_uniform_t &, unsigned, unsigned, const Acc &, long, long,
+            long, int) const {
+        return false;
     }
     __device__ __forceinline__ void quad(const v4i_t &raw, int rs, unsigned ntab, int col, float (&f)[4]) const {
         int v[4] = {raw[0], raw[1], raw[2], raw[3]};
@@ -246,7 +86,7 @@ struct i8_conv_t {
 extern __shared__ __attribute__((aligned(16))) char i8_smem[];
 
 template <bool SRC_U8, bool WEI_U8, class G>
-__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::NW * G::WG_PER_CU / 4))) i8_gemm_kernel(const problem_t P_, const i8_extra_t X) {
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::NW / 4))) i8_gemm_kernel(const problem_t P_, const i8_extra_t X) {
     using Mma = i8_mma_t<SRC_U8, WEI_U8, G>;
     const auto &P = MI355_KERNARG_PROBLEM();
     char *smem = i8_smem;
@@ -276,8 +116,8 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::N
     cv.rowsum = X.rowsum ? X.rowsum + bs * P.M : nullptr;
     cv.colsum = X.colsum ? X.colsum + bw * P.N : nullptr;
     cv.has_comp = X.rowsum != nullptr || X.colsum != nullptr || cv.a_c != 0 || WEI_U8 || P.wei_zp.dt != MI355_DT_UNDEF;
-    const unsigned ntab = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem + G::NSTAGE * G::STAGE_BYTES;
-    fill_ntab<G::NT>(P, cv, ntab, b, n0);
+    const unsigned ntab = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem + line_loader_t<Mma>::LDS_BYTES;
+    auto fill = [&]() __attribute__((always_inline)) { fill_ntab<G::NT>(P, cv, ntab, b, n0); };
 
     v4i acc[Mma::ROWS][Mma::COLS];
 #pragma unroll
@@ -287,17 +127,15 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::N
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][j][r] = 0;
 
-    main_loop<G::NSTAGE, 1, Mma>(acc, smem, A, Bt, lda, X.ldb, P.M - m0, P.N - n0,
-            (int)(P.K / BK), i8_ctx_t {});
+    main_loop_lines<Mma>(acc, smem, A, Bt, lda, X.ldb, P.M - m0, P.N - n0, P.K, line_scales_t {}, fill);
 
     store_quadrant<layout16_t, G::WCOLS>(P, smem, ntab, acc, b, m0 + wm * 128, n0 + wn * G::WCOLS, wn * G::WCOLS, cv);
 }
 
 
-// ---- few tiles or a K that is not a multiple of the stage: 32 x 32 dst tiles
+// ---- few tiles: 32 x 32 dst tiles
 // without LDS staging.  The 256 x 256 tiles above leave the device idle when
-// M x N holds only a handful of them (4 workgroups for 256 x 1024), and their
-// stage loads want K in units of 64.  Here a workgroup of four wavefronts owns a
+// M x N holds only a handful of them (4 workgroups for 256 x 1024).  Here a workgroup of four wavefronts owns a
 // 32 x 32 tile, the wavefronts take every fourth 64-byte step of K, each lane
 // loads its MFMA operands (16 bytes of a src row, 16 bytes of a weights
 // column, K contiguous in both) straight from memory, four steps ahead of the
@@ -491,9 +329,8 @@ i8_plan_t make_plan(const mi355_matmul_desc_t &d) {
     p.Bw = d.wei_stride[0] ? d.batch : 1;
     p.Bs = d.src_stride[0] ? d.batch : 1;
     p.need_transpose = !(d.wei_stride[1] == 1);
-    // the small tiles when the LDS tiles would occupy too little of the device, or
-    // when the LDS tiles cannot step through K (the small tiles compute their own
-    // sums and have no dynamic dst quantization).  Up to 128 large tiles the LDS
+    // the small tiles when the LDS tiles would occupy too little of the device (the
+    // small tiles compute their own sums and have no dynamic dst quantization).  Up to 128 large tiles the LDS
     // tiles' time depends on K alone; the small tiles' grows with their number, in
     // steps of three a CU.  Counted in small tiles and not in large ones, because a
     // short M fills few rows of a large tile.  K = 1024 / 4096 / 16384, small against
@@ -517,12 +354,12 @@ i8_plan_t make_plan(const mi355_matmul_desc_t &d) {
     const bool three_a_cu = !sums && d.N % 128 == 0 && (own_store || d.K > 8192)
             && (d.M >= 32 || d.K < (d.M > 16 ? 2048 : 1024));
     const long crossover = !three_a_cu ? 1024 : d.K < 1024 ? 257 + d.K / 2 : 769;
-    p.small = !d.dst_scale_dynamic && (small_tiles < crossover || d.K % BK != 0);
+    p.small = !d.dst_scale_dynamic && small_tiles < crossover;
     // the MI355_I8_TILES switch overrides the choice where both can run (tests and
     // tuning): large = the LDS tiles, 256 x 128 or 256 x 256 by the number of
     // tiles; wide = the 256 x 256 ones
     const int force = tuning(TUNE_I8_TILES);
-    if ((force == TUNE_LARGE || force == TUNE_WIDE || force == TUNE_NARROW) && d.K % BK == 0) p.small = false;
+    if (force == TUNE_LARGE || force == TUNE_WIDE || force == TUNE_NARROW) p.small = false;
     if (force == TUNE_SMALL && !d.dst_scale_dynamic) p.small = true;
     // a = off_s - zs can be non-zero whenever src is u8 or has a zero point;
     // c likewise for the weights.  The small tiles compute their own sums: a
@@ -549,8 +386,7 @@ i8_plan_t make_plan(const mi355_matmul_desc_t &d) {
 int i8_supported(const mi355_matmul_desc_t &d) {
     if (!is_int8_dt(d.src_dt) || !is_int8_dt(d.wei_dt)) return MI355_UNIMPLEMENTED;
     if (dt_bits(d.dst_dt) < 8) return MI355_UNIMPLEMENTED;
-    // (a K that is not a multiple of the large tiles' stage runs on the small
-    // tiles, whose 16-byte operand loads are whole inside K or beyond it)
+    // whole 16-byte chunks of K
     if (d.K < 16 || d.K % 16 != 0) return MI355_UNIMPLEMENTED;
     if (d.K % BK != 0 && d.dst_scale_dynamic) return MI355_UNIMPLEMENTED;
     if (d.src_stride[2] != 1 || d.src_stride[1] % 16 != 0) return MI355_UNIMPLEMENTED;
@@ -635,38 +471,42 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         if (wu) return go_small(i8_small_kernel<false, true>);
         return go_small(i8_small_kernel<false, false>);
     }
-    X.tiles_m = (int)((d.M + BM - 1) / BM);
-    X.tiles_n = (int)((d.N + i8_geo_t::BN - 1) / i8_geo_t::BN);
-    // Up to 128 large tiles leave half of the CUs or more idle: 256 x 128 tiles of four wavefronts, two workgroups a
-    // CU, put twice as many to work (a wavefront's part, 128 x 64, its fragments and the epilogue are the same).
-    // MI355_I8_TILES=wide keeps the 256 x 256 tiles.
-    using narrow_t = geo_t<4, 128>;
+    // (MI355_I8_TILES: wide / narrow keep one geometry whatever the size: tests, tuning)
     const int force = tuning(TUNE_I8_TILES);
-    if (force == TUNE_NARROW || ((long)X.tiles_m * X.tiles_n * d.batch <= 128 && d.N > 128 && force != TUNE_WIDE)) {
-        X.tiles_n = (int)((d.N + narrow_t::BN - 1) / narrow_t::BN);
-        dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);
-        constexpr int smem_bytes = narrow_t::NSTAGE * narrow_t::STAGE_BYTES + NTAB_BYTES;
-        auto go = [&](auto kern) -> int {
+    const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N) && force != TUNE_WIDE);
+    chain_t C {};
+    if (!wu && P.wei_zp.dt == MI355_DT_UNDEF && chain_from(P, true, false, C)) {
+        C.a = (const char *)P.src; C.lda = P.ss[1]; C.a_bs = P.ss[0];
+        C.bt = (const char *)X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
+        C.kbytes = P.K;
+        C.colsum = X.colsum;
+        C.colsum_bs = plan.Bw > 1 ? d.N : 0;
+        C.src_zp = P.src_zp.dt != MI355_DT_UNDEF ? (const int *)P.src_zp.p : nullptr;
+        C.off_s = su ? 128 : 0;
+        if (P.src_zp.dt == MI355_DT_UNDEF || P.src_zp.dt == MI355_DT_S32) {
+            const int st = chain_launch_i8(su, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
+            if (st != MI355_UNIMPLEMENTED) return st;
+        }
+    }
+    X.tiles_m = (int)((d.M + BM - 1) / BM);
+    auto go = [&](auto su_, auto wu_) -> int {
+        constexpr bool SU = decltype(su_)::value, WU = decltype(wu_)::value;
+        auto run = [&](auto geo) -> int {
+            using G = decltype(geo);
+            constexpr int smem_bytes = line_loader_t<i8_mma_t<SU, WU, G>>::LDS_BYTES + NTAB_BYTES;
+            X.tiles_n = (int)((d.N + G::BN - 1) / G::BN);
+            const dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);
+            const auto kern = i8_gemm_kernel<SU, WU, G>;
             if (const int st = ensure_dynamic_lds((const void *)kern, smem_bytes, "mfma_i8")) return st;
-            hipLaunchKernelGGL(kern, grid, dim3(narrow_t::NT), smem_bytes, stream, P, X);
+            hipLaunchKernelGGL(kern, grid, dim3(G::NT), smem_bytes, stream, P, X);
             return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
         };
-        if (su && wu) return go(i8_gemm_kernel<true, true, narrow_t>);
-        if (su) return go(i8_gemm_kernel<true, false, narrow_t>);
-        if (wu) return go(i8_gemm_kernel<false, true, narrow_t>);
-        return go(i8_gemm_kernel<false, false, narrow_t>);
-    }
-    dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);
-    constexpr int smem_bytes = NSTAGE * i8_geo_t::STAGE_BYTES + NTAB_BYTES;
-    auto go = [&](auto kern) -> int {
-        if (const int st = ensure_dynamic_lds((const void *)kern, smem_bytes, "mfma_i8")) return st;
-        hipLaunchKernelGGL(kern, grid, dim3(i8_geo_t::NT), smem_bytes, stream, P, X);
-        return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
+        return narrow ? run(geo_t<4, 128> {}) : run(i8_geo_t {});
     };
-    if (su && wu) return go(i8_gemm_kernel<true, true, i8_geo_t>);
-    if (su) return go(i8_gemm_kernel<true, false, i8_geo_t>);
-    if (wu) return go(i8_gemm_kernel<false, true, i8_geo_t>);
-    return go(i8_gemm_kernel<false, false, i8_geo_t>);
+    if (su && wu) return go(std::true_type {}, std::true_type {});
+    if (su) return go(std::true_type {}, std::false_type {});
+    if (wu) return go(std::false_type {}, std::true_type {});
+    return go(std::false_type {}, std::false_type {});
 }
 
 } // namespace mi355

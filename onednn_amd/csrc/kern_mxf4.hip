@@ -15,174 +15,24 @@
 // inside a byte is irrelevant as long as both operands agree, because all 32
 // elements of a block share one scale.
 //
-// Scales ride along with the tile stages: per stage and operand one extra
-// direct-to-LDS load per wavefront brings the 4 scale bytes (one dword) of
-// each of its 64 rows.  Two small pre-pass kernels of the launch put both
-// operands' scales into a stage-major order, [K/128][rows] dwords, so that this
-// load is 256 contiguous bytes: from the plain layouts (src [M][K/32] bytes, a
-// row's dword of a stage 256 bytes from the next row's at K = 8192) the same
-// load touched 64 cache lines for 256 useful bytes, and the scales made as many
-// requests to the L2 as the tiles themselves.
-#include "gemm_core.hpp"
+// Two small pre-pass kernels of the launch put both operands' scales into the order that the K loop loads them in
+// (mx_pack_scales): a stage's scales of 64 rows are 256 contiguous bytes.  From the plain layouts (src [M][K/32] bytes, a
+// row's dword of a stage 256 bytes from the next row's at K = 8192) the same load touched 64 cache lines for 256 useful
+// bytes, and the scales made as many requests to the L2 as the tiles themselves.
+#include "chain_gemm.hpp"
+#include "line_policies.hpp"
 
 namespace mi355 {
 namespace {
 
 using namespace gemm;
-#ifndef MI355_MXF4_NW
-#define MI355_MXF4_NW 8
-#endif
-#ifndef MI355_MXF4_AHEAD
-#define MI355_MXF4_AHEAD 1
-#endif
-using mx_geo_t = geo_t<MI355_MXF4_NW, 256>;
-constexpr int NSTAGE = mx_geo_t::NSTAGE;
-constexpr int SCALE_OFF = NSTAGE * mx_geo_t::STAGE_BYTES; // scale ring after the tile ring
-constexpr int SCALE_STAGE = (BM + mx_geo_t::BN) * 4;      // 256 dwords A + BN dwords B
-constexpr int SMEM_RING_BYTES = SCALE_OFF + NSTAGE * SCALE_STAGE;
-constexpr int SMEM_BYTES = SMEM_RING_BYTES + NTAB_BYTES;
+using mx_geo_t = geo_t<8, 256>;
 
 struct mxf4_extra_t {
     const char *bt;       // weights [N][K/2] bytes
     long ldb, bt_bstride; // bytes
-    const char *sa;       // src scales, stage-major copy: [K/128][M] dwords, this batch added in-kernel
-    const char *sb;       // weights scales, stage-major copy: [K/128][N] dwords
-    long sa_bstride, sb_bstride;
-    long sa_pitch, sb_pitch; // bytes between stages: 4 M, 4 N
+    line_scales_args_t sc;
     int tiles_m, tiles_n;
-};
-
-struct mxf4_ctx_t {
-    const char *sa_tile, *sb_tile; // scale dword of tile row 0, stage 0
-    long sa_pitch, sb_pitch;       // bytes between stages
-    unsigned voff_a, voff_b;       // this lane's row offset in the scale arrays
-    const char *s_tile;            // eight wavefronts: the one operand this wavefront brings
-    long s_pitch;
-    unsigned voff_s;
-    unsigned lds_scale0;           // LDS byte address of the scale ring
-    unsigned lds0;                 // LDS byte address of the tile ring
-};
-
-template <class G_>
-struct mxf4_mma_t {
-    using G = G_;
-    static constexpr int EXTRA_DMAS = G::NW == 4 ? 2 : 1;
-    static constexpr int BBLK = G::BN / 64; // 64-row blocks of B^T scales
-    // four wavefronts: wave w brings the scale dwords of tile rows [64w, 64w+64)
-    // of A and those of block w % BBLK of B^T (with BN = 128 two wavefronts
-    // bring the same block: every wavefront issues the same number of loads,
-    // which the outstanding-load accounting relies on); eight wavefronts:
-    // waves 0-3 bring those of A, waves 4-7 those of B^T
-    __device__ static __forceinline__ void issue_extra(const mxf4_ctx_t &c, int g, int slot, int wave,
-            int) {
-        const unsigned dst = c.lds_scale0 + slot * SCALE_STAGE + wave * 256;
-        if (G::NW == 4) {
-            dma4(c.sa_tile + (long)g * c.sa_pitch, c.voff_a, dst);
-            dma4(c.sb_tile + (long)g * c.sb_pitch, c.voff_b,
-                    c.lds_scale0 + slot * SCALE_STAGE + 1024 + (wave % BBLK) * 256);
-        } else {
-            dma4(c.s_tile + (long)g * c.s_pitch, c.voff_s, dst);
-        }
-    }
-    static constexpr int ROWS = 8, COLS = G::WCOLS / 16, A_READS = 2, B_READS = 2; // data + scale dword
-    static constexpr int SA = ROWS / 4, SB = (COLS + 3) / 4; // scale dwords: one per four fragments
-    struct frag_t {
-        v4i a[ROWS], b[COLS];
-        int sa[SA], sb[SB];
-    };
-    __device__ static __forceinline__ frag_t zero_frag() { return frag_t {}; } // e2m1 zero is all-zero bits
-    // LDS byte address of the scale dwords that belong to the stage at S[0]
-    __device__ static __forceinline__ unsigned scales(const unsigned (&S)[1], const mxf4_ctx_t &c) {
-        const unsigned slot = (S[0] - c.lds0) / G::STAGE_BYTES;
-        return c.lds_scale0 + slot * SCALE_STAGE;
-    }
-    // Per-lane LDS offsets of fragment 0 (data; fragment i is 16 rows further) and of
-    // the scale dword of the lane's first group of 64 rows.  A group of 64 rows holds
-    // its stage's scales as 64 dwords, dword 4 r + q = the bytes of block q of rows r,
-    // 16 + r, 32 + r and 48 + r (the pre-pass kernels of the launch write that order):
-    // lane (r, q) of an MFMA operand reads one dword and has the scale bytes of four
-    // fragments, which the instruction picks by its op_sel bits -- a dword and a read
-    // per four fragments, nothing to shift or mask.
-    struct addr_t {
-        unsigned a, b, sa, sb;
-    };
-    __device__ static __forceinline__ addr_t lane_addr(int wm, int wn, int lane) {
-        const int frow = lane & 15, q = lane >> 4;
-        const int ra = wm * 128 + frow, rb = wn * G::WCOLS + frow;
-        const int cell = (frow * 4 + q) * 4;
-        return addr_t {(unsigned)swz(ra, q), (unsigned)(B_OFF + swz(rb, q)), (unsigned)(wm * 2 * 256 + cell),
-                (unsigned)(1024 + (wn * G::WCOLS / 64) * 256 + cell)};
-    }
-    static constexpr bool READS_AHEAD = MI355_MXF4_AHEAD;
-    __device__ static __forceinline__ void prepare(frag_t &) {}
-    __device__ static __forceinline__ void load_b_one(frag_t &f, int j, const unsigned (&S)[1], const addr_t &ad,
-            const mxf4_ctx_t &c, int) {
-        f.b[j] = lds_read16(S[0] + ad.b + j * 1024);
-        if (j % 4 == 0) f.sb[j / 4] = (int)lds_read4(scales(S, c) + ad.sb + (j / 4) * 256);
-    }
-    __device__ static __forceinline__ void load_b(frag_t &f, const unsigned (&S)[1], const addr_t &ad,
-            const mxf4_ctx_t &c, int g) {
-#pragma unroll
-        for (int j = 0; j < COLS; ++j) load_b_one(f, j, S, ad, c, g);
-    }
-    __device__ static __forceinline__ void load_a(frag_t &f, int i, const unsigned (&S)[1], const addr_t &ad,
-            const mxf4_ctx_t &c, int) {
-        f.a[i] = lds_read16(S[0] + ad.a + i * 1024);
-        if (i % 4 == 0) f.sa[i / 4] = (int)lds_read4(scales(S, c) + ad.sa + (i / 4) * 256);
-    }
-    // The instruction is written out with the accumulator tied to one operand: left
-    // to itself the compiler accumulates out of place in the loops that alternate
-    // between fragment sets or wavefront groups and then moves accumulators through
-    // scratch memory in every iteration (one wavefront per SIMD: the accumulation
-    // registers; two: plain ones, which the epilogue can work on directly).  No
-    // wait states are owed inside the loop: an accumulator is next touched 31 or 63
-    // instructions later.  OW / OS: the byte of the scale dwords that belongs to the
-    // weights / src fragment (op_sel bit 0, op_sel_hi bit 1 of each).
-    template <int OW, int OS>
-    __device__ static __forceinline__ void mma_one(v4f &acc, const v4i &w, const v4i &s, int sw, int ss) {
-        // operands exchanged: the tile comes out transposed, a lane holds four
-        // consecutive n of one row (tile_epilogue.hpp)
-        if constexpr (G::NW == 4)
-            asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%8,0] cbsz:4 blgp:4"
-                         : "+a"(acc)
-                         : "v"(w), "v"(s), "v"(sw), "v"(ss), "n"(OW & 1), "n"(OS & 1), "n"(OW >> 1), "n"(OS >> 1));
-        else
-            asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%8,0] cbsz:4 blgp:4"
-                         : "+v"(acc)
-                         : "v"(w), "v"(s), "v"(sw), "v"(ss), "n"(OW & 1), "n"(OS & 1), "n"(OW >> 1), "n"(OS >> 1));
-    }
-    template <int I, int J>
-    __device__ static __forceinline__ void mma_cols(v4f (&acc)[ROWS][COLS], const frag_t &f) {
-        if constexpr (J < COLS) {
-            mma_one<J % 4, I % 4>(acc[I][J], f.b[J], f.a[I], f.sb[J / 4], f.sa[I / 4]);
-            mma_cols<I, J + 1>(acc, f);
-        }
-    }
-    template <int I>
-    __device__ static __forceinline__ void mma_rows(v4f (&acc)[ROWS][COLS], const frag_t &f, int i) {
-        if constexpr (I < ROWS) {
-            if (i == I) mma_cols<I, 0>(acc, f);
-            else mma_rows<I + 1>(acc, f, i);
-        }
-    }
-    // K that ends inside a stage (gemm_core.hpp tail_step): the lane's chunk is block lane / 16 of the stage
-    static constexpr bool K_TAIL = true;
-    __device__ static __forceinline__ void zero_tail(frag_t &f, int nz, int lane) {
-        const bool z = (lane >> 4) < nz;
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f.a[i][e] = z ? 0 : f.a[i][e];
-#pragma unroll
-        for (int j = 0; j < COLS; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f.b[j][e] = z ? 0 : f.b[j][e];
-    }
-    // (i is a constant after unrolling: the chain of comparisons folds away)
-    __device__ static __forceinline__ void mma_row(v4f (&acc)[ROWS][COLS], const frag_t &f, int i,
-            const mxf4_ctx_t &, int) {
-        mma_rows<0>(acc, f, i);
-    }
 };
 
 struct mxf4_conv_t {
@@ -190,16 +40,7 @@ struct mxf4_conv_t {
     template <class PT>
     __device__ __forceinline__ void per_n(const PT &, long, long, float &, int &, int &) const {}
     __device__ __forceinline__ int row_data(long) const { return 0; }
-    // The configuration's own chain: the accumulators as they are -> bf16, no bias, no post-ops.  Global memory sees
-    // whole 128-byte rows only: in the accumulator layout a lane owns 8 bytes of a dst row and a wavefront-wide store
-    // touches 16 rows, 32 bytes each (the memory pipeline's cost is per line touched).  The wavefront's 128 x 64 part
-    // goes through its 16 KB share of the idle tile ring instead -- 8-byte writes at row * 128 + ((slot ^ (row / 2 & 7))
-    // << 4), which spread over all banks -- and leaves as 16 stores of 8 whole rows.
-    template <class PT>
-    __device__ __forceinline__ bool hot_chain(const PT &P, const epi_uniform_t &H, unsigned, unsigned lds_part,
-            const v4f (&acc)[8][4], long b, long m_base, long n_base, int) const {
-        return store_rows_bf16_tile16(P, H, lds_part, acc, b, m_base, n_base);
-    }
+    // (the chains that layers are made of run on the kernels of chain_gemm.hpp)
     template <class PT, class Acc>
     __device__ __forceinline__ bool hot_chain(const PT &, const epi_uniform_t &, unsigned, unsigned, const Acc &, long,
             long, long, int) const {
@@ -214,7 +55,7 @@ struct mxf4_conv_t {
 extern __shared__ __attribute__((aligned(16))) char mxf4_smem[];
 
 template <class G>
-__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::NW * G::WG_PER_CU / 4))) mxf4_gemm_kernel(const problem_t P_, const mxf4_extra_t X) {
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::NW / 4))) mxf4_gemm_kernel(const problem_t P_, const mxf4_extra_t X) {
     using Mma = mxf4_mma_t<G>;
     const auto &P = MI355_KERNARG_PROBLEM();
     char *smem = mxf4_smem;
@@ -228,27 +69,9 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::N
     const char *A = (const char *)P.src + (P.ss[0] ? b * (P.ss[0] / 2) : 0) + m0 * lda;
     const char *Bt = X.bt + b * X.bt_bstride + n0 * X.ldb;
 
-    mxf4_ctx_t ctx;
-    ctx.lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem;
-    ctx.lds_scale0 = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem + SCALE_OFF;
-    ctx.sa_tile = X.sa + b * X.sa_bstride + m0 * 4;
-    ctx.sb_tile = X.sb + b * X.sb_bstride + n0 * 4;
-    ctx.sa_pitch = X.sa_pitch;
-    ctx.sb_pitch = X.sb_pitch;
-    {
-        // (the packed scales are padded to whole tiles of 256 rows: nothing to clamp)
-        const long ra = (wave & 3) * 64 + lane, rb = ((wave & 3) % (G::BN / 64)) * 64 + lane;
-        ctx.voff_a = (unsigned)(ra * 4);
-        ctx.voff_b = (unsigned)(rb * 4);
-        const bool brings_a = __builtin_amdgcn_readfirstlane(wave) < 4; // uniform: the base stays scalar
-        ctx.s_tile = brings_a ? ctx.sa_tile : ctx.sb_tile;
-        ctx.s_pitch = brings_a ? ctx.sa_pitch : ctx.sb_pitch;
-        ctx.voff_s = brings_a ? ctx.voff_a : ctx.voff_b;
-    }
-
-    // the epilogue's per-column operands go into their LDS table now
-    const unsigned ntab = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem + SMEM_RING_BYTES;
-    fill_ntab<G::NT>(P, mxf4_conv_t {}, ntab, b, n0);
+    // the epilogue's per-column operands go into their LDS table behind the first loads
+    const unsigned ntab = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem + line_loader_t<Mma>::LDS_BYTES;
+    auto fill = [&]() __attribute__((always_inline)) { fill_ntab<G::NT>(P, mxf4_conv_t {}, ntab, b, n0); };
 
     v4f acc[Mma::ROWS][Mma::COLS];
 #pragma unroll
@@ -258,13 +81,7 @@ __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::N
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
 
-    main_loop<NSTAGE, 1, Mma>(acc, smem, A, Bt, lda, X.ldb, P.M - m0, P.N - n0,
-            (int)(P.K / 128), ctx);
-    // the rest of a K that is whole blocks of 32 but not whole stages of 128: the row's last 64 bytes, the blocks
-    // multiplied before zeroed; the scales of those four blocks are the stage after the whole ones in the packed order
-    if (const int rem = (int)(P.K % 128))
-        tail_step<Mma>(acc, smem, A + P.K / 2 - BKB, Bt + P.K / 2 - BKB, lda, X.ldb, P.M - m0, P.N - n0,
-                (128 - rem) / 32, (int)(P.K / 128), ctx);
+    main_loop_lines<Mma>(acc, smem, A, Bt, lda, X.ldb, P.M - m0, P.N - n0, P.K / 2, X.sc.tile(b, m0, n0), fill);
 
     store_quadrant<layout16_t, G::WCOLS>(P, smem, ntab, acc, b, m0 + wm * 128, n0 + wn * G::WCOLS, wn * G::WCOLS,
             mxf4_conv_t {});
@@ -289,7 +106,7 @@ __global__ void __launch_bounds__(256) transpose_nibbles_kernel(const uint8_t *i
 // e8m0 scales of `rows` rows x KB blocks of 32 k, element (r, kb) at in[r * rs + kb * ks], into the order the tile
 // kernel loads: per stage of 128 k (four blocks) and group of 64 rows 64 dwords, dword 4 r + q = the bytes of block q
 // of rows r, 16 + r, 32 + r, 48 + r of the group; groups padded to whole tiles of 256 rows (rows beyond the last
-// repeat it).  out[stage][group][64] dwords.
+// repeat it).  out[set][group][64] dwords; blocks beyond KB have the scale 1.
 // Rows contiguous in the input (weights scales [K/32][N], rs = 1): a thread per dword.
 __global__ void __launch_bounds__(256) mx_scales_rows_kernel(const uint8_t *in, long rows, long prows, long KB, long ks,
         long in_bstride, uint32_t *out, long out_bstride) {
@@ -299,15 +116,13 @@ __global__ void __launch_bounds__(256) mx_scales_rows_kernel(const uint8_t *in, 
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
         const long st = i / prows, w = i % prows, grp = w / 64;
         const int cell = (int)(w % 64), r = cell >> 2, q = cell & 3;
-        // a last stage that K does not fill holds the last four blocks (the tile kernel multiplies the row's last
-        // 64 bytes there)
-        const long blk = 4 * st + 4 <= KB ? 4 * st + q : KB - 4 + q;
+        const long blk = 4 * st + q;
         uint32_t v = 0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             long row = grp * 64 + 16 * e + r;
             row = row < rows ? row : rows - 1;
-            v |= (uint32_t)in[blk * ks + row] << (8 * e);
+            v |= (blk < KB ? (uint32_t)in[blk * ks + row] : 127u) << (8 * e);
         }
         out[i] = v;
     }
@@ -321,19 +136,19 @@ __global__ void __launch_bounds__(256) mx_scales_blocks_kernel(const uint8_t *in
     out += blockIdx.z * out_bstride;
     const long grp = blockIdx.x, r0 = grp * 64, q0 = (long)blockIdx.y * 16, nq = (KB + 3) / 4;
     const int t = threadIdx.x;
-    const bool aligned = ((uintptr_t)in & 3) == 0 && (rs & 3) == 0;
+    const bool aligned = ((uintptr_t)in & 3) == 0 && (rs & 3) == 0 && (KB & 3) == 0;
     {
         const int r = t >> 2, c = t & 3; // row, group of four stages
         const long row = r0 + r < rows ? r0 + r : rows - 1;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const long q = q0 + 4 * c + e;
-            // (a last stage that K does not fill: the row's last four blocks)
-            const uint8_t *p = in + row * rs + (4 * q + 4 <= KB ? 4 * q : KB - 4);
+            const uint8_t *p = in + row * rs + 4 * q;
             uint32_t v = 0u;
             if (q < nq) {
-                if (aligned) v = *(const uint32_t *)p;
-                else v = (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
+                if (aligned) v = *(const uint32_t *)p; // (KB = rs is whole dwords)
+                else
+                    for (int x = 3; x >= 0; --x) v = (v << 8) | (4 * q + x < KB ? (uint32_t)p[x] : 127u);
             }
             tile[4 * c + e][r] = v;
         }
@@ -382,10 +197,31 @@ mxf4_plan_t make_plan(const mi355_matmul_desc_t &d) {
 
 } // namespace
 
+// Packs the e8m0 scales of both operands (src [M][K/32], weights [K/32][N], Bsa / Bsb batches of them) into sa / sb:
+// sets of four blocks, (K + 127) / 128 of them, of M / N rounded up to 256 rows, a dword each.
+int mx_pack_scales(const mi355_matmul_desc_t &d, const problem_t &P, long Bsa, long Bsb, char *sa, char *sb,
+        gemm::line_scales_args_t &sc, hipStream_t stream) {
+    const long kb = d.K / 32, sets = (d.K + 127) / 128, pm = (d.M + 255) / 256 * 256, pn = (d.N + 255) / 256 * 256;
+    long blocks = (pn * sets + 255) / 256;
+    if (blocks > 65535) blocks = 65535;
+    hipLaunchKernelGGL(mx_scales_rows_kernel, dim3((unsigned)blocks, 1, (unsigned)Bsb), dim3(256), 0, stream,
+            (const uint8_t *)P.wei_scale.p, d.N, pn, kb, d.N, kb * d.N, (uint32_t *)sb, pn * sets);
+    hipLaunchKernelGGL(mx_scales_blocks_kernel, dim3((unsigned)(pm / 64), (unsigned)((sets + 15) / 16), (unsigned)Bsa),
+            dim3(256), 0, stream, (const uint8_t *)P.src_scale.p, d.M, pm, kb, kb, d.M * kb, (uint32_t *)sa, pm * sets);
+    sc.a = sa;
+    sc.b = sb;
+    sc.a_bs = Bsa > 1 ? pm * sets * 4 : 0;
+    sc.b_bs = Bsb > 1 ? pn * sets * 4 : 0;
+    sc.a_pitch = pm * 4;
+    sc.b_pitch = pn * 4;
+    sc.sets = (int)sets;
+    return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
+}
+
 int mxf4_supported(const mi355_matmul_desc_t &d) {
     if (d.src_dt != MI355_DT_F4_E2M1 || d.wei_dt != MI355_DT_F4_E2M1) return MI355_UNIMPLEMENTED;
     if (dt_bits(d.dst_dt) < 8 && !tile_nibble_dst_ok(d)) return MI355_UNIMPLEMENTED;
-    // whole MX blocks; a K that ends inside a stage of 128 takes one unpipelined step more per tile
+    // whole MX blocks
     if (d.K < 128 || d.K % 32 != 0) return MI355_UNIMPLEMENTED;
     if (d.src_stride[2] != 1 || d.src_stride[1] % 32 != 0 || d.src_stride[0] % 32 != 0)
         return MI355_UNIMPLEMENTED;
@@ -432,30 +268,22 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         X.ldb = d.wei_stride[2] / 2;
         X.bt_bstride = d.wei_stride[0] / 2;
     }
-    // scales into the tile kernel's order (see mx_scales_rows_kernel)
-    const long kb = d.K / 32;
-    {
-        long blocks = (plan.pn * plan.nst + 255) / 256;
-        if (blocks > 65535) blocks = 65535;
-        hipLaunchKernelGGL(mx_scales_rows_kernel, dim3((unsigned)blocks, 1, (unsigned)plan.Bsb), dim3(256), 0, stream,
-                (const uint8_t *)P.wei_scale.p, d.N, plan.pn, kb, d.N, kb * d.N, (uint32_t *)(sc + plan.off_sb),
-                plan.pn * plan.nst);
-        hipLaunchKernelGGL(mx_scales_blocks_kernel,
-                dim3((unsigned)(plan.pm / 64), (unsigned)((plan.nst + 15) / 16), (unsigned)plan.Bsa), dim3(256), 0, stream,
-                (const uint8_t *)P.src_scale.p, d.M, plan.pm, kb, kb, d.M * kb, (uint32_t *)(sc + plan.off_sa),
-                plan.pm * plan.nst);
+    if (const int st = mx_pack_scales(d, P, plan.Bsa, plan.Bsb, sc + plan.off_sa, sc + plan.off_sb, X.sc, stream)) return st;
+    chain_t C {};
+    if (chain_from_mx(P, true, C)) {
+        C.a = (const char *)P.src; C.lda = P.ss[1] / 2; C.a_bs = P.ss[0] / 2;
+        C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
+        C.kbytes = P.K / 2;
+        C.sc = X.sc;
+        const int st = chain_launch_mx(true, P.dst_dt, C, (unsigned)d.batch, stream);
+        if (st != MI355_UNIMPLEMENTED) return st;
     }
-    X.sb = sc + plan.off_sb;
-    X.sb_bstride = plan.Bsb > 1 ? plan.pn * plan.nst * 4 : 0;
-    X.sb_pitch = plan.pn * 4;
-    X.sa = sc + plan.off_sa;
-    X.sa_bstride = plan.Bsa > 1 ? plan.pm * plan.nst * 4 : 0;
-    X.sa_pitch = plan.pm * 4;
     X.tiles_m = (int)((d.M + BM - 1) / BM);
     X.tiles_n = (int)((d.N + mx_geo_t::BN - 1) / mx_geo_t::BN);
     dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);
-    if (const int st = ensure_dynamic_lds((const void *)mxf4_gemm_kernel<mx_geo_t>, SMEM_BYTES, "mfma_mxf4")) return st;
-    hipLaunchKernelGGL(mxf4_gemm_kernel<mx_geo_t>, grid, dim3(mx_geo_t::NT), SMEM_BYTES, stream, P, X);
+    constexpr int smem_bytes = line_loader_t<mxf4_mma_t<mx_geo_t>>::LDS_BYTES + NTAB_BYTES;
+    if (const int st = ensure_dynamic_lds((const void *)mxf4_gemm_kernel<mx_geo_t>, smem_bytes, "mfma_mxf4")) return st;
+    hipLaunchKernelGGL(mxf4_gemm_kernel<mx_geo_t>, grid, dim3(mx_geo_t::NT), smem_bytes, stream, P, X);
     return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
 }
 

@@ -1,0 +1,561 @@
+// The K loops of the tiles that read whole 128-byte lines: int8, fp8, MXFP8, MXFP4 and the 16-bit types.
+//
+// A step is 128 bytes of K of every row, so that a wavefront's direct-to-LDS load brings 8 whole lines.  The loops
+// before these took 64 bytes a step: a load then touches 16 half lines, the L2 is asked twice for every line, and the
+// loads hold their wavefronts and burn the power budget of the matrix cores.  Same tiles, same MFMAs, 8192^3 on one
+// device, 64-byte steps against these: bf16 0.81 -> 0.72 ms, int8 0.47 -> 0.37; matrix cores busy 0.64 -> 0.82 of the
+// cycles at an unchanged 1.75-1.8 GHz.
+//
+// The LDS ring holds two steps (A: 256 rows, B^T: BN rows, 128 bytes each).  What makes two enough is that a step is
+// released in four parts: the rows and columns of a wavefront's part are halved, a step's products are taken as four
+// quadrants (64 rows x half of the columns), and the part of the ring that holds a half is loaded again, for two
+// steps on, as soon as every wavefront has that half in registers: loads lead their use by 1.5 to 1.75 steps.
+//
+// LDS rows are 128 bytes, the eight 16-byte chunks XOR-swizzled by bits 1-3 of the row (on the global side of the
+// load), which keeps the fragment reads -- 16 rows x 4 chunks -- free of bank conflicts (SQ_LDS_BANK_CONFLICT = 0).
+//
+// Fragments: 16 rows x 128 bytes, two 16-byte chunks a lane (row lane % 16, chunks lane / 16 and 4 + lane / 16).  An
+// instruction of 64 bytes of K (bf16 / f16 16x16x32, int8 16x16x64, fp4 16x16x128) takes one of them, two a pair; fp8
+// 16x16x128 takes both.
+//
+// A last step that K does not fill (any whole number of 16-byte chunks) loads no chunk beyond the row's end -- the
+// lanes of those chunks repeat the last one -- and they are zeroed in the fragments of both operands (both, so that no
+// Inf or NaN meets a zero).
+#pragma once
+#include "gemm_core.hpp"
+
+namespace mi355 {
+namespace gemm {
+
+constexpr int LKB = 128; // bytes of K per row and step
+
+__device__ __forceinline__ int line_swz(int row) { return (row >> 1) & 7; }
+
+struct line_pair_t {
+    v4i c[2];
+    __device__ __forceinline__ v8i whole() const {
+        return v8i {c[0][0], c[0][1], c[0][2], c[0][3], c[1][0], c[1][1], c[1][2], c[1][3]};
+    }
+};
+
+template <class G>
+struct line_geo_t {
+    static constexpr int NW = G::NW, BN = G::BN, WC = G::WCOLS;
+    static constexpr int QC = WC / 32;                   // 16-column tiles in a half of a wavefront's columns
+    static constexpr int STAGE_BYTES = (BM + BN) * LKB;  // 64 KB, or 48 KB of the 256 x 128 tile
+    static constexpr int RING_BYTES = 2 * STAGE_BYTES;
+    static constexpr int B_OFF = BM * LKB;
+    static constexpr int DPA = 16 / NW;                  // loads per wavefront of a half of the A rows, of the B^T rows
+    static constexpr int DPB = DPA * BN / 256;
+    // the epilogue's 16 KB per wavefront
+    static_assert(RING_BYTES >= NW * 16384, "epilogue LDS");
+};
+
+// e8m0 scales per 32 k of both operands, in the order that mx_scales_rows_kernel / mx_scales_blocks_kernel
+// (mx_scales.hpp) write: per four blocks of k and group of 64 rows 64 dwords, dword 4 r + q = the bytes of block q of rows
+// r, 16 + r, 32 + r, 48 + r.  Lane (r, q) of an instruction's operands reads one dword and has the scales of four
+// fragments, which the instruction picks by its op_sel bits.
+struct line_scales_t {
+    const char *a, *b;     // of the tile's first row and column, step 0
+    long a_pitch, b_pitch; // bytes between sets of four blocks
+    int sets;              // sets of K
+};
+
+struct line_scales_args_t { // of a problem
+    const char *a, *b;
+    long a_bs, b_bs, a_pitch, b_pitch;
+    int sets;
+    __host__ __device__ __forceinline__ line_scales_t tile(long batch, long m0, long n0) const {
+        return line_scales_t {a + batch * a_bs + m0 * 4, b + batch * b_bs + n0 * 4, a_pitch, b_pitch, sets};
+    }
+};
+
+// Loads of one workgroup: every wavefront's addresses, the ring, the scales' ring behind it.
+template <class Mma>
+struct line_loader_t {
+    using G = typename Mma::G;
+    using L = line_geo_t<G>;
+    static constexpr int NS = Mma::SCALE_SETS;                  // sets of four blocks in a step
+    static constexpr int SG = 4 + G::BN / 64;                   // groups of 64 rows in a set, A's first
+    static constexpr int SCALE_BYTES = NS * SG * 256;           // of a step
+    static constexpr int EX = (NS * SG + G::NW - 1) / G::NW;    // scale loads per wavefront and step
+    static constexpr int LDS_BYTES = L::RING_BYTES + 2 * SCALE_BYTES;
+
+    unsigned lds0;
+    const char *a_tile, *b_tile;
+    int nst, lane;
+    unsigned tail_mask;          // all ones if the last step is partial
+    unsigned va[2][L::DPA], vb[2][L::DPB], over[2];
+    unsigned la[2][L::DPA], lb[2][L::DPB]; // uniform
+    const char *sbase[EX ? EX : 1];
+    long spitch[EX ? EX : 1];
+    int sset[EX ? EX : 1], sets;
+    unsigned sdst[EX ? EX : 1];
+
+    __device__ __forceinline__ void init(char *smem, const char *a_, const char *b_, long lda, long ldb, long rows_a_left,
+            long rows_b_left, long kbytes, const line_scales_t &sc) {
+        lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem;
+        a_tile = scalar_ptr(a_);
+        b_tile = scalar_ptr(b_);
+        const int rem = (int)(kbytes % LKB) / 16; // chunks of a partial last step
+        nst = scalar_int((int)(kbytes / LKB) + (rem ? 1 : 0));
+        tail_mask = (unsigned)scalar_int(rem ? -1 : 0);
+        const int t = threadIdx.x;
+        lane = t & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(t >> 6), r8 = lane >> 3;
+        // a load is 8 rows: which of the two parities of row block decides the swizzle
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+            const int c = (lane & 7) ^ line_swz(par * 8 + r8);
+            over[par] = (unsigned)((c - min(c, rem - 1)) * 16); // back to the last whole chunk
+            if (rem == 0) over[par] = 0;
+        }
+        constexpr int BPW = L::WC / 16; // row blocks of a half of a wavefront's columns
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < L::DPA; ++i) {
+                const int j = wave * L::DPA + i, row0 = (j / 8) * 128 + h * 64 + (j % 8) * 8;
+                const int c = (lane & 7) ^ line_swz(row0 + r8);
+                const long r = min((long)(row0 + r8), rows_a_left - 1);
+                va[h][i] = (unsigned)(r * lda + c * 16);
+                la[h][i] = (unsigned)(row0 * LKB);
+            }
+#pragma unroll
+            for (int i = 0; i < L::DPB; ++i) {
+                const int j = wave * L::DPB + i, row0 = (j / BPW) * L::WC + h * (L::WC / 2) + (j % BPW) * 8;
+                const int c = (lane & 7) ^ line_swz(row0 + r8);
+                const long r = min((long)(row0 + r8), rows_b_left - 1);
+                vb[h][i] = (unsigned)(r * ldb + c * 16);
+                lb[h][i] = (unsigned)(L::B_OFF + row0 * LKB);
+            }
+        }
+        if constexpr (NS > 0) {
+            sets = scalar_int(sc.sets);
+#pragma unroll
+            for (int k = 0; k < EX; ++k) {
+                // (every wavefront issues the same number of loads: the surplus ones bring the last group again)
+                const int e = min(wave * EX + k, NS * SG - 1), u = e / SG, g = e % SG;
+                const bool of_a = g < 4;
+                spitch[k] = of_a ? sc.a_pitch : sc.b_pitch;
+                sbase[k] = scalar_ptr(of_a ? sc.a + g * 256 : sc.b + (g - 4) * 256);
+                sset[k] = u;
+                sdst[k] = (unsigned)(L::RING_BYTES + e * 256);
+            }
+        }
+    }
+    // Steps from 0 on that load and multiply whole steps inside K only (a step loads two ahead); the rest are END
+    // steps: loads past the last step are issued all the same, clamped to the last one and into a slot nobody reads
+    // again -- one outstanding-load count fits every step -- and a partial last step is taken care of.
+    __device__ __forceinline__ int steady() const { return nst - (tail_mask ? 3 : 2); }
+    __device__ __forceinline__ int clamp(int s) const { return s < nst ? s : nst - 1; }
+    template <bool END>
+    __device__ __forceinline__ void load_a1(int h, int i, int s, int slot) const {
+        const int sc = END ? clamp(s) : s;
+        const unsigned back = END ? over[block_parity(L::DPA, i)] & (sc == nst - 1 ? tail_mask : 0u) : 0u;
+        dma16(a_tile + (long)sc * LKB, va[h][i] - back, lds0 + slot * L::STAGE_BYTES + la[h][i]);
+    }
+    template <bool END>
+    __device__ __forceinline__ void load_b1(int h, int i, int s, int slot) const {
+        const int sc = END ? clamp(s) : s;
+        const unsigned back = END ? over[block_parity(L::DPB, i)] & (sc == nst - 1 ? tail_mask : 0u) : 0u;
+        dma16(b_tile + (long)sc * LKB, vb[h][i] - back, lds0 + slot * L::STAGE_BYTES + lb[h][i]);
+    }
+    // a wavefront's blocks of 8 rows start at an even one
+    static __device__ __forceinline__ constexpr int block_parity(int per_wave, int i) {
+        return per_wave % 2 == 0 ? i & 1 : 0;
+    }
+    template <bool END>
+    __device__ __forceinline__ void load_a(int h, int s, int slot) const {
+#pragma unroll
+        for (int i = 0; i < L::DPA; ++i) load_a1<END>(h, i, s, slot);
+    }
+    template <bool END>
+    __device__ __forceinline__ void load_b(int h, int s, int slot) const {
+        static_assert(L::DPA % 2 == 0 && L::DPB % 2 == 0, "block parity");
+#pragma unroll
+        for (int i = 0; i < L::DPB; ++i) load_b1<END>(h, i, s, slot);
+    }
+    template <bool END>
+    __device__ __forceinline__ void load_scales(int s, int slot) const {
+        if constexpr (NS > 0) {
+#pragma unroll
+            for (int k = 0; k < EX; ++k)
+                // (a second set that K does not reach: the last one again, its products are with zeroed fragments)
+                dma4(sbase[k] + (long)(END ? min(clamp(s) * NS + sset[k], sets - 1) : s * NS + sset[k]) * spitch[k], (unsigned)lane * 4u, lds0 + sdst[k] + slot * SCALE_BYTES);
+        }
+    }
+};
+
+// A wavefront's fragments: both halves of its rows (four 16-row tiles each) and of its columns.
+template <class Mma>
+struct line_frags_t {
+    using G = typename Mma::G;
+    using L = line_geo_t<G>;
+    using Ld = line_loader_t<Mma>;
+    static constexpr int QC = L::QC, NS = Ld::NS;
+    line_pair_t a[2][4], b[2][QC];
+    int sa[2][NS ? NS : 1], sb[NS ? NS : 1];
+    // LDS addresses of chunk u of fragment 0 by slot (the fragments' offsets ride in the read's offset field, which does
+    // not reach from one slot to the other), and of the lane's scale dword
+    unsigned ra[2][2], rb[2][2], rs;
+    bool out[2];               // chunk u of this lane lies beyond K in a partial last step
+
+    __device__ __forceinline__ void init(const Ld &ld, long kbytes) {
+        const int t = threadIdx.x, lane = t & 63, r = lane & 15, q = lane >> 4;
+        const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = G::wm(wave), wn = G::wn(wave);
+        const int rem = (int)(kbytes % LKB) / 16;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const unsigned c = (unsigned)(((u * 4 + q) ^ line_swz(r)) << 4);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                ra[s][u] = ld.lds0 + s * L::STAGE_BYTES + (wm * 128 + r) * LKB + c;
+                rb[s][u] = ld.lds0 + s * L::STAGE_BYTES + L::B_OFF + (wn * L::WC + r) * LKB + c;
+            }
+            out[u] = rem != 0 && u * 4 + q >= rem;
+        }
+        rs = ld.lds0 + L::RING_BYTES + (r * 4 + q) * 4;
+        if constexpr (NS == 0) sa[0][0] = sa[1][0] = sb[0] = 0;
+    }
+    __device__ __forceinline__ void read_a1(int h, int i, int u, int slot) {
+        a[h][i].c[u] = lds_read16((slot ? ra[1][u] : ra[0][u]) + h * (64 * LKB) + i * (16 * LKB));
+    }
+    __device__ __forceinline__ void read_b1(int g, int j, int u, int slot) {
+        b[g][j].c[u] = lds_read16((slot ? rb[1][u] : rb[0][u]) + g * (L::WC / 2 * LKB) + j * (16 * LKB));
+    }
+    __device__ __forceinline__ void read_a(int h, int slot) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) read_a1(h, i, u, slot);
+    }
+    __device__ __forceinline__ void read_b(int g, int slot) {
+#pragma unroll
+        for (int j = 0; j < QC; ++j)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) read_b1(g, j, u, slot);
+    }
+    __device__ __forceinline__ void read_sa(int h, int slot) {
+        if constexpr (NS > 0) {
+            const int wm = G::wm(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+#pragma unroll
+            for (int u = 0; u < NS; ++u) sa[h][u] = (int)lds_read4(rs + slot * Ld::SCALE_BYTES + (u * Ld::SG + wm * 2 + h) * 256);
+        }
+    }
+    __device__ __forceinline__ void read_sb(int slot) {
+        if constexpr (NS > 0) {
+            const int wn = G::wn(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+            static_assert(L::WC == 64 || NS == 0, "a group of 64 columns a wavefront");
+#pragma unroll
+            for (int u = 0; u < NS; ++u) sb[u] = (int)lds_read4(rs + slot * Ld::SCALE_BYTES + (u * Ld::SG + 4 + wn) * 256);
+        }
+    }
+    __device__ __forceinline__ static void zero(line_pair_t &f, const bool (&out)[2]) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f.c[u][e] = out[u] ? 0 : f.c[u][e];
+    }
+    // what fragments need between their read and their first product
+    __device__ __forceinline__ void ready_a(int h, bool partial) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) Mma::prepare_a(a[h][i]);
+        if (partial) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) zero(a[h][i], out);
+        }
+    }
+    __device__ __forceinline__ void ready_b(int g, bool partial) {
+#pragma unroll
+        for (int j = 0; j < QC; ++j) Mma::prepare_b(b[g][j]);
+        if (partial) {
+#pragma unroll
+            for (int j = 0; j < QC; ++j) zero(b[g][j], out);
+        }
+    }
+};
+
+// f(0), f(1), ... with the index as a constant expression
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        static_for<N, I + 1>(f);
+    }
+}
+
+// Eight wavefronts, two per SIMD, in two groups of four that alternate: while one group multiplies a quadrant, the
+// other reads the fragments of its next one and issues loads, and a barrier ends every such phase.  Two wavefronts of
+// a SIMD that multiply at the same time, with reads and loads spread between the MFMAs and a barrier a phase or two a
+// step, measured the same (bf16 8192^3 0.7205 / 0.7208 ms, int8 0.371 / 0.371) on 250 registers instead of 212; what
+// the registers leave is what the fused epilogues and block scales live on.
+//
+// Phases of step s (its slot s % 2): what is read, what is loaded into the part that the phase before released
+//   0  B half 0, A half 0, scales   A half 1 of step s + 1
+//   1  B half 1                     B half 0 and the scales of step s + 2
+//   2  A half 1                     A half 0 of step s + 2
+//   3                               B half 1 of step s + 2
+// A wavefront has its reads back before the barrier that ends the phase's reading part, so a released part is free
+// for both groups.  A part is complete once every wavefront's own loads of it have landed before a barrier ahead of the
+// phase that reads it: the counts below are what a wavefront has issued after them.
+template <class Mma, class Acc, class Fill>
+__device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const char *a_tile, const char *b_tile, long lda,
+        long ldb, long rows_a_left, long rows_b_left, long kbytes, const line_scales_t &sc, Fill &&fill) {
+    using Ld = line_loader_t<Mma>;
+    using Fr = line_frags_t<Mma>;
+    using G = typename Mma::G;
+    static_assert(G::NW == 8, "two groups of four wavefronts");
+    constexpr int DA = Ld::L::DPA, DB = Ld::L::DPB, EX = Ld::EX, QC = Fr::QC, NU = Mma::NU;
+    Ld ld;
+    ld.init(smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, sc);
+    Fr f;
+    f.init(ld, kbytes);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool late = wave >= 4;
+
+    auto quadrant = [&](auto H, auto Gc) __attribute__((always_inline)) {
+        constexpr int h = decltype(H)::value, g = decltype(Gc)::value;
+        __builtin_amdgcn_s_setprio(1);
+        static_for<NU>([&](auto U) __attribute__((always_inline)) {
+            static_for<4>([&](auto I) __attribute__((always_inline)) {
+                static_for<QC>([&](auto J) __attribute__((always_inline)) {
+                    constexpr int u = decltype(U)::value, i = decltype(I)::value, j = decltype(J)::value;
+                    Mma::template mma<g * QC + j, i>(acc[h * 4 + i][g * QC + j], f.b[g][j], f.a[h][i], U,
+                            f.sb[Fr::NS ? u : 0], f.sa[h][Fr::NS ? u : 0]);
+                });
+            });
+        });
+        __builtin_amdgcn_s_setprio(0);
+    };
+    constexpr std::integral_constant<int, 0> c0 {};
+    constexpr std::integral_constant<int, 1> c1 {};
+
+    ld.template load_scales<true>(0, 0);
+    ld.template load_b<true>(0, 0, 0);
+    ld.template load_a<true>(0, 0, 0);
+    ld.template load_b<true>(1, 0, 0);
+    ld.template load_a<true>(1, 0, 0);
+    ld.template load_b<true>(0, 1, 1);
+    ld.template load_scales<true>(1, 1);
+    ld.template load_a<true>(0, 1, 1);
+    ld.template load_b<true>(1, 1, 1);
+    fill();
+    constexpr int STEP = 2 * DA + 2 * DB + EX; // loads of a step
+    wait_vmcnt<STEP + DB>();                   // after A 0 of step 0: B 1, A 1, then step 1 without its A 1
+    phase_barrier();
+    if (late) phase_barrier();
+    auto step = [&](auto End, int s, int slot) __attribute__((always_inline)) {
+        constexpr bool END = decltype(End)::value;
+        const bool partial = END && ld.tail_mask != 0 && s == ld.nst - 1;
+        f.read_sb(slot);
+        f.read_b(0, slot);
+        f.read_sa(0, slot);
+        f.read_sa(1, slot);
+        f.read_a(0, slot);
+        ld.template load_a<END>(1, s + 1, slot ^ 1);
+        wait_vmcnt<STEP + DA>(); // after B 1 of s: A 1, then all of s + 1
+        wait_lds_reads();
+        f.ready_b(0, partial);
+        f.ready_a(0, partial);
+        phase_barrier();
+        quadrant(c0, c0);
+        phase_barrier();
+        f.read_b(1, slot);
+        ld.template load_b<END>(0, s + 2, slot);
+        ld.template load_scales<END>(s + 2, slot);
+        wait_vmcnt<STEP + DB + EX>(); // after A 1 of s: all of s + 1, B 0 and scales of s + 2
+        wait_lds_reads();
+        f.ready_b(1, partial);
+        phase_barrier();
+        quadrant(c0, c1);
+        phase_barrier();
+        f.read_a(1, slot);
+        ld.template load_a<END>(0, s + 2, slot);
+        wait_lds_reads();
+        f.ready_a(1, partial);
+        phase_barrier();
+        quadrant(c1, c1);
+        phase_barrier();
+        ld.template load_b<END>(1, s + 2, slot);
+        wait_vmcnt<STEP + DB>(); // after A 0 of s + 1: B 1 and A 1 of s + 1, s + 2 without its A 1
+        phase_barrier();
+        quadrant(c1, c0);
+        phase_barrier();
+    };
+    int s = 0;
+    const int steady = ld.steady();
+#pragma nounroll
+    for (; s + 1 < steady; s += 2) {
+        step(std::false_type {}, s, 0);
+        step(std::false_type {}, s + 1, 1);
+    }
+#pragma nounroll
+    for (; s < ld.nst; ++s) step(std::true_type {}, s, s & 1);
+    if (!late) phase_barrier();
+    // every load has landed (the clamped ones included) before the ring's memory is used for something else
+    wait_vmcnt<0>();
+    phase_barrier();
+}
+
+// Four wavefronts, one per SIMD, for the 256 x 128 tile.  Nobody covers for a wavefront that waits, so nothing a
+// quadrant needs is requested in it: the fragments of the next half step are read between the MFMAs of this one, and
+// the loads with them.  One wavefront with 128 accumulators keeps a matrix core as busy as two of the eight-wavefront
+// tile (bf16 2048 x 4096 x 14336, 256 tiles: 168 us; the same tile on eight wavefronts of 128 x 32, which read 1.7
+// times as much from LDS, 212 us; the 64-byte steps that this loop took the place of 247).
+//
+// A step s is two halves, x and y the column halves with y = s % 2 (so that a step begins with the columns that the
+// step before released first):
+//          products              reads                                 loads
+//   X(s)   (A 0, B y) (A 0, B x)   B x, A 1 of step s                  B y, A 0 of step s + 2
+//   Y(s)   (A 1, B x) (A 1, B y)   A 0 of s + 1, B of s + 1's y (= x)  B x, A 1 of step s + 2
+// with one barrier before each: every read of the half before is back, so what it read may be loaded again, and what
+// this one reads landed (loads of four parts have been issued after it).
+//
+// The MFMAs are inline assembly with the accumulator tied to one operand: left to itself the compiler accumulates out
+// of place in the two-fold unrolled loop and moves 192 accumulator registers a step.  The accumulators are accumulation
+// registers, of which nothing else wants any: among the plain ones the allocator parked a few elsewhere between steps, and
+// what it read right behind an MFMA that it does not know as one was not written yet.  A VALU result needs two wait
+// states before an MFMA reads it, which the compiler cannot place either (s_nop below).
+template <class Mma, class Acc, class Fill>
+__device__ __forceinline__ void main_loop_lines4(Acc &acc, char *smem, const char *a_tile, const char *b_tile, long lda,
+        long ldb, long rows_a_left, long rows_b_left, long kbytes, Fill &&fill) {
+    using Ld = line_loader_t<Mma>;
+    using Fr = line_frags_t<Mma>;
+    static_assert(Mma::G::NW == 4 && Mma::SCALE_SETS == 0, "four wavefronts, no block scales");
+    constexpr int DA = Ld::L::DPA, DB = Ld::L::DPB, QC = Fr::QC, NU = Mma::NU;
+    Ld ld;
+    ld.init(smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, line_scales_t {});
+    Fr f;
+    f.init(ld, kbytes);
+
+    ld.template load_a<true>(0, 0, 0);
+    ld.template load_b<true>(0, 0, 0);
+    ld.template load_b<true>(1, 0, 0);
+    ld.template load_a<true>(1, 0, 0);
+    ld.template load_b<true>(1, 1, 1);
+    ld.template load_a<true>(0, 1, 1);
+    ld.template load_b<true>(0, 1, 1);
+    ld.template load_a<true>(1, 1, 1);
+    fill();
+    wait_vmcnt<3 * (DA + DB)>();
+    phase_barrier();
+    f.read_a(0, 0);
+    f.read_b(0, 0);
+
+    // two wait states behind everything that ready_a / ready_b compute (the scheduler would sink it to its use)
+    auto settle = []() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_nop 1");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // FIRST: X, otherwise Y; G0: the column half of the first quadrant; slot of step s
+    auto half = [&](auto End, auto First, auto G0, int s, int slot) __attribute__((always_inline)) {
+        constexpr bool END = decltype(End)::value, first = decltype(First)::value;
+        constexpr int g0 = decltype(G0)::value, h = first ? 0 : 1;
+        constexpr int rb = first ? 1 - g0 : g0, ra = first ? 1 : 0; // halves that are read ...
+        constexpr int lb = g0, la = first ? 0 : 1;                  // ... and loaded
+        const int rslot = first ? slot : slot ^ 1;
+        const bool partial = END && ld.tail_mask != 0 && s == ld.nst - 1;
+        wait_vmcnt<2 * (DA + DB)>();
+        wait_lds_reads();
+        phase_barrier();
+        f.ready_a(h, partial);
+        if (first) f.ready_b(g0, partial);
+        settle();
+        constexpr int NB = 2 * QC, NR = NB + 8, NM = 4 * QC * NU, ND = DA + DB;
+        constexpr int PER = NM >= 16 ? 1 : 2; // reads ahead of an MFMA
+        int n = 0, read = 0, loaded = 0;
+#pragma unroll
+        for (int qd = 0; qd < 2; ++qd) {
+            const int g = qd ? 1 - g0 : g0;
+            if (first && qd == 1) {
+                f.ready_b(1 - g0, partial);
+                settle();
+            }
+#pragma unroll
+            for (int u = 0; u < NU; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < QC; ++j) {
+#pragma unroll
+                        for (int p = 0; p < PER; ++p) {
+                            // X: the columns first, its second quadrant wants them; Y: they replace those of its first
+                            const bool cols = first ? read < NB : read >= 8;
+                            if (read < NR && (first || !cols || qd == 1)) {
+                                const int e = first ? (cols ? read : read - NB) : (cols ? read - 8 : read);
+                                if (cols) f.read_b1(rb, e / 2, e % 2, rslot);
+                                else f.read_a1(ra, e / 2, e % 2, rslot);
+                                ++read;
+                            }
+                        }
+                        if (loaded < ND && n == (2 * loaded + 1) * NM / ND) {
+                            if (loaded < DB) ld.template load_b1<END>(lb, loaded, s + 2, slot);
+                            else ld.template load_a1<END>(la, loaded - DB, s + 2, slot);
+                            ++loaded;
+                        }
+                        Mma::mma_tied(acc[h * 4 + i][g * QC + j], f.b[g][j], f.a[h][i], u);
+                        __builtin_amdgcn_sched_barrier(0); // keeps the reads and loads spread between the MFMAs
+                        ++n;
+                    }
+        }
+    };
+    constexpr std::integral_constant<int, 0> c0 {};
+    constexpr std::integral_constant<int, 1> c1 {};
+    auto even = [&](auto End, int s) __attribute__((always_inline)) {
+        half(End, std::true_type {}, c0, s, 0);
+        half(End, std::false_type {}, c1, s, 0);
+    };
+    auto odd = [&](auto End, int s) __attribute__((always_inline)) {
+        half(End, std::true_type {}, c1, s, 1);
+        half(End, std::false_type {}, c0, s, 1);
+    };
+    int s = 0;
+    const int steady = ld.steady();
+#pragma nounroll
+    for (; s + 1 < steady; s += 2) {
+        even(std::false_type {}, s);
+        odd(std::false_type {}, s + 1);
+    }
+#pragma nounroll
+    for (; s < ld.nst; s += 2) {
+        even(std::true_type {}, s);
+        if (s + 1 < ld.nst) odd(std::true_type {}, s + 1);
+    }
+    // every load has landed and every read is back before the ring's memory is used for something else; the wait
+    // states between the last MFMA and the first read of its result
+    wait_vmcnt<0>();
+    wait_lds_reads();
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    phase_barrier();
+}
+
+// fill(): what the kernel prepares for its epilogue; its loads wait behind the first steps' and not in front of them
+// (1.5 us a tile)
+template <class Mma, class Acc, class Fill>
+__device__ __forceinline__ void main_loop_lines(Acc &acc, char *smem, const char *a_tile, const char *b_tile, long lda,
+        long ldb, long rows_a_left, long rows_b_left, long kbytes, const line_scales_t &sc, Fill &&fill) {
+    if constexpr (Mma::G::NW == 8)
+        main_loop_lines8<Mma>(acc, smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, sc, fill);
+    else
+        main_loop_lines4<Mma>(acc, smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, fill);
+}
+
+// operand policies of these loops
+template <class Mma, class = void>
+struct reads_lines : std::false_type {};
+template <class Mma>
+struct reads_lines<Mma, std::enable_if_t<(Mma::NU > 0)>> : std::true_type {};
+
+// Which of the two tiles a problem of `batch` x M x N takes: rounds of 256 workgroups, one a CU, at 9 / 16 of the
+// large tile's time for the 256 x 128 one (bf16 / int8 / fp8, K = 4096: 39 / 23.4 / 22.7 us a round against 69 / 40 /
+// 39).  Beyond two rounds of large tiles the chip is power-limited and the small tile's 1.5 loads per MFMA cost 10 %.
+inline bool line_tiles_narrow(long batch, long M, long N) {
+    if (N <= 128) return false;
+    const long tm = (M + BM - 1) / BM, wide = batch * tm * ((N + 255) / 256), narrow = batch * tm * ((N + 127) / 128);
+    return wide <= 512 && 9 * ((narrow + 255) / 256) < 16 * ((wide + 255) / 256);
+}
+
+} // namespace gemm
+} // namespace mi355

@@ -1,0 +1,114 @@
+"""The K loops of 128-byte steps (onednn_amd/csrc/line_loops.hpp) and the kernels with a compiled-in epilogue on top of
+them (chain_gemm.hpp): where the steps end, on both tile geometries, and where the rows of dst do.
+
+Exact data (small integers, power-of-two scales: any order of the sum gives the same bits) against the oracle, bit for
+bit.  K in bytes: a lone partial step, one chunk short of a step and one past it, one / two / three / four steps (the
+loops load two ahead and are unrolled by two) and a partial step behind each count."""
+import numpy as np
+import pytest
+
+from onednn_amd import cabi, configs
+from onednn_amd import dtypes as dtp
+from onednn_amd.problem import MatmulProblem, PostOp, QuantParam, run_gpu, strides_for
+from tests.helpers import assert_bit_exact
+
+pytestmark = pytest.mark.gpu
+DT = cabi.DT_NAMES
+BYTES = {"bf16": 2, "f16": 2, "s8": 1, "u8": 1, "f8_e4m3": 1}
+SWITCH = {"bf16": "MI355_H16_TILES", "f16": "MI355_H16_TILES", "s8": "MI355_I8_TILES", "u8": "MI355_I8_TILES",
+          "f8_e4m3": "MI355_F8_TILES"}
+FAMILY = {"bf16": "hip:mfma_h16", "f16": "hip:mfma_h16", "s8": "hip:mfma_i8", "u8": "hip:mfma_i8", "f8_e4m3": "hip:mfma_f8"}
+
+
+def encode(v, dt):
+    v = np.asarray(v, np.float32)
+    if dt == "bf16":
+        return dtp.f32_to_bf16(v.reshape(-1)).reshape(v.shape)
+    if dt == "f16":
+        return v.astype(np.float16).view(np.uint16)
+    if dt == "f8_e4m3":
+        return dtp.f32_to_e4m3(v.reshape(-1)).reshape(v.shape)
+    return v.astype(np.int8 if dt == "s8" else np.uint8)
+
+
+def problem(M, N, K, dt, ddt, *, bias=False, post=(), batch=1, pitch=0, dst_scale=None, src_zp=None, row_scales=False):
+    r = np.random.default_rng(M + N + K)
+    lo, hi = (0, 7) if dt == "u8" else (-3, 4)
+    src = encode(r.integers(lo, hi, size=(batch, M, K)), dt)
+    wdt = "s8" if dt == "u8" else dt
+    wei = encode(r.integers(-2, 3, size=(batch, N, K)), wdt)
+    quant = {}
+    if dt in ("s8", "u8", "f8_e4m3"):
+        quant["src_scale"] = QuantParam(cabi.DT_F32, 0, np.array([0.5], np.float32))
+        quant["wei_scale"] = QuantParam(cabi.DT_F32, configs.MASK_COL, r.choice([0.25, 0.5, 1.0], size=N).astype(np.float32))
+    if row_scales:
+        quant["src_scale"] = QuantParam(cabi.DT_F32, 2, r.choice([0.25, 0.5, 1.0], size=M).astype(np.float32))
+    if src_zp is not None:
+        quant["src_zp"] = QuantParam(cabi.DT_S32, 0, np.array([src_zp], np.int32))
+    if dst_scale is not None:
+        quant["dst_scale"] = QuantParam(cabi.DT_F32, 0, np.array([dst_scale], np.float32))
+    b = (r.integers(-8, 9, size=N) / 4).astype(np.float32) if bias else None
+    kw = {}
+    if pitch:
+        kw = dict(dst_stride=(M * pitch, pitch, 1), dst_init=np.zeros(batch * M * pitch, np.uint16))
+    return MatmulProblem(M=M, N=N, K=K, batch=batch, src_dt=DT[dt], wei_dt=DT[wdt], dst_dt=DT[ddt], src=src, wei=wei,
+                         wei_stride=strides_for("ba", batch, K, N), bias_dt=cabi.DT_F32 if bias else cabi.DT_UNDEF, bias=b,
+                         quant=quant, post_ops=list(post), name=f"lines-{dt}-{ddt}-{M}x{N}x{K}", **kw)
+
+
+def check(oracle, p, dt, tiles=None):
+    with cabi.tuning(SWITCH[dt], tiles):
+        got, name = run_gpu(p)
+    assert name.startswith(FAMILY[dt]), name
+    assert_bit_exact(p, got, oracle.run_oracle(p), f"{name} {tiles}")
+
+
+# 300 x 328 runs on 256 x 128 tiles by itself (int8: when told to), on 256 x 256 ones when told to
+@pytest.mark.parametrize("kbytes", [64, 112, 128, 144, 192, 256, 272, 384, 448, 496, 512, 640, 656])
+@pytest.mark.parametrize("dt,ddt", [("bf16", "bf16"), ("f16", "f16"), ("s8", "f32"), ("u8", "bf16"), ("f8_e4m3", "bf16")])
+@pytest.mark.parametrize("tiles", ["wide", "narrow"])
+def test_where_the_steps_end(gpu, oracle, kbytes, dt, ddt, tiles):
+    p = problem(300, 328, kbytes // BYTES[dt], dt, ddt, bias=True, src_zp=3 if dt == "u8" else None)
+    check(oracle, p, dt, "wide" if tiles == "wide" else None if BYTES[dt] == 2 else "narrow")
+
+
+RELU = PostOp(cabi.PO_ELTWISE, alg=cabi.ELTWISE["relu"], alpha=0.0)
+
+
+# rows of dst that end inside a wavefront's 64 columns or a 16-byte piece, dst pitches of whole and of no whole pieces,
+# M inside a wavefront's 128 rows, every compiled-in dst type, batches
+@pytest.mark.parametrize("M,N", [(1, 136), (129, 200), (130, 268), (257, 388)])
+@pytest.mark.parametrize("dt,ddt,kw", [
+    ("bf16", "bf16", {}), ("bf16", "f32", dict(bias=True)), ("f16", "f16", dict(bias=True, post=[RELU])),
+    ("f16", "f32", dict(post=[RELU])), ("s8", "s8", dict(post=[RELU], dst_scale=3.0)), ("s8", "u8", dict(bias=True, dst_scale=0.7)),
+    ("u8", "s8", dict(bias=True, src_zp=5)), ("u8", "f32", dict(src_zp=2, post=[RELU])), ("f8_e4m3", "f32", dict(bias=True)),
+    ("f8_e4m3", "bf16", dict(row_scales=True, post=[RELU]))])
+def test_where_the_rows_of_dst_end(gpu, oracle, M, N, dt, ddt, kw):
+    for tiles in ("wide", "narrow"):
+        p = problem(M, N, 256 // BYTES[dt], dt, ddt, batch=2, **kw)
+        check(oracle, p, dt, "wide" if tiles == "wide" else None if BYTES[dt] == 2 else "narrow")
+
+
+@pytest.mark.parametrize("act", [None, "gelu_tanh", "swish"])
+@pytest.mark.parametrize("alg", ["add", "mul"])
+@pytest.mark.parametrize("dt", ["bf16", "f8_e4m3"])
+def test_a_staged_tensor_at_ragged_edges(gpu, oracle, act, alg, dt):
+    """N = 200: the last wavefront's columns end after one chunk of eight; rows end inside a row block.  Without an
+    activation the sums are exact; with one the result is within the activation's few ulp of the oracle, rounded to
+    bf16: two units of bf16."""
+    M, N, K = 150, 200, 128
+    r = np.random.default_rng(5)
+    other = dtp.f32_to_bf16(r.integers(-4, 5, size=M * N).astype(np.float32)).reshape(M, N)
+    post = [PostOp(cabi.PO_ELTWISE, alg=cabi.ELTWISE[act], alpha=1.0)] if act else []
+    post.append(PostOp(cabi.PO_BINARY, alg=cabi.BINARY[alg], dt=cabi.DT_BF16, stride=(0, N, 1), data=other))
+    p = problem(M, N, K, dt, "bf16", bias=True, post=post)
+    if dt == "f8_e4m3":
+        p.quant["src_scale"].data[:] = 1 / 64
+    got, name = run_gpu(p)
+    assert name.startswith(FAMILY[dt]), name
+    want = oracle.run_oracle(p)
+    if not act:
+        assert_bit_exact(p, got, want, name)
+        return
+    g, w = (dtp.bf16_to_f32(np.asarray(x).view(np.uint16).reshape(-1)) for x in (got, want))
+    assert np.all(np.abs(g - w) <= 2.0 ** -7 * np.abs(w) + 2.0 ** -20)
