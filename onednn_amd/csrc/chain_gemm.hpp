@@ -64,6 +64,9 @@ int mx_pack_scales(const mi355_matmul_desc_t &d, const problem_t &P, long Bsa, l
 // The families' launchers on the chain kernels, a translation unit each; C as chain_from and the family left it.
 // wide: the 256 x 256 tiles whatever the size
 int chain_launch_h16(bool bf16, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
+// ... with the weights (across = 1), or src and the weights (2, 256 x 256 tiles only), contiguous across K: lda / ldb are the
+// bytes from one k to the next
+int chain_launch_h16_across(bool bf16, int dst_dt, int across, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
 int chain_launch_i8(bool src_u8, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
 int chain_launch_f8(int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream); // e4m3 x e4m3
 int chain_launch_mx(bool fp4, int dst_dt, chain_t &C, unsigned batch, hipStream_t stream);  // e4m3 x e4m3 or fp4
@@ -346,7 +349,8 @@ __global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = V {0, 0, 0, 0};
     const line_scales_t sc = C.sc.tile(b, tp.m0, tp.n0);
-    main_loop_lines<Mma>(acc, smem, C.a + b * C.a_bs + tp.m0 * C.lda, C.bt + b * C.b_bs + tp.n0 * C.ldb, C.lda, C.ldb,
+    main_loop_lines<Mma>(acc, smem, C.a + b * C.a_bs + tp.m0 * (line_form<Mma>::AKM ? 2 : C.lda),
+            C.bt + b * C.b_bs + tp.n0 * (line_form<Mma>::BKM ? 2 : C.ldb), C.lda, C.ldb,
             C.M - tp.m0, C.N - tp.n0, C.kbytes, sc, fill);
 
     const int wm = G::wm(wave), wn = G::wn(wave);

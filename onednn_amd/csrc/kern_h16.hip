@@ -368,6 +368,19 @@ static int h16_convert(const void *in, int from, long B, long R, long C, const i
     return MI355_SUCCESS;
 }
 
+// Operands that the chain kernels read where they lie although they are contiguous across K (16-byte pieces of every
+// line, 32-bit offsets inside a step): 0 none, 1 the weights, 2 src and the weights.
+static int h16_across(const mi355_matmul_desc_t &d, const h16_plan_t &p, const problem_t &P) {
+    if (p.woq || (p.op_dt != MI355_DT_BF16 && p.op_dt != MI355_DT_F16) || p.op_dt != d.src_dt) return 0;
+    auto lines = [&](const void *ptr, long unit, long pitch, long batch, long width) {
+        return unit == 1 && pitch % 8 == 0 && pitch > 0 && pitch < (1L << 23) && (d.batch == 1 || batch % 8 == 0) && width % 8 == 0
+                && ((uintptr_t)ptr & 15) == 0;
+    };
+    if (!p.copy_wei || d.wei_stride[1] == 1 || !lines(P.wei, d.wei_stride[2], d.wei_stride[1], d.wei_stride[0], d.N)) return 0;
+    if (!p.copy_src) return 1;
+    return d.src_stride[2] != 1 && lines(P.src, d.src_stride[1], d.src_stride[2], d.src_stride[0], d.M) ? 2 : 0;
+}
+
 int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratch, hipStream_t stream) {
     const h16_plan_t plan = h16_plan(d);
     if (!plan.ok) {
@@ -381,6 +394,30 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
     f8_extra_t X {};
     problem_t P = P_in;
     const long EB = plan.EB;
+    // (the MI355_H16_TILES switch keeps the 256 x 256 tiles: tests, tuning)
+    const bool narrow = line_tiles_narrow(d.batch, d.M, d.N) && tuning(TUNE_H16_TILES) != TUNE_WIDE;
+    chain_t C {};
+    int across = h16_across(d, plan, P);
+    // the 256 x 128 tile takes weights across K only: src is copied there (whole chunks of K)
+    if (across == 2 && narrow) across = d.K % 8 == 0 ? 1 : 0;
+    if (across && (P.dst_dt == plan.op_dt || P.dst_dt == MI355_DT_F32) && chain_from(P, false, true, C)) {
+        C.a = (const char *)P.src;
+        C.a_bs = d.src_stride[0] * EB;
+        C.lda = (across == 2 ? d.src_stride[2] : d.src_stride[1]) * EB;
+        if (across == 1 && plan.copy_src) {
+            if (const int st = h16_convert(P.src, d.src_dt, plan.Bs, d.M, d.K, d.src_stride, false, plan.op_dt, scratch, plan.pitch,
+                        stream))
+                return st;
+            C.a = (const char *)scratch;
+            C.a_bs = plan.Bs > 1 ? d.M * plan.pitch * EB : 0;
+            C.lda = plan.pitch * EB;
+        }
+        C.bt = (const char *)P.wei;
+        C.b_bs = d.wei_stride[0] * EB;
+        C.ldb = d.wei_stride[1] * EB;
+        C.kbytes = d.K * EB;
+        return chain_launch_h16_across(plan.op_dt == MI355_DT_BF16, P.dst_dt, across, C, (unsigned)d.batch, !narrow, stream);
+    }
     char *a_copy = (char *)scratch, *b_copy = (char *)scratch + plan.off_wei;
     if (plan.copy_src) {
         if (const int st = h16_convert(P.src, d.src_dt, plan.Bs, d.M, d.K, d.src_stride, false, plan.op_dt, a_copy, plan.pitch,
@@ -445,9 +482,6 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
     using narrow_t = narrow_geo_t;
     using f32_t = f32_mma_t<f8_geo_t>;
     if (plan.op_dt == MI355_DT_F32) return go(f32_t {}, f8_gemm_kernel<f32_t>);
-    // (the MI355_H16_TILES switch keeps the 256 x 256 tiles: tests, tuning)
-    const bool narrow = line_tiles_narrow(d.batch, d.M, d.N) && tuning(TUNE_H16_TILES) != TUNE_WIDE;
-    chain_t C {};
     if (chain_from(P, false, true, C)) {
         C.a = (const char *)P.src; C.lda = P.ss[1] * EB; C.a_bs = P.ss[0] * EB;
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;

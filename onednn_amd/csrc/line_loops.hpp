@@ -18,7 +18,16 @@
 // instruction of 64 bytes of K (bf16 / f16 16x16x32, int8 16x16x64, fp4 16x16x128) takes one of them, two a pair; fp8
 // 16x16x128 takes both.
 //
-// A last step that K does not fill (any whole number of 16-byte chunks) loads no chunk beyond the row's end -- the
+// An operand of the 16-bit types may also lie the other way round, its rows (of src) or columns (of the weights)
+// contiguous and K across them: what a transposed layer has, backward by data in its weights and backward by weights in
+// both operands.  Its part of a step is 64 k of whole 512- or 256-byte lines, halved by k (32 each) where the other kind is
+// halved by rows; a fragment comes out of LDS through ds_read_b64_tr_b16, which hands lane (r, q) the four k of its row
+// from four lines, and is then the same as the other kind's.  Copying such operands K-contiguous first took 144 of the
+// 735 us of a training step (2048 x 14336 x 4096).  The 32-byte units of a line are XOR-swizzled by bits 0, 1 and 3 of k:
+// the eight lines that half a wavefront reads 32 bytes of start at one bank.
+//
+// A last step that K does not fill (any whole number of 16-byte chunks, any K where both operands lie the other way
+// round) loads no chunk beyond the row's end -- the
 // lanes of those chunks repeat the last one -- and they are zeroed in the fragments of both operands (both, so that no
 // Inf or NaN meets a zero).
 #pragma once
@@ -30,6 +39,25 @@ namespace gemm {
 constexpr int LKB = 128; // bytes of K per row and step
 
 __device__ __forceinline__ int line_swz(int row) { return (row >> 1) & 7; }
+
+// operands whose rows / columns are contiguous instead of K
+template <class Mma, class = void>
+struct line_form {
+    static constexpr bool AKM = false, BKM = false;
+};
+template <class Mma>
+struct line_form<Mma, std::enable_if_t<(Mma::A_KM || Mma::B_KM)>> {
+    static constexpr bool AKM = Mma::A_KM, BKM = Mma::B_KM;
+};
+// the swizzle of a line of such an operand, in 32-byte units
+__device__ __forceinline__ int kline_swz(int k) { return (k & 3) | ((k >> 3) & 1) << 2; }
+
+typedef short v4s_t __attribute__((ext_vector_type(4)));
+typedef v4s_t __attribute__((address_space(3))) *lds_v4s_ptr_t;
+typedef int v2i_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ v2i_t lds_read_tr16(unsigned addr) {
+    return __builtin_bit_cast(v2i_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_ptr_t)(size_t)addr));
+}
 
 struct line_pair_t {
     v4i c[2];
@@ -81,9 +109,13 @@ struct line_loader_t {
     static constexpr int EX = (NS * SG + G::NW - 1) / G::NW;    // scale loads per wavefront and step
     static constexpr int LDS_BYTES = L::RING_BYTES + 2 * SCALE_BYTES;
 
+    static constexpr bool AKM = line_form<Mma>::AKM, BKM = line_form<Mma>::BKM;
+    static constexpr int ARB = 2 * BM, BRB = 2 * G::BN; // bytes of a line of 64 k's operand part
+
     unsigned lds0;
     const char *a_tile, *b_tile;
-    int nst, lane;
+    int nst, lane, wave, krows;
+    long lda, ldb;
     unsigned tail_mask;          // all ones if the last step is partial
     unsigned va[2][L::DPA], vb[2][L::DPB], over[2];
     unsigned la[2][L::DPA], lb[2][L::DPB]; // uniform
@@ -92,17 +124,31 @@ struct line_loader_t {
     int sset[EX ? EX : 1], sets;
     unsigned sdst[EX ? EX : 1];
 
-    __device__ __forceinline__ void init(char *smem, const char *a_, const char *b_, long lda, long ldb, long rows_a_left,
+    // row (of 32) that instruction i of this wavefront brings to this lane, lines of RB bytes
+    template <int RB, int D>
+    __device__ __forceinline__ int krow(int i) const {
+        return (wave * D + i) * (1024 / RB) + lane / (RB / 16);
+    }
+    template <int RB, int D>
+    __device__ __forceinline__ unsigned kvoff(int i, long ld, long left) const {
+        const int r = krow<RB, D>(i), chunk = (lane & (RB / 16 - 1)) ^ (kline_swz(r) << 1);
+        return (unsigned)(r * ld + min((long)chunk, left / 8 - 1) * 16); // (columns beyond the last: it again)
+    }
+    __device__ __forceinline__ void init(char *smem, const char *a_, const char *b_, long lda_, long ldb_, long rows_a_left,
             long rows_b_left, long kbytes, const line_scales_t &sc) {
+        lda = lda_;
+        ldb = ldb_;
+        krows = scalar_int((int)(kbytes / 2));
         lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem;
         a_tile = scalar_ptr(a_);
         b_tile = scalar_ptr(b_);
-        const int rem = (int)(kbytes % LKB) / 16; // chunks of a partial last step
+        const int rem = (int)(kbytes % LKB + 15) / 16; // chunks of a partial last step
         nst = scalar_int((int)(kbytes / LKB) + (rem ? 1 : 0));
         tail_mask = (unsigned)scalar_int(rem ? -1 : 0);
         const int t = threadIdx.x;
         lane = t & 63;
-        const int wave = __builtin_amdgcn_readfirstlane(t >> 6), r8 = lane >> 3;
+        wave = __builtin_amdgcn_readfirstlane(t >> 6);
+        const int r8 = lane >> 3;
         // a load is 8 rows: which of the two parities of row block decides the swizzle
 #pragma unroll
         for (int par = 0; par < 2; ++par) {
@@ -115,6 +161,11 @@ struct line_loader_t {
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
             for (int i = 0; i < L::DPA; ++i) {
+                if constexpr (AKM) {
+                    va[h][i] = kvoff<ARB, L::DPA>(i, lda, rows_a_left);
+                    la[h][i] = (unsigned)(h * 32 * ARB + (wave * L::DPA + i) * 1024);
+                    continue;
+                }
                 const int j = wave * L::DPA + i, row0 = (j / 8) * 128 + h * 64 + (j % 8) * 8;
                 const int c = (lane & 7) ^ line_swz(row0 + r8);
                 const long r = min((long)(row0 + r8), rows_a_left - 1);
@@ -123,6 +174,11 @@ struct line_loader_t {
             }
 #pragma unroll
             for (int i = 0; i < L::DPB; ++i) {
+                if constexpr (BKM) {
+                    vb[h][i] = kvoff<BRB, L::DPB>(i, ldb, rows_b_left);
+                    lb[h][i] = (unsigned)(L::B_OFF + h * 32 * BRB + (wave * L::DPB + i) * 1024);
+                    continue;
+                }
                 const int j = wave * L::DPB + i, row0 = (j / BPW) * L::WC + h * (L::WC / 2) + (j % BPW) * 8;
                 const int c = (lane & 7) ^ line_swz(row0 + r8);
                 const long r = min((long)(row0 + r8), rows_b_left - 1);
@@ -149,15 +205,33 @@ struct line_loader_t {
     // again -- one outstanding-load count fits every step -- and a partial last step is taken care of.
     __device__ __forceinline__ int steady() const { return nst - (tail_mask ? 3 : 2); }
     __device__ __forceinline__ int clamp(int s) const { return s < nst ? s : nst - 1; }
+    // instruction i of half h (32 k) of a step's part of an operand whose lines run across K; lines beyond K: the last one
+    template <bool END, int RB, int D>
+    __device__ __forceinline__ void load_k1(const char *tile, long ld, unsigned voff, int h, int i, int sc, unsigned dst) const {
+        if (END) {
+            const int r = krow<RB, D>(i), row = min(h * 32 + r, krows - 1 - sc * 64);
+            dma16(tile + (long)sc * 64 * ld, voff + (unsigned)((row - r) * (int)ld), dst);
+        } else {
+            dma16(tile + ((long)sc * 64 + h * 32) * ld, voff, dst);
+        }
+    }
     template <bool END>
     __device__ __forceinline__ void load_a1(int h, int i, int s, int slot) const {
         const int sc = END ? clamp(s) : s;
+        if constexpr (AKM) {
+            load_k1<END, ARB, L::DPA>(a_tile, lda, va[h][i], h, i, sc, lds0 + slot * L::STAGE_BYTES + la[h][i]);
+            return;
+        }
         const unsigned back = END ? over[block_parity(L::DPA, i)] & (sc == nst - 1 ? tail_mask : 0u) : 0u;
         dma16(a_tile + (long)sc * LKB, va[h][i] - back, lds0 + slot * L::STAGE_BYTES + la[h][i]);
     }
     template <bool END>
     __device__ __forceinline__ void load_b1(int h, int i, int s, int slot) const {
         const int sc = END ? clamp(s) : s;
+        if constexpr (BKM) {
+            load_k1<END, BRB, L::DPB>(b_tile, ldb, vb[h][i], h, i, sc, lds0 + slot * L::STAGE_BYTES + lb[h][i]);
+            return;
+        }
         const unsigned back = END ? over[block_parity(L::DPB, i)] & (sc == nst - 1 ? tail_mask : 0u) : 0u;
         dma16(b_tile + (long)sc * LKB, vb[h][i] - back, lds0 + slot * L::STAGE_BYTES + lb[h][i]);
     }
@@ -199,12 +273,18 @@ struct line_frags_t {
     // LDS addresses of chunk u of fragment 0 by slot (the fragments' offsets ride in the read's offset field, which does
     // not reach from one slot to the other), and of the lane's scale dword
     unsigned ra[2][2], rb[2][2], rs;
-    bool out[2];               // chunk u of this lane lies beyond K in a partial last step
+    int inside[2]; // bytes of this lane's chunk u that lie inside K in a partial last step
+    // the other kind of operand: this lane's address inside a slot, but for the tile (XOR of its 32-byte unit), the lines
+    // of 4 further k and the half
+    unsigned ka, kb, slot0;
 
     __device__ __forceinline__ void init(const Ld &ld, long kbytes) {
         const int t = threadIdx.x, lane = t & 63, r = lane & 15, q = lane >> 4;
         const int wave = __builtin_amdgcn_readfirstlane(t >> 6), wm = G::wm(wave), wn = G::wn(wave);
-        const int rem = (int)(kbytes % LKB) / 16;
+        const int rem = (int)(kbytes % LKB), i4 = (lane & 15) >> 2, g = i4 | (q & 1) << 2;
+        slot0 = ld.lds0;
+        ka = (unsigned)((8 * q + i4) * Ld::ARB + ((wm * 8 ^ g) << 5) + (lane & 3) * 8);
+        kb = (unsigned)((8 * q + i4) * Ld::BRB + ((wn * (L::WC / 16) ^ g) << 5) + (lane & 3) * 8);
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const unsigned c = (unsigned)(((u * 4 + q) ^ line_swz(r)) << 4);
@@ -213,7 +293,7 @@ struct line_frags_t {
                 ra[s][u] = ld.lds0 + s * L::STAGE_BYTES + (wm * 128 + r) * LKB + c;
                 rb[s][u] = ld.lds0 + s * L::STAGE_BYTES + L::B_OFF + (wn * L::WC + r) * LKB + c;
             }
-            out[u] = rem != 0 && u * 4 + q >= rem;
+            inside[u] = min(max(rem - (u * 4 + q) * 16, 0), 16);
         }
         rs = ld.lds0 + L::RING_BYTES + (r * 4 + q) * 4;
         if constexpr (NS == 0) sa[0][0] = sa[1][0] = sb[0] = 0;
@@ -251,11 +331,50 @@ struct line_frags_t {
             for (int u = 0; u < NS; ++u) sb[u] = (int)lds_read4(rs + slot * Ld::SCALE_BYTES + (u * Ld::SG + 4 + wn) * 256);
         }
     }
-    __device__ __forceinline__ static void zero(line_pair_t &f, const bool (&out)[2]) {
+    // (chunks are whole but where K is any number of 16-bit elements)
+    __device__ __forceinline__ void zero1(v4i &c, int u) const {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int e = 0; e < 4; ++e) {
+            const int n = inside[u] - 4 * e;
+            c[e] = n >= 4 ? c[e] : (Ld::AKM && n == 2) ? c[e] & 0xffff : 0;
+        }
+    }
+    __device__ __forceinline__ void zero(line_pair_t &f) const {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) f.c[u][e] = out[u] ? 0 : f.c[u][e];
+        for (int u = 0; u < 2; ++u) zero1(f.c[u], u);
+    }
+    // half t (4 of 8 k) of tile j's fragment for half u of the step, its lines across K
+    __device__ __forceinline__ void read_bk1(int u, int j, int t, int slot) {
+        const v2i_t x = lds_read_tr16(slot0 + slot * L::STAGE_BYTES + L::B_OFF + (kb ^ (unsigned)(j << 5)) + (u * 32 + t * 4) * Ld::BRB);
+        b[j / QC][j % QC].c[u][2 * t] = x[0];
+        b[j / QC][j % QC].c[u][2 * t + 1] = x[1];
+    }
+    __device__ __forceinline__ void read_ak1(int u, int h, int i, int t, int slot) {
+        const v2i_t x = lds_read_tr16(slot0 + slot * L::STAGE_BYTES + (ka ^ (unsigned)((h * 4 + i) << 5)) + (u * 32 + t * 4) * Ld::ARB);
+        a[h][i].c[u][2 * t] = x[0];
+        a[h][i].c[u][2 * t + 1] = x[1];
+    }
+    __device__ __forceinline__ void read_bk(int u, int slot) {
+#pragma unroll
+        for (int j = 0; j < 2 * QC; ++j)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) read_bk1(u, j, t, slot);
+    }
+    __device__ __forceinline__ void read_ak(int u, int h, int slot) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) read_ak1(u, h, i, t, slot);
+    }
+    __device__ __forceinline__ void ready_bk(int u, bool partial) {
+        if (!partial) return;
+#pragma unroll
+        for (int j = 0; j < 2 * QC; ++j) zero1(b[j / QC][j % QC].c[u], u);
+    }
+    __device__ __forceinline__ void ready_ak(int u, int h, bool partial) {
+        if (!partial) return;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) zero1(a[h][i].c[u], u);
     }
     // what fragments need between their read and their first product
     __device__ __forceinline__ void ready_a(int h, bool partial) {
@@ -263,7 +382,7 @@ struct line_frags_t {
         for (int i = 0; i < 4; ++i) Mma::prepare_a(a[h][i]);
         if (partial) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) zero(a[h][i], out);
+            for (int i = 0; i < 4; ++i) zero(a[h][i]);
         }
     }
     __device__ __forceinline__ void ready_b(int g, bool partial) {
@@ -271,7 +390,7 @@ struct line_frags_t {
         for (int j = 0; j < QC; ++j) Mma::prepare_b(b[g][j]);
         if (partial) {
 #pragma unroll
-            for (int j = 0; j < QC; ++j) zero(b[g][j], out);
+            for (int j = 0; j < QC; ++j) zero(b[g][j]);
         }
     }
 };
@@ -330,6 +449,29 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
     };
     constexpr std::integral_constant<int, 0> c0 {};
     constexpr std::integral_constant<int, 1> c1 {};
+    // Operands with their lines across K (B, or both): a quadrant is a half of the rows and a half of the 64 k, and what a
+    // phase reads follows: B half 0 and A half 0 | B half 1 | A half 1 | -  becomes, with k halves,
+    //   B only   B k 0 and A rows 0 | B k 1 | A rows 1 | -
+    //   both     B k 0 and A k 0, rows 0 | A k 0, rows 1 | B k 1 and A k 1, rows 0 | A k 1, rows 1
+    // The schedule of the loads, and with it the counts, are the same.
+    constexpr bool AKM = Ld::AKM, BKM = Ld::BKM;
+    static_assert(BKM || !AKM, "src across K comes with weights across K");
+    auto quadrant_k = [&](auto H, auto U) __attribute__((always_inline)) {
+        constexpr int h = decltype(H)::value, u = decltype(U)::value;
+        __builtin_amdgcn_s_setprio(1);
+        static_for<4>([&](auto I) __attribute__((always_inline)) {
+            static_for<2 * QC>([&](auto J) __attribute__((always_inline)) {
+                constexpr int i = decltype(I)::value, j = decltype(J)::value;
+                Mma::template mma<j, i>(acc[h * 4 + i][j], f.b[j / QC][j % QC], f.a[h][i], std::integral_constant<int, u>(), 0, 0);
+            });
+        });
+        __builtin_amdgcn_s_setprio(0);
+    };
+    auto products = [&](auto First, auto Second) __attribute__((always_inline)) {
+        if constexpr (AKM) quadrant_k(Second, First);
+        else if constexpr (BKM) quadrant_k(First, Second);
+        else quadrant(First, Second);
+    };
 
     ld.template load_scales<true>(0, 0);
     ld.template load_b<true>(0, 0, 0);
@@ -349,38 +491,63 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
         constexpr bool END = decltype(End)::value;
         const bool partial = END && ld.tail_mask != 0 && s == ld.nst - 1;
         f.read_sb(slot);
-        f.read_b(0, slot);
+        if constexpr (BKM) f.read_bk(0, slot);
+        else f.read_b(0, slot);
         f.read_sa(0, slot);
         f.read_sa(1, slot);
-        f.read_a(0, slot);
+        if constexpr (AKM) f.read_ak(0, 0, slot);
+        else f.read_a(0, slot);
         ld.template load_a<END>(1, s + 1, slot ^ 1);
         wait_vmcnt<STEP + DA>(); // after B 1 of s: A 1, then all of s + 1
         wait_lds_reads();
-        f.ready_b(0, partial);
-        f.ready_a(0, partial);
+        if constexpr (BKM) f.ready_bk(0, partial);
+        else f.ready_b(0, partial);
+        if constexpr (AKM) f.ready_ak(0, 0, partial);
+        else f.ready_a(0, partial);
         phase_barrier();
-        quadrant(c0, c0);
+        products(c0, c0);
         phase_barrier();
-        f.read_b(1, slot);
+        if constexpr (AKM) f.read_ak(0, 1, slot);
+        else if constexpr (BKM) f.read_bk(1, slot);
+        else f.read_b(1, slot);
         ld.template load_b<END>(0, s + 2, slot);
         ld.template load_scales<END>(s + 2, slot);
         wait_vmcnt<STEP + DB + EX>(); // after A 1 of s: all of s + 1, B 0 and scales of s + 2
         wait_lds_reads();
-        f.ready_b(1, partial);
+        if constexpr (AKM) f.ready_ak(0, 1, partial);
+        else if constexpr (BKM) f.ready_bk(1, partial);
+        else f.ready_b(1, partial);
         phase_barrier();
-        quadrant(c0, c1);
+        products(c0, c1);
         phase_barrier();
-        f.read_a(1, slot);
+        if constexpr (AKM) {
+            f.read_bk(1, slot);
+            f.read_ak(1, 0, slot);
+        } else {
+            f.read_a(1, slot);
+        }
         ld.template load_a<END>(0, s + 2, slot);
         wait_lds_reads();
-        f.ready_a(1, partial);
+        if constexpr (AKM) {
+            f.ready_bk(1, partial);
+            f.ready_ak(1, 0, partial);
+        } else {
+            f.ready_a(1, partial);
+        }
         phase_barrier();
-        quadrant(c1, c1);
+        if constexpr (BKM) products(c1, c0);
+        else products(c1, c1);
         phase_barrier();
+        if constexpr (AKM) f.read_ak(1, 1, slot);
         ld.template load_b<END>(1, s + 2, slot);
         wait_vmcnt<STEP + DB>(); // after A 0 of s + 1: B 1 and A 1 of s + 1, s + 2 without its A 1
+        if constexpr (AKM) {
+            wait_lds_reads();
+            f.ready_ak(1, 1, partial);
+        }
         phase_barrier();
-        quadrant(c1, c0);
+        if constexpr (BKM) products(c1, c1); // (every sum takes its k in the order that copied operands give)
+        else products(c1, c0);
         phase_barrier();
     };
     int s = 0;
@@ -404,11 +571,10 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
 // tile (bf16 2048 x 4096 x 14336, 256 tiles: 168 us; the same tile on eight wavefronts of 128 x 32, which read 1.7
 // times as much from LDS, 212 us; the 64-byte steps that this loop took the place of 247).
 //
-// A step s is two halves, x and y the column halves with y = s % 2 (so that a step begins with the columns that the
-// step before released first):
-//          products              reads                                 loads
-//   X(s)   (A 0, B y) (A 0, B x)   B x, A 1 of step s                  B y, A 0 of step s + 2
-//   Y(s)   (A 1, B x) (A 1, B y)   A 0 of s + 1, B of s + 1's y (= x)  B x, A 1 of step s + 2
+// A step s is two halves:
+//          products              reads                     loads
+//   X(s)   (A 0, B 0) (A 0, B 1)   B 1, A 1 of step s        B 0, A 0 of step s + 2
+//   Y(s)   (A 1, B 0) (A 1, B 1)   A 0, B 0 of step s + 1    B 1, A 1 of step s + 2
 // with one barrier before each: every read of the half before is back, so what it read may be loaded again, and what
 // this one reads landed (loads of four parts have been issued after it).
 //
@@ -422,7 +588,8 @@ __device__ __forceinline__ void main_loop_lines4(Acc &acc, char *smem, const cha
         long ldb, long rows_a_left, long rows_b_left, long kbytes, Fill &&fill) {
     using Ld = line_loader_t<Mma>;
     using Fr = line_frags_t<Mma>;
-    static_assert(Mma::G::NW == 4 && Mma::SCALE_SETS == 0, "four wavefronts, no block scales");
+    constexpr bool BKM = Ld::BKM; // weights across K: a column half is a half of the 64 k instead
+    static_assert(Mma::G::NW == 4 && Mma::SCALE_SETS == 0 && !Ld::AKM, "four wavefronts, no block scales");
     constexpr int DA = Ld::L::DPA, DB = Ld::L::DPB, QC = Fr::QC, NU = Mma::NU;
     Ld ld;
     ld.init(smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, line_scales_t {});
@@ -433,15 +600,16 @@ __device__ __forceinline__ void main_loop_lines4(Acc &acc, char *smem, const cha
     ld.template load_b<true>(0, 0, 0);
     ld.template load_b<true>(1, 0, 0);
     ld.template load_a<true>(1, 0, 0);
-    ld.template load_b<true>(1, 1, 1);
-    ld.template load_a<true>(0, 1, 1);
     ld.template load_b<true>(0, 1, 1);
+    ld.template load_a<true>(0, 1, 1);
+    ld.template load_b<true>(1, 1, 1);
     ld.template load_a<true>(1, 1, 1);
     fill();
     wait_vmcnt<3 * (DA + DB)>();
     phase_barrier();
     f.read_a(0, 0);
-    f.read_b(0, 0);
+    if constexpr (BKM) f.read_bk(0, 0);
+    else f.read_b(0, 0);
 
     // two wait states behind everything that ready_a / ready_b compute (the scheduler would sink it to its use)
     auto settle = []() __attribute__((always_inline)) {
@@ -449,79 +617,76 @@ __device__ __forceinline__ void main_loop_lines4(Acc &acc, char *smem, const cha
         asm volatile("s_nop 1");
         __builtin_amdgcn_sched_barrier(0);
     };
-    // FIRST: X, otherwise Y; G0: the column half of the first quadrant; slot of step s
-    auto half = [&](auto End, auto First, auto G0, int s, int slot) __attribute__((always_inline)) {
+    // First: X, otherwise Y; slot of step s
+    auto half = [&](auto End, auto First, int s, int slot) __attribute__((always_inline)) {
         constexpr bool END = decltype(End)::value, first = decltype(First)::value;
-        constexpr int g0 = decltype(G0)::value, h = first ? 0 : 1;
-        constexpr int rb = first ? 1 - g0 : g0, ra = first ? 1 : 0; // halves that are read ...
-        constexpr int lb = g0, la = first ? 0 : 1;                  // ... and loaded
+        constexpr int h = first ? 0 : 1, read_half = 1 - h, load_half = h;
         const int rslot = first ? slot : slot ^ 1;
         const bool partial = END && ld.tail_mask != 0 && s == ld.nst - 1;
         wait_vmcnt<2 * (DA + DB)>();
         wait_lds_reads();
         phase_barrier();
         f.ready_a(h, partial);
-        if (first) f.ready_b(g0, partial);
+        auto ready_cols = [&](int g) __attribute__((always_inline)) {
+            if constexpr (BKM) f.ready_bk(g, partial);
+            else f.ready_b(g, partial);
+        };
+        if (first) ready_cols(0);
         settle();
-        constexpr int NB = 2 * QC, NR = NB + 8, NM = 4 * QC * NU, ND = DA + DB;
+        constexpr int NB = BKM ? 4 * QC : 2 * QC, NR = NB + 8, NM = BKM ? 8 * QC : 4 * QC * NU, ND = DA + DB;
         constexpr int PER = NM >= 16 ? 1 : 2; // reads ahead of an MFMA
         int n = 0, read = 0, loaded = 0;
 #pragma unroll
         for (int qd = 0; qd < 2; ++qd) {
-            const int g = qd ? 1 - g0 : g0;
             if (first && qd == 1) {
-                f.ready_b(1 - g0, partial);
+                ready_cols(1);
                 settle();
             }
 #pragma unroll
-            for (int u = 0; u < NU; ++u)
+            for (int u = 0; u < (BKM ? 1 : NU); ++u)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int j = 0; j < QC; ++j) {
+                    for (int j = 0; j < (BKM ? 2 * QC : QC); ++j) {
 #pragma unroll
                         for (int p = 0; p < PER; ++p) {
-                            // X: the columns first, its second quadrant wants them; Y: they replace those of its first
+                            // X: the columns first, its second quadrant wants them; Y: they replace its first quadrant's
                             const bool cols = first ? read < NB : read >= 8;
                             if (read < NR && (first || !cols || qd == 1)) {
                                 const int e = first ? (cols ? read : read - NB) : (cols ? read - 8 : read);
-                                if (cols) f.read_b1(rb, e / 2, e % 2, rslot);
-                                else f.read_a1(ra, e / 2, e % 2, rslot);
+                                if (!cols) f.read_a1(read_half, e / 2, e % 2, rslot);
+                                else if (BKM) f.read_bk1(read_half, e / 2, e % 2, rslot);
+                                else f.read_b1(read_half, e / 2, e % 2, rslot);
                                 ++read;
                             }
                         }
                         if (loaded < ND && n == (2 * loaded + 1) * NM / ND) {
-                            if (loaded < DB) ld.template load_b1<END>(lb, loaded, s + 2, slot);
-                            else ld.template load_a1<END>(la, loaded - DB, s + 2, slot);
+                            if (loaded < DB) ld.template load_b1<END>(load_half, loaded, s + 2, slot);
+                            else ld.template load_a1<END>(load_half, loaded - DB, s + 2, slot);
                             ++loaded;
                         }
-                        Mma::mma_tied(acc[h * 4 + i][g * QC + j], f.b[g][j], f.a[h][i], u);
+                        if (BKM) Mma::mma_tied(acc[h * 4 + i][j], f.b[j / QC][j % QC], f.a[h][i], qd);
+                        else Mma::mma_tied(acc[h * 4 + i][BKM ? j : qd * QC + j], f.b[qd][BKM ? 0 : j], f.a[h][i], u);
                         __builtin_amdgcn_sched_barrier(0); // keeps the reads and loads spread between the MFMAs
                         ++n;
                     }
         }
     };
-    constexpr std::integral_constant<int, 0> c0 {};
-    constexpr std::integral_constant<int, 1> c1 {};
-    auto even = [&](auto End, int s) __attribute__((always_inline)) {
-        half(End, std::true_type {}, c0, s, 0);
-        half(End, std::false_type {}, c1, s, 0);
-    };
-    auto odd = [&](auto End, int s) __attribute__((always_inline)) {
-        half(End, std::true_type {}, c1, s, 1);
-        half(End, std::false_type {}, c0, s, 1);
+    auto step = [&](auto End, int s, int slot) __attribute__((always_inline)) {
+        half(End, std::true_type {}, s, slot);
+        half(End, std::false_type {}, s, slot);
     };
     int s = 0;
     const int steady = ld.steady();
 #pragma nounroll
     for (; s + 1 < steady; s += 2) {
-        even(std::false_type {}, s);
-        odd(std::false_type {}, s + 1);
+        step(std::false_type {}, s, 0);
+        step(std::false_type {}, s + 1, 1);
     }
 #pragma nounroll
     for (; s < ld.nst; s += 2) {
-        even(std::true_type {}, s);
-        if (s + 1 < ld.nst) odd(std::true_type {}, s + 1);
+        step(std::true_type {}, s, 0);
+        if (s + 1 < ld.nst) step(std::true_type {}, s + 1, 1);
     }
     // every load has landed and every read is back before the ring's memory is used for something else; the wait
     // states between the last MFMA and the first read of its result

@@ -51,6 +51,12 @@ struct h16x16_mma_t {
     }
 };
 
+// the same with the weights (ACROSS = 1), or src and the weights (2), contiguous across K
+template <bool BF16, class G_, int ACROSS>
+struct h16_across_mma_t : h16x16_mma_t<BF16, G_> {
+    static constexpr bool A_KM = ACROSS == 2, B_KM = true;
+};
+
 // int8 on v_mfma_i32_16x16x64_i8 (sustains ~4.0 POPS on this hardware, the 32 x 32 x 32 shape ~3.0).  u8 operands are
 // re-biased to s8 in registers; bytes beyond K are zeroed after that.
 template <bool SRC_U8, bool WEI_U8, class G_>

@@ -112,3 +112,38 @@ def test_a_staged_tensor_at_ragged_edges(gpu, oracle, act, alg, dt):
         return
     g, w = (dtp.bf16_to_f32(np.asarray(x).view(np.uint16).reshape(-1)) for x in (got, want))
     assert np.all(np.abs(g - w) <= 2.0 ** -7 * np.abs(w) + 2.0 ** -20)
+
+
+def across_problem(M, N, K, dt, ddt, src_across, *, batch=1, wei_pad=0, src_pad=0, bias=True):
+    """weights row-major ([K][N], a pitch of N + wei_pad), src row-major or ([K][M], a pitch of M + src_pad)"""
+    r = np.random.default_rng(M * 3 + N * 5 + K)
+    sv = r.integers(-3, 4, size=(batch, M, K)).astype(np.float32)
+    wv = np.full((batch, K, N + wei_pad), 99, np.float32)
+    wv[:, :, :N] = r.integers(-2, 3, size=(batch, K, N))
+    ss = (M * K, K, 1)
+    if src_across:
+        full = np.full((batch, K, M + src_pad), 77, np.float32)
+        full[:, :, :M] = sv.transpose(0, 2, 1)
+        sv, ss = full, (K * (M + src_pad), 1, M + src_pad)
+    b = (r.integers(-8, 9, size=N) / 4).astype(np.float32) if bias else None
+    return MatmulProblem(M=M, N=N, K=K, batch=batch, src_dt=DT[dt], wei_dt=DT[dt], dst_dt=DT[ddt], src=encode(sv, dt),
+                         wei=encode(wv, dt), src_stride=ss, wei_stride=(K * (N + wei_pad), N + wei_pad, 1),
+                         bias_dt=cabi.DT_F32 if bias else cabi.DT_UNDEF, bias=b, name=f"across-{dt}-{ddt}-{M}x{N}x{K}")
+
+
+# operands that are contiguous across K: every place where a step, a half of its 64 k or a 32-byte unit of a line can end
+@pytest.mark.parametrize("K", [8, 24, 32, 56, 64, 72, 96, 104, 128, 160, 192, 200, 320])
+@pytest.mark.parametrize("dt,ddt", [("bf16", "bf16"), ("f16", "f16"), ("bf16", "f32")])
+@pytest.mark.parametrize("tiles", [None, "wide"])
+@pytest.mark.parametrize("src_across", [False, True])
+def test_operands_contiguous_across_k(gpu, oracle, K, dt, ddt, tiles, src_across):
+    check(oracle, across_problem(304, 328, K, dt, ddt, src_across), dt, tiles)
+
+
+# both across K: any K; row pitches beyond the rows; ragged edges in steps of eight; what is not whole 16-byte pieces is
+# copied as before
+@pytest.mark.parametrize("M,N,K,pads", [(264, 264, 1, (0, 0)), (512, 136, 63, (8, 16)), (520, 392, 65, (0, 8)), (8, 264, 127, (16, 0)),
+                                        (296, 520, 193, (0, 0)), (300, 328, 70, (0, 0)), (304, 330, 70, (0, 0)), (304, 328, 70, (3, 5))])
+def test_both_across_k_ragged(gpu, oracle, M, N, K, pads):
+    for tiles in (None, "wide"):
+        check(oracle, across_problem(M, N, K, "bf16", "bf16", True, batch=2, src_pad=pads[0], wei_pad=pads[1]), "bf16", tiles)
