@@ -5,12 +5,16 @@
 
 namespace mi355 {
 
-int chain_launch_mx(bool fp4, int dst_dt, chain_t &C, unsigned batch, hipStream_t stream) {
+int chain_launch_mx(bool fp4, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream) {
     using wide_t = geo_t<8, 256>;
+    using narrow_t = geo_t<4, 128>;
     auto go = [&](auto dst) -> int {
         constexpr int D = decltype(dst)::value;
-        return fp4 ? chain_go<mxf4_mma_t<wide_t>, D>(C, batch, stream, "mfma_mxf4")
-                   : chain_go<mxf8_mma_t<0, 0, wide_t>, D>(C, batch, stream, "mfma_f8");
+        if (fp4)
+            return wide ? chain_go<mxf4_mma_t<wide_t>, D>(C, batch, stream, "mfma_mxf4")
+                        : chain_go<mxf4_mma_t<narrow_t>, D>(C, batch, stream, "mfma_mxf4");
+        return wide ? chain_go<mxf8_mma_t<0, 0, wide_t>, D>(C, batch, stream, "mfma_f8")
+                    : chain_go<mxf8_mma_t<0, 0, narrow_t>, D>(C, batch, stream, "mfma_f8");
     };
     if (dst_dt == MI355_DT_BF16) return go(std::integral_constant<int, CHAIN_BF16> {});
     if (dst_dt == MI355_DT_F32) return go(std::integral_constant<int, CHAIN_F32> {});

@@ -120,18 +120,18 @@ int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, h
     }
     // (MI355_F8_TILES: wide / narrow keep one geometry whatever the size: tests, tuning)
     const int force = tuning(TUNE_F8_TILES);
-    const bool narrow = !plan.mx && (force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N) && force != TUNE_WIDE));
+    const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N) && force != TUNE_WIDE);
     chain_t C {};
     if (!fa && !fb && chain_from_mx(P, plan.mx, C)) {
         C.a = (const char *)P.src; C.lda = P.ss[1]; C.a_bs = P.ss[0];
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K;
         C.sc = X.sc;
-        const int st = plan.mx ? chain_launch_mx(false, P.dst_dt, C, (unsigned)d.batch, stream)
+        const int st = plan.mx ? chain_launch_mx(false, P.dst_dt, C, (unsigned)d.batch, !narrow, stream)
                                : chain_launch_f8(P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }
-    if (narrow) return f8_launch_narrow(fa, fb, P, X.bt, X.ldb, X.bt_bstride, (unsigned)d.batch, stream);
+    if (narrow && !plan.mx) return f8_launch_narrow(fa, fb, P, X.bt, X.ldb, X.bt_bstride, (unsigned)d.batch, stream);
     X.tiles_m = (int)((d.M + BM - 1) / BM);
     X.tiles_n = (int)((d.N + f8_geo_t::BN - 1) / f8_geo_t::BN);
     const dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);

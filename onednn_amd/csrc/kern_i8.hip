@@ -335,25 +335,17 @@ i8_plan_t make_plan(const mi355_matmul_desc_t &d) {
     // steps of three a CU.  Counted in small tiles and not in large ones, because a
     // short M fills few rows of a large tile.  K = 1024 / 4096 / 16384, small against
     // LDS tiles: with zero points, whose sums are kernels of their own in front of the
-    // latter (256 x 3840, f32 dst), 17.4 / 36.4 / 119 us against 31 / 57 / 155; without
-    // (bf16 dst, K = 8192 / 16384) 63 / 119 against 71 / 120 for 256 x 3712, 64 / 125 against
-    // 69 / 118 for 128 x 8064: the line is lower for the longest K.  So it is where the
-    // LDS tiles have the 8-bit dst's own store (i8_conv_t::hot_chain) and whole columns,
-    // 13.5 / 28.7 / 91 us against 16.3 / 34.4 / 110 on 768 tiles (256 x 3072), but 18.0 /
-    // 35.9 / 119 against 16.3 / 34.5 / 111 on 800; with K = 256 10.3 against 9.9 on
-    // 384 (32 x 12288), 12.6 against 10.1 on 640.  Of fewer rows than
-    // 32 a small tile loads the last one again and again: 16 x 29696 x 1024, 928 tiles, still
-    // takes 14.5 us against 16, but with K = 256 13.1 against 10.5; 22 x 28672, K = 1024 /
-    // 2048 / 14336 17.6 / 23.9 / 126 against 15.3 / 23.3 / 138.
+    // latter (f32 dst), 13 / 29 / 90 us against 22 / 37 / 103 on 768 tiles, 18 / 37 / 118
+    // against 22 / 37 / 106 on 1024; without and with a chain of chain_gemm.hpp (bf16 dst),
+    // 10.6 / 21 / 63 against 14 / 25 / 72 on 512, 13.0 / 28.7 / 90 against 14.1 / 25.3 / 73
+    // on 768, 18 / 37 / 119 against 14 / 26 / 74 on 1024; K = 512 10.3 against 12.0 on 512
+    // and 12.7 against 12.1 on 768.
     const long small_tiles = ((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch;
     const bool sums = d.src_dt == MI355_DT_U8 || d.wei_dt == MI355_DT_U8 || !quant_absent(d.src_zp) || !quant_absent(d.wei_zp);
-    const bool plain_chain = d.n_post_ops == 0
-            || (d.n_post_ops == 1 && d.post_ops[0].kind == MI355_PO_ELTWISE && d.post_ops[0].alg == MI355_ELTWISE_RELU);
-    const bool own_store = !quant_absent(d.src_scale) && !quant_absent(d.wei_scale) && quant_absent(d.dst_zp)
-            && d.bias_dt == MI355_DT_UNDEF && plain_chain && is_int8_dt(d.dst_dt);
-    const bool three_a_cu = !sums && d.N % 128 == 0 && (own_store || d.K > 8192)
-            && (d.M >= 32 || d.K < (d.M > 16 ? 2048 : 1024));
-    const long crossover = !three_a_cu ? 1024 : d.K < 1024 ? 257 + d.K / 2 : 769;
+    const bool chain = (is_int8_dt(d.dst_dt) || d.dst_dt == MI355_DT_BF16 || d.dst_dt == MI355_DT_F32) && quant_absent(d.dst_zp)
+            && (d.n_post_ops == 0
+                    || (d.n_post_ops == 1 && d.post_ops[0].kind == MI355_PO_ELTWISE && d.post_ops[0].alg == MI355_ELTWISE_RELU));
+    const long crossover = sums ? (d.K > 8192 ? 769 : 1024) : !chain ? 1024 : d.K < 1024 ? 257 + d.K / 2 : d.K < 2048 ? 769 : 513;
     p.small = !d.dst_scale_dynamic && small_tiles < crossover;
     // the MI355_I8_TILES switch overrides the choice where both can run (tests and
     // tuning): large = the LDS tiles, 256 x 128 or 256 x 256 by the number of

@@ -275,7 +275,10 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K / 2;
         C.sc = X.sc;
-        const int st = chain_launch_mx(true, P.dst_dt, C, (unsigned)d.batch, stream);
+        // (MI355_F8_TILES keeps one geometry here as well)
+        const int force = tuning(TUNE_F8_TILES);
+        const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N) && force != TUNE_WIDE);
+        const int st = chain_launch_mx(true, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }
     X.tiles_m = (int)((d.M + BM - 1) / BM);

@@ -269,7 +269,7 @@ struct line_frags_t {
     using Ld = line_loader_t<Mma>;
     static constexpr int QC = L::QC, NS = Ld::NS;
     line_pair_t a[2][4], b[2][QC];
-    int sa[2][NS ? NS : 1], sb[NS ? NS : 1];
+    int sa[2][NS ? NS : 1], sb[2][NS ? NS : 1]; // sb: of this step and, read ahead, of the next
     // LDS addresses of chunk u of fragment 0 by slot (the fragments' offsets ride in the read's offset field, which does
     // not reach from one slot to the other), and of the lane's scale dword
     unsigned ra[2][2], rb[2][2], rs;
@@ -296,7 +296,7 @@ struct line_frags_t {
             inside[u] = min(max(rem - (u * 4 + q) * 16, 0), 16);
         }
         rs = ld.lds0 + L::RING_BYTES + (r * 4 + q) * 4;
-        if constexpr (NS == 0) sa[0][0] = sa[1][0] = sb[0] = 0;
+        if constexpr (NS == 0) sa[0][0] = sa[1][0] = sb[0][0] = sb[1][0] = 0;
     }
     __device__ __forceinline__ void read_a1(int h, int i, int u, int slot) {
         a[h][i].c[u] = lds_read16((slot ? ra[1][u] : ra[0][u]) + h * (64 * LKB) + i * (16 * LKB));
@@ -323,12 +323,12 @@ struct line_frags_t {
             for (int u = 0; u < NS; ++u) sa[h][u] = (int)lds_read4(rs + slot * Ld::SCALE_BYTES + (u * Ld::SG + wm * 2 + h) * 256);
         }
     }
-    __device__ __forceinline__ void read_sb(int slot) {
+    __device__ __forceinline__ void read_sb(int at, int slot) {
         if constexpr (NS > 0) {
             const int wn = G::wn(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
             static_assert(L::WC == 64 || NS == 0, "a group of 64 columns a wavefront");
 #pragma unroll
-            for (int u = 0; u < NS; ++u) sb[u] = (int)lds_read4(rs + slot * Ld::SCALE_BYTES + (u * Ld::SG + 4 + wn) * 256);
+            for (int u = 0; u < NS; ++u) sb[at][u] = (int)lds_read4(rs + slot * Ld::SCALE_BYTES + (u * Ld::SG + 4 + wn) * 256);
         }
     }
     // (chunks are whole but where K is any number of 16-bit elements)
@@ -441,7 +441,7 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
                 static_for<QC>([&](auto J) __attribute__((always_inline)) {
                     constexpr int u = decltype(U)::value, i = decltype(I)::value, j = decltype(J)::value;
                     Mma::template mma<g * QC + j, i>(acc[h * 4 + i][g * QC + j], f.b[g][j], f.a[h][i], U,
-                            f.sb[Fr::NS ? u : 0], f.sa[h][Fr::NS ? u : 0]);
+                            f.sb[0][Fr::NS ? u : 0], f.sa[h][Fr::NS ? u : 0]);
                 });
             });
         });
@@ -490,7 +490,7 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
     auto step = [&](auto End, int s, int slot) __attribute__((always_inline)) {
         constexpr bool END = decltype(End)::value;
         const bool partial = END && ld.tail_mask != 0 && s == ld.nst - 1;
-        f.read_sb(slot);
+        f.read_sb(0, slot);
         if constexpr (BKM) f.read_bk(0, slot);
         else f.read_b(0, slot);
         f.read_sa(0, slot);
@@ -574,7 +574,7 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
 // A step s is two halves:
 //          products              reads                     loads
 //   X(s)   (A 0, B 0) (A 0, B 1)   B 1, A 1 of step s        B 0, A 0 of step s + 2
-//   Y(s)   (A 1, B 0) (A 1, B 1)   A 0, B 0 of step s + 1    B 1, A 1 of step s + 2
+//   Y(s)   (A 1, B 0) (A 1, B 1)   A 0, B 0 of step s + 1    scales, B 1, A 1 of step s + 2
 // with one barrier before each: every read of the half before is back, so what it read may be loaded again, and what
 // this one reads landed (loads of four parts have been issued after it).
 //
@@ -585,28 +585,32 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
 // states before an MFMA reads it, which the compiler cannot place either (s_nop below).
 template <class Mma, class Acc, class Fill>
 __device__ __forceinline__ void main_loop_lines4(Acc &acc, char *smem, const char *a_tile, const char *b_tile, long lda,
-        long ldb, long rows_a_left, long rows_b_left, long kbytes, Fill &&fill) {
+        long ldb, long rows_a_left, long rows_b_left, long kbytes, const line_scales_t &sc, Fill &&fill) {
     using Ld = line_loader_t<Mma>;
     using Fr = line_frags_t<Mma>;
     constexpr bool BKM = Ld::BKM; // weights across K: a column half is a half of the 64 k instead
-    static_assert(Mma::G::NW == 4 && Mma::SCALE_SETS == 0 && !Ld::AKM, "four wavefronts, no block scales");
-    constexpr int DA = Ld::L::DPA, DB = Ld::L::DPB, QC = Fr::QC, NU = Mma::NU;
+    static_assert(Mma::G::NW == 4 && !Ld::AKM, "four wavefronts");
+    constexpr int DA = Ld::L::DPA, DB = Ld::L::DPB, EX = Ld::EX, QC = Fr::QC, NU = Mma::NU, NS = Fr::NS;
     Ld ld;
-    ld.init(smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, line_scales_t {});
+    ld.init(smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, sc);
     Fr f;
     f.init(ld, kbytes);
 
     ld.template load_a<true>(0, 0, 0);
     ld.template load_b<true>(0, 0, 0);
+    ld.template load_scales<true>(0, 0);
     ld.template load_b<true>(1, 0, 0);
     ld.template load_a<true>(1, 0, 0);
     ld.template load_b<true>(0, 1, 1);
     ld.template load_a<true>(0, 1, 1);
+    ld.template load_scales<true>(1, 1);
     ld.template load_b<true>(1, 1, 1);
     ld.template load_a<true>(1, 1, 1);
     fill();
-    wait_vmcnt<3 * (DA + DB)>();
+    wait_vmcnt<3 * (DA + DB) + EX>();
     phase_barrier();
+    f.read_sb(0, 0);
+    f.read_sa(0, 0);
     f.read_a(0, 0);
     if constexpr (BKM) f.read_bk(0, 0);
     else f.read_b(0, 0);
@@ -623,9 +627,16 @@ __device__ __forceinline__ void main_loop_lines4(Acc &acc, char *smem, const cha
         constexpr int h = first ? 0 : 1, read_half = 1 - h, load_half = h;
         const int rslot = first ? slot : slot ^ 1;
         const bool partial = END && ld.tail_mask != 0 && s == ld.nst - 1;
-        wait_vmcnt<2 * (DA + DB)>();
+        wait_vmcnt<2 * (DA + DB) + (first ? EX : 0)>(); // (the scales go in front of Y's loads)
         wait_lds_reads();
         phase_barrier();
+        if (first) {
+            f.read_sa(1, slot);
+        } else {
+            f.read_sa(0, slot ^ 1);
+            f.read_sb(slot ^ 1, slot ^ 1);
+            ld.template load_scales<END>(s + 2, slot);
+        }
         f.ready_a(h, partial);
         auto ready_cols = [&](int g) __attribute__((always_inline)) {
             if constexpr (BKM) f.ready_bk(g, partial);
@@ -636,41 +647,42 @@ __device__ __forceinline__ void main_loop_lines4(Acc &acc, char *smem, const cha
         constexpr int NB = BKM ? 4 * QC : 2 * QC, NR = NB + 8, NM = BKM ? 8 * QC : 4 * QC * NU, ND = DA + DB;
         constexpr int PER = NM >= 16 ? 1 : 2; // reads ahead of an MFMA
         int n = 0, read = 0, loaded = 0;
-#pragma unroll
-        for (int qd = 0; qd < 2; ++qd) {
+        static_for<2>([&](auto Qd) __attribute__((always_inline)) {
+            constexpr int qd = decltype(Qd)::value;
             if (first && qd == 1) {
                 ready_cols(1);
                 settle();
             }
+            static_for<BKM ? 1 : NU>([&](auto U) __attribute__((always_inline)) {
+            static_for<4>([&](auto I) __attribute__((always_inline)) {
+            static_for<BKM ? 2 * QC : QC>([&](auto J) __attribute__((always_inline)) {
+                constexpr int u = BKM ? qd : decltype(U)::value, i = decltype(I)::value;
+                constexpr int j = BKM ? decltype(J)::value : qd * QC + decltype(J)::value; // column tile
 #pragma unroll
-            for (int u = 0; u < (BKM ? 1 : NU); ++u)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < (BKM ? 2 * QC : QC); ++j) {
-#pragma unroll
-                        for (int p = 0; p < PER; ++p) {
-                            // X: the columns first, its second quadrant wants them; Y: they replace its first quadrant's
-                            const bool cols = first ? read < NB : read >= 8;
-                            if (read < NR && (first || !cols || qd == 1)) {
-                                const int e = first ? (cols ? read : read - NB) : (cols ? read - 8 : read);
-                                if (!cols) f.read_a1(read_half, e / 2, e % 2, rslot);
-                                else if (BKM) f.read_bk1(read_half, e / 2, e % 2, rslot);
-                                else f.read_b1(read_half, e / 2, e % 2, rslot);
-                                ++read;
-                            }
-                        }
-                        if (loaded < ND && n == (2 * loaded + 1) * NM / ND) {
-                            if (loaded < DB) ld.template load_b1<END>(load_half, loaded, s + 2, slot);
-                            else ld.template load_a1<END>(load_half, loaded - DB, s + 2, slot);
-                            ++loaded;
-                        }
-                        if (BKM) Mma::mma_tied(acc[h * 4 + i][j], f.b[j / QC][j % QC], f.a[h][i], qd);
-                        else Mma::mma_tied(acc[h * 4 + i][BKM ? j : qd * QC + j], f.b[qd][BKM ? 0 : j], f.a[h][i], u);
-                        __builtin_amdgcn_sched_barrier(0); // keeps the reads and loads spread between the MFMAs
-                        ++n;
+                for (int p = 0; p < PER; ++p) {
+                    // X: the columns first, its second quadrant wants them; Y: they replace its first quadrant's
+                    const bool cols = first ? read < NB : read >= 8;
+                    if (read < NR && (first || !cols || qd == 1)) {
+                        const int e = first ? (cols ? read : read - NB) : (cols ? read - 8 : read);
+                        if (!cols) f.read_a1(read_half, e / 2, e % 2, rslot);
+                        else if (BKM) f.read_bk1(read_half, e / 2, e % 2, rslot);
+                        else f.read_b1(read_half, e / 2, e % 2, rslot);
+                        ++read;
                     }
-        }
+                }
+                if (loaded < ND && n == (2 * loaded + 1) * NM / ND) {
+                    if (loaded < DB) ld.template load_b1<END>(load_half, loaded, s + 2, slot);
+                    else ld.template load_a1<END>(load_half, loaded - DB, s + 2, slot);
+                    ++loaded;
+                }
+                Mma::template mma_tied<j, i>(acc[h * 4 + i][j], f.b[j / QC][j % QC], f.a[h][i], u, f.sb[slot][NS ? u : 0],
+                        f.sa[h][NS ? u : 0]);
+                __builtin_amdgcn_sched_barrier(0); // keeps the reads and loads spread between the MFMAs
+                ++n;
+            });
+            });
+            });
+        });
     };
     auto step = [&](auto End, int s, int slot) __attribute__((always_inline)) {
         half(End, std::true_type {}, s, slot);
@@ -704,7 +716,7 @@ __device__ __forceinline__ void main_loop_lines(Acc &acc, char *smem, const char
     if constexpr (Mma::G::NW == 8)
         main_loop_lines8<Mma>(acc, smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, sc, fill);
     else
-        main_loop_lines4<Mma>(acc, smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, fill);
+        main_loop_lines4<Mma>(acc, smem, a_tile, b_tile, lda, ldb, rows_a_left, rows_b_left, kbytes, sc, fill);
 }
 
 // operand policies of these loops

@@ -43,7 +43,8 @@ struct h16x16_mma_t {
             acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h_t, b.c[u]), __builtin_bit_cast(v8h_t, a.c[u]),
                     acc, 0, 0, 0);
     }
-    __device__ static __forceinline__ void mma_tied(v4f &acc, const line_pair_t &b, const line_pair_t &a, int u) {
+    template <int, int>
+    __device__ static __forceinline__ void mma_tied(v4f &acc, const line_pair_t &b, const line_pair_t &a, int u, int, int) {
         if constexpr (BF16)
             asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(b.c[u]), "v"(a.c[u]));
         else
@@ -80,7 +81,8 @@ struct i8_mma_t {
     __device__ static __forceinline__ void mma(v4i &acc, const line_pair_t &b, const line_pair_t &a, U, int, int) {
         acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(b.c[U::value], a.c[U::value], acc, 0, 0, 0);
     }
-    __device__ static __forceinline__ void mma_tied(v4i &acc, const line_pair_t &b, const line_pair_t &a, int u) {
+    template <int, int>
+    __device__ static __forceinline__ void mma_tied(v4i &acc, const line_pair_t &b, const line_pair_t &a, int u, int, int) {
         asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(acc) : "v"(b.c[u]), "v"(a.c[u]));
     }
 };
@@ -104,7 +106,8 @@ struct f8_mma_t {
     __device__ static __forceinline__ void mma(v4f &acc, const line_pair_t &b, const line_pair_t &a, U, int, int) {
         acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b.whole(), a.whole(), acc, FMT_B, FMT_A, 0, 0, 0, 0);
     }
-    __device__ static __forceinline__ void mma_tied(v4f &acc, const line_pair_t &b, const line_pair_t &a, int) {
+    template <int, int>
+    __device__ static __forceinline__ void mma_tied(v4f &acc, const line_pair_t &b, const line_pair_t &a, int, int, int) {
         const v8i B = b.whole(), A = a.whole();
         asm volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0 cbsz:%3 blgp:%4"
                      : "+a"(acc)
@@ -124,6 +127,14 @@ struct mxf8_mma_t : f8_mma_t<FMT_A, FMT_B, G_> {
     template <int J, int I, class U>
     __device__ static __forceinline__ void mma(v4f &acc, const line_pair_t &b, const line_pair_t &a, U, int sb, int sa) {
         acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b.whole(), a.whole(), acc, FMT_B, FMT_A, J, sb, I, sa);
+    }
+    // (the scale's byte: op_sel its bit 0, op_sel_hi its bit 1)
+    template <int J, int I>
+    __device__ static __forceinline__ void mma_tied(v4f &acc, const line_pair_t &b, const line_pair_t &a, int, int sb, int sa) {
+        const v8i B = b.whole(), A = a.whole();
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%8,0] cbsz:%9 blgp:%10"
+                     : "+a"(acc)
+                     : "v"(B), "v"(A), "v"(sb), "v"(sa), "n"(J & 1), "n"(I & 1), "n"(J >> 1), "n"(I >> 1), "n"(FMT_B), "n"(FMT_A));
     }
 };
 
@@ -145,6 +156,12 @@ struct mxf4_mma_t {
         const v4i &x = b.c[U::value], &y = a.c[U::value];
         acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(v8i {x[0], x[1], x[2], x[3], 0, 0, 0, 0},
                 v8i {y[0], y[1], y[2], y[3], 0, 0, 0, 0}, acc, 4, 4, J, sb, I, sa);
+    }
+    template <int J, int I>
+    __device__ static __forceinline__ void mma_tied(v4f &acc, const line_pair_t &b, const line_pair_t &a, int u, int sb, int sa) {
+        asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%8,0] cbsz:4 blgp:4"
+                     : "+a"(acc)
+                     : "v"(b.c[u]), "v"(a.c[u]), "v"(sb), "v"(sa), "n"(J & 1), "n"(I & 1), "n"(J >> 1), "n"(I >> 1));
     }
 };
 

@@ -147,3 +147,36 @@ def test_operands_contiguous_across_k(gpu, oracle, K, dt, ddt, tiles, src_across
 def test_both_across_k_ragged(gpu, oracle, M, N, K, pads):
     for tiles in (None, "wide"):
         check(oracle, across_problem(M, N, K, "bf16", "bf16", True, batch=2, src_pad=pads[0], wei_pad=pads[1]), "bf16", tiles)
+
+
+# block scales on both geometries (their loads ride along with the steps'): a scale of its own for every block
+@pytest.mark.parametrize("K", [64, 96, 128, 160, 256, 288, 384, 512, 672])
+@pytest.mark.parametrize("tiles", [None, "wide"])
+def test_mxfp8_steps(gpu, oracle, K, tiles):
+    from tests.test_mxf8_gemm import problem as mx_problem
+    for M, N, ddt in ((300, 328, "f32"), (129, 200, "bf16")):
+        p = mx_problem(M, N, K, ddt=ddt, seed=K)
+        with cabi.tuning("MI355_F8_TILES", tiles):
+            got, name = run_gpu(p)
+        assert name.startswith("hip:mfma_f8"), name
+        assert_bit_exact(p, got, oracle.run_oracle(p), f"{name} {tiles}")
+
+
+@pytest.mark.parametrize("K", [128, 160, 256, 288, 512, 544, 768, 1024, 1120])
+@pytest.mark.parametrize("tiles", [None, "wide"])
+def test_mxfp4_steps(gpu, oracle, K, tiles):
+    """one block of some rows and columns scaled up: every block of every step has to meet its own scale"""
+    p = configs.config5(M=300, N=328, K=K)
+    p.dst_dt = cabi.DT_F32
+    ss, ws = p.quant["src_scale"].data, p.quant["wei_scale"].data
+    ss[:] = 127
+    ws[:] = 126
+    kb = K // 32
+    s2, w2 = ss.reshape(300, kb), ws.reshape(kb, 328)
+    for i in range(kb):
+        s2[(37 * i) % 300, i] = 129
+        w2[i, (53 * i) % 328] = 128
+    with cabi.tuning("MI355_F8_TILES", tiles):
+        got, name = run_gpu(p)
+    assert name.startswith("hip:mfma_mxf4"), name
+    assert_bit_exact(p, got, oracle.run_oracle(p), f"{name} {tiles}")
