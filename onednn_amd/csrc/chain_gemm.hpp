@@ -68,6 +68,8 @@ int chain_launch_h16(bool bf16, int dst_dt, chain_t &C, unsigned batch, bool wid
 // bytes from one k to the next
 int chain_launch_h16_across(bool bf16, int dst_dt, int across, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
 int chain_launch_i8(bool src_u8, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
+// ... on 32 x 32 tiles that make their own column sums (C.colsum is not read)
+int chain_launch_i8_small(bool src_u8, int dst_dt, chain_t &C, unsigned batch, hipStream_t stream);
 int chain_launch_f8(int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream); // e4m3 x e4m3
 int chain_launch_mx(bool fp4, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream); // e4m3 x e4m3 or fp4
 

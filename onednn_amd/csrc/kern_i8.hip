@@ -333,19 +333,22 @@ i8_plan_t make_plan(const mi355_matmul_desc_t &d) {
     // small tiles compute their own sums and have no dynamic dst quantization).  Up to 128 large tiles the LDS
     // tiles' time depends on K alone; the small tiles' grows with their number, in
     // steps of three a CU.  Counted in small tiles and not in large ones, because a
-    // short M fills few rows of a large tile.  K = 1024 / 4096 / 16384, small against
-    // LDS tiles: with zero points, whose sums are kernels of their own in front of the
-    // latter (f32 dst), 13 / 29 / 90 us against 22 / 37 / 103 on 768 tiles, 18 / 37 / 118
-    // against 22 / 37 / 106 on 1024; without and with a chain of chain_gemm.hpp (bf16 dst),
-    // 10.6 / 21 / 63 against 14 / 25 / 72 on 512, 13.0 / 28.7 / 90 against 14.1 / 25.3 / 73
-    // on 768, 18 / 37 / 119 against 14 / 26 / 74 on 1024; K = 512 10.3 against 12.0 on 512
-    // and 12.7 against 12.1 on 768.
+    // short M fills few rows of a large tile.  With a chain of chain_gemm.hpp on both
+    // (bf16 dst; K = 512 / 1024 / 4096 / 16384), small against LDS tiles: 6.4 / 6.6 / 17.2 / 60
+    // us against 12.1 / 14.2 / 25.6 / 72 on 512 of them, 8.5 / 8.8 / 24.9 / 86 against 12.6 /
+    // 14.7 / 26.1 / 74 on 768, 10.7 / 10.7 / 31.9 / 116 against 12.5 / 14.6 / 26.0 / 74 on
+    // 1024, 19.1 / 18.5 / 59 against 12.8 / 14.8 / 26.9 on 2048.  With zero points, whose
+    // sums are a kernel of their own in front of the LDS tiles (f32 dst), the latter take
+    // 19 / 22 / 37 / 105.  Other epilogues cost the small tiles about 4 us more a launch and
+    // the LDS tiles about 8.
     const long small_tiles = ((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch;
     const bool sums = d.src_dt == MI355_DT_U8 || d.wei_dt == MI355_DT_U8 || !quant_absent(d.src_zp) || !quant_absent(d.wei_zp);
     const bool chain = (is_int8_dt(d.dst_dt) || d.dst_dt == MI355_DT_BF16 || d.dst_dt == MI355_DT_F32) && quant_absent(d.dst_zp)
             && (d.n_post_ops == 0
                     || (d.n_post_ops == 1 && d.post_ops[0].kind == MI355_PO_ELTWISE && d.post_ops[0].alg == MI355_ELTWISE_RELU));
-    const long crossover = sums ? (d.K > 8192 ? 769 : 1024) : !chain ? 1024 : d.K < 1024 ? 257 + d.K / 2 : d.K < 2048 ? 769 : 513;
+    const long crossover = !chain ? 1024
+            : sums                ? (d.K < 512 ? 1024 : d.K < 2048 ? 1793 : d.K <= 8192 ? 1153 : 897)
+                                  : (d.K < 512 ? 1025 : d.K < 2048 ? 1281 : d.K <= 8192 ? 769 : 513);
     p.small = !d.dst_scale_dynamic && small_tiles < crossover;
     // the MI355_I8_TILES switch overrides the choice where both can run (tests and
     // tuning): large = the LDS tiles, 256 x 128 or 256 x 256 by the number of
@@ -445,7 +448,23 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         X.rowsum = rs;
     }
     const bool su = d.src_dt == MI355_DT_U8, wu = d.wei_dt == MI355_DT_U8;
+    chain_t C {};
+    const bool chain = !wu && P.wei_zp.dt == MI355_DT_UNDEF && (P.src_zp.dt == MI355_DT_UNDEF || P.src_zp.dt == MI355_DT_S32)
+            && chain_from(P, true, false, C);
+    if (chain) {
+        C.a = (const char *)P.src; C.lda = P.ss[1]; C.a_bs = P.ss[0];
+        C.bt = (const char *)X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
+        C.kbytes = P.K;
+        C.colsum = X.colsum;
+        C.colsum_bs = plan.Bw > 1 ? d.N : 0;
+        C.src_zp = P.src_zp.dt != MI355_DT_UNDEF ? (const int *)P.src_zp.p : nullptr;
+        C.off_s = su ? 128 : 0;
+    }
     if (plan.small) {
+        if (chain) {
+            const int st = chain_launch_i8_small(su, P.dst_dt, C, (unsigned)d.batch, stream);
+            if (st != MI355_UNIMPLEMENTED) return st;
+        }
         X.tiles_m = (int)((d.M + ST - 1) / ST);
         X.tiles_n = (int)((d.N + ST - 1) / ST);
         const long tiles = (long)X.tiles_m * X.tiles_n;
@@ -466,19 +485,9 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
     // (MI355_I8_TILES: wide / narrow keep one geometry whatever the size: tests, tuning)
     const int force = tuning(TUNE_I8_TILES);
     const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N) && force != TUNE_WIDE);
-    chain_t C {};
-    if (!wu && P.wei_zp.dt == MI355_DT_UNDEF && chain_from(P, true, false, C)) {
-        C.a = (const char *)P.src; C.lda = P.ss[1]; C.a_bs = P.ss[0];
-        C.bt = (const char *)X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
-        C.kbytes = P.K;
-        C.colsum = X.colsum;
-        C.colsum_bs = plan.Bw > 1 ? d.N : 0;
-        C.src_zp = P.src_zp.dt != MI355_DT_UNDEF ? (const int *)P.src_zp.p : nullptr;
-        C.off_s = su ? 128 : 0;
-        if (P.src_zp.dt == MI355_DT_UNDEF || P.src_zp.dt == MI355_DT_S32) {
-            const int st = chain_launch_i8(su, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
-            if (st != MI355_UNIMPLEMENTED) return st;
-        }
+    if (chain) {
+        const int st = chain_launch_i8(su, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
+        if (st != MI355_UNIMPLEMENTED) return st;
     }
     X.tiles_m = (int)((d.M + BM - 1) / BM);
     auto go = [&](auto su_, auto wu_) -> int {
