@@ -36,12 +36,6 @@ struct f8_conv_t {
         return ssc_p ? load_float(ssc_dt, ssc_p, m) : ssc_common;
     }
 
-    // (the chains that layers are made of run on the kernels of chain_gemm.hpp)
-    template <class PT, class Acc>
-    __device__ __forceinline__ bool hot_chain(const PT &, const epi_uniform_t &, unsigned, unsigned, const Acc &, long, long,
-            long, int) const {
-        return false;
-    }
     __device__ __forceinline__ void quad(const v4i_t &raw, float ssc, unsigned ntab, int col, float (&f)[4]) const {
 #pragma unroll
         for (int e = 0; e < 4; ++e) f[e] = __int_as_float(raw[e]);

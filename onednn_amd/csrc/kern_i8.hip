@@ -56,12 +56,6 @@ struct i8_conv_t {
     }
     __device__ __forceinline__ int row_data(long m) const { return rowsum ? rowsum[m] : 0; }
 
-    // (the chains that layers are made of run on the kernels of chain_gemm.hpp)
-    template <class PT, class Acc>
-    __device__ __forceinline__ bool hot_chain(const PT &, const epi_uniform_t &, unsigned, unsigned, const Acc &, long, long,
-            long, int) const {
-        return false;
-    }
     __device__ __forceinline__ void quad(const v4i_t &raw, int rs, unsigned ntab, int col, float (&f)[4]) const {
         int v[4] = {raw[0], raw[1], raw[2], raw[3]};
         if (has_comp) {
