@@ -62,7 +62,7 @@ int mx_pack_scales(const mi355_matmul_desc_t &d, const problem_t &P, long Bsa, l
         gemm::line_scales_args_t &sc, hipStream_t stream);
 
 // The families' launchers on the chain kernels, a translation unit each; C as chain_from and the family left it.
-// wide: the 256 x 256 tiles whatever the size
+// wide: the 256 x 256 tiles whatever the size.  A 16-bit dst of the operands' other type takes a C of full = false.
 int chain_launch_h16(bool bf16, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
 // ... with the weights (across = 1), or src and the weights (2, 256 x 256 tiles only), contiguous across K: lda / ldb are the
 // bytes from one k to the next

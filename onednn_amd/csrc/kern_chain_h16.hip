@@ -87,10 +87,20 @@ int chain_launch_h16(bool bf16, int dst_dt, chain_t &C, unsigned batch, bool wid
         return wide ? chain_go<h16x16_mma_t<B, wide_t>, D>(C, batch, stream, "mfma_h16")
                     : chain_go<h16x16_mma_t<B, narrow_t>, D>(C, batch, stream, "mfma_h16");
     };
+    auto go_mixed = [&](auto b16, auto dst) -> int {
+        constexpr bool B = decltype(b16)::value;
+        constexpr int D = decltype(dst)::value;
+        return wide ? chain_go<h16_mixed_mma_t<B, wide_t>, D>(C, batch, stream, "mfma_h16")
+                    : chain_go<h16_mixed_mma_t<B, narrow_t>, D>(C, batch, stream, "mfma_h16");
+    };
     constexpr std::integral_constant<int, CHAIN_F32> f32 {};
-    if (bf16 && dst_dt == MI355_DT_BF16) return go(std::true_type {}, std::integral_constant<int, CHAIN_BF16> {});
+    constexpr std::integral_constant<int, CHAIN_BF16> b {};
+    constexpr std::integral_constant<int, CHAIN_F16> h {};
+    if (bf16 && dst_dt == MI355_DT_BF16) return go(std::true_type {}, b);
+    if (bf16 && dst_dt == MI355_DT_F16) return go_mixed(std::true_type {}, h);
     if (bf16 && dst_dt == MI355_DT_F32) return go(std::true_type {}, f32);
-    if (!bf16 && dst_dt == MI355_DT_F16) return go(std::false_type {}, std::integral_constant<int, CHAIN_F16> {});
+    if (!bf16 && dst_dt == MI355_DT_BF16) return go_mixed(std::false_type {}, b);
+    if (!bf16 && dst_dt == MI355_DT_F16) return go(std::false_type {}, h);
     if (!bf16 && dst_dt == MI355_DT_F32) return go(std::false_type {}, f32);
     return MI355_UNIMPLEMENTED;
 }

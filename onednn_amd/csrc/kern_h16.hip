@@ -482,7 +482,7 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
     using narrow_t = narrow_geo_t;
     using f32_t = f32_mma_t<f8_geo_t>;
     if (plan.op_dt == MI355_DT_F32) return go(f32_t {}, f8_gemm_kernel<f32_t>);
-    if (chain_from(P, false, true, C)) {
+    if (chain_from(P, false, P.dst_dt == plan.op_dt, C)) {
         C.a = (const char *)P.src; C.lda = P.ss[1] * EB; C.a_bs = P.ss[0] * EB;
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K * EB;

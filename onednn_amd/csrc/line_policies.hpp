@@ -52,6 +52,12 @@ struct h16x16_mma_t {
     }
 };
 
+// the same for a dst of the other 16-bit type: chains without the activations that take a hardware exponential
+template <bool BF16, class G_>
+struct h16_mixed_mma_t : h16x16_mma_t<BF16, G_> {
+    static constexpr bool FULL = false;
+};
+
 // the same with the weights (ACROSS = 1), or src and the weights (2), contiguous across K
 template <bool BF16, class G_, int ACROSS>
 struct h16_across_mma_t : h16x16_mma_t<BF16, G_> {

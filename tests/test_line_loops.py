@@ -80,7 +80,7 @@ RELU = PostOp(cabi.PO_ELTWISE, alg=cabi.ELTWISE["relu"], alpha=0.0)
 @pytest.mark.parametrize("M,N", [(1, 136), (129, 200), (130, 268), (257, 388)])
 @pytest.mark.parametrize("dt,ddt,kw", [
     ("bf16", "bf16", {}), ("bf16", "f32", dict(bias=True)), ("f16", "f16", dict(bias=True, post=[RELU])),
-    ("f16", "f32", dict(post=[RELU])), ("s8", "s8", dict(post=[RELU], dst_scale=3.0)), ("s8", "u8", dict(bias=True, dst_scale=0.7)),
+    ("f16", "f32", dict(post=[RELU])), ("f16", "bf16", dict(bias=True)), ("bf16", "f16", dict(post=[RELU])), ("s8", "s8", dict(post=[RELU], dst_scale=3.0)), ("s8", "u8", dict(bias=True, dst_scale=0.7)),
     ("u8", "s8", dict(bias=True, src_zp=5)), ("u8", "f32", dict(src_zp=2, post=[RELU])), ("f8_e4m3", "f32", dict(bias=True)),
     ("f8_e4m3", "bf16", dict(row_scales=True, post=[RELU]))])
 def test_where_the_rows_of_dst_end(gpu, oracle, M, N, dt, ddt, kw):
