@@ -54,8 +54,8 @@ struct chain_t {
 // weights scales are the epilogue's; full: activations other than relu and the bf16 tensor are carried.
 bool chain_from(const problem_t &P, bool scaled, bool full, chain_t &C);
 
-// the same for a block-scaled problem (mx), whose scales are operands of the instruction
-bool chain_from_mx(const problem_t &P, bool mx, chain_t &C);
+// the same for a family with block scales: where mx is set they are operands of the instruction
+bool chain_from_mx(const problem_t &P, bool mx, bool full, chain_t &C);
 
 // mx_pack_scales (kern_mxf4.hip): the pre-pass of the block-scaled types
 int mx_pack_scales(const mi355_matmul_desc_t &d, const problem_t &P, long Bsa, long Bsb, char *sa, char *sb,

@@ -71,11 +71,11 @@ bool chain_from(const problem_t &P, bool scaled, bool full, chain_t &C) {
     return at == P.n_po;
 }
 
-bool chain_from_mx(const problem_t &P, bool mx, chain_t &C) {
-    if (!mx) return chain_from(P, true, true, C);
+bool chain_from_mx(const problem_t &P, bool mx, bool full, chain_t &C) {
+    if (!mx) return chain_from(P, true, full, C);
     problem_t Q = P;
     Q.src_scale.dt = Q.wei_scale.dt = MI355_DT_UNDEF;
-    return chain_from(Q, false, false, C);
+    return chain_from(Q, false, full, C);
 }
 
 int chain_launch_h16(bool bf16, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream) {

@@ -264,7 +264,7 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
     }
     if (const int st = mx_pack_scales(d, P, plan.Bsa, plan.Bsb, sc + plan.off_sa, sc + plan.off_sb, X.sc, stream)) return st;
     chain_t C {};
-    if (chain_from_mx(P, true, C)) {
+    if (chain_from_mx(P, true, false, C)) {
         C.a = (const char *)P.src; C.lda = P.ss[1] / 2; C.a_bs = P.ss[0] / 2;
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K / 2;

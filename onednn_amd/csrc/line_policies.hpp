@@ -129,7 +129,7 @@ template <int FMT_A, int FMT_B, class G_>
 struct mxf8_mma_t : f8_mma_t<FMT_A, FMT_B, G_> {
     static constexpr bool MX = true;
     static constexpr int SCALE_SETS = 1;
-    static constexpr bool SCALED = false, FULL = false;
+    static constexpr bool SCALED = false;
     template <int J, int I, class U>
     __device__ static __forceinline__ void mma(v4f &acc, const line_pair_t &b, const line_pair_t &a, U, int sb, int sa) {
         acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(b.whole(), a.whole(), acc, FMT_B, FMT_A, J, sb, I, sa);

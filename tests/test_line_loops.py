@@ -91,7 +91,7 @@ def test_where_the_rows_of_dst_end(gpu, oracle, M, N, dt, ddt, kw):
 
 @pytest.mark.parametrize("act", [None, "gelu_tanh", "swish"])
 @pytest.mark.parametrize("alg", ["add", "mul"])
-@pytest.mark.parametrize("dt", ["bf16", "f8_e4m3"])
+@pytest.mark.parametrize("dt", ["bf16", "f8_e4m3", "mxfp8"])
 def test_a_staged_tensor_at_ragged_edges(gpu, oracle, act, alg, dt):
     """N = 200: the last wavefront's columns end after one chunk of eight; rows end inside a row block.  Without an
     activation the sums are exact; with one the result is within the activation's few ulp of the oracle, rounded to
@@ -101,11 +101,17 @@ def test_a_staged_tensor_at_ragged_edges(gpu, oracle, act, alg, dt):
     other = dtp.f32_to_bf16(r.integers(-4, 5, size=M * N).astype(np.float32)).reshape(M, N)
     post = [PostOp(cabi.PO_ELTWISE, alg=cabi.ELTWISE[act], alpha=1.0)] if act else []
     post.append(PostOp(cabi.PO_BINARY, alg=cabi.BINARY[alg], dt=cabi.DT_BF16, stride=(0, N, 1), data=other))
-    p = problem(M, N, K, dt, "bf16", bias=True, post=post)
+    if dt == "mxfp8":
+        from tests.test_mxf8_gemm import problem as mx_problem
+        p = mx_problem(M, N, K, ddt="bf16", bias=True, post_ops=post)
+        p.quant["src_scale"].data[:] = 127 - 6
+        p.quant["wei_scale"].data[:] = 127
+    else:
+        p = problem(M, N, K, dt, "bf16", bias=True, post=post)
     if dt == "f8_e4m3":
         p.quant["src_scale"].data[:] = 1 / 64
     got, name = run_gpu(p)
-    assert name.startswith(FAMILY[dt]), name
+    assert name.startswith(FAMILY.get(dt, "hip:mfma_f8")), name
     want = oracle.run_oracle(p)
     if not act:
         assert_bit_exact(p, got, want, name)
