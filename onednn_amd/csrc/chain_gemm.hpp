@@ -318,7 +318,7 @@ struct chain_part_t {
     }
 };
 
-extern __shared__ __attribute__((aligned(16))) char chain_smem[];
+extern __shared__ __attribute__((aligned(128))) char chain_smem[];
 
 template <class Mma, int DST>
 __global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu(Mma::G::NW / 4))) chain_gemm_kernel(const chain_t C) {

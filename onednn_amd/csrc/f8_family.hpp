@@ -83,7 +83,7 @@ struct ring_of<Mma, std::enable_if_t<reads_lines<Mma>::value>> {
     static constexpr int WAVES = Mma::G::NW / 4;
 };
 
-extern __shared__ __attribute__((aligned(16))) char f8_smem[];
+extern __shared__ __attribute__((aligned(128))) char f8_smem[];
 
 template <class Mma>
 __global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu(ring_of<Mma>::WAVES))) f8_gemm_kernel(const problem_t P_, const f8_extra_t X) {

@@ -77,7 +77,7 @@ struct i8_conv_t {
     }
 };
 
-extern __shared__ __attribute__((aligned(16))) char i8_smem[];
+extern __shared__ __attribute__((aligned(128))) char i8_smem[];
 
 template <bool SRC_U8, bool WEI_U8, class G>
 __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::NW / 4))) i8_gemm_kernel(const problem_t P_, const i8_extra_t X) {

@@ -27,6 +27,7 @@ namespace {
 
 using namespace gemm;
 using mx_geo_t = geo_t<8, 256>;
+using mx_narrow_t = geo_t<4, 128>;
 
 struct mxf4_extra_t {
     const char *bt;       // weights [N][K/2] bytes
@@ -46,7 +47,7 @@ struct mxf4_conv_t {
     }
 };
 
-extern __shared__ __attribute__((aligned(16))) char mxf4_smem[];
+extern __shared__ __attribute__((aligned(128))) char mxf4_smem[];
 
 template <class G>
 __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(G::NW / 4))) mxf4_gemm_kernel(const problem_t P_, const mxf4_extra_t X) {
@@ -263,25 +264,33 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         X.bt_bstride = d.wei_stride[0] / 2;
     }
     if (const int st = mx_pack_scales(d, P, plan.Bsa, plan.Bsb, sc + plan.off_sa, sc + plan.off_sb, X.sc, stream)) return st;
+    // (MI355_F8_TILES keeps one geometry here as well)
+    const int force = tuning(TUNE_F8_TILES);
+    const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N) && force != TUNE_WIDE);
     chain_t C {};
     if (chain_from_mx(P, true, false, C)) {
         C.a = (const char *)P.src; C.lda = P.ss[1] / 2; C.a_bs = P.ss[0] / 2;
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K / 2;
         C.sc = X.sc;
-        // (MI355_F8_TILES keeps one geometry here as well)
-        const int force = tuning(TUNE_F8_TILES);
-        const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N) && force != TUNE_WIDE);
         const int st = chain_launch_mx(true, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }
     X.tiles_m = (int)((d.M + BM - 1) / BM);
-    X.tiles_n = (int)((d.N + mx_geo_t::BN - 1) / mx_geo_t::BN);
-    dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);
-    constexpr int smem_bytes = line_loader_t<mxf4_mma_t<mx_geo_t>>::LDS_BYTES + NTAB_BYTES;
-    if (const int st = ensure_dynamic_lds((const void *)mxf4_gemm_kernel<mx_geo_t>, smem_bytes, "mfma_mxf4")) return st;
-    hipLaunchKernelGGL(mxf4_gemm_kernel<mx_geo_t>, grid, dim3(mx_geo_t::NT), smem_bytes, stream, P, X);
-    return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
+    auto go = [&](auto geo) -> int {
+        using G = decltype(geo);
+        constexpr int smem_bytes = line_loader_t<mxf4_mma_t<G>>::LDS_BYTES + NTAB_BYTES;
+        X.tiles_n = (int)((d.N + G::BN - 1) / G::BN);
+        const dim3 grid((unsigned)(X.tiles_m * X.tiles_n), 1, (unsigned)d.batch);
+        const auto kern = mxf4_gemm_kernel<G>;
+        if (const int st = ensure_dynamic_lds((const void *)kern, smem_bytes, "mfma_mxf4")) return st;
+        hipLaunchKernelGGL(kern, grid, dim3(G::NT), smem_bytes, stream, P, X);
+        return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
+    };
+    // The general epilogue on both tiles: by rounds like the chains, and the narrow one also where one column of them
+    // holds N (64 x 4096 x 1024, f16 dst: 25.4 us wide, 21.8 narrow; 300 x 100 x 2048, bf16: 50.6 and 44.5; but 4096 x 4096 x
+    // 256, two rounds of narrow tiles: 27.2 and 39.3).
+    return narrow || (d.N <= mx_narrow_t::BN && force != TUNE_WIDE) ? go(mx_narrow_t {}) : go(mx_geo_t {});
 }
 
 } // namespace mi355

@@ -298,23 +298,34 @@ struct line_frags_t {
         rs = ld.lds0 + L::RING_BYTES + (r * 4 + q) * 4;
         if constexpr (NS == 0) sa[0][0] = sa[1][0] = sb[0][0] = sb[1][0] = 0;
     }
+    // MXFP4's last steps (END), where the slot is not a constant, work the address out from one: its two sets of scales
+    // leave the eight-wavefront loop no registers, and the general epilogue's kernel kept 22 in scratch memory, whose
+    // reloads wait for every load in flight (64 x 4096 x 1024, f16 dst: 29.4 -> 25.4 us; the other types have the room and
+    // lose 1 us to the arithmetic).  (The ring starts at a multiple of 128 bytes.)
+    static constexpr bool ONE_ADDRESS = NS == 2;
+    template <bool END = false>
     __device__ __forceinline__ void read_a1(int h, int i, int u, int slot) {
-        a[h][i].c[u] = lds_read16((slot ? ra[1][u] : ra[0][u]) + h * (64 * LKB) + i * (16 * LKB));
+        const unsigned at = END && ONE_ADDRESS ? (ra[0][0] ^ (unsigned)(u << 6)) + slot * L::STAGE_BYTES : slot ? ra[1][u] : ra[0][u];
+        a[h][i].c[u] = lds_read16(at + h * (64 * LKB) + i * (16 * LKB));
     }
+    template <bool END = false>
     __device__ __forceinline__ void read_b1(int g, int j, int u, int slot) {
-        b[g][j].c[u] = lds_read16((slot ? rb[1][u] : rb[0][u]) + g * (L::WC / 2 * LKB) + j * (16 * LKB));
+        const unsigned at = END && ONE_ADDRESS ? (rb[0][0] ^ (unsigned)(u << 6)) + slot * L::STAGE_BYTES : slot ? rb[1][u] : rb[0][u];
+        b[g][j].c[u] = lds_read16(at + g * (L::WC / 2 * LKB) + j * (16 * LKB));
     }
+    template <bool END>
     __device__ __forceinline__ void read_a(int h, int slot) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int u = 0; u < 2; ++u) read_a1(h, i, u, slot);
+            for (int u = 0; u < 2; ++u) read_a1<END>(h, i, u, slot);
     }
+    template <bool END>
     __device__ __forceinline__ void read_b(int g, int slot) {
 #pragma unroll
         for (int j = 0; j < QC; ++j)
 #pragma unroll
-            for (int u = 0; u < 2; ++u) read_b1(g, j, u, slot);
+            for (int u = 0; u < 2; ++u) read_b1<END>(g, j, u, slot);
     }
     __device__ __forceinline__ void read_sa(int h, int slot) {
         if constexpr (NS > 0) {
@@ -492,11 +503,11 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
         const bool partial = END && ld.tail_mask != 0 && s == ld.nst - 1;
         f.read_sb(0, slot);
         if constexpr (BKM) f.read_bk(0, slot);
-        else f.read_b(0, slot);
+        else f.template read_b<END>(0, slot);
         f.read_sa(0, slot);
         f.read_sa(1, slot);
         if constexpr (AKM) f.read_ak(0, 0, slot);
-        else f.read_a(0, slot);
+        else f.template read_a<END>(0, slot);
         ld.template load_a<END>(1, s + 1, slot ^ 1);
         wait_vmcnt<STEP + DA>(); // after B 1 of s: A 1, then all of s + 1
         wait_lds_reads();
@@ -509,7 +520,7 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
         phase_barrier();
         if constexpr (AKM) f.read_ak(0, 1, slot);
         else if constexpr (BKM) f.read_bk(1, slot);
-        else f.read_b(1, slot);
+        else f.template read_b<END>(1, slot);
         ld.template load_b<END>(0, s + 2, slot);
         ld.template load_scales<END>(s + 2, slot);
         wait_vmcnt<STEP + DB + EX>(); // after A 1 of s: all of s + 1, B 0 and scales of s + 2
@@ -524,7 +535,7 @@ __device__ __forceinline__ void main_loop_lines8(Acc &acc, char *smem, const cha
             f.read_bk(1, slot);
             f.read_ak(1, 0, slot);
         } else {
-            f.read_a(1, slot);
+            f.template read_a<END>(1, slot);
         }
         ld.template load_a<END>(0, s + 2, slot);
         wait_lds_reads();
@@ -611,9 +622,9 @@ __device__ __forceinline__ void main_loop_lines4(Acc &acc, char *smem, const cha
     phase_barrier();
     f.read_sb(0, 0);
     f.read_sa(0, 0);
-    f.read_a(0, 0);
+    f.template read_a<false>(0, 0);
     if constexpr (BKM) f.read_bk(0, 0);
-    else f.read_b(0, 0);
+    else f.template read_b<false>(0, 0);
 
     // two wait states behind everything that ready_a / ready_b compute (the scheduler would sink it to its use)
     auto settle = []() __attribute__((always_inline)) {

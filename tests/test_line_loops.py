@@ -170,10 +170,12 @@ def test_mxfp8_steps(gpu, oracle, K, tiles):
 
 @pytest.mark.parametrize("K", [128, 160, 256, 288, 512, 544, 768, 1024, 1120])
 @pytest.mark.parametrize("tiles", [None, "wide"])
-def test_mxfp4_steps(gpu, oracle, K, tiles):
-    """one block of some rows and columns scaled up: every block of every step has to meet its own scale"""
+@pytest.mark.parametrize("ddt", ["f32", "f16"])
+def test_mxfp4_steps(gpu, oracle, K, tiles, ddt):
+    """one block of some rows and columns scaled up: every block of every step has to meet its own scale; f16: the general
+    epilogue's kernels"""
     p = configs.config5(M=300, N=328, K=K)
-    p.dst_dt = cabi.DT_F32
+    p.dst_dt = DT[ddt]
     ss, ws = p.quant["src_scale"].data, p.quant["wei_scale"].data
     ss[:] = 127
     ws[:] = 126
