@@ -287,9 +287,11 @@ __global__ void __launch_bounds__(SNW * 64) i8_small_kernel(const problem_t P_, 
     store4(P, P.ds[2] == 1 && vec_ok_store(P.dst, P.ds[0], P.ds[1], dt_bits(P.dst_dt)), v, b, m, nbase, nvalid);
 }
 
-// out[r] = sum_k (bytes[r][k] ^ flip) as signed bytes; one wave per row
+// out[b][r] = sum_k (bytes[b][r][k] ^ flip) as signed bytes; one wave per row
 __global__ void __launch_bounds__(256) i8_rowsum_kernel(const int8_t *p, long rows, long K,
-        long ld, int flip, int *out) {
+        long ld, long bs, int flip, int *out) {
+    p += blockIdx.y * bs;
+    out += blockIdx.y * rows;
     const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (r >= rows) return;
     const int lane = threadIdx.x & 63;
@@ -427,18 +429,14 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
     }
     if (plan.need_colsum) {
         int *cs = (int *)(sc + plan.off_colsum);
-        for (long b = 0; b < plan.Bw; ++b)
-            hipLaunchKernelGGL(i8_rowsum_kernel, dim3((unsigned)((d.N + 3) / 4)), dim3(256), 0,
-                    stream, X.bt + b * X.bt_bstride, d.N, d.K, X.ldb,
-                    wei_u8 ? (int)0x80808080 : 0, cs + b * d.N);
+        hipLaunchKernelGGL(i8_rowsum_kernel, dim3((unsigned)((d.N + 3) / 4), (unsigned)plan.Bw), dim3(256), 0, stream, X.bt, d.N,
+                d.K, X.ldb, X.bt_bstride, wei_u8 ? (int)0x80808080 : 0, cs);
         X.colsum = cs;
     }
     if (plan.need_rowsum) {
         int *rs = (int *)(sc + plan.off_rowsum);
-        for (long b = 0; b < plan.Bs; ++b)
-            hipLaunchKernelGGL(i8_rowsum_kernel, dim3((unsigned)((d.M + 3) / 4)), dim3(256), 0,
-                    stream, (const int8_t *)P.src + b * d.src_stride[0], d.M, d.K,
-                    d.src_stride[1], src_u8 ? (int)0x80808080 : 0, rs + b * d.M);
+        hipLaunchKernelGGL(i8_rowsum_kernel, dim3((unsigned)((d.M + 3) / 4), (unsigned)plan.Bs), dim3(256), 0, stream,
+                (const int8_t *)P.src, d.M, d.K, d.src_stride[1], d.src_stride[0], src_u8 ? (int)0x80808080 : 0, rs);
         X.rowsum = rs;
     }
     const bool su = d.src_dt == MI355_DT_U8, wu = d.wei_dt == MI355_DT_U8;

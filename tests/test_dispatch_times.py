@@ -48,8 +48,12 @@ def in_turn(*launches, n=20, turns=12):
 
 
 def launches(p, switch=None, value=None):
-    """A launch of p for in_turn, a tuning switch set around it."""
-    g = GpuRun(p)
+    """A launch of p for in_turn, a tuning switch set around it (and around the scratch query)."""
+    if switch is None:
+        g = GpuRun(p)
+    else:
+        with cabi.tuning(switch, value):
+            g = GpuRun(p)
 
     def go(s):
         g.stream = s
@@ -82,6 +86,17 @@ def test_int8_layers_with_a_short_m(gpu, M, N, K):
 
     chosen, lds = in_turn(*(launches(p, "MI355_I8_TILES", tiles) for tiles in (None, "large")))
     assert chosen <= 1.06 * lds, (chosen, lds)
+
+
+@pytest.mark.parametrize("src_dt,wei_dt,dims", [(cabi.DT_U8, cabi.DT_S8, (64, 128, 128, 256)), (cabi.DT_S8, cabi.DT_U8, (64, 128, 128, 256)),
+                                                (cabi.DT_U8, cabi.DT_S8, (256, 128, 128, 48))])
+def test_int8_sums_of_a_batch_are_one_launch(gpu, src_dt, wei_dt, dims):
+    """Column or row sums in front of the LDS tiles, against signed operands without: one kernel more of a few us (and the
+    general epilogue's terms, for u8 weights), not one of 2 us for every batch."""
+    B, M, N, K = dims
+    with_sums, plain = in_turn(*(launches(int8_problem(M, N, K, s, w, cabi.DT_F32, batch=B), "MI355_I8_TILES", "large")
+                                 for s, w in ((src_dt, wei_dt), (cabi.DT_S8, cabi.DT_S8))))
+    assert with_sums <= plain + 20, (with_sums, plain)
 
 
 @pytest.mark.parametrize("pitch,offset", [(8196, 0), (8192, 4), (8200, 8)])
