@@ -239,15 +239,14 @@ static int choose_impl(const mi355_matmul_desc_t &d, int *chosen) {
     return MI355_UNIMPLEMENTED;
 }
 
-static void fill_quant(quant_dev_t &q, const mi355_quant_t &s, const void *p) {
+static void fill_quant(quant_dev_t &q, const mi355_quant_t &s) {
     q.dt = s.dt;
     q.mask = s.mask;
     q.g0 = s.dt == MI355_DT_UNDEF ? 1 : s.group[0];
     q.g1 = s.dt == MI355_DT_UNDEF ? 1 : s.group[1];
-    q.p = p;
 }
 
-static int build_problem(const mi355_matmul_desc_t &d, const mi355_matmul_args_t &a, problem_t &P) {
+void problem_of_desc(const mi355_matmul_desc_t &d, problem_t &P) {
     memset(&P, 0, sizeof(P));
     P.B = d.batch; P.M = d.M; P.N = d.N; P.K = d.K;
     P.src_dt = d.src_dt; P.wei_dt = d.wei_dt; P.dst_dt = d.dst_dt; P.bias_dt = d.bias_dt;
@@ -255,21 +254,37 @@ static int build_problem(const mi355_matmul_desc_t &d, const mi355_matmul_args_t
         P.ss[i] = d.src_stride[i]; P.ws[i] = d.wei_stride[i];
         P.ds[i] = d.dst_stride[i]; P.bs[i] = d.bias_stride[i];
     }
-    fill_quant(P.src_scale, d.src_scale, a.src_scale);
-    fill_quant(P.wei_scale, d.wei_scale, a.wei_scale);
-    fill_quant(P.dst_scale, d.dst_scale, a.dst_scale);
-    fill_quant(P.src_zp, d.src_zp, a.src_zp);
-    fill_quant(P.wei_zp, d.wei_zp, a.wei_zp);
-    fill_quant(P.dst_zp, d.dst_zp, a.dst_zp);
-    fill_quant(P.src_pr, d.src_pr, a.src_pr);
+    fill_quant(P.src_scale, d.src_scale);
+    fill_quant(P.wei_scale, d.wei_scale);
+    fill_quant(P.dst_scale, d.dst_scale);
+    fill_quant(P.src_zp, d.src_zp);
+    fill_quant(P.wei_zp, d.wei_zp);
+    fill_quant(P.dst_zp, d.dst_zp);
+    fill_quant(P.src_pr, d.src_pr);
     P.apply_to_int = d.fpmath_apply_to_int;
     P.dst_scale_mode = d.dst_scale_mode;
     P.n_po = d.n_post_ops;
     P.sum_dt = MI355_DT_UNDEF;
     P.wei_packing = d.wei_packing;
     P.dst_dynamic = d.dst_scale_dynamic;
-    P.src = a.src; P.wei = a.wei; P.bias = a.bias; P.dst = a.dst;
     P.rnd_flags = d.rnd_flags;
+    for (int i = 0; i < d.n_post_ops; ++i) {
+        const mi355_post_op_t &s = d.post_ops[i];
+        po_dev_t &o = P.po[i];
+        o.kind = s.kind; o.alg = s.alg; o.alpha = s.alpha; o.beta = s.beta; o.scale = s.scale;
+        o.zp = s.zero_point; o.dt = s.dt;
+        o.s0 = s.stride[0]; o.s1 = s.stride[1]; o.s2 = s.stride[2];
+        if (s.kind == MI355_PO_SUM && P.sum_dt == MI355_DT_UNDEF)
+            P.sum_dt = s.dt ? s.dt : d.dst_dt;
+    }
+}
+
+static int build_problem(const mi355_matmul_desc_t &d, const mi355_matmul_args_t &a, problem_t &P) {
+    problem_of_desc(d, P);
+    P.src_scale.p = a.src_scale; P.wei_scale.p = a.wei_scale; P.dst_scale.p = a.dst_scale;
+    P.src_zp.p = a.src_zp; P.wei_zp.p = a.wei_zp; P.dst_zp.p = a.dst_zp;
+    P.src_pr.p = a.src_pr;
+    P.src = a.src; P.wei = a.wei; P.bias = a.bias; P.dst = a.dst;
     P.drop_p = a.dropout_p; P.drop_seed = a.dropout_seed; P.drop_offset = a.dropout_offset; P.drop_mask = a.dropout_mask;
     if ((d.rnd_flags & MI355_RND_DROPOUT)
             && (!a.dropout_p || !a.dropout_seed || ((d.rnd_flags & MI355_RND_DROPOUT_OFFSET) && !a.dropout_offset)
@@ -292,18 +307,12 @@ static int build_problem(const mi355_matmul_desc_t &d, const mi355_matmul_args_t
         return MI355_INVALID_ARGUMENTS;
     }
     for (int i = 0; i < d.n_post_ops; ++i) {
-        const mi355_post_op_t &s = d.post_ops[i];
-        po_dev_t &o = P.po[i];
-        o.kind = s.kind; o.alg = s.alg; o.alpha = s.alpha; o.beta = s.beta; o.scale = s.scale;
-        o.zp = s.zero_point; o.dt = s.dt;
-        o.s0 = s.stride[0]; o.s1 = s.stride[1]; o.s2 = s.stride[2];
-        o.p = a.po_arg[i];
-        if ((s.kind == MI355_PO_BINARY || s.kind == MI355_PO_PRELU || s.kind == MI355_PO_SELECT_COND) && !o.p) {
+        const int kind = d.post_ops[i].kind;
+        P.po[i].p = a.po_arg[i];
+        if ((kind == MI355_PO_BINARY || kind == MI355_PO_PRELU || kind == MI355_PO_SELECT_COND) && !a.po_arg[i]) {
             set_error("missing post-op argument %d", i);
             return MI355_INVALID_ARGUMENTS;
         }
-        if (s.kind == MI355_PO_SUM && P.sum_dt == MI355_DT_UNDEF)
-            P.sum_dt = s.dt ? s.dt : d.dst_dt;
     }
     return MI355_SUCCESS;
 }

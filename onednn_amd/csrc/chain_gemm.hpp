@@ -53,6 +53,10 @@ struct chain_t {
 // bt, lda, ldb, the batches' strides, kbytes, block scales, colsum) is the family's to fill in.  scaled: src and
 // weights scales are the epilogue's; full: activations other than relu and the bf16 tensor are carried.
 bool chain_from(const problem_t &P, bool scaled, bool full, chain_t &C);
+// ... in two parts: what the descriptor decides (problem_of_desc, kernels.hpp, is enough of a problem), and whether dst lies
+// where whole pieces of its rows can be stored
+bool chain_form(const problem_t &P, bool scaled, bool full, chain_t &C);
+inline bool chain_dst_aligned(const chain_t &C, int dst_dt) { return ((uintptr_t)C.dst & (dt_bits(dst_dt) == 8 ? 3 : 15)) == 0; }
 
 // the same for a family with block scales: where mx is set they are operands of the instruction
 bool chain_from_mx(const problem_t &P, bool mx, bool full, chain_t &C);

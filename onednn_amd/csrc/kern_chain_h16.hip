@@ -5,7 +5,7 @@
 
 namespace mi355 {
 
-bool chain_from(const problem_t &P, bool scaled, bool full, chain_t &C) {
+bool chain_form(const problem_t &P, bool scaled, bool full, chain_t &C) {
     const int db = dt_bits(P.dst_dt);
     if (P.dst_dt != MI355_DT_BF16 && P.dst_dt != MI355_DT_F16 && P.dst_dt != MI355_DT_F32 && !is_int8_dt(P.dst_dt)) return false;
     if (P.rnd_flags || P.dst_dynamic || P.dst_zp.dt != MI355_DT_UNDEF || P.ds[2] != 1) return false;
@@ -15,7 +15,7 @@ bool chain_from(const problem_t &P, bool scaled, bool full, chain_t &C) {
     C.dst = (char *)P.dst;
     C.dst_pitch = P.ds[1] * esz;
     C.dst_bs = P.B > 1 ? P.ds[0] * esz : 0;
-    if (((uintptr_t)C.dst | (uintptr_t)C.dst_pitch | (uintptr_t)C.dst_bs) & (uintptr_t)(align - 1)) return false;
+    if ((C.dst_pitch | C.dst_bs) & (align - 1)) return false;
     C.M = P.M;
     C.N = P.N;
     auto readable = [](int dt) { return dt == MI355_DT_F32 || dt == MI355_DT_BF16 || dt == MI355_DT_F16; };
@@ -69,6 +69,10 @@ bool chain_from(const problem_t &P, bool scaled, bool full, chain_t &C) {
         ++at;
     }
     return at == P.n_po;
+}
+
+bool chain_from(const problem_t &P, bool scaled, bool full, chain_t &C) {
+    return chain_form(P, scaled, full, C) && chain_dst_aligned(C, P.dst_dt);
 }
 
 bool chain_from_mx(const problem_t &P, bool mx, bool full, chain_t &C) {

@@ -320,32 +320,47 @@ struct i8_plan_t {
     long Bw, Bs;
 };
 
-i8_plan_t make_plan(const mi355_matmul_desc_t &d) {
+// The epilogue as a chain of chain_gemm.hpp that the int8 kernels have, as far as the descriptor tells (where dst lies is the
+// launch's to look at); false: the general kernels.
+bool i8_chain(const problem_t &P, chain_t &C) {
+    return P.wei_dt == MI355_DT_S8 && P.wei_zp.dt == MI355_DT_UNDEF && (P.src_zp.dt == MI355_DT_UNDEF || P.src_zp.dt == MI355_DT_S32)
+            && P.dst_dt != MI355_DT_F16 && chain_form(P, true, false, C);
+}
+
+// The small tiles' time grows with their number, the LDS tiles' -- up to 128 of them -- hardly at all, so the line between
+// the two is a number of small tiles.  (Not of large ones: a short M fills few rows of a large tile.)  What moves it, with
+// small against LDS tiles in us:
+//   K       1024 tiles (256 x 4096, s8 -> s8 with K = 1024 / 4096 / 16384): 10.7 / 14.5, 31.5 / 26.0, 115 / 74
+//   a K that ends inside 64 bytes: the small tiles' rows then start in different channels, and the LDS tiles have a
+//           partial last step (the same with K = 1040 / 4112 / 16400): 8.8 / 15.4, 25.4 / 27.2, 89 / 107
+//   sums    that are kernels of their own in front of the LDS tiles (u8 -> bf16, 256 x 4096 x 4096): 31.9 / 34.8 against 31.5 /
+//           26.0 without
+//   the general epilogue, 4 us of a launch of small tiles and 8 to 12 of LDS tiles (f16 dst, 256 x 6144 x 1024): 21.5 /
+//           23.5 against 14.4 / 14.7 of a chain
+//   up to 32 rows: an LDS tile is seven eighths empty or more, and a second round of them costs as much as the first (16 x
+//           65536 x 1024, s8 -> s8): 18.2 / 23.1 against 18.1 / 14.7 for 256 x 8192
+// The lines lie where the two meet in a grid of 12 K x 7 M x 11 numbers of tiles x 4 epilogues, the lowest over the M of a
+// row; the choice is within 1.1 times the better one's time nearly everywhere.
+bool small_tiles_better(const mi355_matmul_desc_t &d, bool chain) {
+    constexpr int ALL = 1 << 30;
+    static const int line[2][2][2][2][5] = {
+            // [32 rows or fewer][whole 64 bytes of K][general epilogue][sums][K < 512, < 2048, < 4096, < 8192, longer]
+            {{{{1793, 2049, 1537, 1025, 1025}, {2561, 3073, 2049, 1537, 1153}}, {{1793, 2049, 1537, 1281, 1025}, {2561, 2561, 2049, 1537, 1153}}},
+                    {{{897, 1281, 1025, 769, 513}, {1281, 1793, 1281, 1025, 769}}, {{1281, 1537, 1025, 769, 641}, {1537, 2049, 1537, 1153, 769}}}},
+            {{{{ALL, ALL, ALL, 2049, 1153}, {ALL, ALL, ALL, 2561, 2049}}, {{ALL, ALL, ALL, 2049, 1153}, {ALL, ALL, ALL, 2561, 1281}}},
+                    {{{1025, ALL, ALL, 1025, 769}, {1024, ALL, ALL, 2561, 2049}}, {{1281, ALL, ALL, 1025, 769}, {ALL, ALL, ALL, 1537, 1025}}}}};
+    const bool sums = d.src_dt == MI355_DT_U8 || d.wei_dt == MI355_DT_U8 || !quant_absent(d.src_zp) || !quant_absent(d.wei_zp);
+    const int band = d.K < 512 ? 0 : d.K < 2048 ? 1 : d.K < 4096 ? 2 : d.K < 8192 ? 3 : 4;
+    return ((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch < line[d.M <= 32][d.K % BK == 0][!chain][sums][band];
+}
+
+// chain: what i8_chain says, the same of the descriptor's problem and of the launch's
+i8_plan_t make_plan(const mi355_matmul_desc_t &d, bool chain) {
     i8_plan_t p {};
     p.Bw = d.wei_stride[0] ? d.batch : 1;
     p.Bs = d.src_stride[0] ? d.batch : 1;
     p.need_transpose = !(d.wei_stride[1] == 1);
-    // the small tiles when the LDS tiles would occupy too little of the device (the
-    // small tiles compute their own sums and have no dynamic dst quantization).  Up to 128 large tiles the LDS
-    // tiles' time depends on K alone; the small tiles' grows with their number, in
-    // steps of three a CU.  Counted in small tiles and not in large ones, because a
-    // short M fills few rows of a large tile.  With a chain of chain_gemm.hpp on both
-    // (bf16 dst; K = 512 / 1024 / 4096 / 16384), small against LDS tiles: 6.4 / 6.6 / 17.2 / 60
-    // us against 12.1 / 14.2 / 25.6 / 72 on 512 of them, 8.5 / 8.8 / 24.9 / 86 against 12.6 /
-    // 14.7 / 26.1 / 74 on 768, 10.7 / 10.7 / 31.9 / 116 against 12.5 / 14.6 / 26.0 / 74 on
-    // 1024, 19.1 / 18.5 / 59 against 12.8 / 14.8 / 26.9 on 2048.  With zero points, whose
-    // sums are a kernel of their own in front of the LDS tiles (f32 dst), the latter take
-    // 19 / 22 / 37 / 105.  Other epilogues cost the small tiles about 4 us more a launch and
-    // the LDS tiles about 8.
-    const long small_tiles = ((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch;
-    const bool sums = d.src_dt == MI355_DT_U8 || d.wei_dt == MI355_DT_U8 || !quant_absent(d.src_zp) || !quant_absent(d.wei_zp);
-    const bool chain = (is_int8_dt(d.dst_dt) || d.dst_dt == MI355_DT_BF16 || d.dst_dt == MI355_DT_F32) && quant_absent(d.dst_zp)
-            && (d.n_post_ops == 0
-                    || (d.n_post_ops == 1 && d.post_ops[0].kind == MI355_PO_ELTWISE && d.post_ops[0].alg == MI355_ELTWISE_RELU));
-    const long crossover = !chain ? 1024
-            : sums                ? (d.K < 512 ? 1024 : d.K < 2048 ? 1793 : d.K <= 8192 ? 1153 : 897)
-                                  : (d.K < 512 ? 1025 : d.K < 2048 ? 1281 : d.K <= 8192 ? 769 : 513);
-    p.small = !d.dst_scale_dynamic && small_tiles < crossover;
+    p.small = !d.dst_scale_dynamic && small_tiles_better(d, chain);
     // the MI355_I8_TILES switch overrides the choice where both can run (tests and
     // tuning): large = the LDS tiles, 256 x 128 or 256 x 256 by the number of
     // tiles; wide = the 256 x 256 ones
@@ -402,12 +417,17 @@ int i8_supported(const mi355_matmul_desc_t &d) {
 }
 
 size_t i8_scratch_bytes(const mi355_matmul_desc_t &d) {
-    return make_plan(d).total;
+    problem_t P;
+    problem_of_desc(d, P);
+    chain_t C;
+    return make_plan(d, i8_chain(P, C)).total;
 }
 
 int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         hipStream_t stream) {
-    const i8_plan_t plan = make_plan(d);
+    chain_t C {};
+    bool chain = i8_chain(P, C);
+    const i8_plan_t plan = make_plan(d, chain);
     if (plan.total > 0 && !scratch) {
         set_error("mfma_i8: %zu bytes of scratch required", plan.total);
         return MI355_INVALID_ARGUMENTS;
@@ -440,9 +460,7 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         X.rowsum = rs;
     }
     const bool su = d.src_dt == MI355_DT_U8, wu = d.wei_dt == MI355_DT_U8;
-    chain_t C {};
-    const bool chain = !wu && P.wei_zp.dt == MI355_DT_UNDEF && (P.src_zp.dt == MI355_DT_UNDEF || P.src_zp.dt == MI355_DT_S32)
-            && chain_from(P, true, false, C);
+    chain = chain && chain_dst_aligned(C, P.dst_dt);
     if (chain) {
         C.a = (const char *)P.src; C.lda = P.ss[1]; C.a_bs = P.ss[0];
         C.bt = (const char *)X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;

@@ -46,6 +46,9 @@ int f8_launch_narrow(int fa, int fb, const problem_t &P, const char *bt, long ld
 
 void set_error(const char *fmt, ...);
 
+// the problem of a descriptor, its pointers null: what a plan can know before the launch
+void problem_of_desc(const mi355_matmul_desc_t &d, problem_t &P);
+
 // Tuning switches (tests and measurements force a tile geometry where several can run a problem).  Each starts from
 // the environment variable of its name, read once per process, and changes only through mi355_tuning_set: no getenv on a
 // launch path.  Values: 0 = the library's own choice.

@@ -99,6 +99,19 @@ def test_int8_sums_of_a_batch_are_one_launch(gpu, src_dt, wei_dt, dims):
     assert with_sums <= plain + 20, (with_sums, plain)
 
 
+# what decides between the small and the LDS tiles: K, whole 64 bytes of it or not, M, sums of their own and the epilogue.  (u8
+# weights, a zero point that is not s32 and relu with a slope are the general kernels'.)
+@pytest.mark.parametrize("M,N,K", [(256, 4096, 8208), (256, 6144, 1040), (256, 4096, 4112), (256, 5120, 1024), (256, 3840, 16384),
+                                   (16, 32768, 2176), (32, 49152, 1040)])
+@pytest.mark.parametrize("form", ["s8", "u8 src", "u8 weights", "f16 dst", "slope"])
+def test_int8_small_or_lds_tiles(gpu, M, N, K, form):
+    kw = {"s8": dict(dst_dt=cabi.DT_S8, dst_scale=20.0), "u8 src": dict(src_dt=cabi.DT_U8), "u8 weights": dict(wei_dt=cabi.DT_U8),
+          "f16 dst": dict(dst_dt=cabi.DT_F16), "slope": dict(post_ops=[PostOp(kind=cabi.PO_ELTWISE, alg=cabi.ELTWISE["relu"], alpha=0.1)])}
+    p = int8_problem(M, N, K, **{**dict(src_dt=cabi.DT_S8, wei_dt=cabi.DT_S8, dst_dt=cabi.DT_BF16), **kw[form]})
+    chosen, small, lds = in_turn(*(launches(p, "MI355_I8_TILES", tiles) for tiles in (None, "small", "large")))
+    assert chosen <= 1.12 * min(small, lds), (chosen, small, lds)
+
+
 @pytest.mark.parametrize("pitch,offset", [(8196, 0), (8192, 4), (8200, 8)])
 def test_transposition_out_of_rows_that_are_4_byte_aligned(gpu, pitch, offset):
     """Four elements a load: about half of what rows off a 4-byte boundary, an element a load, take."""
