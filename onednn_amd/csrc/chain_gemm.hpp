@@ -172,14 +172,16 @@ struct chain_part_t {
         typedef const v4f __attribute__((address_space(3))) *lds_v4f_t;
         return *(lds_v4f_t)(size_t)(tab + (unsigned)((slot * 256 + col0 + 16 * k + 4 * (lane >> 4)) * 4));
     }
-    template <int DST, int ACT, class V>
+    // STAGED: the chain may have a bf16 tensor
+    template <int DST, int ACT, bool STAGED, class V>
     __device__ __forceinline__ void store(const V (&acc)[8][4]) const {
         constexpr int SHIFT = DST == CHAIN_I8 ? 0 : DST == CHAIN_F32 ? 2 : 1;
+        const bool staged = STAGED && C.staged;
         const int lrow = lane & 15;
         const long rows_left = C.M - m_base, cols_left = C.N - n_base;
         if (rows_left <= 0 || cols_left <= 0) return;
         char *base = C.dst + b * C.dst_bs + m_base * C.dst_pitch + (n_base << SHIFT);
-        if (SHIFT == 1 && C.staged) {
+        if (staged) {
             const char *from = scalar_ptr(C.st + b * C.st_bs + m_base * C.st_pitch + n_base * 2);
             // (columns in whole chunks, chain_from; those beyond N repeat the last chunk, rows beyond M the last row)
             const int last = (int)(cols_left < 64 ? cols_left : 64) / 8 - 1;
@@ -205,7 +207,7 @@ struct chain_part_t {
         for (int i = 0; i < 8; ++i) {
             const int r = 16 * i + lrow;
             if (Mma::SCALED && C.ssc.per) ssc = chain_load(C.ssc, b * C.ssc.bs + m_base + (r < rows_left ? r : rows_left - 1));
-            if (SHIFT == 1 && C.staged) {
+            if (staged) {
                 wait_vmcnt_upto(14 - 2 * i); // the two loads of this row block have landed
                 asm volatile("" ::: "memory"); // no LDS read moves above the wait
             }
@@ -244,7 +246,7 @@ struct chain_part_t {
                     }
                     x[k][e] = t;
                 }
-            if (SHIFT == 1 && C.staged) {
+            if (staged) {
                 const bool add = C.staged == 1;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
@@ -368,14 +370,25 @@ __global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu
         const float as = fabsf(E.ds);
         E.ds_mode = C.ds_mode == 2 ? 2 : as >= 0x1p-20f && as <= 0x1p20f ? 3 : 1;
     }
-    if constexpr (DST == CHAIN_I8 || DST == CHAIN_F32 || !Mma::FULL) {
-        if (C.act == CHAIN_RELU) E.template store<DST, CHAIN_RELU>(acc);
-        else E.template store<DST, CHAIN_NONE>(acc);
+    constexpr bool FULL = DST != CHAIN_I8 && DST != CHAIN_F32 && Mma::FULL;
+    // A launch of few steps is bound by its epilogue's instruction fetches, and the second tensor's code is in the way of a
+    // chain without one: the 16-bit types have both (1 x 512 x 64, bf16: 9.4 -> 8.4 us).  fp8's scales leave no registers
+    // for that (4096 x 28672 x 8192 with gelu and residual: 706 -> 723 us, 72 bytes a lane in scratch memory).
+    constexpr bool BOTH = FULL && !Mma::SCALED && Mma::SCALE_SETS == 0;
+    auto store = [&](auto staged) __attribute__((always_inline)) {
+        constexpr bool S = decltype(staged)::value;
+        if constexpr (FULL) {
+            if (C.act == CHAIN_GELU) return E.template store<DST, CHAIN_GELU, S>(acc);
+            if (C.act == CHAIN_SWISH) return E.template store<DST, CHAIN_SWISH, S>(acc);
+        }
+        if (C.act == CHAIN_RELU) E.template store<DST, CHAIN_RELU, S>(acc);
+        else E.template store<DST, CHAIN_NONE, S>(acc);
+    };
+    if constexpr (BOTH) {
+        if (C.staged) store(std::true_type {});
+        else store(std::false_type {});
     } else {
-        if (C.act == CHAIN_GELU) E.template store<DST, CHAIN_GELU>(acc);
-        else if (C.act == CHAIN_SWISH) E.template store<DST, CHAIN_SWISH>(acc);
-        else if (C.act == CHAIN_RELU) E.template store<DST, CHAIN_RELU>(acc);
-        else E.template store<DST, CHAIN_NONE>(acc);
+        store(std::integral_constant<bool, FULL> {});
     }
 }
 

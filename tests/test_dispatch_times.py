@@ -145,11 +145,20 @@ def test_a_dst_of_the_other_16_bit_type(gpu, M, N, K, dt, ddt):
     assert mixed <= 1.15 * same, (mixed, same)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 512, 64), (64, 4096, 128)])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_a_16_bit_dst_of_a_small_product(gpu, M, N, K, dt):
+    """A launch of one round and few steps is its epilogue's instruction fetches: against an f32 dst, which knows no second
+    tensor, 1.1 to 1.6 us for the conversion; 2.1 to 2.6 with that tensor's code in the way of a chain that has none."""
+    half, f32 = in_turn(*(launches(float_problem(M, N, K, dt, d)) for d in (dt, "f32")))
+    assert half <= f32 + 1.9, (half, f32)
+
+
 @pytest.mark.parametrize("M,N,K", [(1024, 4096, 512), (64, 4096, 1024), (4096, 4096, 256)])
 @pytest.mark.parametrize("act,residual", [(True, False), (False, True), (True, True)])
 def test_mxfp8_layers_with_an_activation_or_a_residual(gpu, M, N, K, act, residual):
-    """Against the same sums with a bias alone.  The two together are a tile more to read and about 20 instructions an
-    element more, 4 us at most of these 17 to 24; through the general epilogue they cost 13 to 20."""
+    """Against the same sums with a bias alone.  The two together are a tensor more to read (at 5 TB/s), behind a latency of
+    its own, and about 20 instructions an element more (5.5 us in all); through the general epilogue they cost 13 to 20."""
     def scaled(**kw):
         p = float_problem(M, N, K, "f8_e4m3", "bf16", bias_dt=cabi.DT_BF16, bias=np.zeros(N, np.uint16), **kw)
         for name, rows, groups in (("src_scale", M, (1, 32)), ("wei_scale", N, (32, 1))):
@@ -160,7 +169,7 @@ def test_mxfp8_layers_with_an_activation_or_a_residual(gpu, M, N, K, act, residu
     if residual:
         post.append(PostOp(cabi.PO_BINARY, alg=cabi.BINARY["add"], dt=cabi.DT_BF16, stride=(0, N, 1), data=np.zeros(M * N, np.uint16)))
     with_post, plain = in_turn(scaled(post_ops=post), scaled())
-    assert with_post <= 1.35 * plain, (with_post, plain)
+    assert with_post <= plain + (2 * M * N / 5e6 if residual else 0) + 5.5, (with_post, plain)
 
 
 @pytest.mark.parametrize("M,N,K", [(64, 4096, 1024), (512, 4096, 1024), (1024, 4096, 512), (64, 4096, 4096)])
