@@ -577,6 +577,10 @@ int mi355_matmul_launch_noalloc(const mi355_matmul_desc_t *desc, const mi355_mat
     size_t bytes = 0;
     int st = mi355_matmul_scratch_bytes(desc, &bytes);
     if (st) return st;
+    int impl = 0;
+    if (bytes > (size_t)MI355_NOALLOC_SCRATCH_BYTES && choose_impl(*desc, &impl) == MI355_SUCCESS && impl == MI355_IMPL_I8_MFMA
+            && i8_scratch_optional(*desc))
+        bytes = 0;
     if (bytes > (size_t)MI355_NOALLOC_SCRATCH_BYTES) {
         set_error("mi355_matmul_launch_noalloc: the problem needs %zu bytes of scratch, the static buffer holds %zu "
                   "(use mi355_matmul_launch with a caller-owned buffer, or K-contiguous weights)",

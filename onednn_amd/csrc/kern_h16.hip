@@ -221,7 +221,7 @@ static int h16_down_dt(const mi355_matmul_desc_t &d) {
 // K to Kp, K rounded up to whole chunks -- so any K and any plain layout with a unit stride runs here, at the price of
 // the copy.  pitch: elements between the rows of a copy, whole 64 bytes.
 struct h16_plan_t {
-    bool ok, woq;
+    bool ok, woq, inside;
     int op_dt;
     long EB, Kp, pitch, Bs, Bw;
     bool copy_src, copy_wei;
@@ -252,13 +252,13 @@ static h16_plan_t h16_plan(const mi355_matmul_desc_t &d) {
     // byte offsets inside a tile are 32-bit
     const long lda = p.copy_src ? p.pitch : d.src_stride[1], ldb = p.copy_wei ? p.pitch : d.wei_stride[2];
     if (lda * p.EB * BM >= (1L << 31) || ldb * p.EB * f8_geo_t::BN >= (1L << 31)) return p;
-    // (a K that ends inside 64 bytes is read where it lies as well; the scratch such a problem asks for, room for the
-    // copies, stays what callers that allocate by it have been told)
-    const bool inside = p.pitch != d.K;
+    // (a K that ends inside 64 bytes is read where it lies as well, but copied where it starts off a 16-byte boundary, which
+    // only the launch can see: its scratch has room for that)
+    p.inside = p.pitch != d.K;
     size_t off = 0;
-    if (p.copy_src || inside) off += align_up((size_t)p.Bs * d.M * p.pitch * p.EB, 256);
+    if (p.copy_src || p.inside) off += align_up((size_t)p.Bs * d.M * p.pitch * p.EB, 256);
     p.off_wei = off;
-    if (p.copy_wei || inside) off += align_up((size_t)p.Bw * d.N * p.pitch * p.EB, 256);
+    if (p.copy_wei || p.inside) off += align_up((size_t)p.Bw * d.N * p.pitch * p.EB, 256);
     p.total = off;
     p.ok = true;
     return p;
@@ -382,10 +382,14 @@ static int h16_across(const mi355_matmul_desc_t &d, const h16_plan_t &p, const p
 }
 
 int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratch, hipStream_t stream) {
-    const h16_plan_t plan = h16_plan(d);
+    h16_plan_t plan = h16_plan(d);
     if (!plan.ok) {
         set_error("mfma_h16: the problem is not one this family takes");
         return MI355_UNIMPLEMENTED;
+    }
+    if (plan.inside) {
+        plan.copy_src |= ((uintptr_t)P_in.src & 15) != 0;
+        plan.copy_wei |= ((uintptr_t)P_in.wei & 15) != 0;
     }
     if ((plan.copy_src || plan.copy_wei) && !scratch) {
         set_error("mfma_h16: %zu bytes of scratch required", plan.total);

@@ -416,6 +416,8 @@ int i8_supported(const mi355_matmul_desc_t &d) {
     return MI355_SUCCESS;
 }
 
+bool i8_scratch_optional(const mi355_matmul_desc_t &d) { return d.K % BK != 0 && d.wei_stride[1] == 1; }
+
 size_t i8_scratch_bytes(const mi355_matmul_desc_t &d) {
     problem_t P;
     problem_of_desc(d, P);
@@ -427,7 +429,14 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         hipStream_t stream) {
     chain_t C {};
     bool chain = i8_chain(P, C);
-    const i8_plan_t plan = make_plan(d, chain);
+    i8_plan_t plan = make_plan(d, chain);
+    // A K that ends inside 64 bytes also takes operands off 16-byte boundaries, which the LDS tiles' loads cannot, and
+    // K-contiguous weights without scratch: the small tiles'.
+    if (!plan.small && d.K % BK != 0) {
+        const uintptr_t at = (uintptr_t)P.src | (plan.need_transpose ? 0 : (uintptr_t)P.wei);
+        if ((at & 15) || (!scratch && i8_scratch_optional(d))) plan.small = true, plan.need_colsum = plan.need_rowsum = false;
+        if (i8_scratch_optional(d)) plan.total = 0;
+    }
     if (plan.total > 0 && !scratch) {
         set_error("mfma_i8: %zu bytes of scratch required", plan.total);
         return MI355_INVALID_ARGUMENTS;

@@ -14,6 +14,7 @@ int ref_launch(const problem_t &P, hipStream_t stream);
 
 int i8_supported(const mi355_matmul_desc_t &d);
 size_t i8_scratch_bytes(const mi355_matmul_desc_t &d);
+bool i8_scratch_optional(const mi355_matmul_desc_t &d); // i8_launch takes a null scratch all the same
 int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         hipStream_t stream);
 
