@@ -342,6 +342,8 @@ const char *mi355_last_error(void); /* thread-local text of the last failure */
  *                      instruction for 16-bit types too, tall / wide = a workgroup takes one / eight
  *                      column tiles in turn)
  *   MI355_GEMM_ORDER   0..63                  tile order of the large GEMMs
+ *   MI355_EPILOGUE     chain                  MI355_UNIMPLEMENTED where a GEMM would run a kernel with the general
+ *                      epilogue instead of a compiled-in one
  * value NULL, "" or "auto" restores the library's own choice.  A switch can
  * change a problem's scratch need (the 32 x 32 int8 tiles need none, the LDS
  * tiles want column / row sums): set it before mi355_matmul_scratch_bytes, not

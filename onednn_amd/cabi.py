@@ -349,7 +349,7 @@ def scratch_bytes(desc):
 
 def tuning_set(name, value=None):
     """Set one of the library's tuning switches (MI355_I8_TILES, MI355_F8_TILES, MI355_H16_TILES,
-    MI355_GROUPED_IMPL, MI355_GEMM_ORDER); None restores the library's own choice.  The switches start from the
+    MI355_GROUPED_IMPL, MI355_GEMM_ORDER, MI355_EPILOGUE); None restores the library's own choice.  The switches start from the
     environment variables of the same names, read once per process."""
     lib = load_kernels()
     check(lib.mi355_tuning_set(name.encode(), None if value is None else str(value).encode()))

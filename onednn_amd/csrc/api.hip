@@ -36,6 +36,7 @@ const tune_name_t TUNE_NAMES[TUNE_COUNT] = {
         {"MI355_H16_TILES", "wide"},
         {"MI355_GROUPED_IMPL", "ref short tall wide"},
         {"MI355_GEMM_ORDER", ""},
+        {"MI355_EPILOGUE", "chain"},
 };
 std::atomic<int> g_tune[TUNE_COUNT];
 std::once_flag g_tune_once;
@@ -52,7 +53,7 @@ int tune_parse(int key, const char *v) {
         const char *w;
         int val;
     } words[] = {{"large", TUNE_LARGE}, {"wide", TUNE_WIDE}, {"small", TUNE_SMALL}, {"ref", TUNE_REF},
-            {"short", TUNE_SHORT}, {"tall", TUNE_TALL}, {"narrow", TUNE_NARROW}};
+            {"short", TUNE_SHORT}, {"tall", TUNE_TALL}, {"narrow", TUNE_NARROW}, {"chain", TUNE_CHAIN}};
     for (const auto &w : words) {
         if (strcmp(v, w.w)) continue;
         const char *hit = strstr(TUNE_NAMES[key].values, v);

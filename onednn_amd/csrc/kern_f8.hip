@@ -131,6 +131,7 @@ int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, h
                                : chain_launch_f8(P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }
+    if (general_refused("mfma_f8")) return MI355_UNIMPLEMENTED;
     if (narrow && !plan.mx) return f8_launch_narrow(fa, fb, P, X.bt, X.ldb, X.bt_bstride, (unsigned)d.batch, stream);
     X.tiles_m = (int)((d.M + BM - 1) / BM);
     X.tiles_n = (int)((d.N + f8_geo_t::BN - 1) / f8_geo_t::BN);

@@ -493,6 +493,7 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
         const int st = chain_launch_h16(plan.op_dt == MI355_DT_BF16, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }
+    if (general_refused("mfma_h16")) return MI355_UNIMPLEMENTED;
     using bf16_t = h16x16_mma_t<true, f8_geo_t>;
     using bf16_narrow_t = h16x16_mma_t<true, narrow_t>;
     using f16_t = h16x16_mma_t<false, f8_geo_t>;

@@ -484,6 +484,7 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
             const int st = chain_launch_i8_small(su, P.dst_dt, C, (unsigned)d.batch, stream);
             if (st != MI355_UNIMPLEMENTED) return st;
         }
+        if (general_refused("mfma_i8")) return MI355_UNIMPLEMENTED;
         X.tiles_m = (int)((d.M + ST - 1) / ST);
         X.tiles_n = (int)((d.N + ST - 1) / ST);
         const long tiles = (long)X.tiles_m * X.tiles_n;
@@ -508,6 +509,7 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         const int st = chain_launch_i8(su, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }
+    if (general_refused("mfma_i8")) return MI355_UNIMPLEMENTED;
     X.tiles_m = (int)((d.M + BM - 1) / BM);
     auto go = [&](auto su_, auto wu_) -> int {
         constexpr bool SU = decltype(su_)::value, WU = decltype(wu_)::value;

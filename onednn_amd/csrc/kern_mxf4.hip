@@ -276,6 +276,7 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         const int st = chain_launch_mx(true, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }
+    if (general_refused("mfma_mxf4")) return MI355_UNIMPLEMENTED;
     X.tiles_m = (int)((d.M + BM - 1) / BM);
     auto go = [&](auto geo) -> int {
         using G = decltype(geo);

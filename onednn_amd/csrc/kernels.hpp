@@ -45,17 +45,24 @@ int woqp_launch(const mi355_matmul_desc_t &d, const problem_t &P, hipStream_t st
 // the family's instantiations side by side); bt = the weights as [N][K] bytes, K contiguous
 int f8_launch_narrow(int fa, int fb, const problem_t &P, const char *bt, long ldb, long bt_bstride, unsigned batch, hipStream_t stream);
 
-void set_error(const char *fmt, ...);
-
 // the problem of a descriptor, its pointers null: what a plan can know before the launch
 void problem_of_desc(const mi355_matmul_desc_t &d, problem_t &P);
 
 // Tuning switches (tests and measurements force a tile geometry where several can run a problem).  Each starts from
 // the environment variable of its name, read once per process, and changes only through mi355_tuning_set: no getenv on a
 // launch path.  Values: 0 = the library's own choice.
-enum tune_key_t { TUNE_I8_TILES = 0, TUNE_F8_TILES, TUNE_H16_TILES, TUNE_GROUPED_IMPL, TUNE_GEMM_ORDER, TUNE_COUNT };
-enum { TUNE_AUTO = 0, TUNE_LARGE = 1, TUNE_WIDE = 2, TUNE_SMALL = 3, TUNE_REF = 4, TUNE_SHORT = 5, TUNE_TALL = 6, TUNE_NARROW = 7 };
+enum tune_key_t { TUNE_I8_TILES = 0, TUNE_F8_TILES, TUNE_H16_TILES, TUNE_GROUPED_IMPL, TUNE_GEMM_ORDER, TUNE_EPILOGUE, TUNE_COUNT };
+enum { TUNE_AUTO = 0, TUNE_LARGE = 1, TUNE_WIDE = 2, TUNE_SMALL = 3, TUNE_REF = 4, TUNE_SHORT = 5, TUNE_TALL = 6, TUNE_NARROW = 7, TUNE_CHAIN = 8 };
 int tuning(tune_key_t key);
+
+void set_error(const char *fmt, ...);
+
+// MI355_EPILOGUE=chain: a launch that comes past the chain kernels ends here
+inline bool general_refused(const char *who) {
+    if (tuning(TUNE_EPILOGUE) != TUNE_CHAIN) return false;
+    set_error("%s: the epilogue is not a chain (MI355_EPILOGUE=chain)", who);
+    return true;
+}
 
 // hipFuncSetAttribute(MaxDynamicSharedMemorySize) for a kernel, once per
 // (kernel, device, size) of this process.  Safe to call from several host

@@ -9,7 +9,7 @@ import pytest
 
 from onednn_amd import cabi, configs
 from onednn_amd import dtypes as dtp
-from onednn_amd.problem import MatmulProblem, PostOp, QuantParam, run_gpu, strides_for
+from onednn_amd.problem import MatmulProblem, PostOp, QuantParam, decode, run_gpu, storage_dtype, strides_for
 from tests.helpers import assert_bit_exact
 
 pytestmark = pytest.mark.gpu
@@ -49,15 +49,17 @@ def problem(M, N, K, dt, ddt, *, bias=False, post=(), batch=1, pitch=0, dst_scal
         quant["dst_scale"] = QuantParam(cabi.DT_F32, 0, np.array([dst_scale], np.float32))
     b = (r.integers(-8, 9, size=N) / 4).astype(np.float32) if bias else None
     kw = {}
-    if pitch:
-        kw = dict(dst_stride=(M * pitch, pitch, 1), dst_init=np.zeros(batch * M * pitch, np.uint16))
+    if pitch:  # what lies between the rows stays as it is
+        kw = dict(dst_stride=(M * pitch, pitch, 1),
+                  dst_init=np.full((batch * M - 1) * pitch + N, 0x5A, storage_dtype(DT[ddt])))
     return MatmulProblem(M=M, N=N, K=K, batch=batch, src_dt=DT[dt], wei_dt=DT[wdt], dst_dt=DT[ddt], src=src, wei=wei,
                          wei_stride=strides_for("ba", batch, K, N), bias_dt=cabi.DT_F32 if bias else cabi.DT_UNDEF, bias=b,
                          quant=quant, post_ops=list(post), name=f"lines-{dt}-{ddt}-{M}x{N}x{K}", **kw)
 
 
-def check(oracle, p, dt, tiles=None):
-    with cabi.tuning(SWITCH[dt], tiles):
+def check(oracle, p, dt, tiles=None, chain=False):
+    """chain: a compiled-in epilogue's kernel or an error"""
+    with cabi.tuning(SWITCH[dt], tiles), cabi.tuning("MI355_EPILOGUE", "chain" if chain else None):
         got, name = run_gpu(p)
     assert name.startswith(FAMILY[dt]), name
     assert_bit_exact(p, got, oracle.run_oracle(p), f"{name} {tiles}")
@@ -75,8 +77,8 @@ def test_where_the_steps_end(gpu, oracle, kbytes, dt, ddt, tiles):
 RELU = PostOp(cabi.PO_ELTWISE, alg=cabi.ELTWISE["relu"], alpha=0.0)
 
 
-# rows of dst that end inside a wavefront's 64 columns or a 16-byte piece, dst pitches of whole and of no whole pieces,
-# M inside a wavefront's 128 rows, every compiled-in dst type, batches
+# rows of dst that end inside a wavefront's 64 columns, dense ones of whole and of no whole 16-byte pieces (a 16-bit or f32
+# dst of the latter is the general epilogue's), M inside a wavefront's 128 rows, every compiled-in dst type, batches
 @pytest.mark.parametrize("M,N", [(1, 136), (129, 200), (130, 268), (257, 388)])
 @pytest.mark.parametrize("dt,ddt,kw", [
     ("bf16", "bf16", {}), ("bf16", "f32", dict(bias=True)), ("f16", "f16", dict(bias=True, post=[RELU])),
@@ -89,28 +91,48 @@ def test_where_the_rows_of_dst_end(gpu, oracle, M, N, dt, ddt, kw):
         check(oracle, p, dt, "wide" if tiles == "wide" else None if BYTES[dt] == 2 else "narrow")
 
 
+# ... and that end inside a 16-byte piece of a pitch of whole ones (8-bit: of dwords, too): every length of the last piece,
+# on each tile's chain
+@pytest.mark.parametrize("dt,ddt,kw", [
+    ("bf16", "bf16", dict(bias=True)), ("bf16", "f16", {}), ("f16", "f16", dict(post=[RELU])), ("f16", "f32", {}),
+    ("s8", "s8", dict(post=[RELU], dst_scale=3.0)), ("s8", "f32", dict(bias=True)), ("u8", "u8", dict(bias=True, src_zp=5)),
+    ("u8", "bf16", dict(src_zp=2)), ("f8_e4m3", "bf16", dict(row_scales=True)), ("f8_e4m3", "f32", {})])
+@pytest.mark.parametrize("N", [257, 258, 259, 260, 261, 262, 263, 195])
+def test_rows_of_dst_that_end_inside_a_piece(gpu, oracle, dt, ddt, kw, N):
+    piece = {"f32": 4, "s8": 16, "u8": 16}.get(ddt, 8)
+    for tiles in ("wide", "narrow", "small")[:3 if BYTES[dt] == 1 and dt != "f8_e4m3" else 2]:
+        for pitch in {-(-N // piece) * piece, -(-N // 4) * 4 if piece == 16 else -(-N // piece) * piece + piece}:
+            p = problem(131, N, 256 // BYTES[dt], dt, ddt, batch=2, pitch=pitch, **kw)
+            check(oracle, p, dt, None if BYTES[dt] == 2 and tiles == "narrow" else tiles, chain=True)
+
+
 @pytest.mark.parametrize("act", [None, "gelu_tanh", "swish"])
 @pytest.mark.parametrize("alg", ["add", "mul"])
-@pytest.mark.parametrize("dt", ["bf16", "f8_e4m3", "mxfp8"])
-def test_a_staged_tensor_at_ragged_edges(gpu, oracle, act, alg, dt):
-    """N = 200: the last wavefront's columns end after one chunk of eight; rows end inside a row block.  Without an
-    activation the sums are exact; with one the result is within the activation's few ulp of the oracle, rounded to
+@pytest.mark.parametrize("dt", ["bf16", "f8_e4m3", "f8_e4m3 rows", "mxfp8"])
+@pytest.mark.parametrize("tiles", ["wide", None])
+@pytest.mark.parametrize("M,N,batch", [(150, 200, 1), (300, 328, 2)])
+def test_a_staged_tensor_at_ragged_edges(gpu, oracle, act, alg, dt, tiles, M, N, batch):
+    """Both tiles (the narrow one by itself at these sizes); the last wavefront's columns end after one chunk of eight, rows
+    inside a row block; scales per row, whose loads the waits for the tensor's have to reckon with; a tensor of two batches.
+    Without an activation the sums are exact; with one the result is within the activation's few ulp of the oracle, rounded to
     bf16: two units of bf16."""
-    M, N, K = 150, 200, 128
+    K, rows = 128, dt.endswith("rows")
+    dt = dt.split()[0]
     r = np.random.default_rng(5)
-    other = dtp.f32_to_bf16(r.integers(-4, 5, size=M * N).astype(np.float32)).reshape(M, N)
+    other = dtp.f32_to_bf16(r.integers(-4, 5, size=batch * M * N).astype(np.float32)).reshape(batch, M, N)
     post = [PostOp(cabi.PO_ELTWISE, alg=cabi.ELTWISE[act], alpha=1.0)] if act else []
-    post.append(PostOp(cabi.PO_BINARY, alg=cabi.BINARY[alg], dt=cabi.DT_BF16, stride=(0, N, 1), data=other))
+    post.append(PostOp(cabi.PO_BINARY, alg=cabi.BINARY[alg], dt=cabi.DT_BF16, stride=(M * N, N, 1), data=other))
     if dt == "mxfp8":
         from tests.test_mxf8_gemm import problem as mx_problem
-        p = mx_problem(M, N, K, ddt="bf16", bias=True, post_ops=post)
+        p = mx_problem(M, N, K, ddt="bf16", bias=True, post_ops=post, batch=batch)
         p.quant["src_scale"].data[:] = 127 - 6
         p.quant["wei_scale"].data[:] = 127
     else:
-        p = problem(M, N, K, dt, "bf16", bias=True, post=post)
+        p = problem(M, N, K, dt, "bf16", bias=True, post=post, batch=batch, row_scales=rows)
     if dt == "f8_e4m3":
-        p.quant["src_scale"].data[:] = 1 / 64
-    got, name = run_gpu(p)
+        p.quant["src_scale"].data[:] /= 64
+    with cabi.tuning(SWITCH.get(dt, "MI355_F8_TILES"), tiles), cabi.tuning("MI355_EPILOGUE", "chain"):
+        got, name = run_gpu(p)
     assert name.startswith(FAMILY.get(dt, "hip:mfma_f8")), name
     want = oracle.run_oracle(p)
     if not act:
@@ -120,15 +142,15 @@ def test_a_staged_tensor_at_ragged_edges(gpu, oracle, act, alg, dt):
     assert np.all(np.abs(g - w) <= 2.0 ** -7 * np.abs(w) + 2.0 ** -20)
 
 
-def across_problem(M, N, K, dt, ddt, src_across, *, batch=1, wei_pad=0, src_pad=0, bias=True):
+def across_problem(M, N, K, dt, ddt, src_across, *, batch=1, wei_pad=0, src_pad=0, bias=True, pads=(77, 99)):
     """weights row-major ([K][N], a pitch of N + wei_pad), src row-major or ([K][M], a pitch of M + src_pad)"""
     r = np.random.default_rng(M * 3 + N * 5 + K)
     sv = r.integers(-3, 4, size=(batch, M, K)).astype(np.float32)
-    wv = np.full((batch, K, N + wei_pad), 99, np.float32)
+    wv = np.full((batch, K, N + wei_pad), pads[1], np.float32)
     wv[:, :, :N] = r.integers(-2, 3, size=(batch, K, N))
     ss = (M * K, K, 1)
     if src_across:
-        full = np.full((batch, K, M + src_pad), 77, np.float32)
+        full = np.full((batch, K, M + src_pad), pads[0], np.float32)
         full[:, :, :M] = sv.transpose(0, 2, 1)
         sv, ss = full, (K * (M + src_pad), 1, M + src_pad)
     b = (r.integers(-8, 9, size=N) / 4).astype(np.float32) if bias else None
@@ -188,3 +210,53 @@ def test_mxfp4_steps(gpu, oracle, K, tiles, ddt):
         got, name = run_gpu(p)
     assert name.startswith("hip:mfma_mxf4"), name
     assert_bit_exact(p, got, oracle.run_oracle(p), f"{name} {tiles}")
+
+
+def check_with_nan(oracle, p, tiles):
+    """NaN and infinities where the oracle has them, the rest bit for bit"""
+    switch = "MI355_H16_TILES" if p.src_dt in (cabi.DT_BF16, cabi.DT_F16) else "MI355_F8_TILES"
+    with cabi.tuning(switch, tiles):
+        got, name = run_gpu(p)
+    n = p.batch * p.M * p.N
+    g, w = decode(p.dst_dt, got, n), decode(p.dst_dt, oracle.run_oracle(p), n)
+    assert np.isnan(w).any() and np.isfinite(w).any()
+    assert np.array_equal(g, w, equal_nan=True), (p.name, name, tiles)
+
+
+# What lies behind K, or is loaded twice by the lanes of a partial last step, adds nothing, whatever it is: NaN behind the
+# rows of both operands, and infinities and NaN in the last chunk of some rows and columns.
+@pytest.mark.parametrize("tiles", [None, "wide"])
+@pytest.mark.parametrize("K", [8, 40, 72, 104, 136, 200, 328])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_nan_at_the_end_of_k(gpu, oracle, tiles, K, dt):
+    p = problem(300, 328, K, dt, "f32", bias=True)
+    inf, nan = (0x7F80, 0x7FC0) if dt == "bf16" else (0x7C00, 0x7E00)
+    for name, rows in (("src", 300), ("wei", 328)):
+        wide = np.full((rows, K + 24), nan, np.uint16)
+        wide[:, :K] = np.asarray(getattr(p, name)).reshape(rows, K)
+        wide[rows // 3, K - 1], wide[rows // 2, K - 5] = inf, nan
+        setattr(p, name, wide.reshape(-1))
+    p.src_stride, p.wei_stride = (0, K + 24, 1), (0, 1, K + 24)
+    check_with_nan(oracle, p, tiles)
+
+
+@pytest.mark.parametrize("tiles", [None, "wide"])
+@pytest.mark.parametrize("K", [8, 24, 40, 72, 136, 200])
+@pytest.mark.parametrize("src_across", [False, True])
+def test_nan_across_k(gpu, oracle, tiles, K, src_across):
+    p = across_problem(304, 328, K, "bf16", "f32", src_across, wei_pad=8, src_pad=16, pads=(np.nan, np.nan))
+    wei = p.wei.reshape(K, 336)
+    wei[K - 1, 17], wei[K - 3, 200] = 0x7F80, 0x7FC0
+    src = p.src.reshape(K, 320) if src_across else p.src.reshape(304, K).T
+    src[K - 1, 40], src[K - 2, 250] = 0x7F80, 0x7FC0
+    check_with_nan(oracle, p, tiles)
+
+
+@pytest.mark.parametrize("tiles", [None, "wide"])
+@pytest.mark.parametrize("K", [96, 160, 224, 288])
+def test_nan_at_the_end_of_block_scaled_k(gpu, oracle, tiles, K):
+    from tests.test_mxf8_gemm import problem as mx_problem
+    p = mx_problem(300, 328, K, seed=K)
+    p.src.reshape(300, K)[70, K - 9] = p.wei.reshape(328, K)[201, K - 2] = 0x7F
+    p.quant["src_scale"].data.reshape(300, K // 32)[155, K // 32 - 1] = 0xFF
+    check_with_nan(oracle, p, tiles)
