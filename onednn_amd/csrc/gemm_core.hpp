@@ -42,10 +42,9 @@ struct geo_t {
 
 // Chunk swizzle.  Measured on MI355X with a read-only micro-benchmark over all
 // XOR-of-row-bits functions: this one is free of bank conflicts for both
-// fragment read patterns in use (16 rows x 4 chunks across the 64 lanes, the
-// 16x16 MFMA shapes; 32 rows x 2 chunks in two reads, the 32x32 shape), where
-// e.g. ((row >> 1) & 3) ^ ((row >> 3) & 1) costs the 16-row pattern a factor
-// of two (SQ_LDS_BANK_CONFLICT = half of SQ_LDS_IDX_ACTIVE in the int8 kernel).
+// fragment read patterns of 64-byte rows (16 rows x 4 chunks across the 64
+// lanes; 32 rows x 2 chunks in two reads, what the f32 tiles' 32x32 shape reads),
+// where e.g. ((row >> 1) & 3) ^ ((row >> 3) & 1) costs the 16-row one a factor of two.
 __device__ __forceinline__ int swz_f(int row) {
     return ((row >> 2) & 1) | ((((row >> 2) ^ (row >> 3)) & 1) << 1);
 }
@@ -184,9 +183,7 @@ __device__ __forceinline__ void main_loop_two_groups(Acc &acc, char *smem, const
 
     int slot = 0;
     // Group 1 carries the fragments from one iteration to the next; they start
-    // as the operands' zero (Mma::zero_frag: bytes the MFMA row reads as 0 --
-    // not all-zero bits for an operand type whose bytes are re-biased at use), so
-    // that its first iteration, which has no stage to multiply yet, adds zero
+    // as zeros (Mma::zero_frag), so that its first iteration, which has no stage to multiply yet, adds zero
     // products instead of branching around the MFMAs (one MFMA sequence on every
     // path keeps the accumulators where they are).
     typename Mma::frag_t f = Mma::zero_frag();

@@ -16,16 +16,18 @@
 // of log2): p <= 256 loses nothing in either type.
 //
 // Two forms.  Long rows of queries (NWQ = 4): four wavefronts, 128 rows, share every tile of 64 keys through LDS, two
-// tiles in flight; two workgroups a CU, so that one's softmax runs under the other's matrix instructions.  Few rows
+// tiles in flight, two workgroups a CU.  Few rows
 // (NWQ = 1, decode): one block of 32 rows, every wavefront walks tiles of 32 keys of its own -- no barriers, 64 KB of
 // keys and values in flight a CU -- and the four partial results meet in LDS.  Queries that share one key / value head
 // are rows of one problem (row = query * heads + head).  Where that leaves CUs idle the keys are split over workgroups
 // and sdpa_combine_kernel adds the parts.
 //
-// Bound: vector arithmetic next to the matrix instructions for long queries (16 heads, 4096 x 4096, d 128, causal, bf16:
-// the composition 1221 us, of which 729 were the softmax over scores in memory, this 95 us = 725 TFLOP/s, the matrix
-// cores and the vector units busy 43 % of the time each, a wavefront waiting 24 %; 8 x 8 heads, 1918 x 2942, d 64:
-// 4024 -> 119 us); memory for few (8 x 16 heads, one query, 8192 keys: 653 -> 103 us, 5.2 TB/s; a wavefront waits 55 %).
+// Bound: for long queries the series of K Q, softmax and P V in a wavefront, behind a wait for all loads and a barrier every
+// 64 keys (16 heads, 4096 x 4096, d 128, causal, bf16: the composition 1221 us, of which 729 were the softmax over scores in
+// memory, this 91 us = 755 TFLOP/s; the matrix cores and the vector units busy 43 % of the time each, which adds up to the
+// 86 % that are not stalls: the two workgroups of a CU hardly run one's softmax under the other's products; 8 x 8 heads,
+// 1918 x 2942, d 64: 4024 -> 119 us); memory for few (8 x 16 heads, one query, 8192 keys: 653 -> 103 us, 5.2 TB/s; a wavefront
+// waits 55 %).
 // 64 rows is where the forms cross: at 64 rows half of the large form's wavefronts have none.  The form for few rows
 // reads every mask buffer element by element (the decode above: 172 us with one).
 #include "kernels.hpp"

@@ -25,7 +25,6 @@ struct h16x16_mma_t {
     using G = G_;
     static constexpr bool TILE16 = true;
     static constexpr int ELEM_BYTES = 2;
-    static constexpr bool HOT = false;
     static constexpr int ROWS = 8, COLS = G::WCOLS / 16;
     static constexpr int NU = 2, SCALE_SETS = 0;
     typedef v4f acc_t;
@@ -101,7 +100,6 @@ struct f8_mma_t {
     using G = G_;
     static constexpr bool TILE16 = true;
     static constexpr int ELEM_BYTES = 1;
-    static constexpr int HOT = 0;
     static constexpr int ROWS = 8, COLS = G::WCOLS / 16;
     static constexpr int NU = 1, SCALE_SETS = 0;
     typedef v4f acc_t;
