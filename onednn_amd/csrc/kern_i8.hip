@@ -434,8 +434,9 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
     // K-contiguous weights without scratch: the small tiles'.
     if (!plan.small && d.K % BK != 0) {
         const uintptr_t at = (uintptr_t)P.src | (plan.need_transpose ? 0 : (uintptr_t)P.wei);
-        if ((at & 15) || (!scratch && i8_scratch_optional(d))) plan.small = true, plan.need_colsum = plan.need_rowsum = false;
-        if (i8_scratch_optional(d)) plan.total = 0;
+        const bool without = plan.total > 0 && !scratch && i8_scratch_optional(d);
+        if ((at & 15) || without) plan.small = true, plan.need_colsum = plan.need_rowsum = false;
+        if (without) plan.total = 0;
     }
     if (plan.total > 0 && !scratch) {
         set_error("mfma_i8: %zu bytes of scratch required", plan.total);

@@ -183,3 +183,11 @@ def test_mxfp4_through_the_general_epilogue(gpu, M, N, K):
 
     general, chain = in_turn(launch("f16"), launch("bf16"))
     assert general <= chain + 7.5, (general, chain)
+
+
+def test_int8_sums_are_no_reason_for_small_tiles_without_them(gpu):
+    """A K that ends inside 64 bytes, signed operands: nothing to add up, so no scratch, and the LDS tiles all the same."""
+    p = int8_problem(2048, 4096, 2064, cabi.DT_S8, cabi.DT_S8, cabi.DT_S8, dst_scale=20.0)
+    assert cabi.scratch_bytes(p.desc()) == 0
+    chosen, small = in_turn(*(launches(p, "MI355_I8_TILES", t) for t in (None, "small")))
+    assert chosen <= 0.6 * small, (chosen, small)
