@@ -120,9 +120,10 @@ int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, h
     }
     // (MI355_F8_TILES: wide / narrow keep one geometry whatever the size: tests, tuning)
     const int force = tuning(TUNE_F8_TILES);
-    const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N) && force != TUNE_WIDE);
     chain_t C {};
-    if (!fa && !fb && chain_from_mx(P, plan.mx, true, C)) {
+    const bool chain = !fa && !fb && chain_from_mx(P, plan.mx, true, C) && (P.dst_dt == MI355_DT_BF16 || P.dst_dt == MI355_DT_F32);
+    const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N, d.K, chain) && force != TUNE_WIDE);
+    if (chain) {
         C.a = (const char *)P.src; C.lda = P.ss[1]; C.a_bs = P.ss[0];
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K;

@@ -399,7 +399,10 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
     problem_t P = P_in;
     const long EB = plan.EB;
     // (the MI355_H16_TILES switch keeps the 256 x 256 tiles: tests, tuning)
-    const bool narrow = line_tiles_narrow(d.batch, d.M, d.N) && tuning(TUNE_H16_TILES) != TUNE_WIDE;
+    auto narrow_for = [&](bool chain) {
+        return line_tiles_narrow(d.batch, d.M, d.N, plan.Kp * EB, chain) && tuning(TUNE_H16_TILES) != TUNE_WIDE;
+    };
+    bool narrow = narrow_for(true);
     chain_t C {};
     int across = h16_across(d, plan, P);
     // the 256 x 128 tile takes weights across K only: src is copied there (whole chunks of K)
@@ -494,6 +497,7 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
         if (st != MI355_UNIMPLEMENTED) return st;
     }
     if (general_refused("mfma_h16")) return MI355_UNIMPLEMENTED;
+    narrow = narrow_for(false);
     using bf16_t = h16x16_mma_t<true, f8_geo_t>;
     using bf16_narrow_t = h16x16_mma_t<true, narrow_t>;
     using f16_t = h16x16_mma_t<false, f8_geo_t>;

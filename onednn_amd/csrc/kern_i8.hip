@@ -505,7 +505,7 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
     }
     // (MI355_I8_TILES: wide / narrow keep one geometry whatever the size: tests, tuning)
     const int force = tuning(TUNE_I8_TILES);
-    const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N) && force != TUNE_WIDE);
+    const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N, d.K, chain) && force != TUNE_WIDE);
     if (chain) {
         const int st = chain_launch_i8(su, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;

@@ -736,15 +736,19 @@ struct reads_lines : std::false_type {};
 template <class Mma>
 struct reads_lines<Mma, std::enable_if_t<(Mma::NU > 0)>> : std::true_type {};
 
-// Which of the two tiles a problem of `batch` x M x N takes: rounds of 256 workgroups, one a CU, at 9 / 16 of the
-// large tile's time for the 256 x 128 one (bf16 / int8 / fp8, K = 4096: 39 / 23.4 / 22.7 us a round against 69 / 40 /
-// 39).  Beyond two rounds of large tiles the chip is power-limited and the small tile's 1.5 loads per MFMA cost 10 %.
+// Which of the two tiles a problem of `batch` x M x N takes: rounds of 256 workgroups, one a CU.  A round of 256 x 128 tiles
+// is the cheaper one, so no more of them than of large ones are taken always.  Three against two take as long or less
+// only where K is long, 9 / 16 of the time for a round (bf16 / int8 / fp8, K = 4096: 39 / 23.4 / 22.7 us against 69 / 40 / 39),
+// and the epilogue is a chain: 4096 x 5120, narrow against wide, bf16 with K = 256 / 1024 / 4096 32.5 / 29.3, 56.9 / 56.9, 149 / 164
+// us, fp8 with K = 1024 / 4096 42.7 / 40.9, 89.8 / 94.2, and through the general epilogue 69.8 / 59.1, 116 / 111.  Beyond two
+// rounds of large tiles the chip is power-limited and the small tile's 1.5 loads per MFMA cost 10 %.
 // (N up to 128, half of a large tile at most, has stayed on them since the tiles were chosen by count alone.  The narrow one
 // measures 0.66 to 0.89 of their time there, fp8: 4096 x 128 x 1024 13.4 / 17.5 us, 70000 x 100 x 2048 96.5 / 108.)
-inline bool line_tiles_narrow(long batch, long M, long N) {
+inline bool line_tiles_narrow(long batch, long M, long N, long kbytes, bool chain) {
     if (N <= 128) return false;
     const long tm = (M + BM - 1) / BM, wide = batch * tm * ((N + 255) / 256), narrow = batch * tm * ((N + 127) / 128);
-    return wide <= 512 && 9 * ((narrow + 255) / 256) < 16 * ((wide + 255) / 256);
+    const long rounds_wide = (wide + 255) / 256, rounds_narrow = (narrow + 255) / 256;
+    return wide <= 512 && (rounds_narrow <= rounds_wide || (chain && kbytes >= 4096 && 9 * rounds_narrow < 16 * rounds_wide));
 }
 
 } // namespace gemm

@@ -185,6 +185,16 @@ def test_mxfp4_through_the_general_epilogue(gpu, M, N, K):
     assert general <= chain + 7.5, (general, chain)
 
 
+@pytest.mark.parametrize("M,N,K", [(4096, 5120, 256), (3072, 8192, 1024), (4096, 4352, 2048), (2560, 8192, 4096)])
+@pytest.mark.parametrize("dt,ddt", [("bf16", "bf16"), ("bf16", "f8_e4m3"), ("f8_e4m3", "bf16"), ("f8_e4m3", "f16")])
+def test_three_rounds_of_narrow_tiles_or_two_of_wide(gpu, M, N, K, dt, ddt):
+    """257 to 384 large tiles: the wide tiles are never better by more than 7 %, where three narrow rounds cost a short K or
+    the general epilogue a quarter and more."""
+    p = float_problem(M, N, K, dt, ddt)
+    chosen, wide = in_turn(*(launches(p, "MI355_H16_TILES" if dt == "bf16" else "MI355_F8_TILES", t) for t in (None, "wide")), n=10)
+    assert chosen <= 1.07 * wide, (chosen, wide)
+
+
 def test_int8_sums_are_no_reason_for_small_tiles_without_them(gpu):
     """A K that ends inside 64 bytes, signed operands: nothing to add up, so no scratch, and the LDS tiles all the same."""
     p = int8_problem(2048, 4096, 2064, cabi.DT_S8, cabi.DT_S8, cabi.DT_S8, dst_scale=20.0)
