@@ -331,27 +331,28 @@ bool i8_chain(const problem_t &P, chain_t &C) {
 // the two is a number of small tiles.  (Not of large ones: a short M fills few rows of a large tile.)  What moves it, with
 // small against LDS tiles in us:
 //   K       1024 tiles (256 x 4096, s8 -> s8 with K = 1024 / 4096 / 16384): 10.7 / 14.5, 31.5 / 26.0, 115 / 74
-//   a K that ends inside 64 bytes: the small tiles' rows then start in different channels, and the LDS tiles have a
-//           partial last step (the same with K = 1040 / 4112 / 16400): 8.8 / 15.4, 25.4 / 27.2, 89 / 107
+//   a K of no whole 128-byte lines: the small tiles' rows then start in different channels, and the LDS tiles have a
+//           partial last step (the same with K = 1040 / 4112 / 16400): 8.8 / 15.4, 25.4 / 27.2, 89 / 107.  (Sums: 64 bytes.)
 //   sums    that are kernels of their own in front of the LDS tiles (u8 -> bf16, 256 x 4096 x 4096): 31.9 / 34.8 against 31.5 /
 //           26.0 without
 //   the general epilogue, 4 us of a launch of small tiles and 8 to 12 of LDS tiles (f16 dst, 256 x 6144 x 1024): 21.5 /
 //           23.5 against 14.4 / 14.7 of a chain
-//   up to 32 rows: an LDS tile is seven eighths empty or more, and a second round of them costs as much as the first (16 x
-//           65536 x 1024, s8 -> s8): 18.2 / 23.1 against 18.1 / 14.7 for 256 x 8192
-// The lines lie where the two meet in a grid of 12 K x 7 M x 11 numbers of tiles x 4 epilogues, the lowest over the M of a
+//   few rows: an LDS tile is seven eighths empty or more (16 x 65536 x 1024, s8 -> s8): 18.2 / 23.1 against 18.1 / 14.7 for 256 x
+//           8192; with sums, whose time follows N, up to 64 of them (64 x 40960 x 2064, u8 -> bf16): 36.8 / 53.8
+// The lines lie where the two meet in a grid of 26 K x 8 M x 11 numbers of tiles x 4 epilogues, the lowest over the M of a
 // row; the choice is within 1.1 times the better one's time nearly everywhere.
 bool small_tiles_better(const mi355_matmul_desc_t &d, bool chain) {
     constexpr int ALL = 1 << 30;
     static const int line[2][2][2][2][5] = {
-            // [32 rows or fewer][whole 64 bytes of K][general epilogue][sums][K < 512, < 2048, < 4096, < 8192, longer]
-            {{{{1793, 2049, 1537, 1025, 1025}, {2561, 3073, 2049, 1537, 1153}}, {{1793, 2049, 1537, 1281, 1025}, {2561, 2561, 2049, 1537, 1153}}},
-                    {{{897, 1281, 1025, 769, 513}, {1281, 1793, 1281, 1025, 769}}, {{1281, 1537, 1025, 769, 641}, {1537, 2049, 1537, 1153, 769}}}},
+            // [few rows][whole lines of K][general epilogue][sums][K < 512, < 2048, < 4096, < 8192, longer]
+            {{{{1665, 2049, 1537, 1025, 1025}, {2561, 3073, 2049, 1537, 1153}}, {{1665, 2049, 1537, 1281, 1025}, {2561, 2561, 2049, 1537, 1153}}},
+                    {{{769, 1281, 897, 641, 513}, {1281, 1793, 1281, 1025, 769}}, {{1281, 1537, 1025, 769, 641}, {1537, 2049, 1537, 1153, 769}}}},
             {{{{ALL, ALL, ALL, 2049, 1153}, {ALL, ALL, ALL, 2561, 2049}}, {{ALL, ALL, ALL, 2049, 1153}, {ALL, ALL, ALL, 2561, 1281}}},
-                    {{{1025, ALL, ALL, 1025, 769}, {1024, ALL, ALL, 2561, 2049}}, {{1281, ALL, ALL, 1025, 769}, {ALL, ALL, ALL, 1537, 1025}}}}};
+                    {{{897, ALL, ALL, 1025, 769}, {1024, ALL, 2561, 1537, 1025}}, {{1025, ALL, ALL, 1025, 769}, {3073, ALL, ALL, 1537, 1025}}}}};
     const bool sums = d.src_dt == MI355_DT_U8 || d.wei_dt == MI355_DT_U8 || !quant_absent(d.src_zp) || !quant_absent(d.wei_zp);
     const int band = d.K < 512 ? 0 : d.K < 2048 ? 1 : d.K < 4096 ? 2 : d.K < 8192 ? 3 : 4;
-    return ((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch < line[d.M <= 32][d.K % BK == 0][!chain][sums][band];
+    const bool few = d.M <= (chain && sums ? 64 : 32), whole = d.K % (sums ? BK : LKB) == 0;
+    return ((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch < line[few][whole][!chain][sums][band];
 }
 
 // chain: what i8_chain says, the same of the descriptor's problem and of the launch's
