@@ -201,6 +201,9 @@ MX_SHAPES = [
     ([1, 2, 4, 8, 16], 2048, 132),
     ([0, 1, 2, 0, 3, 0], 1024, 20),
     ([70, 3, 129], 1024, 40),
+    ([10, 20, 30, 40], 768, 36),       # whole 128-byte steps that are not whole 512-byte chunks: the src scales' rows are no
+    ([70, 3, 129], 1536, 260),         # 16-byte pieces (768), and fp4's last chunk is a half (1536, 2560)
+    ([1, 2, 4, 8, 16], 2560, 132),
 ]
 MX_TYPES = [("mxfp8 e4m3", E4M3, E4M3), ("mxfp8 e5m2 x e4m3", E5M2, E4M3), ("mxfp4", cabi.DT_F4_E2M1, cabi.DT_F4_E2M1)]
 
