@@ -1,5 +1,5 @@
 // "hip:woq_packed" -- the weight-only-quantized decode of kern_woq.hip over
-// weights in the MI355_WEI_PACK_WOQ64 layout: bf16 activations (M <= 32 rows)
+// weights in the MI355_WEI_PACK_WOQ64 layout: bf16 or f16 activations (M <= 32 rows)
 // times 4-bit weights, per-group scales and zero points along K, fpmath
 // "apply_to_int" weight decompression.
 //
@@ -42,8 +42,14 @@
 //    steps each keep this tail short;
 //  - the parameter decode at a group's end is straight-line code (candidate
 //    conversions selected by uniform masks), no data-type switch.
+//
+// f16 activations: the same with 64 in the place of 128, whose f16 has a nibble's
+// place four bits up (0x5400 | w << 4 = 64 + w), on the f16 instruction.  Before
+// it the GEMM tiles ran on a decompressed copy of the weights (14336 x 4096, M = 1 / 32:
+// 127 / 129 us; here 7.5 / 14.4).
 #include "kernels.hpp"
 #include "tile_epilogue.hpp"
+#include "woq_ops.hpp"
 
 #include <type_traits>
 
@@ -62,7 +68,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned v16u __attribute__((ext_vector_type(16)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 constexpr int CHUNK = 64;      // columns per workgroup
 constexpr int KBLK = 32;       // rows per step (one MFMA depth)
@@ -70,7 +75,7 @@ constexpr int NO_GROUPS = 1 << 30;
 
 struct woqp_extra_t {
     const uint8_t *wei;  // packed, K * N / 2 bytes
-    const uint8_t *src;  // bf16 [M][src_ld]
+    const uint8_t *src;  // bf16 or f16 [M][src_ld]
     const uint8_t *sc, *zp; // weights scales / zero points (NULL when absent)
     uint8_t *dst;        // the plain store: dst_dt in {f32, bf16, f16}, rows dst_ld elements apart
     int dst_dt, dst_ld;
@@ -92,8 +97,7 @@ struct woqp_args_t {
     problem_t P;
 };
 typedef const __attribute__((address_space(4))) woqp_args_t kernarg_woqp_t;
-
-__device__ __forceinline__ v8bf as_bf(const v4i &x) { return __builtin_bit_cast(v8bf, x); }
+typedef const __attribute__((address_space(4))) woqp_extra_t kernarg_woqp_extra_t; // (first in either form of the argument)
 
 // Loads through pointers of the global address space.  The kernel's pointers come out of a block of scalar
 // registers filled by inline assembly, so the compiler cannot tell that they point to global memory and would
@@ -222,7 +226,7 @@ __device__ __forceinline__ float decode_zp(int dt, int bits, unsigned raw) {
 // super-step holds whole groups, 0 when a group holds whole super-steps.
 // NWV wavefronts per workgroup.  PLAIN: nothing follows the K sum but the
 // conversion to the dst type.
-template <int NWV, int MT, int SS, int SPG, bool PLAIN>
+template <int NWV, int MT, int SS, int SPG, bool PLAIN, bool F16>
 __global__ void __launch_bounds__(NWV * 64)
         woqp_kernel(const std::conditional_t<PLAIN, woqp_extra_t, woqp_args_t> A_) {
     __shared__ v4f red4[NWV * MT * 4 * 64];
@@ -358,14 +362,15 @@ __global__ void __launch_bounds__(NWV * 64)
             tot[mt][tt] = v4f {0.f, 0.f, 0.f, 0.f};
         }
     }
-    // 0x4300 | nibble = bf16(128 + nibble).  The constant is kept in a vector
+    // OFFSET + nibble in the activations' type.  The constant is kept in a vector
     // register: a VOP3 instruction takes one scalar operand at most, so
     // (x & mask) | magic fuses into v_and_or_b32 only when `magic` is not scalar.
+    typedef woq_ops_t<F16> ops;
     unsigned magic;
-    asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
-    const v4i ones = {0x3F803F80, 0x3F803F80, 0x3F803F80, 0x3F803F80};
+    asm volatile("v_mov_b32 %0, %1" : "=v"(magic) : "n"(ops::MAGIC));
+    const v4i ones = {ops::ONES, ops::ONES, ops::ONES, ops::ONES};
     const unsigned flip = X.signed_w ? 0x88888888u : 0u; // s4 -> offset-binary
-    const float zbase = X.signed_w ? 136.f : 128.f;
+    const float zbase = X.signed_w ? ops::OFFSET + 8.f : ops::OFFSET;
     // s4 weights go to offset-binary before they are unpacked: a uniform branch around the exclusive-ors, so the
     // unsigned case does not pay an instruction per dword for them
     auto flip_signed = [&](auto &ws) __attribute__((always_inline)) {
@@ -387,7 +392,7 @@ __global__ void __launch_bounds__(NWV * 64)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             av[mt] = v4i {(int)a[mt][0], (int)a[mt][1], (int)a[mt][2], (int)a[mt][3]};
-            rsum[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf(av[mt]), as_bf(ones), first ? zero : rsum[mt], 0, 0, 0);
+            rsum[mt] = ops::mma(av[mt], ones, first ? zero : rsum[mt]);
         }
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) {
@@ -395,10 +400,10 @@ __global__ void __launch_bounds__(NWV * 64)
             v4i b;
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                b[u] = MI355_WOQP_ABL == 5 ? (int)(d + u) : (int)(((d >> (4 * u)) & 0x000F000Fu) | magic);
+                b[u] = MI355_WOQP_ABL == 5 ? (int)(d + u) : (int)ops::unpack(d, u, magic);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
-                acc[mt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf(av[mt]), as_bf(b), first ? zero : acc[mt][tt], 0, 0, 0);
+                acc[mt][tt] = ops::mma(av[mt], b, first ? zero : acc[mt][tt]);
         }
     };
 
@@ -552,6 +557,15 @@ __global__ void __launch_bounds__(NWV * 64)
         }
     }
 
+    // an element whose sums came out as NaN, from its terms (woq_ops.hpp); cold code
+    auto term_sum = [&](int m, int n) __attribute__((always_inline)) {
+        const kernarg_woqp_extra_t &Y = *(kernarg_woqp_extra_t *)__builtin_amdgcn_kernarg_segment_ptr();
+        return woq_term_sum(Y, Y.spg == NO_GROUPS ? Y.K : Y.spg * KBLK, m, n, [&](int k) {
+            const unsigned at = (k / 8) * 512 + (n % 16) * 32 + (n % CHUNK) / 16 * 8 + (k % 2) * 4 + (k % 8) / 2; // in nibbles
+            return Y.wei[(long)(n / CHUNK) * Y.K * (CHUNK / 2) + at / 2] >> (at % 2 * 4);
+        });
+    };
+
     // ---- add the wavefronts' sums in wavefront order and store.  LDS holds
     // [wavefront][row][column] floats; a thread then owns four consecutive
     // columns of one row and runs the four-wide epilogue of the GEMM tiles.
@@ -575,6 +589,7 @@ __global__ void __launch_bounds__(NWV * 64)
             float v = cell[0];
 #pragma unroll
             for (int wv = 1; wv < NWV; ++wv) v += cell[wv * WSTRIDE];
+            if (F16 && v != v) v = term_sum(m, chunk * CHUNK + nl);
             const unsigned bits = X.dst_dt == MI355_DT_F32 ? f2u(v)
                     : X.dst_dt == MI355_DT_BF16 ? (unsigned)f32_to_bf16(v) : (unsigned)f32_to_f16(v);
             const long off = (long)m * X.dst_ld + chunk * CHUNK + nl;
@@ -596,6 +611,7 @@ __global__ void __launch_bounds__(NWV * 64)
             float v = cell[0];
 #pragma unroll
             for (int wv = 1; wv < NWV; ++wv) v += cell[wv * WSTRIDE];
+            if (F16 && v != v) v = term_sum(m, chunk * CHUNK + nl);
             epilogue_store(P, v, 0, m, chunk * CHUNK + nl);
         }
         return;
@@ -610,6 +626,11 @@ __global__ void __launch_bounds__(NWV * 64)
         for (int wv = 1; wv < NWV; ++wv) sum += cell[wv * (WSTRIDE / 4)];
         float v[4] = {sum[0], sum[1], sum[2], sum[3]};
         const long n = (long)chunk * CHUNK + nq * 4;
+        if constexpr (F16) {
+#pragma unroll 1
+            for (int i = 0; i < 4; ++i)
+                if (v[i] != v[i]) v[i] = term_sum(m, (int)n + i);
+        }
         gemm::apply_epilogue4(P, v, 0, m, n, 4);
         gemm::store4(P, P.ds[2] == 1 && gemm::vec_ok_store(P.dst, P.ds[0], P.ds[1], dt_bits(P.dst_dt)), v, 0, m, n, 4);
     }
@@ -679,7 +700,7 @@ woqp_geo_t pick_geo(int mt, long G, long K) {
 
 int woqp_supported(const mi355_matmul_desc_t &d) {
     if (!woq64_layout_ok(d)) return MI355_UNIMPLEMENTED;
-    if (d.src_dt != MI355_DT_BF16 || !d.fpmath_apply_to_int) return MI355_UNIMPLEMENTED;
+    if ((d.src_dt != MI355_DT_BF16 && d.src_dt != MI355_DT_F16) || !d.fpmath_apply_to_int) return MI355_UNIMPLEMENTED;
     if (dt_bits(d.dst_dt) < 8) return MI355_UNIMPLEMENTED;
     if (d.M < 1 || d.M > 32) return MI355_UNIMPLEMENTED;
     // 16-byte loads of src rows at 32-bit byte offsets
@@ -737,13 +758,14 @@ int woqp_launch(const mi355_matmul_desc_t &d, const problem_t &P, hipStream_t st
     X.zp_common = X.zp_dt && d.wei_zp.mask == 0;
     X.signed_w = d.wei_dt == MI355_DT_S4;
     const dim3 grid((unsigned)(d.N / CHUNK)), block(nw * 64);
+    auto go = [&](auto kern, auto kern_f16, const auto &arg) {
+        hipLaunchKernelGGL(d.src_dt == MI355_DT_F16 ? kern_f16 : kern, grid, block, 0, stream, arg);
+        return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
+    };
 #define MI355_WOQP_CASE(NW_, MT_, SS_, SPG_) \
     if (nw == NW_ && mt == MT_ && geo.ss == SS_ && geo.spg == SPG_) { \
-        if (plain) \
-            hipLaunchKernelGGL((woqp_kernel<NW_, MT_, SS_, SPG_, true>), grid, block, 0, stream, A.X); \
-        else \
-            hipLaunchKernelGGL((woqp_kernel<NW_, MT_, SS_, SPG_, false>), grid, block, 0, stream, A); \
-        return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR; \
+        if (plain) return go(woqp_kernel<NW_, MT_, SS_, SPG_, true, false>, woqp_kernel<NW_, MT_, SS_, SPG_, true, true>, A.X); \
+        return go(woqp_kernel<NW_, MT_, SS_, SPG_, false, false>, woqp_kernel<NW_, MT_, SS_, SPG_, false, true>, A); \
     }
     MI355_WOQP_CASE(16, 1, 8, 4)
     MI355_WOQP_CASE(16, 1, 8, 0)

@@ -1884,7 +1884,7 @@ DNNL_EXPORT dnnl_status_t dnnl_matmul_primitive_desc_create(dnnl_primitive_desc_
         // 4-bit decode weights: the 64-column packing, if the packed decode
         // kernel takes the problem and N gives it enough workgroups to fill
         // the device (decided below, once the descriptor is lowered)
-        try_packed = pd->src.dt == dnnl_bf16 && (w.dt == dnnl_s4 || w.dt == dnnl_u4) && pd->attr.apply_to_int
+        try_packed = (pd->src.dt == dnnl_bf16 || pd->src.dt == dnnl_f16) && (w.dt == dnnl_s4 || w.dt == dnnl_u4) && pd->attr.apply_to_int
                 && w.ndims == 2 && w.dims[1] >= 64 * 128;
         const bool mfma_operands = (is_int8(pd->src.dt) && is_int8(w.dt)) || (is_fp8(pd->src.dt) && is_fp8(w.dt))
                 || (pd->src.dt == dnnl_f4_e2m1 && w.dt == dnnl_f4_e2m1)

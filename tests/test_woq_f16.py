@@ -1,0 +1,92 @@
+"""The decode kernels with f16 activations: against the oracle under the bound of the factored sum (the f16 form keeps
+64 + w where the bf16 form keeps 128 + w, so tests/helpers.py decode_bound covers it), one-hot rows bit for bit, and
+infinite activations, whose factored sums are NaN where the terms' sum is an infinity.
+"""
+import numpy as np
+import pytest
+
+from onednn_amd import cabi, configs
+from onednn_amd import dtypes as dtp
+from onednn_amd.problem import run_gpu
+from tests.helpers import assert_bit_exact, assert_decode_close, decode
+
+IMPLS = {"plain": (cabi.IMPL_WOQ_GEMV, "hip:woq_gemv"), "packed": (cabi.IMPL_WOQ_PACKED, "hip:woq_packed")}
+
+
+def f16_problem(M, N, K, group, layout, wdt="u4", sdt="f16", zdt="u4", zkind="grouped", ddt="f16", relu_bias=False):
+    p = configs.woq_variant(M, N, K, group, wei_dt=wdt, sc_dt=sdt, zp_dt=zdt, zp_kind=zkind, dst_dt=ddt, relu_bias=relu_bias)
+    src = decode(p.src_dt, p.src, M * K).astype(np.float32).reshape(M, K)
+    p.src, p.src_dt = src.astype(np.float16).view(np.uint16), cabi.DT_F16
+    if layout == "packed":
+        p.wei_packing = cabi.WEI_PACK_WOQ64
+    return p
+
+
+def test_f16_activations_take_the_decode_kernels():
+    for layout, (_, name) in IMPLS.items():
+        for M, N, K, group in [(1, 128, 128, 128), (32, 192, 8320, 64)]:
+            st, impl = cabi.query(f16_problem(M, N, K, group, layout).desc())
+            assert st == cabi.SUCCESS and cabi.impl_name(impl).startswith(name)
+    assert cabi.impl_name(cabi.query(f16_problem(33, 128, 128, 128, "plain").desc())[1]).startswith("hip:mfma_h16")
+
+
+CASES = [
+    # M, N, K, group, weights, scales, zero points, dst, bias + relu
+    (1, 64, 32, 32, "u4", "f16", "u4", "grouped", "f16", False),
+    (1, 1280, 7680, 64, "s4", "f16", "u4", "none", "f16", False),
+    (4, 320, 8320, 128, "u4", "f16", "u4", "grouped", "f32", False),
+    (8, 192, 1056, 1056, "u4", "f32", "u8", "common", "f32", True),
+    (13, 256, 2048, 512, "s4", "f16", "s8", "grouped", "f16", True),
+    (16, 4160, 384, 128, "u4", "f32", "s32", "grouped", "f32", False),
+    (17, 256, 2048, 128, "s4", "bf16", "s4", "column", "f16", False),
+    (32, 128, 3072, 64, "u4", "f16", "u4", "grouped", "f16", False),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", IMPLS)
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x) for x in c))
+def test_f16_attribute_variants(gpu, oracle, case, layout):
+    M, N, K, group, wdt, sdt, zdt, zkind, ddt, relu_bias = case
+    p = f16_problem(M, N, K, group, layout, wdt, sdt, zdt, zkind, ddt, relu_bias)
+    got, name = run_gpu(p, cabi.IMPL_AUTO)
+    assert name.startswith(IMPLS[layout][1])
+    _, ideal, asum = oracle.run_oracle(p, want_ideal=True)
+    assert_decode_close(p, got, ideal, asum, what=name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", IMPLS)
+@pytest.mark.parametrize("K,group", [(32, 32), (256, 64), (512, 128), (2048, 2048)])
+def test_f16_one_hot_rows_are_exact(gpu, oracle, layout, K, group):
+    M = 32
+    p = f16_problem(M, 128, K, group, layout, ddt="f32")
+    hot = np.zeros((M, K), np.float16)
+    r = np.random.default_rng(K)
+    hot[np.arange(M), r.choice(K, size=M, replace=K < M)] = 1.0
+    p.src = hot.view(np.uint16)
+    got, name = run_gpu(p, IMPLS[layout][0])
+    assert_bit_exact(p, got, oracle.run_oracle(p), name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", IMPLS)
+@pytest.mark.parametrize("M,K,wdt,zkind,ddt,relu_bias", [(3, 512, "u4", "grouped", "f32", False), (20, 512, "s4", "none", "f16", True),
+                                                         (12, 4096, "s4", "common", "f16", False)])
+def test_f16_infinite_activations(gpu, oracle, layout, M, K, wdt, zkind, ddt, relu_bias):
+    # weights and zero points that never meet (w - zp is not 0), infinities of one sign per row: no term is NaN
+    p = f16_problem(M, 192, K, 128, layout, wdt=wdt, zkind=zkind, zdt="u4" if wdt == "u4" else "s8", ddt=ddt, relu_bias=relu_bias)
+    r = np.random.default_rng(5)
+    p.wei = dtp.pack_nibbles(r.integers(1, 8, size=(K, 192), dtype=np.uint8))
+    if "wei_zp" in p.quant:
+        z = p.quant["wei_zp"].data
+        z[...] = 0x99 if wdt == "u4" else -3
+    src = np.asarray(p.src).view(np.float16).reshape(M, K)
+    src[0, K - 1] = np.inf
+    src[1, 0] = -np.inf
+    src[2, K // 2] = np.nan
+    p.src = src.view(np.uint16)
+    got, name = run_gpu(p, IMPLS[layout][0])
+    want = oracle.run_oracle(p)
+    g, w = (decode(p.dst_dt, x, M * 192).astype(np.float64).reshape(M, 192)[:3] for x in (got, want))
+    np.testing.assert_array_equal(g, w)
