@@ -369,9 +369,10 @@ int mi355_matmul_scratch_bytes(const mi355_matmul_desc_t *desc, size_t *bytes);
 
 /* Enqueue the matmul on `stream` (a hipStream_t passed as void*, NULL =
  * default stream).  Asynchronous.  `scratch` may be NULL when
- * mi355_matmul_scratch_bytes reports 0, and for hip:mfma_i8 with K-contiguous
+ * mi355_matmul_scratch_bytes reports 0, for hip:mfma_i8 with K-contiguous
  * weights and a K that is not a multiple of 64 (which then runs on the tiles
- * that need none). */
+ * that need none), and where all of it is for the partial sums of a K split
+ * over workgroups (which is then not split: slower). */
 int mi355_matmul_launch(const mi355_matmul_desc_t *desc,
         const mi355_matmul_args_t *args, void *scratch, void *stream);
 
@@ -380,8 +381,9 @@ int mi355_matmul_launch(const mi355_matmul_desc_t *desc,
  * counterpart in the reference.  The scratch is a static device array of
  * MI355_NOALLOC_SCRATCH_BYTES inside the library, one per GPU, held until the
  * process ends; the call allocates and frees nothing.  A problem whose
- * mi355_matmul_scratch_bytes exceeds it (and that mi355_matmul_launch does
- * not take without) is refused with
+ * mi355_matmul_scratch_bytes, less the partial sums of a split K (no K is
+ * split here), exceeds it (and that mi355_matmul_launch does not take without)
+ * is refused with
  * MI355_INVALID_ARGUMENTS (mi355_last_error names both sizes).  All calls on
  * one GPU share that array: calls that overlap on one GPU (different streams,
  * or threads) race on it -- order them, or use mi355_matmul_launch with a

@@ -527,7 +527,7 @@ int mi355_matmul_query(const mi355_matmul_desc_t *desc, int impl, int *chosen_im
     return st;
 }
 
-int mi355_matmul_scratch_bytes(const mi355_matmul_desc_t *desc, size_t *bytes) {
+static int scratch_bytes(const mi355_matmul_desc_t *desc, bool parts, size_t *bytes) {
     if (!bytes) return MI355_INVALID_ARGUMENTS;
     *bytes = 0;
     int st = validate(desc);
@@ -535,18 +535,19 @@ int mi355_matmul_scratch_bytes(const mi355_matmul_desc_t *desc, size_t *bytes) {
     int impl = 0;
     if ((st = choose_impl(*desc, &impl))) return st;
     switch (impl) {
-        case MI355_IMPL_I8_MFMA: *bytes = i8_scratch_bytes(*desc); break;
-        case MI355_IMPL_F8_MFMA: *bytes = f8_scratch_bytes(*desc); break;
-        case MI355_IMPL_H16_MFMA: *bytes = h16_scratch_bytes(*desc); break;
-        case MI355_IMPL_MXF4_MFMA: *bytes = mxf4_scratch_bytes(*desc); break;
+        case MI355_IMPL_I8_MFMA: *bytes = i8_scratch_bytes(*desc, parts); break;
+        case MI355_IMPL_F8_MFMA: *bytes = f8_scratch_bytes(*desc, parts); break;
+        case MI355_IMPL_H16_MFMA: *bytes = h16_scratch_bytes(*desc, parts); break;
+        case MI355_IMPL_MXF4_MFMA: *bytes = mxf4_scratch_bytes(*desc, parts); break;
         case MI355_IMPL_WOQ_GEMV: *bytes = woq_scratch_bytes(*desc); break;
         default: break;
     }
     return MI355_SUCCESS;
 }
 
-int mi355_matmul_launch(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *args,
-        void *scratch, void *stream) {
+int mi355_matmul_scratch_bytes(const mi355_matmul_desc_t *desc, size_t *bytes) { return scratch_bytes(desc, true, bytes); }
+
+static int launch(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *args, void *scratch, bool parts, void *stream) {
     int st = validate(desc);
     if (st) return st;
     if (!args) {
@@ -563,26 +564,33 @@ int mi355_matmul_launch(const mi355_matmul_desc_t *desc, const mi355_matmul_args
     hipStream_t s = (hipStream_t)stream;
     switch (impl) {
         case MI355_IMPL_REF: return ref_launch(P, s);
-        case MI355_IMPL_I8_MFMA: return i8_launch(*desc, P, scratch, s);
-        case MI355_IMPL_F8_MFMA: return f8_launch(*desc, P, scratch, s);
-        case MI355_IMPL_H16_MFMA: return h16_launch(*desc, P, scratch, s);
-        case MI355_IMPL_MXF4_MFMA: return mxf4_launch(*desc, P, scratch, s);
+        case MI355_IMPL_I8_MFMA: return i8_launch(*desc, P, scratch, parts, s);
+        case MI355_IMPL_F8_MFMA: return f8_launch(*desc, P, scratch, parts, s);
+        case MI355_IMPL_H16_MFMA: return h16_launch(*desc, P, scratch, parts, s);
+        case MI355_IMPL_MXF4_MFMA: return mxf4_launch(*desc, P, scratch, parts, s);
         case MI355_IMPL_WOQ_GEMV: return woq_launch(*desc, P, scratch, s);
         case MI355_IMPL_WOQ_PACKED: return woqp_launch(*desc, P, s);
         default: return MI355_UNIMPLEMENTED;
     }
 }
 
+int mi355_matmul_launch(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *args,
+        void *scratch, void *stream) {
+    return launch(desc, args, scratch, scratch != nullptr, stream);
+}
+
+// (without parts: problems that need no scratch stay free to overlap on one GPU)
 int mi355_matmul_launch_noalloc(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *args,
         void *stream) {
     size_t bytes = 0;
-    int st = mi355_matmul_scratch_bytes(desc, &bytes);
+    int st = scratch_bytes(desc, false, &bytes);
     if (st) return st;
     int impl = 0;
     if (bytes > (size_t)MI355_NOALLOC_SCRATCH_BYTES && choose_impl(*desc, &impl) == MI355_SUCCESS && impl == MI355_IMPL_I8_MFMA
             && i8_scratch_optional(*desc))
         bytes = 0;
     if (bytes > (size_t)MI355_NOALLOC_SCRATCH_BYTES) {
+        (void)mi355_matmul_scratch_bytes(desc, &bytes); // what the buffer it asks for has to hold
         set_error("mi355_matmul_launch_noalloc: the problem needs %zu bytes of scratch, the static buffer holds %zu "
                   "(use mi355_matmul_launch with a caller-owned buffer, or K-contiguous weights)",
                 bytes, (size_t)MI355_NOALLOC_SCRATCH_BYTES);
@@ -593,7 +601,7 @@ int mi355_matmul_launch_noalloc(const mi355_matmul_desc_t *desc, const mi355_mat
     // every kernel family writes the part of its scratch it reads within the same
     // launch (transposed weights, row / column sums, split-K partial sums): nothing
     // has to start at zero
-    return mi355_matmul_launch(desc, args, scratch, stream);
+    return launch(desc, args, scratch, false, stream);
 }
 
 } // extern "C"

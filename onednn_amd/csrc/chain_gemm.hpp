@@ -19,7 +19,7 @@
 
 namespace mi355 {
 
-enum chain_dst_t { CHAIN_BF16, CHAIN_F16, CHAIN_F32, CHAIN_I8 };
+enum chain_dst_t { CHAIN_BF16, CHAIN_F16, CHAIN_F32, CHAIN_I8, CHAIN_PART }; // CHAIN_PART: a part of K, no epilogue
 enum chain_act_t { CHAIN_NONE, CHAIN_RELU, CHAIN_GELU, CHAIN_SWISH };
 
 struct chain_vec_t { // f32 / bf16 / f16 values; dt UNDEF = absent
@@ -47,7 +47,45 @@ struct chain_t {
     const void *dsc;
     int dsc_dt, ds_mode; // 0 none, 1 divide, 2 multiply by the reciprocal
     int lo, hi;          // 8-bit dst
+    // split > 1: K in parts of part_steps steps, a workgroup each; their accumulators go to parts and chain_sum_kernel
+    // (kern_chain_sum.hip) adds them and does the rest
+    char *parts;
+    int split, part_steps;
 };
+
+// Into how many parts of K a problem of few tiles is split, 1 = not at all.  One workgroup a CU and round: with T tiles
+// (256 x 128, or 256 x 256) a launch takes its K steps one after the other on T of 256 CUs.  S parts make that steps / S, for
+// a second kernel (3 us and more of a launch), the parts' way out and in again (a part of a tile 128 / 256 KB each way) and
+// a workgroup's fixed cost, which is why S is not 256 / T: per step_ns + S T part_ns + CHAIN_SPLIT_NS is what a launch of S
+// parts of `per` steps takes beyond one without, and the S of the least is within 1.05 of the best S measured on 20 shapes of every
+// type.  Unsplit / split, us: fp8 256 x 4352 x 12224 73.7 / 30.4, 64 x 640 x 16384 66.6 / 18.3, 512 x 7168 x 16384 (two parts) 73.0 / 60.0;
+// MXFP4 100 x 1040 x 16352 58.3 / 27.1; bf16 4096 x 960 x 13312 125 / 95.6, f16 300 x 2048 x 4096 38.8 / 23.0; int8 256 x 6272 x
+// 6528 (u8) 53.0 / 36.3; where steps are few the second kernel costs more than it gives (bf16 512 x 3600 x 704 15.0 / 23.2).
+constexpr long CHAIN_SPLIT_NS = 5000;
+struct chain_split_t {
+    int split, part_steps;
+};
+inline chain_split_t chain_split(long batch, long M, long N, long kbytes, bool wide, long step_ns) {
+    const long bn = wide ? 256 : 128, tiles = batch * ((M + 255) / 256) * ((N + bn - 1) / bn), steps = (kbytes + 127) / 128;
+    const long part_ns = wide ? 104 : 52;
+    chain_split_t r {1, (int)steps};
+    if (tiles < 1 || tiles > 128) return r;
+    long best = steps * step_ns - CHAIN_SPLIT_NS;
+    for (long s = 2; s * tiles <= 256; ++s) {
+        const long per = (steps + s - 1) / s;
+        if (per < 2) break;
+        if ((steps + per - 1) / per != s) continue; // (the same steps a part with fewer of them)
+        const long ns = per * step_ns + s * tiles * part_ns;
+        if (ns < best) best = ns, r = chain_split_t {(int)s, (int)per};
+    }
+    return r;
+}
+inline size_t chain_parts_bytes(long batch, long M, long N, bool wide, int split) {
+    const long bn = wide ? 256 : 128;
+    return split > 1 ? (size_t)(batch * ((M + 255) / 256) * ((N + bn - 1) / bn)) * split * (size_t)(256 * bn * 4) : 0;
+}
+// the sums of a problem whose parts lie at C.parts, and its epilogue (integer: they are s32)
+int chain_launch_sum(bool integer, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
 
 // The problem's epilogue as a chain; false: not one of them (the general kernels run it).  What the K loop reads (a,
 // bt, lda, ldb, the batches' strides, kbytes, block scales, colsum) is the family's to fill in.  scaled: src and
@@ -333,11 +371,14 @@ __global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu
     static_assert(G::WCOLS == 64, "a wavefront's part is 128 x 64");
     char *smem = chain_smem;
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const long b = blockIdx.z;
+    constexpr bool PART = DST == CHAIN_PART;
+    const long b = PART ? blockIdx.z / C.split : blockIdx.z;
+    const long step0 = PART ? (long)(blockIdx.z % C.split) * C.part_steps : 0; // the first step of the part
     const tile_pos_t tp = tile_position<G>((int)blockIdx.x, C.tiles_m, C.tiles_n);
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem;
     const unsigned tab = lds0 + line_loader_t<Mma>::LDS_BYTES;
     auto fill = [&]() __attribute__((always_inline)) {
+        if constexpr (PART) return;
         typedef int __attribute__((address_space(3))) *lds_i_t;
         static_assert(G::NT % 256 == 0, "every column has a thread");
         const int col = t & 255;
@@ -356,10 +397,26 @@ __global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu
     for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = V {0, 0, 0, 0};
-    const line_scales_t sc = C.sc.tile(b, tp.m0, tp.n0);
-    main_loop_lines<Mma>(acc, smem, C.a + b * C.a_bs + tp.m0 * (line_form<Mma>::AKM ? 2 : C.lda),
-            C.bt + b * C.b_bs + tp.n0 * (line_form<Mma>::BKM ? 2 : C.ldb), C.lda, C.ldb,
-            C.M - tp.m0, C.N - tp.n0, C.kbytes, sc, fill);
+    line_scales_t sc = C.sc.tile(b, tp.m0, tp.n0);
+    long kbytes = C.kbytes;
+    if constexpr (PART) {
+        kbytes = min(kbytes - step0 * LKB, (long)C.part_steps * LKB);
+        sc.a += step0 * Mma::SCALE_SETS * sc.a_pitch;
+        sc.b += step0 * Mma::SCALE_SETS * sc.b_pitch;
+        sc.sets -= (int)step0 * Mma::SCALE_SETS;
+    }
+    main_loop_lines<Mma>(acc, smem,
+            C.a + b * C.a_bs + (line_form<Mma>::AKM ? tp.m0 * 2 + step0 * 64 * C.lda : tp.m0 * C.lda + step0 * LKB),
+            C.bt + b * C.b_bs + (line_form<Mma>::BKM ? tp.n0 * 2 + step0 * 64 * C.ldb : tp.n0 * C.ldb + step0 * LKB), C.lda, C.ldb,
+            C.M - tp.m0, C.N - tp.n0, kbytes, sc, fill);
+    if constexpr (PART) { // [part][tile][wavefront][accumulator quad][lane]
+        char *to = C.parts + (((long)blockIdx.z * gridDim.x + blockIdx.x) * G::NW + wave) * 32768 + (t & 63) * 16;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) *(V *)(to + (i * 4 + j) * 1024) = acc[i][j];
+        return;
+    } else {
 
     const int wm = G::wm(wave), wn = G::wn(wave);
     chain_part_t<Mma> E {C, tab, lds0 + (unsigned)wave * 16384u, b, tp.m0 + wm * 128, tp.n0 + wn * 64, t & 63, wn * 64, 1.f, 1.f, 0};
@@ -390,6 +447,7 @@ __global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu
     } else {
         store(std::integral_constant<bool, FULL> {});
     }
+    }
 }
 
 template <class Mma, int DST>
@@ -397,10 +455,16 @@ int chain_go(chain_t &C, unsigned batch, hipStream_t stream, const char *who) {
     constexpr int smem_bytes = line_loader_t<Mma>::LDS_BYTES + CT_BYTES;
     C.tiles_m = (int)((C.M + BM - 1) / BM);
     C.tiles_n = (int)((C.N + Mma::G::BN - 1) / Mma::G::BN);
-    const dim3 grid((unsigned)(C.tiles_m * C.tiles_n), 1, batch);
+    const dim3 grid((unsigned)(C.tiles_m * C.tiles_n), 1, DST == CHAIN_PART ? batch * C.split : batch);
     if (const int st = ensure_dynamic_lds((const void *)chain_gemm_kernel<Mma, DST>, smem_bytes, who)) return st;
     hipLaunchKernelGGL((chain_gemm_kernel<Mma, DST>), grid, dim3(Mma::G::NT), smem_bytes, stream, C);
     return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
+}
+// K in parts (C.split of them), then their sums and the epilogue
+template <class Mma>
+int chain_go_parts(int dst_dt, chain_t &C, unsigned batch, hipStream_t stream, const char *who) {
+    if (const int st = chain_go<Mma, CHAIN_PART>(C, batch, stream, who)) return st;
+    return chain_launch_sum(Mma::INTEGER, dst_dt, C, batch, Mma::G::BN == 256, stream);
 }
 } // namespace
 #endif

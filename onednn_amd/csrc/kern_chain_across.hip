@@ -16,6 +16,14 @@ int chain_launch_h16_across(bool bf16, int dst_dt, int across, chain_t &C, unsig
         return wide ? chain_go<h16_across_mma_t<B, wide_t, 1>, D>(C, batch, stream, "mfma_h16")
                     : chain_go<h16_across_mma_t<B, narrow_t, 1>, D>(C, batch, stream, "mfma_h16");
     };
+    if (C.split > 1) {
+        auto parts = [&](auto b16) -> int {
+            constexpr bool B = decltype(b16)::value;
+            return across == 2 ? chain_go_parts<h16_across_mma_t<B, wide_t, 2>>(dst_dt, C, batch, stream, "mfma_h16")
+                               : chain_go_parts<h16_across_mma_t<B, narrow_t, 1>>(dst_dt, C, batch, stream, "mfma_h16");
+        };
+        return bf16 ? parts(std::true_type {}) : parts(std::false_type {});
+    }
     constexpr std::integral_constant<int, CHAIN_F32> f32 {};
     if (bf16 && dst_dt == MI355_DT_BF16) return go(std::true_type {}, std::integral_constant<int, CHAIN_BF16> {});
     if (bf16 && dst_dt == MI355_DT_F32) return go(std::true_type {}, f32);

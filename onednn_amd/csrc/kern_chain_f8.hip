@@ -11,6 +11,7 @@ int chain_launch_f8(int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream
         return wide ? chain_go<f8_mma_t<0, 0, geo_t<8, 256>>, D>(C, batch, stream, "mfma_f8")
                     : chain_go<f8_mma_t<0, 0, geo_t<4, 128>>, D>(C, batch, stream, "mfma_f8");
     };
+    if (C.split > 1) return chain_go_parts<f8_mma_t<0, 0, geo_t<4, 128>>>(dst_dt, C, batch, stream, "mfma_f8");
     if (dst_dt == MI355_DT_BF16) return go(std::integral_constant<int, CHAIN_BF16> {});
     if (dst_dt == MI355_DT_F32) return go(std::integral_constant<int, CHAIN_F32> {});
     return MI355_UNIMPLEMENTED;

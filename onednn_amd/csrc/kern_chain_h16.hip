@@ -97,6 +97,9 @@ int chain_launch_h16(bool bf16, int dst_dt, chain_t &C, unsigned batch, bool wid
         return wide ? chain_go<h16_mixed_mma_t<B, wide_t>, D>(C, batch, stream, "mfma_h16")
                     : chain_go<h16_mixed_mma_t<B, narrow_t>, D>(C, batch, stream, "mfma_h16");
     };
+    if (C.split > 1)
+        return bf16 ? chain_go_parts<h16x16_mma_t<true, narrow_t>>(dst_dt, C, batch, stream, "mfma_h16")
+                    : chain_go_parts<h16x16_mma_t<false, narrow_t>>(dst_dt, C, batch, stream, "mfma_h16");
     constexpr std::integral_constant<int, CHAIN_F32> f32 {};
     constexpr std::integral_constant<int, CHAIN_BF16> b {};
     constexpr std::integral_constant<int, CHAIN_F16> h {};

@@ -190,6 +190,9 @@ int chain_launch_i8(bool src_u8, int dst_dt, chain_t &C, unsigned batch, bool wi
         if (dst_dt == MI355_DT_F32) return go(u8, std::integral_constant<int, CHAIN_F32> {});
         return MI355_UNIMPLEMENTED;
     };
+    if (C.split > 1)
+        return src_u8 ? chain_go_parts<i8_mma_t<true, false, geo_t<4, 128>>>(dst_dt, C, batch, stream, "mfma_i8")
+                      : chain_go_parts<i8_mma_t<false, false, geo_t<4, 128>>>(dst_dt, C, batch, stream, "mfma_i8");
     return src_u8 ? by_dst(std::true_type {}) : by_dst(std::false_type {});
 }
 

@@ -16,6 +16,9 @@ int chain_launch_mx(bool fp4, int dst_dt, chain_t &C, unsigned batch, bool wide,
         return wide ? chain_go<mxf8_mma_t<0, 0, wide_t>, D>(C, batch, stream, "mfma_f8")
                     : chain_go<mxf8_mma_t<0, 0, narrow_t>, D>(C, batch, stream, "mfma_f8");
     };
+    if (C.split > 1)
+        return fp4 ? chain_go_parts<mxf4_mma_t<narrow_t>>(dst_dt, C, batch, stream, "mfma_mxf4")
+                   : chain_go_parts<mxf8_mma_t<0, 0, narrow_t>>(dst_dt, C, batch, stream, "mfma_f8");
     if (dst_dt == MI355_DT_BF16) return go(std::integral_constant<int, CHAIN_BF16> {});
     if (dst_dt == MI355_DT_F32) return go(std::integral_constant<int, CHAIN_F32> {});
     return MI355_UNIMPLEMENTED;

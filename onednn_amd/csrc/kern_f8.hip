@@ -24,7 +24,8 @@ namespace {
 // pre-pass of the launch packs the scales (mx_pack_scales, kern_mxf4.hip).
 struct f8_plan_t {
     bool need_transpose, mx;
-    size_t off_sa, off_sb, total;
+    size_t off_sa, off_sb, off_parts, total;
+    chain_split_t split; // of K, where the scratch has room for the parts
     long Bw, Bsa, Bsb;
     long sets, pm, pn; // MX: sets of four blocks of K; M, N rounded up to whole tiles
 };
@@ -36,7 +37,13 @@ bool f8_is_mx(const mi355_matmul_desc_t &d) {
             && ws.dt == MI355_DT_E8M0 && (ws.mask & 6) == 6 && ws.group[0] == 32 && ws.group[1] == 1;
 }
 
-f8_plan_t make_plan(const mi355_matmul_desc_t &d) {
+bool is_e4m3_pair(const mi355_matmul_desc_t &d) { return d.src_dt == MI355_DT_F8_E4M3 && d.wei_dt == MI355_DT_F8_E4M3; }
+bool f8_chain(const problem_t &P, bool mx, chain_t &C) {
+    return chain_from_mx(P, mx, true, C) && (P.dst_dt == MI355_DT_BF16 || P.dst_dt == MI355_DT_F32);
+}
+constexpr long F8_STEP_NS = 700; // of a 256 x 128 tile (chain_split)
+
+f8_plan_t make_plan(const mi355_matmul_desc_t &d, bool parts) {
     f8_plan_t p {};
     p.Bw = d.wei_stride[0] ? d.batch : 1;
     p.need_transpose = !(d.wei_stride[1] == 1);
@@ -56,6 +63,13 @@ f8_plan_t make_plan(const mi355_matmul_desc_t &d) {
         p.off_sb = off;
         off += align_up((size_t)p.Bsb * std::max(p.pn * p.sets * 4, p.pn * 4 * stages), 256);
     }
+    p.off_parts = off;
+    p.split = chain_split_t {1, 0};
+    problem_t P;
+    chain_t C;
+    if (parts && is_e4m3_pair(d) && tuning(TUNE_F8_TILES) == TUNE_AUTO && (problem_of_desc(d, P), f8_chain(P, p.mx, C)))
+        p.split = chain_split(d.batch, d.M, d.N, d.K, false, F8_STEP_NS);
+    off += chain_parts_bytes(d.batch, d.M, d.N, false, p.split.split);
     p.total = off;
     return p;
 }
@@ -91,12 +105,12 @@ int f8_supported(const mi355_matmul_desc_t &d) {
     return MI355_SUCCESS;
 }
 
-size_t f8_scratch_bytes(const mi355_matmul_desc_t &d) {
-    return make_plan(d).total;
+size_t f8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts) {
+    return make_plan(d, parts).total;
 }
 
-int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, hipStream_t stream) {
-    const f8_plan_t plan = make_plan(d);
+int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts, hipStream_t stream) {
+    const f8_plan_t plan = make_plan(d, parts);
     if (plan.total > 0 && !scratch) {
         set_error("mfma_f8: %zu bytes of scratch required", plan.total);
         return MI355_INVALID_ARGUMENTS;
@@ -121,13 +135,16 @@ int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, h
     // (MI355_F8_TILES: wide / narrow keep one geometry whatever the size: tests, tuning)
     const int force = tuning(TUNE_F8_TILES);
     chain_t C {};
-    const bool chain = !fa && !fb && chain_from_mx(P, plan.mx, true, C) && (P.dst_dt == MI355_DT_BF16 || P.dst_dt == MI355_DT_F32);
+    const bool chain = is_e4m3_pair(d) && f8_chain(P, plan.mx, C);
     const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N, d.K, chain) && force != TUNE_WIDE);
     if (chain) {
         C.a = (const char *)P.src; C.lda = P.ss[1]; C.a_bs = P.ss[0];
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K;
         C.sc = X.sc;
+        C.parts = (char *)scratch + plan.off_parts;
+        C.split = plan.split.split;
+        C.part_steps = plan.split.part_steps;
         const int st = plan.mx ? chain_launch_mx(false, P.dst_dt, C, (unsigned)d.batch, !narrow, stream)
                                : chain_launch_f8(P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;

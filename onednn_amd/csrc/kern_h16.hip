@@ -4,6 +4,7 @@
 // plain loop, whose matrix instructions take eight times the cycles per byte.
 #include <cstdlib>
 #include <cstring>
+#include <algorithm>
 #include "f8_family.hpp"
 #include "chain_gemm.hpp"
 #include "line_policies.hpp"
@@ -225,10 +226,13 @@ struct h16_plan_t {
     int op_dt;
     long EB, Kp, pitch, Bs, Bw;
     bool copy_src, copy_wei;
-    size_t off_wei, total;
+    size_t off_wei, off_parts, total;
+    // of K, where the scratch has room for the parts: on 256 x 128 tiles, and on 256 x 256 ones with both operands across K
+    chain_split_t split, split_across;
 };
+constexpr long H16_STEP_NS = 600, H16_WIDE_STEP_NS = 1080; // of either tile (chain_split)
 
-static h16_plan_t h16_plan(const mi355_matmul_desc_t &d) {
+static h16_plan_t h16_plan(const mi355_matmul_desc_t &d, bool parts) {
     h16_plan_t p {};
     if (d.K < 1) return p;
     p.Bs = d.src_stride[0] ? d.batch : 1;
@@ -259,6 +263,21 @@ static h16_plan_t h16_plan(const mi355_matmul_desc_t &d) {
     if (p.copy_src || p.inside) off += align_up((size_t)p.Bs * d.M * p.pitch * p.EB, 256);
     p.off_wei = off;
     if (p.copy_wei || p.inside) off += align_up((size_t)p.Bw * d.N * p.pitch * p.EB, 256);
+    p.off_parts = off;
+    p.split = p.split_across = chain_split_t {1, 0};
+    if (parts && (p.op_dt == MI355_DT_BF16 || p.op_dt == MI355_DT_F16) && tuning(TUNE_H16_TILES) == TUNE_AUTO) {
+        problem_t P;
+        chain_t C;
+        problem_of_desc(d, P);
+        if (p.woq) P.wei_scale.dt = P.wei_zp.dt = MI355_DT_UNDEF; // applied by the copy
+        if (chain_from(P, false, P.dst_dt == p.op_dt, C) && !is_int8_dt(P.dst_dt)) {
+            p.split = chain_split(d.batch, d.M, d.N, p.Kp * p.EB, false, H16_STEP_NS);
+            if (!p.woq && d.src_stride[2] != 1 && d.wei_stride[1] != 1)
+                p.split_across = chain_split(d.batch, d.M, d.N, d.K * p.EB, true, H16_WIDE_STEP_NS);
+        }
+    }
+    off += std::max(chain_parts_bytes(d.batch, d.M, d.N, false, p.split.split),
+            chain_parts_bytes(d.batch, d.M, d.N, true, p.split_across.split));
     p.total = off;
     p.ok = true;
     return p;
@@ -308,7 +327,7 @@ static int h16_woq_fast(const mi355_matmul_desc_t &d, const h16_plan_t &p) {
 int h16_supported(const mi355_matmul_desc_t &d) {
     if (dt_bits(d.dst_dt) < 8 && !tile_nibble_dst_ok(d)) return MI355_UNIMPLEMENTED;
     if (d.batch > 65535) return MI355_UNIMPLEMENTED;
-    if (h16_woq(d)) return h16_plan(d).ok ? MI355_SUCCESS : MI355_UNIMPLEMENTED;
+    if (h16_woq(d)) return h16_plan(d, false).ok ? MI355_SUCCESS : MI355_UNIMPLEMENTED;
     if (d.src_dt != d.wei_dt || (d.src_dt != MI355_DT_BF16 && d.src_dt != MI355_DT_F16 && d.src_dt != MI355_DT_F32))
         return MI355_UNIMPLEMENTED;
     if (!quant_absent(d.src_zp) || !quant_absent(d.wei_zp) || !quant_absent(d.src_pr)) return MI355_UNIMPLEMENTED;
@@ -319,11 +338,11 @@ int h16_supported(const mi355_matmul_desc_t &d) {
             && ((d.wei_scale.mask & 2) || d.wei_scale.group[0] > 1 || d.wei_scale.group[1] > 1))
         return MI355_UNIMPLEMENTED;
     if (d.batch > 65535) return MI355_UNIMPLEMENTED;
-    return h16_plan(d).ok ? MI355_SUCCESS : MI355_UNIMPLEMENTED;
+    return h16_plan(d, false).ok ? MI355_SUCCESS : MI355_UNIMPLEMENTED;
 }
 
-size_t h16_scratch_bytes(const mi355_matmul_desc_t &d) {
-    const h16_plan_t p = h16_plan(d);
+size_t h16_scratch_bytes(const mi355_matmul_desc_t &d, bool parts) {
+    const h16_plan_t p = h16_plan(d, parts);
     return p.ok ? p.total : 0;
 }
 
@@ -381,8 +400,8 @@ static int h16_across(const mi355_matmul_desc_t &d, const h16_plan_t &p, const p
     return d.src_stride[2] != 1 && lines(P.src, d.src_stride[1], d.src_stride[2], d.src_stride[0], d.M) ? 2 : 0;
 }
 
-int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratch, hipStream_t stream) {
-    h16_plan_t plan = h16_plan(d);
+int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratch, bool parts, hipStream_t stream) {
+    h16_plan_t plan = h16_plan(d, parts);
     if (!plan.ok) {
         set_error("mfma_h16: the problem is not one this family takes");
         return MI355_UNIMPLEMENTED;
@@ -406,7 +425,13 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
     chain_t C {};
     int across = h16_across(d, plan, P);
     // the 256 x 128 tile takes weights across K only: src is copied there (whole chunks of K)
-    if (across == 2 && narrow) across = d.K % 8 == 0 ? 1 : 0;
+    const bool split_both = across == 2 && plan.split_across.split > 1;
+    if (across == 2 && narrow && !split_both) across = d.K % 8 == 0 ? 1 : 0;
+    auto split = [&](const chain_split_t &s) {
+        C.parts = (char *)scratch + plan.off_parts;
+        C.split = s.split;
+        C.part_steps = s.part_steps;
+    };
     if (across && (P.dst_dt == plan.op_dt || P.dst_dt == MI355_DT_F32) && chain_from(P, false, true, C)) {
         C.a = (const char *)P.src;
         C.a_bs = d.src_stride[0] * EB;
@@ -423,6 +448,7 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
         C.b_bs = d.wei_stride[0] * EB;
         C.ldb = d.wei_stride[1] * EB;
         C.kbytes = d.K * EB;
+        split(across == 2 ? plan.split_across : plan.split);
         return chain_launch_h16_across(plan.op_dt == MI355_DT_BF16, P.dst_dt, across, C, (unsigned)d.batch, !narrow, stream);
     }
     char *a_copy = (char *)scratch, *b_copy = (char *)scratch + plan.off_wei;
@@ -493,6 +519,7 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
         C.a = (const char *)P.src; C.lda = P.ss[1] * EB; C.a_bs = P.ss[0] * EB;
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K * EB;
+        split(plan.split);
         const int st = chain_launch_h16(plan.op_dt == MI355_DT_BF16, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }

@@ -316,7 +316,8 @@ __global__ void __launch_bounds__(256) i8_rowsum_kernel(const int8_t *p, long ro
 struct i8_plan_t {
     bool small; // 32 x 32 tiles
     bool need_transpose, need_colsum, need_rowsum;
-    size_t off_bt, off_colsum, off_rowsum, total;
+    size_t off_bt, off_colsum, off_rowsum, off_parts, total;
+    chain_split_t split; // of K on the LDS tiles, where the scratch has room for the parts
     long Bw, Bs;
 };
 
@@ -356,7 +357,20 @@ bool small_tiles_better(const mi355_matmul_desc_t &d, bool chain) {
 }
 
 // chain: what i8_chain says, the same of the descriptor's problem and of the launch's
-i8_plan_t make_plan(const mi355_matmul_desc_t &d, bool chain) {
+// The line of small_tiles_better is drawn against LDS tiles that take all of K; with K split (chain_gemm.hpp) they are the better
+// ones from fewer small tiles on where K is long.  Both sides in ns, from a dozen shapes: 128 x 4096 x 4096 17.1 us small, 20.2
+// split, 1024 x 1024 x 4096 31 and 20.3, with sums 64 x 2048 x 16384 31.0 and 33.4; a tenth in favour of the small tiles, one launch.
+bool split_tiles_better(const mi355_matmul_desc_t &d, const chain_split_t &s) {
+    const bool sums = d.src_dt == MI355_DT_U8 || !quant_absent(d.src_zp);
+    const double small_tiles = (double)((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch;
+    const double tiles = (double)((d.M + 255) / 256) * ((d.N + 127) / 128) * d.batch;
+    const double small = 3500 + (small_tiles < 256 ? 256 : small_tiles) * d.K * (d.K % LKB == 0 ? 6.6e-3 : 5.2e-3);
+    const double split = 9000 + s.part_steps * 700. + s.split * tiles * 52 + (sums ? 3500 + (double)d.N * d.K * 1e-4 : 0);
+    return 1.1 * split < small;
+}
+constexpr long I8_STEP_NS = 700; // of a 256 x 128 tile (chain_split)
+
+i8_plan_t make_plan(const mi355_matmul_desc_t &d, bool chain, bool parts) {
     i8_plan_t p {};
     p.Bw = d.wei_stride[0] ? d.batch : 1;
     p.Bs = d.src_stride[0] ? d.batch : 1;
@@ -368,6 +382,12 @@ i8_plan_t make_plan(const mi355_matmul_desc_t &d, bool chain) {
     const int force = tuning(TUNE_I8_TILES);
     if (force == TUNE_LARGE || force == TUNE_WIDE || force == TUNE_NARROW) p.small = false;
     if (force == TUNE_SMALL && !d.dst_scale_dynamic) p.small = true;
+    p.split = chain_split_t {1, 0};
+    if (chain && parts && force == TUNE_AUTO) {
+        const chain_split_t split = chain_split(d.batch, d.M, d.N, d.K, false, I8_STEP_NS);
+        if (p.small && split.split > 1 && split_tiles_better(d, split)) p.small = false;
+        if (!p.small) p.split = split;
+    }
     // a = off_s - zs can be non-zero whenever src is u8 or has a zero point;
     // c likewise for the weights.  The small tiles compute their own sums: a
     // problem they run on K-contiguous weights needs no scratch at all.
@@ -384,6 +404,8 @@ i8_plan_t make_plan(const mi355_matmul_desc_t &d, bool chain) {
     if (colsum) off += align_up((size_t)p.Bw * d.N * 4, 256);
     p.off_rowsum = off;
     if (rowsum) off += align_up((size_t)p.Bs * d.M * 4, 256);
+    p.off_parts = off;
+    off += chain_parts_bytes(d.batch, d.M, d.N, false, p.split.split);
     p.total = off;
     return p;
 }
@@ -419,18 +441,18 @@ int i8_supported(const mi355_matmul_desc_t &d) {
 
 bool i8_scratch_optional(const mi355_matmul_desc_t &d) { return d.K % BK != 0 && d.wei_stride[1] == 1; }
 
-size_t i8_scratch_bytes(const mi355_matmul_desc_t &d) {
+size_t i8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts) {
     problem_t P;
     problem_of_desc(d, P);
     chain_t C;
-    return make_plan(d, i8_chain(P, C)).total;
+    return make_plan(d, i8_chain(P, C), parts).total;
 }
 
-int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
+int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts,
         hipStream_t stream) {
     chain_t C {};
     bool chain = i8_chain(P, C);
-    i8_plan_t plan = make_plan(d, chain);
+    i8_plan_t plan = make_plan(d, chain, parts);
     // A K that ends inside 64 bytes also takes operands off 16-byte boundaries, which the LDS tiles' loads cannot, and
     // K-contiguous weights without scratch: the small tiles'.
     if (!plan.small && d.K % BK != 0) {
@@ -480,6 +502,9 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         C.colsum_bs = plan.Bw > 1 ? d.N : 0;
         C.src_zp = P.src_zp.dt != MI355_DT_UNDEF ? (const int *)P.src_zp.p : nullptr;
         C.off_s = su ? 128 : 0;
+        C.parts = sc + plan.off_parts;
+        C.split = plan.split.split;
+        C.part_steps = plan.split.part_steps;
     }
     if (plan.small) {
         if (chain) {

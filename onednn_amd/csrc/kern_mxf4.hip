@@ -163,13 +163,19 @@ __global__ void __launch_bounds__(256) mx_scales_blocks_kernel(const uint8_t *in
 
 struct mxf4_plan_t {
     bool need_transpose;
-    size_t off_bt, off_sb, off_sa, total;
+    size_t off_bt, off_sb, off_sa, off_parts, total;
+    chain_split_t split; // of K, where the scratch has room for the parts
     long Bw, Bsb, Bsa;
     long pm, pn; // M, N rounded up to whole tiles
     long nst;
 };
 
-mxf4_plan_t make_plan(const mi355_matmul_desc_t &d) {
+bool mxf4_chain(const problem_t &P, chain_t &C) {
+    return chain_from_mx(P, true, false, C) && (P.dst_dt == MI355_DT_BF16 || P.dst_dt == MI355_DT_F32);
+}
+constexpr long MXF4_STEP_NS = 800; // of a 256 x 128 tile (chain_split)
+
+mxf4_plan_t make_plan(const mi355_matmul_desc_t &d, bool parts) {
     mxf4_plan_t p {};
     p.Bw = d.wei_stride[0] ? d.batch : 1;
     p.Bsb = (d.wei_scale.mask & 1) ? p.Bw : 1;
@@ -186,6 +192,13 @@ mxf4_plan_t make_plan(const mi355_matmul_desc_t &d) {
     p.Bsa = ((d.src_scale.mask & 1) && d.src_stride[0]) ? d.batch : 1;
     p.off_sa = off;
     off += align_up((size_t)p.Bsa * p.pm * p.nst * 4, 256);
+    p.off_parts = off;
+    p.split = chain_split_t {1, 0};
+    problem_t P;
+    chain_t C;
+    if (parts && tuning(TUNE_F8_TILES) == TUNE_AUTO && (problem_of_desc(d, P), mxf4_chain(P, C)))
+        p.split = chain_split(d.batch, d.M, d.N, d.K / 2, false, MXF4_STEP_NS);
+    off += chain_parts_bytes(d.batch, d.M, d.N, false, p.split.split);
     p.total = off;
     return p;
 }
@@ -236,12 +249,12 @@ int mxf4_supported(const mi355_matmul_desc_t &d) {
     return MI355_SUCCESS;
 }
 
-size_t mxf4_scratch_bytes(const mi355_matmul_desc_t &d) {
-    return make_plan(d).total;
+size_t mxf4_scratch_bytes(const mi355_matmul_desc_t &d, bool parts) {
+    return make_plan(d, parts).total;
 }
 
-int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, hipStream_t stream) {
-    const mxf4_plan_t plan = make_plan(d);
+int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts, hipStream_t stream) {
+    const mxf4_plan_t plan = make_plan(d, parts);
     if (!scratch) {
         set_error("mfma_mxf4: %zu bytes of scratch required", plan.total);
         return MI355_INVALID_ARGUMENTS;
@@ -267,13 +280,16 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
     // (MI355_F8_TILES keeps one geometry here as well)
     const int force = tuning(TUNE_F8_TILES);
     chain_t C {};
-    const bool chain = chain_from_mx(P, true, false, C) && (P.dst_dt == MI355_DT_BF16 || P.dst_dt == MI355_DT_F32);
+    const bool chain = mxf4_chain(P, C);
     const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N, d.K / 2, chain) && force != TUNE_WIDE);
     if (chain) {
         C.a = (const char *)P.src; C.lda = P.ss[1] / 2; C.a_bs = P.ss[0] / 2;
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K / 2;
         C.sc = X.sc;
+        C.parts = sc + plan.off_parts;
+        C.split = plan.split.split;
+        C.part_steps = plan.split.part_steps;
         const int st = chain_launch_mx(true, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }

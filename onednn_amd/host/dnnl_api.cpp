@@ -2943,7 +2943,8 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
     if (pd0.runtime) {
         scratch = rt_scratch;
     } else if (pd.attr.scratchpad_mode == dnnl_scratchpad_mode_user) {
-        if ((st = handle(DNNL_ARG_SCRATCHPAD, pd.scratch_bytes > 0, &scratch))) return st;
+        // (the launch refuses a problem that cannot do without)
+        if ((st = handle(DNNL_ARG_SCRATCHPAD, false, &scratch))) return st;
     } else if (scratch) {
         // the library-mode scratchpad belongs to the primitive: executions of
         // one primitive object are serialised on the host while they enqueue
