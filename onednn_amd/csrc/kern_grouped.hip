@@ -238,12 +238,13 @@ __device__ __forceinline__ g4u gk_frag16(const gk_u2 (&raw)[8], int r) {
 }
 
 // lane (j, q) of a wavefront's 64 x 64: acc[r][c][e] is row 4 (4 q + e) + r, column 4 j + c
-template <int DT>
+// WHOLE: dst's rows are whole 128-byte lines (the launch's rule)
+template <int DT, bool WHOLE>
 __device__ __forceinline__ void gk_store(const grouped_k_dev_t &P, const gk_f4 (&acc)[4][4], long g, long m_w, long n_w,
         int j, int q) {
     const long col = n_w + 4 * j;
     // dst is written once and not read again by the launch: non-temporal stores, which do not take lines of the
-    // L2s (a quarter faster on a launch that writes 1.3 GB: 0.325 -> 0.25 ms)
+    // L2s (a quarter faster on a launch that writes 1.3 GB: 0.325 -> 0.25 ms), where dst's rows are whole lines
     // bf16: v_cvt_pk_bf16_f32 unless the wavefront holds a NaN or an f32 subnormal, which the software conversion
     // (the reference's: subnormals flush, NaNs are quieted its way) treats differently; f16: v_cvt_f16_f32 unless it
     // holds a NaN (the 64 software roundings a lane were the kernel's bound: 435 rows over 64 groups, 3712 x 8064, f16,
@@ -261,6 +262,10 @@ __device__ __forceinline__ void gk_store(const grouped_k_dev_t &P, const gk_f4 (
         hw = __builtin_amdgcn_ballot_w64(special) == 0;
     }
     if (col >= P.NB) return;
+    auto put = [](const auto &v, auto *to) __attribute__((always_inline)) {
+        if constexpr (WHOLE) __builtin_nontemporal_store(v, to);
+        else *to = v;
+    };
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -270,30 +275,30 @@ __device__ __forceinline__ void gk_store(const grouped_k_dev_t &P, const gk_f4 (
             const long off = g * P.dst_g + row * P.dst_ld + col;
             const float v0 = acc[r][0][e], v1 = acc[r][1][e], v2 = acc[r][2][e], v3 = acc[r][3][e];
             if (DT == MI355_DT_F32) {
-                __builtin_nontemporal_store(gk_f4 {v0, v1, v2, v3}, (gk_f4 *)((float *)P.dst + off));
+                put(gk_f4 {v0, v1, v2, v3}, (gk_f4 *)((float *)P.dst + off));
             } else if (DT == MI355_DT_BF16 && hw) {
                 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
                 typedef float f32x2_t __attribute__((ext_vector_type(2)));
                 gk_u2 o;
                 o.x = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2_t {v0, v1}, bf16x2_t));
                 o.y = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2_t {v2, v3}, bf16x2_t));
-                __builtin_nontemporal_store(o, (gk_u2 *)((uint16_t *)P.dst + off));
+                put(o, (gk_u2 *)((uint16_t *)P.dst + off));
             } else if (DT == MI355_DT_F16 && hw) {
                 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
                 gk_u2 o;
                 o.x = __builtin_bit_cast(unsigned, f16x2_t {(_Float16)v0, (_Float16)v1});
                 o.y = __builtin_bit_cast(unsigned, f16x2_t {(_Float16)v2, (_Float16)v3});
-                __builtin_nontemporal_store(o, (gk_u2 *)((uint16_t *)P.dst + off));
+                put(o, (gk_u2 *)((uint16_t *)P.dst + off));
             } else {
                 gk_u2 o;
                 o.x = (cvt_store_bits(DT, v0) & 0xffffu) | (cvt_store_bits(DT, v1) << 16);
                 o.y = (cvt_store_bits(DT, v2) & 0xffffu) | (cvt_store_bits(DT, v3) << 16);
-                __builtin_nontemporal_store(o, (gk_u2 *)((uint16_t *)P.dst + off));
+                put(o, (gk_u2 *)((uint16_t *)P.dst + off));
             }
         }
 }
 
-template <int DT>
+template <int DT, bool WHOLE>
 __global__ void __launch_bounds__(256) grouped_k_tile_kernel(const grouped_k_dev_t P) {
     typedef gk_f4 f4;
     typedef gk_step_t<DT> step_t;
@@ -338,7 +343,7 @@ __global__ void __launch_bounds__(256) grouped_k_tile_kernel(const grouped_k_dev
         }
     }
 
-    gk_store<DT>(P, acc, g, m_w, n_w, i, q);
+    gk_store<DT, WHOLE>(P, acc, g, m_w, n_w, i, q);
 }
 
 // ---- "hip:mfma_grouped" -- the 2Dx3D pattern on the matrix cores for fp8,
@@ -996,7 +1001,7 @@ __device__ __forceinline__ void gk_wait_vm(int n) {
     }
 }
 
-template <int DT, int GK_NST>
+template <int DT, int GK_NST, bool WHOLE>
 __global__ void __launch_bounds__(256) grouped_k_lds_kernel(const grouped_k_dev_t P) {
     typedef gk_f4 f4;
     extern __shared__ __attribute__((aligned(16))) unsigned char gk_smem[];
@@ -1113,7 +1118,7 @@ __global__ void __launch_bounds__(256) grouped_k_lds_kernel(const grouped_k_dev_
             first_stages(n_t + 128);
         }
         const long n_w = n_t + (wave & 1) * 64;
-        if (m_w < P.MA && n_w < P.NB) gk_store<DT>(P, acc, g, m_w, n_w, i, q);
+        if (m_w < P.MA && n_w < P.NB) gk_store<DT, WHOLE>(P, acc, g, m_w, n_w, i, q);
         stores_behind = m_w >= P.MA || n_w >= P.NB ? 0 : (m_w + 64 <= P.MA && n_w + 64 <= P.NB ? 16 : -1);
     }
 }
@@ -1481,6 +1486,11 @@ int launch_k_tiles(int plan, const grouped_dev_t &G, hipStream_t stream) {
     const bool h16 = d.src_dt != MI355_DT_F32;
     bool lds_path = h16 && P.MA % 8 == 0 && P.NB % 8 == 0 && d.total * (P.MA > P.NB ? P.MA : P.NB) * 2 < (1L << 32);
     if (tuning(TUNE_GROUPED_IMPL) == TUNE_SHORT) lds_path = false;
+    // Non-temporal stores where dst's rows are whole 128-byte lines; where they are not a wavefront's 128 bytes of a row are
+    // pieces of two lines, which the L2s have to put together (bf16, 64 rows over 32 groups, 1472 x 6768: 300 us non-temporal,
+    // 201 so; 594 rows, 2944 x 2864: 248 and 188).
+    const long esz = d.src_dt == MI355_DT_F32 ? 4 : 2;
+    const bool whole = (((uintptr_t)P.dst | (uintptr_t)(P.dst_ld * esz) | (uintptr_t)(P.dst_g * esz)) & 127) == 0;
     if (lds_path) {
         const bool brief = d.total <= 48 * d.group_count; // (k per group on average)
         // runs of up to 8 column tiles a workgroup, while some thousands of workgroups remain
@@ -1496,16 +1506,22 @@ int launch_k_tiles(int plan, const grouped_dev_t &G, hipStream_t stream) {
             hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, P);
             return hipGetLastError() == hipSuccess ? (int)MI355_SUCCESS : (int)MI355_RUNTIME_ERROR;
         };
-        if (d.src_dt == MI355_DT_BF16)
-            return brief ? launch(grouped_k_lds_kernel<MI355_DT_BF16, 2>, 2) : launch(grouped_k_lds_kernel<MI355_DT_BF16, 4>, 4);
-        return brief ? launch(grouped_k_lds_kernel<MI355_DT_F16, 2>, 2) : launch(grouped_k_lds_kernel<MI355_DT_F16, 4>, 4);
+        auto by_depth = [&](auto dt) -> int {
+            constexpr int DT = decltype(dt)::value;
+            if (brief) return whole ? launch(grouped_k_lds_kernel<DT, 2, true>, 2) : launch(grouped_k_lds_kernel<DT, 2, false>, 2);
+            return whole ? launch(grouped_k_lds_kernel<DT, 4, true>, 4) : launch(grouped_k_lds_kernel<DT, 4, false>, 4);
+        };
+        return d.src_dt == MI355_DT_BF16 ? by_depth(std::integral_constant<int, MI355_DT_BF16> {})
+                                         : by_depth(std::integral_constant<int, MI355_DT_F16> {});
     }
-    if (d.src_dt == MI355_DT_F32)
-        hipLaunchKernelGGL(grouped_k_tile_kernel<MI355_DT_F32>, grid, dim3(256), 0, stream, P);
-    else if (d.src_dt == MI355_DT_BF16)
-        hipLaunchKernelGGL(grouped_k_tile_kernel<MI355_DT_BF16>, grid, dim3(256), 0, stream, P);
-    else
-        hipLaunchKernelGGL(grouped_k_tile_kernel<MI355_DT_F16>, grid, dim3(256), 0, stream, P);
+    auto tiles = [&](auto dt) {
+        constexpr int DT = decltype(dt)::value;
+        if (whole) hipLaunchKernelGGL((grouped_k_tile_kernel<DT, true>), grid, dim3(256), 0, stream, P);
+        else hipLaunchKernelGGL((grouped_k_tile_kernel<DT, false>), grid, dim3(256), 0, stream, P);
+    };
+    if (d.src_dt == MI355_DT_F32) tiles(std::integral_constant<int, MI355_DT_F32> {});
+    else if (d.src_dt == MI355_DT_BF16) tiles(std::integral_constant<int, MI355_DT_BF16> {});
+    else tiles(std::integral_constant<int, MI355_DT_F16> {});
     return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
 }
 
