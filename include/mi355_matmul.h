@@ -335,8 +335,8 @@ const char *mi355_last_error(void); /* thread-local text of the last failure */
  *   MI355_I8_TILES     large | wide | narrow | small   tile geometry of hip:mfma_i8
  *                      (large: the LDS tiles, 256 x 128 or 256 x 256 by the tile count;
  *                      wide: 256 x 256; narrow: 256 x 128; small: 32 x 32 without LDS)
- *   MI355_F8_TILES     wide | narrow          hip:mfma_f8 on 256 x 256 / 256 x 128 tiles
- *   MI355_H16_TILES    wide                   hip:mfma_h16 on 256 x 256 tiles
+ *   MI355_F8_TILES     wide | narrow | small  hip:mfma_f8, hip:mfma_mxf4 on 256 x 256 / 256 x 128 / 32 x 32 tiles
+ *   MI355_H16_TILES    wide | narrow | small  hip:mfma_h16 on the same
  *   MI355_GROUPED_IMPL ref | short | tall | wide   grouped matmul kernel (ref: a thread per dst element;
  *                      variable M: 16 x 32, 48 x 64 or 64 x 256 tiles; variable K: short = the f32
  *                      instruction for 16-bit types too, tall / wide = a workgroup takes one / eight

@@ -32,8 +32,8 @@ struct tune_name_t {
 };
 const tune_name_t TUNE_NAMES[TUNE_COUNT] = {
         {"MI355_I8_TILES", "large wide small narrow"},
-        {"MI355_F8_TILES", "wide narrow"},
-        {"MI355_H16_TILES", "wide"},
+        {"MI355_F8_TILES", "wide narrow small"},
+        {"MI355_H16_TILES", "wide narrow small"},
         {"MI355_GROUPED_IMPL", "ref short tall wide"},
         {"MI355_GEMM_ORDER", ""},
         {"MI355_EPILOGUE", "chain"},

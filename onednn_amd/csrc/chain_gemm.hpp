@@ -22,37 +22,6 @@ namespace mi355 {
 enum chain_dst_t { CHAIN_BF16, CHAIN_F16, CHAIN_F32, CHAIN_I8, CHAIN_PART }; // CHAIN_PART: a part of K, no epilogue
 enum chain_act_t { CHAIN_NONE, CHAIN_RELU, CHAIN_GELU, CHAIN_SWISH };
 
-struct chain_vec_t { // f32 / bf16 / f16 values; dt UNDEF = absent
-    const void *p;
-    int dt, per; // per: one value for every column (weights scales, bias) or row (src scales) instead of one for all
-    long bs;     // elements between batches
-};
-
-struct chain_t {
-    const char *a, *bt;
-    char *dst;
-    long lda, ldb, a_bs, b_bs, dst_pitch, dst_bs; // bytes
-    long M, N, kbytes;
-    int tiles_m, tiles_n;
-    gemm::line_scales_args_t sc;
-    chain_vec_t ssc, wsc, bias;
-    int act, staged; // staged: 1 = + the bf16 tensor, 2 = * it
-    float alpha;
-    const char *st;
-    long st_pitch, st_bs;
-    // int8: (K sum) + (off_s - src zero point) * colsum[n]
-    const int *colsum, *src_zp;
-    long colsum_bs;
-    int off_s;
-    const void *dsc;
-    int dsc_dt, ds_mode; // 0 none, 1 divide, 2 multiply by the reciprocal
-    int lo, hi;          // 8-bit dst
-    // split > 1: K in parts of part_steps steps, a workgroup each; their accumulators go to parts and chain_sum_kernel
-    // (kern_chain_sum.hip) adds them and does the rest
-    char *parts;
-    int split, part_steps;
-};
-
 // Into how many parts of K a problem of few tiles is split, 1 = not at all.  One workgroup a CU and round: with T tiles
 // (256 x 128, or 256 x 256) a launch takes its K steps one after the other on T of 256 CUs.  S parts make that steps / S, for
 // a second kernel (3 us and more of a launch), the parts' way out and in again (a part of a tile 128 / 256 KB each way) and
@@ -84,6 +53,47 @@ inline size_t chain_parts_bytes(long batch, long M, long N, bool wide, int split
     const long bn = wide ? 256 : 128;
     return split > 1 ? (size_t)(batch * ((M + 255) / 256) * ((N + bn - 1) / bn)) * split * (size_t)(256 * bn * 4) : 0;
 }
+
+struct chain_vec_t { // f32 / bf16 / f16 values; dt UNDEF = absent
+    const void *p;
+    int dt, per; // per: one value for every column (weights scales, bias) or row (src scales) instead of one for all
+    long bs;     // elements between batches
+};
+
+struct chain_t {
+    const char *a, *bt;
+    char *dst;
+    long lda, ldb, a_bs, b_bs, dst_pitch, dst_bs; // bytes
+    long M, N, kbytes;
+    int tiles_m, tiles_n;
+    gemm::line_scales_args_t sc;
+    chain_vec_t ssc, wsc, bias;
+    int act, staged; // staged: 1 = + the bf16 tensor, 2 = * it
+    float alpha;
+    const char *st;
+    long st_pitch, st_bs;
+    // int8: (K sum) + (off_s - src zero point) * colsum[n]
+    const int *colsum, *src_zp;
+    long colsum_bs;
+    int off_s;
+    const void *dsc;
+    int dsc_dt, ds_mode; // 0 none, 1 divide, 2 multiply by the reciprocal
+    int lo, hi;          // 8-bit dst
+    // split > 1: K in parts of part_steps steps, a workgroup each; their accumulators go to parts and chain_sum_kernel
+    // (kern_chain_sum.hip) adds them and does the rest
+    char *parts;
+    int split, part_steps;
+    // e8m0 scales as the caller has them (chain_launch_small): [M][K / 32] and [K / 32][N], values between batches
+    const uint8_t *sa, *sb;
+    long sa_bs, sb_bs;
+};
+
+// A product of few 32 x 32 tiles on chain_small_float_kernel (kern_chain_small.hip): small_tiles_float says whether (mx: 0, or
+// the bits of a block-scaled type).
+enum chain_small_t { CHAIN_SMALL_BF16, CHAIN_SMALL_F16, CHAIN_SMALL_F8, CHAIN_SMALL_MXF8, CHAIN_SMALL_MXF4 };
+bool small_tiles_float(long batch, long M, long N, long kbytes, const chain_split_t &split, long step_ns, const chain_t &C, int mx);
+int chain_launch_small(chain_small_t kind, int dst_dt, chain_t &C, unsigned batch, hipStream_t stream);
+
 // the sums of a problem whose parts lie at C.parts, and its epilogue (integer: they are s32)
 int chain_launch_sum(bool integer, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
 
@@ -460,6 +470,80 @@ int chain_go(chain_t &C, unsigned batch, hipStream_t stream, const char *who) {
     hipLaunchKernelGGL((chain_gemm_kernel<Mma, DST>), grid, dim3(Mma::G::NT), smem_bytes, stream, C);
     return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
 }
+// The chain for four consecutive columns of one row, a thread at a time: what chain_part_t::store does with a tile.
+// load: its operands, ahead of the sums; m and n are inside dst.
+template <int DST>
+struct chain_quad_t {
+    float ssc, w[4], bias[4];
+    v2u_cell_t y;
+    __device__ __forceinline__ void load(const chain_t &C, long b, long m, long n) {
+        ssc = C.ssc.dt != MI355_DT_UNDEF ? chain_load(C.ssc, b * C.ssc.bs + (C.ssc.per ? m : 0)) : 1.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const long ne = min(n + e, C.N - 1);
+            w[e] = C.wsc.dt != MI355_DT_UNDEF ? chain_load(C.wsc, b * C.wsc.bs + (C.wsc.per ? ne : 0)) : 1.f;
+            bias[e] = C.bias.dt != MI355_DT_UNDEF ? chain_load(C.bias, b * C.bias.bs + ne) : 0.f;
+        }
+        if (C.staged) y = *(const v2u_cell_t *)(C.st + b * C.st_bs + m * C.st_pitch + n * 2); // (columns in whole chunks of eight)
+    }
+    __device__ __forceinline__ void finish(const chain_t &C, long b, long m, long n, float (&x)[4]) const {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float f = x[e];
+            f *= ssc;
+            f *= w[e];
+            if (C.bias.dt != MI355_DT_UNDEF) f += bias[e];
+            if (C.act == CHAIN_RELU) f = DST == CHAIN_I8 ? fmaxf(f, 0.f) : f > 0 ? f : f * 0.f;
+            else if (C.act == CHAIN_GELU) f = gelu_tanh_fast(f);
+            else if (C.act == CHAIN_SWISH) f = f * logistic_fast(C.alpha * f);
+            x[e] = f;
+        }
+        if (C.staged) {
+            const float v[4] = {u2f(y.x << 16), u2f(y.x & 0xffff0000u), u2f(y.y << 16), u2f(y.y & 0xffff0000u)};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = C.staged == 1 ? x[e] + v[e] : x[e] * v[e];
+        }
+        constexpr int SHIFT = DST == CHAIN_I8 ? 0 : DST == CHAIN_F32 ? 2 : 1;
+        char *to = C.dst + b * C.dst_bs + m * C.dst_pitch + (n << SHIFT);
+        const int left = C.N - n < 4 ? (int)(C.N - n) : 4;
+        if constexpr (DST == CHAIN_I8) {
+            if (C.ds_mode) {
+                const float ds = chain_load(chain_vec_t {C.dsc, C.dsc_dt, 0, 0}, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = C.ds_mode == 2 ? x[e] * (1.f / ds) : x[e] / ds;
+            }
+            const unsigned word = pack4_i8(x, C.lo, C.hi);
+            if (left == 4) *(unsigned *)to = word;
+            else
+                for (int e = 0; e < left; ++e) to[e] = (char)(word >> (8 * e));
+        } else if constexpr (DST == CHAIN_F32) {
+            if (left == 4) *(v4f *)to = v4f {x[0], x[1], x[2], x[3]};
+            else
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (e < left) ((float *)to)[e] = x[e];
+        } else {
+            v2u_cell_t q;
+            if constexpr (DST == CHAIN_F16) {
+                unsigned h[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) h[e] = __builtin_bit_cast(uint16_t, (_Float16)x[e]);
+                q = v2u_cell_t {h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+            } else {
+                bool special = false;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) special |= __builtin_amdgcn_classf(x[e], 0x93); // NaN or subnormal
+                q = chain_bf16(x, __builtin_amdgcn_ballot_w64(special) != 0);
+            }
+            if (left == 4) *(v2u_cell_t *)to = q;
+            else
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (e < left) ((uint16_t *)to)[e] = (uint16_t)(q[e / 2] >> (16 * (e % 2)));
+        }
+    }
+};
+
 // K in parts (C.split of them), then their sums and the epilogue
 template <class Mma>
 int chain_go_parts(int dst_dt, chain_t &C, unsigned batch, hipStream_t stream, const char *who) {

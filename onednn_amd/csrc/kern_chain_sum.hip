@@ -22,14 +22,8 @@ __global__ void __launch_bounds__(256) chain_sum_kernel(const chain_t C) {
     if (m >= C.M || n >= C.N) return;
     const char *from = C.parts + ((b * C.split * tiles + id) * G::NW + wave) * 32768 + (i * 4 + k) * 1024 + lane * 16;
     const long pitch = tiles * G::NW * 32768;
-    const float ssc = C.ssc.dt != MI355_DT_UNDEF ? chain_load(C.ssc, b * C.ssc.bs + (C.ssc.per ? m : 0)) : 1.f;
-    float w[4], bias[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const long ne = min(n + e, C.N - 1);
-        w[e] = C.wsc.dt != MI355_DT_UNDEF ? chain_load(C.wsc, b * C.wsc.bs + (C.wsc.per ? ne : 0)) : 1.f;
-        bias[e] = C.bias.dt != MI355_DT_UNDEF ? chain_load(C.bias, b * C.bias.bs + ne) : 0.f;
-    }
+    chain_quad_t<DST> Q;
+    Q.load(C, b, m, n);
     V sum = *(const V *)from;
     int p = 1;
     for (; p + 4 <= C.split; p += 4) {
@@ -41,69 +35,17 @@ __global__ void __launch_bounds__(256) chain_sum_kernel(const chain_t C) {
     }
     for (; p < C.split; ++p) sum += *(const V *)(from + p * pitch);
 
-    // the chain, step by step as chain_part_t::store takes it
     float x[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        float f;
         if constexpr (INTEGER) {
             const int a = C.off_s - (C.src_zp ? *C.src_zp : 0);
-            f = (float)(sum[e] + (C.colsum ? a * C.colsum[b * C.colsum_bs + min(n + e, C.N - 1)] : 0));
+            x[e] = (float)(sum[e] + (C.colsum ? a * C.colsum[b * C.colsum_bs + min(n + e, C.N - 1)] : 0));
         } else {
-            f = sum[e];
+            x[e] = sum[e];
         }
-        f *= ssc;
-        f *= w[e];
-        if (C.bias.dt != MI355_DT_UNDEF) f += bias[e];
-        if (C.act == CHAIN_RELU) f = DST == CHAIN_I8 ? fmaxf(f, 0.f) : f > 0 ? f : f * 0.f;
-        else if (C.act == CHAIN_GELU) f = gelu_tanh_fast(f);
-        else if (C.act == CHAIN_SWISH) f = f * logistic_fast(C.alpha * f);
-        x[e] = f;
     }
-    if (C.staged) { // (columns in whole chunks of eight)
-        const v2u_cell_t q = *(const v2u_cell_t *)(C.st + b * C.st_bs + m * C.st_pitch + n * 2);
-        const float y[4] = {u2f(q.x << 16), u2f(q.x & 0xffff0000u), u2f(q.y << 16), u2f(q.y & 0xffff0000u)};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = C.staged == 1 ? x[e] + y[e] : x[e] * y[e];
-    }
-    constexpr int SHIFT = DST == CHAIN_I8 ? 0 : DST == CHAIN_F32 ? 2 : 1;
-    char *to = C.dst + b * C.dst_bs + m * C.dst_pitch + (n << SHIFT);
-    const int left = C.N - n < 4 ? (int)(C.N - n) : 4;
-    if constexpr (DST == CHAIN_I8) {
-        if (C.ds_mode) {
-            const float ds = chain_load(chain_vec_t {C.dsc, C.dsc_dt, 0, 0}, 0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] = C.ds_mode == 2 ? x[e] * (1.f / ds) : x[e] / ds;
-        }
-        const unsigned word = pack4_i8(x, C.lo, C.hi);
-        if (left == 4) *(unsigned *)to = word;
-        else
-            for (int e = 0; e < left; ++e) to[e] = (char)(word >> (8 * e));
-    } else if constexpr (DST == CHAIN_F32) {
-        if (left == 4) *(v4f *)to = v4f {x[0], x[1], x[2], x[3]};
-        else
-#pragma unroll
-            for (int e = 0; e < 3; ++e)
-                if (e < left) ((float *)to)[e] = x[e];
-    } else {
-        v2u_cell_t q;
-        if constexpr (DST == CHAIN_F16) {
-            unsigned h[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) h[e] = __builtin_bit_cast(uint16_t, (_Float16)x[e]);
-            q = v2u_cell_t {h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
-        } else {
-            bool special = false;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) special |= __builtin_amdgcn_classf(x[e], 0x93); // NaN or subnormal
-            q = chain_bf16(x, __builtin_amdgcn_ballot_w64(special) != 0);
-        }
-        if (left == 4) *(v2u_cell_t *)to = q;
-        else
-#pragma unroll
-            for (int e = 0; e < 3; ++e)
-                if (e < left) ((uint16_t *)to)[e] = (uint16_t)(q[e / 2] >> (16 * (e % 2)));
-    }
+    Q.finish(C, b, m, n, x);
 }
 
 } // namespace

@@ -26,6 +26,7 @@ struct f8_plan_t {
     bool need_transpose, mx;
     size_t off_sa, off_sb, off_parts, total;
     chain_split_t split; // of K, where the scratch has room for the parts
+    bool small;          // 32 x 32 tiles
     long Bw, Bsa, Bsb;
     long sets, pm, pn; // MX: sets of four blocks of K; M, N rounded up to whole tiles
 };
@@ -38,8 +39,10 @@ bool f8_is_mx(const mi355_matmul_desc_t &d) {
 }
 
 bool is_e4m3_pair(const mi355_matmul_desc_t &d) { return d.src_dt == MI355_DT_F8_E4M3 && d.wei_dt == MI355_DT_F8_E4M3; }
-bool f8_chain(const problem_t &P, bool mx, chain_t &C) {
-    return chain_from_mx(P, mx, true, C) && (P.dst_dt == MI355_DT_BF16 || P.dst_dt == MI355_DT_F32);
+// (an f16 dst has a chain on the small tiles only)
+bool f8_chain(const problem_t &P, bool mx, bool small, chain_t &C) {
+    return chain_from_mx(P, mx, true, C)
+            && (P.dst_dt == MI355_DT_BF16 || P.dst_dt == MI355_DT_F32 || (small && P.dst_dt == MI355_DT_F16));
 }
 constexpr long F8_STEP_NS = 700; // of a 256 x 128 tile (chain_split)
 
@@ -67,8 +70,13 @@ f8_plan_t make_plan(const mi355_matmul_desc_t &d, bool parts) {
     p.split = chain_split_t {1, 0};
     problem_t P;
     chain_t C;
-    if (parts && is_e4m3_pair(d) && tuning(TUNE_F8_TILES) == TUNE_AUTO && (problem_of_desc(d, P), f8_chain(P, p.mx, C)))
-        p.split = chain_split(d.batch, d.M, d.N, d.K, false, F8_STEP_NS);
+    const int force = tuning(TUNE_F8_TILES);
+    if (is_e4m3_pair(d) && force != TUNE_WIDE && (problem_of_desc(d, P), f8_chain(P, p.mx, true, C))) {
+        if (parts && force != TUNE_SMALL && P.dst_dt != MI355_DT_F16) p.split = chain_split(d.batch, d.M, d.N, d.K, false, F8_STEP_NS);
+        p.small = force == TUNE_SMALL
+                || (force == TUNE_AUTO && small_tiles_float(d.batch, d.M, d.N, d.K, p.split, F8_STEP_NS, C, p.mx ? 8 : 0));
+        if (p.small) p.split = chain_split_t {1, 0};
+    }
     off += chain_parts_bytes(d.batch, d.M, d.N, false, p.split.split);
     p.total = off;
     return p;
@@ -128,14 +136,15 @@ int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, b
         X.bt_bstride = d.wei_stride[0];
     }
     const int fa = d.src_dt == MI355_DT_F8_E5M2, fb = d.wei_dt == MI355_DT_F8_E5M2;
-    if (plan.mx) {
+    chain_t C {};
+    const bool small = plan.small && f8_chain(P, plan.mx, true, C);
+    const bool chain = small || (is_e4m3_pair(d) && f8_chain(P, plan.mx, false, C));
+    if (plan.mx && !small) {
         char *sa = (char *)scratch + plan.off_sa, *sb = (char *)scratch + plan.off_sb;
         if (const int st = mx_pack_scales(d, P, plan.Bsa, plan.Bsb, sa, sb, X.sc, stream)) return st;
     }
     // (MI355_F8_TILES: wide / narrow keep one geometry whatever the size: tests, tuning)
     const int force = tuning(TUNE_F8_TILES);
-    chain_t C {};
-    const bool chain = is_e4m3_pair(d) && f8_chain(P, plan.mx, C);
     const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N, d.K, chain) && force != TUNE_WIDE);
     if (chain) {
         C.a = (const char *)P.src; C.lda = P.ss[1]; C.a_bs = P.ss[0];
@@ -145,6 +154,11 @@ int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, b
         C.parts = (char *)scratch + plan.off_parts;
         C.split = plan.split.split;
         C.part_steps = plan.split.part_steps;
+        if (small) {
+            C.sa = (const uint8_t *)P.src_scale.p; C.sa_bs = plan.Bsa > 1 ? d.M * (d.K / 32) : 0;
+            C.sb = (const uint8_t *)P.wei_scale.p; C.sb_bs = plan.Bsb > 1 ? d.N * (d.K / 32) : 0;
+            return chain_launch_small(plan.mx ? CHAIN_SMALL_MXF8 : CHAIN_SMALL_F8, P.dst_dt, C, (unsigned)d.batch, stream);
+        }
         const int st = plan.mx ? chain_launch_mx(false, P.dst_dt, C, (unsigned)d.batch, !narrow, stream)
                                : chain_launch_f8(P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;

@@ -229,6 +229,7 @@ struct h16_plan_t {
     size_t off_wei, off_parts, total;
     // of K, where the scratch has room for the parts: on 256 x 128 tiles, and on 256 x 256 ones with both operands across K
     chain_split_t split, split_across;
+    bool small; // 32 x 32 tiles
 };
 constexpr long H16_STEP_NS = 600, H16_WIDE_STEP_NS = 1080; // of either tile (chain_split)
 
@@ -265,14 +266,20 @@ static h16_plan_t h16_plan(const mi355_matmul_desc_t &d, bool parts) {
     if (p.copy_wei || p.inside) off += align_up((size_t)p.Bw * d.N * p.pitch * p.EB, 256);
     p.off_parts = off;
     p.split = p.split_across = chain_split_t {1, 0};
-    if (parts && (p.op_dt == MI355_DT_BF16 || p.op_dt == MI355_DT_F16) && tuning(TUNE_H16_TILES) == TUNE_AUTO) {
+    const int force = tuning(TUNE_H16_TILES);
+    if ((p.op_dt == MI355_DT_BF16 || p.op_dt == MI355_DT_F16) && force != TUNE_WIDE) {
         problem_t P;
         chain_t C;
         problem_of_desc(d, P);
         if (p.woq) P.wei_scale.dt = P.wei_zp.dt = MI355_DT_UNDEF; // applied by the copy
         if (chain_from(P, false, P.dst_dt == p.op_dt, C) && !is_int8_dt(P.dst_dt)) {
-            p.split = chain_split(d.batch, d.M, d.N, p.Kp * p.EB, false, H16_STEP_NS);
-            if (!p.woq && d.src_stride[2] != 1 && d.wei_stride[1] != 1)
+            if (parts && force != TUNE_SMALL) p.split = chain_split(d.batch, d.M, d.N, p.Kp * p.EB, false, H16_STEP_NS);
+            // K-contiguous operands only: others are copied where the large tiles do not read them as they lie, and either way
+            // has the same bits
+            p.small = d.src_stride[2] == 1 && (p.woq || d.wei_stride[1] == 1)
+                    && (force == TUNE_SMALL || (force == TUNE_AUTO && small_tiles_float(d.batch, d.M, d.N, p.Kp * p.EB, p.split, H16_STEP_NS, C, 0)));
+            if (p.small) p.split = chain_split_t {1, 0};
+            if (parts && !p.woq && d.src_stride[2] != 1 && d.wei_stride[1] != 1)
                 p.split_across = chain_split(d.batch, d.M, d.N, d.K * p.EB, true, H16_WIDE_STEP_NS);
         }
     }
@@ -417,9 +424,10 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
     f8_extra_t X {};
     problem_t P = P_in;
     const long EB = plan.EB;
-    // (the MI355_H16_TILES switch keeps the 256 x 256 tiles: tests, tuning)
+    // (the MI355_H16_TILES switch keeps one geometry: tests, tuning)
     auto narrow_for = [&](bool chain) {
-        return line_tiles_narrow(d.batch, d.M, d.N, plan.Kp * EB, chain) && tuning(TUNE_H16_TILES) != TUNE_WIDE;
+        const int force = tuning(TUNE_H16_TILES);
+        return force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N, plan.Kp * EB, chain) && force != TUNE_WIDE);
     };
     bool narrow = narrow_for(true);
     chain_t C {};
@@ -519,6 +527,8 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
         C.a = (const char *)P.src; C.lda = P.ss[1] * EB; C.a_bs = P.ss[0] * EB;
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K * EB;
+        if (plan.small)
+            return chain_launch_small(plan.op_dt == MI355_DT_BF16 ? CHAIN_SMALL_BF16 : CHAIN_SMALL_F16, P.dst_dt, C, (unsigned)d.batch, stream);
         split(plan.split);
         const int st = chain_launch_h16(plan.op_dt == MI355_DT_BF16, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;

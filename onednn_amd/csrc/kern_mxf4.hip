@@ -165,13 +165,16 @@ struct mxf4_plan_t {
     bool need_transpose;
     size_t off_bt, off_sb, off_sa, off_parts, total;
     chain_split_t split; // of K, where the scratch has room for the parts
+    bool small;          // 32 x 32 tiles
     long Bw, Bsb, Bsa;
     long pm, pn; // M, N rounded up to whole tiles
     long nst;
 };
 
-bool mxf4_chain(const problem_t &P, chain_t &C) {
-    return chain_from_mx(P, true, false, C) && (P.dst_dt == MI355_DT_BF16 || P.dst_dt == MI355_DT_F32);
+// (an f16 dst has a chain on the small tiles only)
+bool mxf4_chain(const problem_t &P, bool small, chain_t &C) {
+    return chain_from_mx(P, true, false, C)
+            && (P.dst_dt == MI355_DT_BF16 || P.dst_dt == MI355_DT_F32 || (small && P.dst_dt == MI355_DT_F16));
 }
 constexpr long MXF4_STEP_NS = 800; // of a 256 x 128 tile (chain_split)
 
@@ -196,8 +199,13 @@ mxf4_plan_t make_plan(const mi355_matmul_desc_t &d, bool parts) {
     p.split = chain_split_t {1, 0};
     problem_t P;
     chain_t C;
-    if (parts && tuning(TUNE_F8_TILES) == TUNE_AUTO && (problem_of_desc(d, P), mxf4_chain(P, C)))
-        p.split = chain_split(d.batch, d.M, d.N, d.K / 2, false, MXF4_STEP_NS);
+    const int force = tuning(TUNE_F8_TILES);
+    if (force != TUNE_WIDE && (problem_of_desc(d, P), mxf4_chain(P, true, C))) {
+        if (parts && force != TUNE_SMALL && P.dst_dt != MI355_DT_F16) p.split = chain_split(d.batch, d.M, d.N, d.K / 2, false, MXF4_STEP_NS);
+        p.small = force == TUNE_SMALL
+                || (force == TUNE_AUTO && small_tiles_float(d.batch, d.M, d.N, d.K / 2, p.split, MXF4_STEP_NS, C, 4));
+        if (p.small) p.split = chain_split_t {1, 0};
+    }
     off += chain_parts_bytes(d.batch, d.M, d.N, false, p.split.split);
     p.total = off;
     return p;
@@ -276,11 +284,12 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         X.ldb = d.wei_stride[2] / 2;
         X.bt_bstride = d.wei_stride[0] / 2;
     }
-    if (const int st = mx_pack_scales(d, P, plan.Bsa, plan.Bsb, sc + plan.off_sa, sc + plan.off_sb, X.sc, stream)) return st;
     // (MI355_F8_TILES keeps one geometry here as well)
     const int force = tuning(TUNE_F8_TILES);
     chain_t C {};
-    const bool chain = mxf4_chain(P, C);
+    const bool small = plan.small && mxf4_chain(P, true, C), chain = small || mxf4_chain(P, false, C);
+    if (!small)
+        if (const int st = mx_pack_scales(d, P, plan.Bsa, plan.Bsb, sc + plan.off_sa, sc + plan.off_sb, X.sc, stream)) return st;
     const bool narrow = force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N, d.K / 2, chain) && force != TUNE_WIDE);
     if (chain) {
         C.a = (const char *)P.src; C.lda = P.ss[1] / 2; C.a_bs = P.ss[0] / 2;
@@ -290,6 +299,11 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         C.parts = sc + plan.off_parts;
         C.split = plan.split.split;
         C.part_steps = plan.split.part_steps;
+        if (small) {
+            C.sa = (const uint8_t *)P.src_scale.p; C.sa_bs = plan.Bsa > 1 ? d.M * (d.K / 32) : 0;
+            C.sb = (const uint8_t *)P.wei_scale.p; C.sb_bs = plan.Bsb > 1 ? d.N * (d.K / 32) : 0;
+            return chain_launch_small(CHAIN_SMALL_MXF4, P.dst_dt, C, (unsigned)d.batch, stream);
+        }
         const int st = chain_launch_mx(true, P.dst_dt, C, (unsigned)d.batch, !narrow, stream);
         if (st != MI355_UNIMPLEMENTED) return st;
     }
