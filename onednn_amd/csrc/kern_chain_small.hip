@@ -16,6 +16,7 @@
 namespace mi355 {
 namespace {
 constexpr int FST = 32, FSNW = 4;
+constexpr long SMALL_MXF8_PARTS = 256; // MXFP8: up to so many tiles K goes to the four wavefronts in parts
 
 // KIND's policy of line_policies.hpp (the geometry is not used)
 template <int KIND>
@@ -24,26 +25,28 @@ using small_mma_t = std::conditional_t<KIND == CHAIN_SMALL_BF16, h16x16_mma_t<tr
                 std::conditional_t<KIND == CHAIN_SMALL_F8, f8_mma_t<0, 0, geo_t<4, 128>>,
                         std::conditional_t<KIND == CHAIN_SMALL_MXF8, mxf8_mma_t<0, 0, geo_t<4, 128>>, mxf4_mma_t<geo_t<4, 128>>>>>>;
 
-template <int KIND, int DST>
-__global__ void __launch_bounds__(FSNW * 64, KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) chain_small_float_kernel(const chain_t C) {
+// IN_ORDER: a wavefront owns 16 x 16 of the tile and all of K, in the large tiles' order of sums.
+template <int KIND, int DST, bool IN_ORDER>
+__global__ void __launch_bounds__(FSNW * 64, IN_ORDER ? 3 : KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) chain_small_float_kernel(const chain_t C) {
     using Mma = small_mma_t<KIND>;
     constexpr int NU = Mma::NU, NS = Mma::SCALE_SETS; // instructions a pair; scales a lane, fragment and step
     // steps of a wavefront in flight (four, at half the workgroups a CU, took as long or up to 1.8 times as long: 512 x 2048 x 512
     // fp8 19.0 us against 10.7)
-    constexpr int SD = 2;
-    __shared__ float part[FSNW][16][64];
+    constexpr int SD = IN_ORDER ? 3 : 2;
+    constexpr int NF = IN_ORDER ? 1 : 2, STRIDE = IN_ORDER ? 1 : FSNW; // fragments of 16 rows a wavefront; its next step
+    __shared__ float part[IN_ORDER ? 1 : FSNW][16][64];
     const int t = threadIdx.x, lane = t & 63, j = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const long b = blockIdx.z, M = C.M, N = C.N;
     const int kbytes = (int)C.kbytes;
     const long m0 = (long)(blockIdx.x / C.tiles_n) * FST, n0 = (long)(blockIdx.x % C.tiles_n) * FST;
     // rows and columns beyond the edge read the last valid one (never stored)
-    const char *arow[2], *bcol[2];
-    const uint8_t *asc[2], *bsc[2];
+    const char *arow[NF], *bcol[NF];
+    const uint8_t *asc[NF], *bsc[NF];
     const int kblocks = (int)C.kbytes * (KIND == CHAIN_SMALL_MXF4 ? 2 : 1) / 32;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const long m = min(m0 + 16 * i + j, M - 1), n = min(n0 + 16 * i + j, N - 1);
+    for (int i = 0; i < NF; ++i) {
+        const long m = min(m0 + 16 * (IN_ORDER ? wave >> 1 : i) + j, M - 1), n = min(n0 + 16 * (IN_ORDER ? wave & 1 : i) + j, N - 1);
         arow[i] = C.a + b * C.a_bs + m * C.lda;
         bcol[i] = C.bt + b * C.b_bs + n * C.ldb;
         if constexpr (NS > 0) {
@@ -52,8 +55,8 @@ __global__ void __launch_bounds__(FSNW * 64, KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) c
         }
     }
     struct step_t {
-        line_pair_t a[2], b[2];
-        int sa[2][NS ? NS : 1], sb[2][NS ? NS : 1];
+        line_pair_t a[NF], b[NF];
+        int sa[NF][NS ? NS : 1], sb[NF][NS ? NS : 1];
     };
     // kbytes is a multiple of 16: a chunk is inside K or beyond it.  Those beyond are loaded from the row's last one and zeroed
     // in both operands before they are multiplied (a branch around the load would be a wait for everything in flight).
@@ -63,7 +66,7 @@ __global__ void __launch_bounds__(FSNW * 64, KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) c
         for (int u = 0; u < 2; ++u) {
             const int k = min(s * 128 + 64 * u + 16 * q, kbytes - 16);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < NF; ++i) {
                 f.a[i].c[u] = *(const v4i *)(arow[i] + k);
                 f.b[i].c[u] = *(const v4i *)(bcol[i] + k);
             }
@@ -73,7 +76,7 @@ __global__ void __launch_bounds__(FSNW * 64, KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) c
             for (int u = 0; u < NS; ++u) {
                 const int blk = min(s * (4 * NS) + 4 * u + q, kblocks - 1);
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
+                for (int i = 0; i < NF; ++i) {
                     f.sa[i][u] = asc[i][blk];
                     f.sb[i][u] = bsc[i][(unsigned)blk * (unsigned)N];
                 }
@@ -82,11 +85,11 @@ __global__ void __launch_bounds__(FSNW * 64, KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) c
         return f;
     };
     const int nsteps = (kbytes + 127) / 128;
-    int step = wave;
+    int step = IN_ORDER ? 0 : wave;
     step_t st[SD];
 #pragma unroll
     for (int d = 0; d < SD; ++d) {
-        const int sl = step + d * FSNW;
+        const int sl = step + d * STRIDE;
         st[d] = load(sl < nsteps ? sl : 0);
     }
     // this thread's four outputs
@@ -95,54 +98,60 @@ __global__ void __launch_bounds__(FSNW * 64, KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) c
     chain_quad_t<DST> Q;
     if (m < M && n < N) Q.load(C, b, m, n);
 
-    v4f acc[2][2];
+    v4f acc[NF][NF];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NF; ++i)
 #pragma unroll
-        for (int jn = 0; jn < 2; ++jn) acc[i][jn] = v4f {0.f, 0.f, 0.f, 0.f};
+        for (int jn = 0; jn < NF; ++jn) acc[i][jn] = v4f {0.f, 0.f, 0.f, 0.f};
     auto multiply = [&](step_t &f, int s) __attribute__((always_inline)) {
         if (s * 128 + 128 > kbytes) { // (uniform: the last, partial step)
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 const int keep = s * 128 + 64 * u + 16 * q < kbytes ? -1 : 0;
 #pragma unroll
-                for (int i = 0; i < 2; ++i) f.a[i].c[u] &= keep, f.b[i].c[u] &= keep;
+                for (int i = 0; i < NF; ++i) f.a[i].c[u] &= keep, f.b[i].c[u] &= keep;
             }
         }
         static_for<NU>([&](auto U) __attribute__((always_inline)) {
             constexpr int su = NS > 1 ? decltype(U)::value : 0;
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < NF; ++i)
 #pragma unroll
-                for (int jn = 0; jn < 2; ++jn)
+                for (int jn = 0; jn < NF; ++jn)
                     Mma::template mma<0, 0>(acc[i][jn], f.b[jn], f.a[i], U, NS ? f.sb[jn][su] : 0, NS ? f.sa[i][su] : 0);
         });
     };
-    for (; step + (SD - 1) * FSNW < nsteps; step += SD * FSNW) {
+    for (; step + (SD - 1) * STRIDE < nsteps; step += SD * STRIDE) {
 #pragma unroll
         for (int d = 0; d < SD; ++d) {
-            multiply(st[d], step + d * FSNW);
-            const int sl = step + (SD + d) * FSNW;
+            multiply(st[d], step + d * STRIDE);
+            const int sl = step + (SD + d) * STRIDE;
             if (sl < nsteps) st[d] = load(sl); // (uniform over the wavefront)
         }
     }
 #pragma unroll
     for (int d = 0; d < SD; ++d)
-        if (step + d * FSNW < nsteps) multiply(st[d], step + d * FSNW);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int jn = 0; jn < 2; ++jn)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) part[wave][i * 8 + jn * 4 + e][lane] = acc[i][jn][e];
-    __syncthreads();
-    if (m >= M || n >= N) return;
+        if (step + d * STRIDE < nsteps) multiply(st[d], step + d * STRIDE);
     float x[4];
+    if constexpr (IN_ORDER) {
+        if (m >= M || n >= N) return;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        x[e] = part[0][ui * 8 + ujn * 4 + e][lane];
+        for (int e = 0; e < 4; ++e) x[e] = acc[0][0][e];
+    } else {
 #pragma unroll
-        for (int w = 1; w < FSNW; ++w) x[e] += part[w][ui * 8 + ujn * 4 + e][lane];
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int jn = 0; jn < 2; ++jn)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) part[wave][i * 8 + jn * 4 + e][lane] = acc[i][jn][e];
+        __syncthreads();
+        if (m >= M || n >= N) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[e] = part[0][ui * 8 + ujn * 4 + e][lane];
+#pragma unroll
+            for (int w = 1; w < FSNW; ++w) x[e] += part[w][ui * 8 + ujn * 4 + e][lane];
+        }
     }
     Q.finish(C, b, m, n, x);
 }
@@ -152,14 +161,15 @@ __global__ void __launch_bounds__(FSNW * 64, KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) c
 // 1024 5.3 / 12.9, 256 x 2048 x 1024 7.2 / 13.4, 64 x 4096 x 4096 10.7 / 19.8, 916 x 512 x 640 with gelu_tanh and a residual 7.7 / 16.7, but 64 x
 // 640 x 16384 30.7 / 19.0; bf16 32 x 1792 x 768 6.2 / 13.9, 512 x 1024 x 1024 10.2 / 16.3, 128 x 1024 x 8192 (f16) 34.0 / 20.1, 512 x 3600 x
 // 704 23.5 / 14.7; MXFP4 128 x 2048 x 2048 9.4 / 23.0 (whose 7 us of pre-pass kernels it does without), MXFP8 300 x 1040 x 1056 9.0 / 25.9.
+// MXFP8 beyond 256 tiles, in the large tiles' order (data that tests/test_mxf8_gemm.py calls exact takes 25 bits there, so that its
+// bits follow the order of the sums): 128 x 3520 x 1408 15.8 / 24.5, 700 x 1024 x 640 12.9 / 21.5.
 // A workgroup's steps are a chain (1.67 ns a byte of K), its neighbours' traffic comes on top (per tile).
 bool small_tiles_float(long batch, long M, long N, long kbytes, const chain_split_t &split, long step_ns, const chain_t &C, int mx) {
     const double tiles = (double)((M + FST - 1) / FST) * ((N + FST - 1) / FST) * batch;
-    // Four workgroups a CU.  MXFP8, whose data that is called exact in tests/test_mxf8_gemm.py takes 25 bits and so depends on the
-    // order of the sums, keeps the large tiles' order from 256 tiles on (550 of them, 333 x 1600 x 1536: 25.8 us there, 14.4 here).
-    if (tiles > (mx == 8 ? 256 : 1024)) return false;
+    if (tiles > 1024) return false;
     const double large = (double)((M + 255) / 256) * ((N + 127) / 128) * batch;
-    const double small = 3300 + 1.67 * kbytes + tiles * (3 + 0.0025 * kbytes);
+    const double small = mx == 8 && tiles > SMALL_MXF8_PARTS ? 3300 + 8.2 * kbytes + tiles * 9
+                                                              : 3300 + 1.67 * kbytes + tiles * (3 + 0.0025 * kbytes);
     const double rest = (mx ? 7000 : 0) + (C.act >= CHAIN_GELU ? 3000 : 0)
             + (split.split > 1 ? 8000 + split.part_steps * step_ns + split.split * large * 35 : 8500 + (kbytes + 127) / 128 * 500.);
     return small < 0.95 * rest;
@@ -171,7 +181,14 @@ int chain_launch_small(chain_small_t kind, int dst_dt, chain_t &C, unsigned batc
     C.tiles_n = (int)tn;
     auto go = [&](auto k, auto dst) -> int {
         constexpr int K = decltype(k)::value, D = decltype(dst)::value;
-        hipLaunchKernelGGL((chain_small_float_kernel<K, D>), dim3((unsigned)(tm * tn), 1, batch), dim3(FSNW * 64), 0, stream, C);
+        const dim3 grid((unsigned)(tm * tn), 1, batch);
+        if constexpr (K == CHAIN_SMALL_MXF8) {
+            if (tm * tn * batch > SMALL_MXF8_PARTS) {
+                hipLaunchKernelGGL((chain_small_float_kernel<K, D, true>), grid, dim3(FSNW * 64), 0, stream, C);
+                return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
+            }
+        }
+        hipLaunchKernelGGL((chain_small_float_kernel<K, D, false>), grid, dim3(FSNW * 64), 0, stream, C);
         return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
     };
     auto by_dst = [&](auto k) -> int {

@@ -25,7 +25,8 @@
 // Bound: for long queries the series of K Q, softmax and P V in a wavefront, behind a wait for all loads and a barrier every
 // 64 keys (16 heads, 4096 x 4096, d 128, causal, bf16: the composition 1221 us, of which 729 were the softmax over scores in
 // memory, this 91 us = 755 TFLOP/s; the matrix cores and the vector units busy 43 % of the time each, which adds up to the
-// 86 % that are not stalls: the two workgroups of a CU hardly run one's softmax under the other's products; 8 x 8 heads,
+// 86 % that are not stalls: the two workgroups of a CU hardly run one's softmax under the other's products.  Multiplying the next
+// tile's scores among this one's softmax in the wavefront itself was 6 % slower, with and without the order forced.  8 x 8 heads,
 // 1918 x 2942, d 64: 4024 -> 119 us); memory for few (8 x 16 heads, one query, 8192 keys: 653 -> 103 us, 5.2 TB/s; a wavefront
 // waits 55 %).
 // 64 rows is where the forms cross: at 64 rows half of the large form's wavefronts have none.  The form for few rows

@@ -65,6 +65,18 @@ def test_block_scales(gpu, oracle, fmt, K, ddt):
         assert_bit_exact(p, got, oracle.run_oracle(p), name)
 
 
+@pytest.mark.parametrize("K", [64, 96, 384, 416, 544])
+def test_mxfp8_in_the_large_tiles_order(gpu, K):
+    """more than 256 tiles: random data, the bits of the 256 x 128 tiles"""
+    from tests.test_mxf8_gemm import problem as mx_problem
+    p = mx_problem(520, 531, K, ddt="f32", exact=False, seed=K, bias=True)
+    out = []
+    for tiles in ("small", "narrow"):
+        with cabi.tuning("MI355_F8_TILES", tiles):
+            out.append(run_gpu(p)[0])
+    assert np.array_equal(*(np.asarray(o).view(np.uint32) for o in out))
+
+
 # infinities and NaN in the chunks that lanes beyond K load a second time
 @pytest.mark.parametrize("K", [8, 40, 72, 200])
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
