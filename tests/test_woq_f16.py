@@ -30,6 +30,26 @@ def test_f16_activations_take_the_decode_kernels():
     assert cabi.impl_name(cabi.query(f16_problem(33, 128, 128, 128, "plain").desc())[1]).startswith("hip:mfma_h16")
 
 
+def test_format_any_weights_of_fewer_columns():
+    """packed where a workgroup's walk along K beats the two launches of the row-major kernel"""
+    from onednn_amd import dnnl
+    eng = dnnl.engine(dnnl.gpu, 0)
+
+    def kind(M, N, K, dt):
+        attr = dnnl.primitive_attr()
+        attr.set_scales(dnnl.ARG_WEIGHTS, 3, (128, 1), cabi.DT_NAMES[dt])
+        attr.set_fpmath_mode(dnnl.fpmath_bf16 if dt == "bf16" else dnnl.fpmath_f16, True)
+        md = lambda dims, t, tag: dnnl.memory_desc(dims, cabi.DT_NAMES[t], tag=tag)  # noqa: E731
+        pd = dnnl.matmul_primitive_desc(eng, md([M, K], dt, dnnl.tag_ab), md([K, N], "u4", dnnl.tag_any), md([M, N], dt, dnnl.tag_ab), attr=attr)
+        return pd.query_md(dnnl.query_weights_md).format_kind()
+
+    packed, plain = dnnl.format_kind_opaque, dnnl.format_kind_blocked
+    for M, K in ((4, 16384), (16, 12288), (32, 11264)):
+        assert kind(M, 1024, K, "f16") == packed and kind(M, 4160, K, "bf16") == packed and kind(M, 4096, K, "bf16") == plain
+        assert kind(M, 1024, K + 128, "f16") == plain and kind(M, 4160, K + 128, "bf16") == plain and kind(M, 8192, K + 128, "f16") == packed
+    assert kind(33, 1024, 1024, "f16") == plain
+
+
 CASES = [
     # M, N, K, group, weights, scales, zero points, dst, bias + relu
     (1, 64, 32, 32, "u4", "f16", "u4", "grouped", "f16", False),
