@@ -536,11 +536,11 @@ __device__ __forceinline__ uint32_t quantize4(float (&x)[4], const float (&s0)[4
 // template parameters, four rows are in flight per lane, and every load or
 // store instruction moves whole 128-byte lines.
 //
-// flat: no outer dim and no scales along `a` (a dense tensor with a scale for all of it comes here as one row): rows of 1024
+// FLAT: no outer dim and no scales along `a` (a dense tensor with a scale for all of it comes here as one row): rows of 1024
 // elements, the last one shorter.  As one row every lane asked for its four elements four times and had nothing
 // else in flight: 2048 x 12288 f32 -> s8 41.5 us, so 23.5.
-template <int SDT, int DDT>
-__global__ void __launch_bounds__(256) reorder_rows_kernel(const reorder_t R_, unsigned rows_per_wg, unsigned flat) {
+template <int SDT, int DDT, bool FLAT>
+__global__ void __launch_bounds__(256) reorder_rows_kernel(const reorder_t R_, unsigned rows_per_wg) {
     const auto &R = *(const __attribute__((address_space(4))) reorder_t *)__builtin_amdgcn_kernarg_segment_ptr();
     typedef uint32_t u4v __attribute__((ext_vector_type(4)));
     typedef uint32_t u2v __attribute__((ext_vector_type(2)));
@@ -548,8 +548,8 @@ __global__ void __launch_bounds__(256) reorder_rows_kernel(const reorder_t R_, u
     constexpr int U = 4;
     const unsigned a = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (a >= R.a.n) return;
-    const unsigned rows = flat ? (R.a.n - a - 1) / 1024 + 1 : R.n_outer ? R.outer[0].n : 1; // (flat: of this lane)
-    const long rs = flat ? 1024 : R.n_outer ? R.outer[0].ss : 0, rd = flat ? 1024 : R.n_outer ? R.outer[0].ds : 0;
+    const unsigned rows = FLAT ? (R.a.n - a - 1) / 1024 + 1 : R.n_outer ? R.outer[0].n : 1; // (FLAT: of this lane)
+    const long rs = FLAT ? 1024 : R.n_outer ? R.outer[0].ss : 0, rd = FLAT ? 1024 : R.n_outer ? R.outer[0].ds : 0;
     const unsigned r0 = blockIdx.y * rows_per_wg;
     const unsigned r1 = min(rows, r0 + rows_per_wg);
     float s0[4], s1[4], y1[4];
@@ -1264,7 +1264,8 @@ extern "C" int mi355_reorder_launch(const mi355_reorder_desc_t *desc, const mi35
                         && (R.n_outer == 0 || R.outer[0].qs[k] == 0);
             }
             if (rows_ok) {
-                const bool flat = R.n_outer == 0 && R.a.n > 1024 && (!R.qp[0] || R.a.qs[0] == 0) && (!R.qp[1] || R.a.qs[1] == 0);
+                // (below 8192 rows too few workgroups of four rows: 1.9 M elements bf16 -> e4m3 5.8 us as one row, 7.9 so)
+                const bool flat = R.n_outer == 0 && R.a.n > 8192 * 1024 && (!R.qp[0] || R.a.qs[0] == 0) && (!R.qp[1] || R.a.qs[1] == 0);
                 const unsigned rows = flat ? (unsigned)((R.a.n - 1) / 1024 + 1) : R.n_outer ? R.outer[0].n : 1;
                 const unsigned chunks = flat ? 1 : (unsigned)((R.a.n / 4 + 255) / 256);
                 // some 4096 workgroups, at least four rows (one round of loads) each
@@ -1273,7 +1274,10 @@ extern "C" int mi355_reorder_launch(const mi355_reorder_desc_t *desc, const mi35
                 const dim3 rgrid(chunks, (rows + per - 1) / per), block(256);
                 if (rgrid.y <= 65535) {
 #define MI355_ROWS_CASE(S_, D_) \
-    if (d.src_dt == S_ && d.dst_dt == D_) hipLaunchKernelGGL((reorder_rows_kernel<S_, D_>), rgrid, block, 0, hs, R, per, flat ? 1u : 0u);
+    if (d.src_dt == S_ && d.dst_dt == D_) { \
+        if (flat) hipLaunchKernelGGL((reorder_rows_kernel<S_, D_, true>), rgrid, block, 0, hs, R, per); \
+        else hipLaunchKernelGGL((reorder_rows_kernel<S_, D_, false>), rgrid, block, 0, hs, R, per); \
+    }
 #define MI355_ROWS_SRC(S_) \
     MI355_ROWS_CASE(S_, MI355_DT_S8) MI355_ROWS_CASE(S_, MI355_DT_U8) MI355_ROWS_CASE(S_, MI355_DT_F8_E4M3) \
     MI355_ROWS_CASE(S_, MI355_DT_F8_E5M2)

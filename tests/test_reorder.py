@@ -392,6 +392,18 @@ def test_gpu_row_quantization_is_bit_exact(make):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(8192, 1024), (4099, 2052), (8193, 1028)])
+@pytest.mark.parametrize("sdt,ddt", [(cabi.DT_F32, cabi.DT_S8), (cabi.DT_BF16, cabi.DT_U8), (cabi.DT_F16, cabi.DT_F8_E4M3)])
+def test_gpu_row_quantization_of_a_dense_tensor_with_one_scale(dims, sdt, ddt):
+    """the last size that goes as one row, and rows of 1024 elements whose last one ends after 12 or 4"""
+    p = _case("dense, one scale", dims, sdt, ddt, 140, quant={"dst_scale": _qp(141, cabi.DT_F32, 0, (1,), lo=0.5, hi=4.0)})
+    want = oracle.reorder(p)
+    got = run_gpu(p)
+    bad = np.flatnonzero(got != want)
+    assert bad.size == 0, f"{p.name}: {bad.size} of {got.size} storage elements differ, first at {bad[:5]}"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dst_dt", [cabi.DT_S8, cabi.DT_U8, cabi.DT_F8_E4M3])
 def test_gpu_row_quantization_special_values(dst_dt):
     rows, cols = 12, 64
