@@ -356,7 +356,6 @@ bool small_tiles_better(const mi355_matmul_desc_t &d, bool chain) {
     return ((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch < line[few][whole][!chain][sums][band];
 }
 
-// chain: what i8_chain says, the same of the descriptor's problem and of the launch's
 // The line of small_tiles_better is drawn against LDS tiles that take all of K; with K split (chain_gemm.hpp) they are the better
 // ones from fewer small tiles on where K is long.  Both sides in ns, from a dozen shapes: 128 x 4096 x 4096 17.1 us small, 20.2
 // split, 1024 x 1024 x 4096 31 and 20.3, with sums 64 x 2048 x 16384 31.0 and 33.4; a tenth in favour of the small tiles, one launch.
@@ -368,8 +367,13 @@ bool split_tiles_better(const mi355_matmul_desc_t &d, const chain_split_t &s) {
     const double split = 9000 + s.part_steps * 700. + s.split * tiles * 52 + (sums ? 3500 + (double)d.N * d.K * 1e-4 : 0);
     return 1.1 * split < small;
 }
+// (the LDS tiles' offsets from a tile's first row are 32-bit, the small tiles' are not)
+bool rows_fit_lds_tiles(const mi355_matmul_desc_t &d) {
+    return d.src_stride[1] <= (1L << 24) && (d.wei_stride[1] == 1 ? d.wei_stride[2] : d.K) <= (1L << 24);
+}
 constexpr long I8_STEP_NS = 700; // of a 256 x 128 tile (chain_split)
 
+// chain: what i8_chain says, the same of the descriptor's problem and of the launch's
 i8_plan_t make_plan(const mi355_matmul_desc_t &d, bool chain, bool parts) {
     i8_plan_t p {};
     p.Bw = d.wei_stride[0] ? d.batch : 1;
@@ -385,7 +389,7 @@ i8_plan_t make_plan(const mi355_matmul_desc_t &d, bool chain, bool parts) {
     p.split = chain_split_t {1, 0};
     if (chain && parts && force == TUNE_AUTO) {
         const chain_split_t split = chain_split(d.batch, d.M, d.N, d.K, false, I8_STEP_NS);
-        if (p.small && split.split > 1 && split_tiles_better(d, split)) p.small = false;
+        if (p.small && split.split > 1 && rows_fit_lds_tiles(d) && split_tiles_better(d, split)) p.small = false;
         if (!p.small) p.split = split;
     }
     // a = off_s - zs can be non-zero whenever src is u8 or has a zero point;
@@ -453,10 +457,13 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, b
     chain_t C {};
     bool chain = i8_chain(P, C);
     i8_plan_t plan = make_plan(d, chain, parts);
+    const uintptr_t at = (uintptr_t)P.src | (plan.need_transpose ? 0 : (uintptr_t)P.wei);
+    // K is split on the LDS tiles, whose loads bring whole chunks from 16-byte boundaries straight to LDS: operands off one
+    // have the tiles that they have without parts, the small ones where those are the better ones
+    if (plan.split.split > 1 && (at & 15)) plan = make_plan(d, chain, false);
     // A K that ends inside 64 bytes also takes operands off 16-byte boundaries, which the LDS tiles' loads cannot, and
     // K-contiguous weights without scratch: the small tiles'.
     if (!plan.small && d.K % BK != 0) {
-        const uintptr_t at = (uintptr_t)P.src | (plan.need_transpose ? 0 : (uintptr_t)P.wei);
         const bool without = plan.total > 0 && !scratch && i8_scratch_optional(d);
         if ((at & 15) || without) plan.small = true, plan.need_colsum = plan.need_rowsum = false;
         if (without) plan.total = 0;

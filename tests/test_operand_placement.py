@@ -51,6 +51,15 @@ def test_int8_operands(gpu, oracle, dt, ddt, src, wei):
     check(oracle, problem(512, 8192, 80, dt, ddt, src_zp=3 if dt == "u8" else None), "hip:mfma_i8", src, wei)
 
 
+@pytest.mark.parametrize("dt,ddt", [("s8", "s8"), ("u8", "f32")])
+@pytest.mark.parametrize("src,wei", [(1, 0), (0, 4), (8, 7)])
+def test_int8_operands_where_k_would_be_split(gpu, oracle, dt, ddt, src, wei):
+    """1024 small tiles by themselves; K in parts on the LDS tiles only where both operands lie on 16-byte boundaries"""
+    p = problem(1024, 1024, 4096, dt, ddt, src_zp=3 if dt == "u8" else None)
+    assert cabi.scratch_bytes(p.desc()) > 1 << 20
+    check(oracle, p, "hip:mfma_i8", src, wei)
+
+
 @pytest.mark.parametrize("wei_zp", [False, True])
 def test_int8_sums_without_scratch(gpu, oracle, wei_zp):
     p = int8_problem(512, 8192, 80, cabi.DT_U8, cabi.DT_S8, cabi.DT_F32, src_zp=5, wei_zp=wei_zp)

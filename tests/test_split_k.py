@@ -54,6 +54,19 @@ def test_which_problems_are_split():
         assert 2 <= n <= 256
 
 
+@pytest.mark.parametrize("K,parts", [(1 << 24, True), ((1 << 24) + 64, False)])
+def test_int8_rows_beyond_the_offsets_of_the_lds_tiles(K, parts):
+    """their offsets are 32-bit: longer rows stay on the small tiles, which need no scratch (u8: nor column sums)"""
+    d = problem(8, 64, 128, "u8", "f32", src_zp=3).desc()
+    d.K = K
+    for s in (d.src_stride, d.wei_stride):
+        for i in range(2 if s is d.src_stride else 3):
+            if s[i] == 128:
+                s[i] = K
+    assert list(d.wei_stride)[1:] == [1, K] and list(d.src_stride)[1:] == [K, 1]
+    assert (cabi.scratch_bytes(d) > 0) == parts
+
+
 # steps of the last part: whole, one chunk, a chunk short of a step
 @pytest.mark.gpu
 @pytest.mark.parametrize("tail", [0, 16, 112])
