@@ -91,6 +91,8 @@ struct chain_t {
 // A product of few 32 x 32 tiles on chain_small_float_kernel (kern_chain_small.hip): small_tiles_float says whether (mx: 0, or
 // the bits of a block-scaled type).
 enum chain_small_t { CHAIN_SMALL_BF16, CHAIN_SMALL_F16, CHAIN_SMALL_F8, CHAIN_SMALL_MXF8, CHAIN_SMALL_MXF4 };
+// small_tiles_fit: whether its 32-bit steps of K and offsets of block scales reach that far.
+bool small_tiles_fit(long M, long N, long kbytes, int mx);
 bool small_tiles_float(long batch, long M, long N, long kbytes, const chain_split_t &split, long step_ns, const chain_t &C, int mx);
 int chain_launch_small(chain_small_t kind, int dst_dt, chain_t &C, unsigned batch, hipStream_t stream);
 

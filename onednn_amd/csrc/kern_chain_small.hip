@@ -157,6 +157,11 @@ __global__ void __launch_bounds__(FSNW * 64, IN_ORDER ? 3 : KIND >= CHAIN_SMALL_
 }
 } // namespace
 
+bool small_tiles_fit(long M, long N, long kbytes, int mx) {
+    return kbytes < (1L << 30) && (M + FST - 1) / FST * ((N + FST - 1) / FST) < (1L << 31)
+            && (mx == 0 || kbytes * 8 / mx / 32 * N < (1L << 32));
+}
+
 // Both sides in ns, as measured on 64 shapes of every type (small / 256 x 128 tiles, K split where that pays, us): fp8 16 x 2240 x
 // 1024 5.3 / 12.9, 256 x 2048 x 1024 7.2 / 13.4, 64 x 4096 x 4096 10.7 / 19.8, 916 x 512 x 640 with gelu_tanh and a residual 7.7 / 16.7, but 64 x
 // 640 x 16384 30.7 / 19.0; bf16 32 x 1792 x 768 6.2 / 13.9, 512 x 1024 x 1024 10.2 / 16.3, 128 x 1024 x 8192 (f16) 34.0 / 20.1, 512 x 3600 x

@@ -72,9 +72,11 @@ f8_plan_t make_plan(const mi355_matmul_desc_t &d, bool parts) {
     chain_t C;
     const int force = tuning(TUNE_F8_TILES);
     if (is_e4m3_pair(d) && force != TUNE_WIDE && (problem_of_desc(d, P), f8_chain(P, p.mx, true, C))) {
-        if (parts && force != TUNE_SMALL && P.dst_dt != MI355_DT_F16) p.split = chain_split(d.batch, d.M, d.N, d.K, false, F8_STEP_NS);
-        p.small = force == TUNE_SMALL
-                || (force == TUNE_AUTO && small_tiles_float(d.batch, d.M, d.N, d.K, p.split, F8_STEP_NS, C, p.mx ? 8 : 0));
+        const bool fits = small_tiles_fit(d.M, d.N, d.K, p.mx ? 8 : 0);
+        if (parts && !(fits && force == TUNE_SMALL) && P.dst_dt != MI355_DT_F16) p.split = chain_split(d.batch, d.M, d.N, d.K, false, F8_STEP_NS);
+        p.small = fits
+                && (force == TUNE_SMALL
+                        || (force == TUNE_AUTO && small_tiles_float(d.batch, d.M, d.N, d.K, p.split, F8_STEP_NS, C, p.mx ? 8 : 0)));
         if (p.small) p.split = chain_split_t {1, 0};
     }
     off += chain_parts_bytes(d.batch, d.M, d.N, false, p.split.split);

@@ -273,10 +273,11 @@ static h16_plan_t h16_plan(const mi355_matmul_desc_t &d, bool parts) {
         problem_of_desc(d, P);
         if (p.woq) P.wei_scale.dt = P.wei_zp.dt = MI355_DT_UNDEF; // applied by the copy
         if (chain_from(P, false, P.dst_dt == p.op_dt, C) && !is_int8_dt(P.dst_dt)) {
-            if (parts && force != TUNE_SMALL) p.split = chain_split(d.batch, d.M, d.N, p.Kp * p.EB, false, H16_STEP_NS);
+            const bool fits = small_tiles_fit(d.M, d.N, p.Kp * p.EB, 0);
+            if (parts && !(fits && force == TUNE_SMALL)) p.split = chain_split(d.batch, d.M, d.N, p.Kp * p.EB, false, H16_STEP_NS);
             // K-contiguous operands only: others are copied where the large tiles do not read them as they lie, and either way
             // has the same bits
-            p.small = d.src_stride[2] == 1 && (p.woq || d.wei_stride[1] == 1)
+            p.small = fits && d.src_stride[2] == 1 && (p.woq || d.wei_stride[1] == 1)
                     && (force == TUNE_SMALL || (force == TUNE_AUTO && small_tiles_float(d.batch, d.M, d.N, p.Kp * p.EB, p.split, H16_STEP_NS, C, 0)));
             if (p.small) p.split = chain_split_t {1, 0};
             if (parts && !p.woq && d.src_stride[2] != 1 && d.wei_stride[1] != 1)

@@ -201,9 +201,11 @@ mxf4_plan_t make_plan(const mi355_matmul_desc_t &d, bool parts) {
     chain_t C;
     const int force = tuning(TUNE_F8_TILES);
     if (force != TUNE_WIDE && (problem_of_desc(d, P), mxf4_chain(P, true, C))) {
-        if (parts && force != TUNE_SMALL && P.dst_dt != MI355_DT_F16) p.split = chain_split(d.batch, d.M, d.N, d.K / 2, false, MXF4_STEP_NS);
-        p.small = force == TUNE_SMALL
-                || (force == TUNE_AUTO && small_tiles_float(d.batch, d.M, d.N, d.K / 2, p.split, MXF4_STEP_NS, C, 4));
+        const bool fits = small_tiles_fit(d.M, d.N, d.K / 2, 4);
+        if (parts && !(fits && force == TUNE_SMALL) && P.dst_dt != MI355_DT_F16) p.split = chain_split(d.batch, d.M, d.N, d.K / 2, false, MXF4_STEP_NS);
+        p.small = fits
+                && (force == TUNE_SMALL
+                        || (force == TUNE_AUTO && small_tiles_float(d.batch, d.M, d.N, d.K / 2, p.split, MXF4_STEP_NS, C, 4)));
         if (p.small) p.split = chain_split_t {1, 0};
     }
     off += chain_parts_bytes(d.batch, d.M, d.N, false, p.split.split);

@@ -67,6 +67,24 @@ def test_int8_rows_beyond_the_offsets_of_the_lds_tiles(K, parts):
     assert (cabi.scratch_bytes(d) > 0) == parts
 
 
+@pytest.mark.parametrize("dt,shape", [("f8_e4m3", (8, 64, 1 << 30)), ("mxf8", (8, 16384, 1 << 23)), ("mxf4", (8, 16384, 1 << 23))])
+def test_what_the_offsets_of_the_small_tiles_do_not_reach(dt, shape):
+    """by the scratch when they are told to run: K that is split instead is the large tiles'"""
+    M, N, K = shape
+    for k, fits in ((K, False), (K - 256, True)):
+        d = (mx(8, 64, 256, dt, "bf16") if dt.startswith("mx") else problem(8, 64, 256, dt, "bf16")).desc()
+        d.N, d.K = N, k
+        for s in (d.src_stride, d.wei_stride):
+            for i in range(3):
+                if s[i] == 256:
+                    s[i] = k
+        d.dst_stride[1] = N
+        with cabi.tuning("MI355_F8_TILES", "wide"):
+            unsplit = cabi.scratch_bytes(d)
+        with cabi.tuning("MI355_F8_TILES", "small"):
+            assert (cabi.scratch_bytes(d) == unsplit) == fits, k
+
+
 # steps of the last part: whole, one chunk, a chunk short of a step
 @pytest.mark.gpu
 @pytest.mark.parametrize("tail", [0, 16, 112])
