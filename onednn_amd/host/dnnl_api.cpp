@@ -1882,17 +1882,15 @@ DNNL_EXPORT dnnl_status_t dnnl_matmul_primitive_desc_create(dnnl_primitive_desc_
         dnnl_memory_desc &w = pd->wei;
         w.set_dense();
         // 4-bit decode weights: the 64-column packing, if the packed decode
-        // kernel takes the problem (decided below, once the descriptor is
-        // lowered).  From N = 8192 on it has the workgroups to fill the device.
-        // With fewer its launch is a workgroup's walk along K (1.2 ns a row of K,
-        // 2 above 16 rows of src), the row-major kernel's two launches take 15 to 30 us
-        // whatever the size: M 1, N 1024, K 4096 5.5 / 15.1 us, M 24, N 6144, K 11776
-        // 26.5 / 35.6, but M 32, N 2048, K 16384 38.3 / 30.0.  (bf16 src up to N = 4096
-        // has always had row-major weights, and callers may count on that.)
-        const dnnl_dim_t M = pd->src.dims[0], K = w.dims[0], N = w.dims[1];
-        const bool fewer = (pd->src.dt == dnnl_f16 || N > 4096) && K <= (M <= 4 ? 16384 : M <= 16 ? 12288 : 11264);
-        try_packed = (pd->src.dt == dnnl_bf16 || pd->src.dt == dnnl_f16) && (w.dt == dnnl_s4 || w.dt == dnnl_u4) && pd->attr.apply_to_int
-                && w.ndims == 2 && (N >= 64 * 128 || fewer);
+        // kernel takes the problem and N gives it enough workgroups to fill
+        // the device (decided below, once the descriptor is lowered).  Other
+        // types and fewer columns, where the packed kernel would be faster (f16,
+        // M 1, N 14336, K 4096: 7.5 us, row-major 16.9), keep the row-major answer:
+        // it has strides, a quantizing reorder from f32 writes it, and a
+        // primitive of more rows reads it on the matrix cores, none of which an
+        // opaque one does.
+        try_packed = pd->src.dt == dnnl_bf16 && (w.dt == dnnl_s4 || w.dt == dnnl_u4) && pd->attr.apply_to_int
+                && w.ndims == 2 && w.dims[1] >= 64 * 128;
         const bool mfma_operands = (is_int8(pd->src.dt) && is_int8(w.dt)) || (is_fp8(pd->src.dt) && is_fp8(w.dt))
                 || (pd->src.dt == dnnl_f4_e2m1 && w.dt == dnnl_f4_e2m1)
                 || (pd->src.dt == w.dt && (w.dt == dnnl_bf16 || w.dt == dnnl_f16 || w.dt == dnnl_f32));

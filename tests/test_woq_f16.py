@@ -30,26 +30,6 @@ def test_f16_activations_take_the_decode_kernels():
     assert cabi.impl_name(cabi.query(f16_problem(33, 128, 128, 128, "plain").desc())[1]).startswith("hip:mfma_h16")
 
 
-def test_format_any_weights_of_fewer_columns():
-    """packed where a workgroup's walk along K beats the two launches of the row-major kernel"""
-    from onednn_amd import dnnl
-    eng = dnnl.engine(dnnl.gpu, 0)
-
-    def kind(M, N, K, dt):
-        attr = dnnl.primitive_attr()
-        attr.set_scales(dnnl.ARG_WEIGHTS, 3, (128, 1), cabi.DT_NAMES[dt])
-        attr.set_fpmath_mode(dnnl.fpmath_bf16 if dt == "bf16" else dnnl.fpmath_f16, True)
-        md = lambda dims, t, tag: dnnl.memory_desc(dims, cabi.DT_NAMES[t], tag=tag)  # noqa: E731
-        pd = dnnl.matmul_primitive_desc(eng, md([M, K], dt, dnnl.tag_ab), md([K, N], "u4", dnnl.tag_any), md([M, N], dt, dnnl.tag_ab), attr=attr)
-        return pd.query_md(dnnl.query_weights_md).format_kind()
-
-    packed, plain = dnnl.format_kind_opaque, dnnl.format_kind_blocked
-    for M, K in ((4, 16384), (16, 12288), (32, 11264)):
-        assert kind(M, 1024, K, "f16") == packed and kind(M, 4160, K, "bf16") == packed and kind(M, 4096, K, "bf16") == plain
-        assert kind(M, 1024, K + 128, "f16") == plain and kind(M, 4160, K + 128, "bf16") == plain and kind(M, 8192, K + 128, "f16") == packed
-    assert kind(33, 1024, 1024, "f16") == plain
-
-
 CASES = [
     # M, N, K, group, weights, scales, zero points, dst, bias + relu
     (1, 64, 32, 32, "u4", "f16", "u4", "grouped", "f16", False),
@@ -110,3 +90,24 @@ def test_f16_infinite_activations(gpu, oracle, layout, M, K, wdt, zkind, ddt, re
     want = oracle.run_oracle(p)
     g, w = (decode(p.dst_dt, x, M * 192).astype(np.float64).reshape(M, 192)[:3] for x in (got, want))
     np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("dt,M,N,K", [("f16", 1, 14336, 4096), ("f16", 32, 64, 128), ("f16", 4, 1024, 16384), ("bf16", 8, 8128, 4096),
+                                      ("bf16", 24, 6144, 11776)])
+def test_format_any_weights_that_are_row_major(dt, M, N, K):
+    """what a caller does with them: asks for strides, quantizes f32 into them, hands them to a primitive of more rows"""
+    from onednn_amd import dnnl
+    eng = dnnl.engine(dnnl.gpu, 0)
+    attr = dnnl.primitive_attr()
+    attr.set_scales(dnnl.ARG_WEIGHTS, 3, (128, 1), cabi.DT_NAMES[dt])
+    attr.set_fpmath_mode(dnnl.fpmath_bf16 if dt == "bf16" else dnnl.fpmath_f16, True)
+    md = lambda dims, t, tag=dnnl.tag_ab: dnnl.memory_desc(dims, cabi.DT_NAMES[t], tag=tag)  # noqa: E731
+    pd = dnnl.matmul_primitive_desc(eng, md([M, K], dt), md([K, N], "u4", dnnl.tag_any), md([M, N], dt), attr=attr)
+    assert pd.impl_info_str().startswith("hip:woq_gemv")
+    wmd = pd.query_md(dnnl.query_weights_md)
+    assert wmd.strides() == [N, 1]
+    quantize = dnnl.primitive_attr()
+    quantize.set_scales(dnnl.ARG_SRC, 3, (128, 1), cabi.DT_F32)
+    dnnl.reorder_primitive_desc(eng, md([K, N], "f32"), eng, wmd, attr=quantize)
+    prompt = dnnl.matmul_primitive_desc(eng, md([512, K], dt), wmd, md([512, N], dt), attr=attr)
+    assert prompt.impl_info_str().startswith("hip:mfma_h16")
