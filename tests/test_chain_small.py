@@ -6,7 +6,7 @@ import pytest
 
 from onednn_amd import cabi, configs
 from onednn_amd import dtypes as dtp
-from onednn_amd.problem import PostOp, run_gpu
+from onednn_amd.problem import PostOp, decode, run_gpu
 from tests.helpers import assert_bit_exact
 from tests.test_line_loops import BYTES, FAMILY, RELU, SWITCH, check, problem
 
@@ -65,23 +65,38 @@ def test_block_scales(gpu, oracle, fmt, K, ddt):
         assert_bit_exact(p, got, oracle.run_oracle(p), name)
 
 
-@pytest.mark.parametrize("K", [64, 96, 384, 416, 544])
-def test_mxfp8_in_the_large_tiles_order(gpu, K):
-    """more than 256 tiles: random data, the bits of the 256 x 128 tiles"""
+# more than 256 tiles: rows and columns that end inside a tile, steps that K does not fill, up to two rounds of the three in flight
+@pytest.mark.parametrize("K", [64, 96, 128, 384, 416, 544, 800, 1184])
+@pytest.mark.parametrize("ddt,M,N,batch", [("f32", 520, 532, 1), ("bf16", 520, 536, 1), ("f32", 300, 532, 2), ("bf16", 289, 536, 2)])
+def test_mxfp8_in_the_large_tiles_order(gpu, K, ddt, M, N, batch):
+    """random data, the bits of the 256 x 128 tiles; the chain of either or an error"""
     from tests.test_mxf8_gemm import problem as mx_problem
-    p = mx_problem(520, 531, K, ddt="f32", exact=False, seed=K, bias=True)
+    p = mx_problem(M, N, K, ddt=ddt, exact=False, seed=K, bias=True, batch=batch)
     out = []
-    for tiles in ("small", "narrow"):
-        with cabi.tuning("MI355_F8_TILES", tiles):
-            out.append(run_gpu(p)[0])
-    assert np.array_equal(*(np.asarray(o).view(np.uint32) for o in out))
+    with cabi.tuning("MI355_EPILOGUE", "chain"):
+        for tiles in ("small", "narrow"):
+            with cabi.tuning("MI355_F8_TILES", tiles):
+                out.append(np.asarray(run_gpu(p)[0]))
+    bits = np.uint32 if ddt == "f32" else np.uint16
+    assert np.isfinite(decode(p.dst_dt, out[0], out[0].size)).all() and len(np.unique(out[0].view(bits))) > 1000
+    assert np.array_equal(*(o.view(bits) for o in out))
+
+
+@pytest.mark.parametrize("K", [96, 384, 544, 1184])
+@pytest.mark.parametrize("ddt", ["f32", "bf16", "f16"])
+def test_mxfp8_of_more_than_256_tiles(gpu, oracle, K, ddt):
+    """exact data, a scale of its own for every block"""
+    from tests.test_split_k import mx
+    p = mx(520, 536, K, "mxf8", ddt)
+    with cabi.tuning("MI355_F8_TILES", "small"), cabi.tuning("MI355_EPILOGUE", "chain"):
+        got, name = run_gpu(p)
+    assert_bit_exact(p, got, oracle.run_oracle(p), name)
 
 
 # infinities and NaN in the chunks that lanes beyond K load a second time
 @pytest.mark.parametrize("K", [8, 40, 72, 200])
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 def test_nan_at_the_end_of_k(gpu, oracle, K, dt):
-    from onednn_amd.problem import decode
     p = problem(40, 72, K, dt, "f32", bias=True)
     inf, nan = (0x7F80, 0x7FC0) if dt == "bf16" else (0x7C00, 0x7E00)
     for name, rows in (("src", 40), ("wei", 72)):
