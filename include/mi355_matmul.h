@@ -294,9 +294,11 @@ int mi355_mem_d2d(void *dst, const void *src, size_t bytes, void *stream);
 int mi355_stream_create(void **stream);
 int mi355_stream_destroy(void *stream);
 int mi355_stream_sync(void *stream); /* NULL = default stream */
+int mi355_stream_capturing(void *stream, int *capturing);
 int mi355_event_create(void **event);
 int mi355_event_destroy(void *event);
 int mi355_event_record(void *event, void *stream);
+int mi355_event_done(void *event, int *done); /* without waiting */
 int mi355_event_sync(void *event);
 int mi355_event_elapsed_ms(float *ms, void *start, void *stop);
 /* work enqueued on `stream` after this call starts when `event` has completed
@@ -363,9 +365,18 @@ int mi355_matmul_query(const mi355_matmul_desc_t *desc, int impl,
 /* Implementation name in oneDNN's "impl_info_str" style, e.g. "hip:mfma_i8". */
 const char *mi355_matmul_impl_name(int impl);
 
-/* Bytes of device scratch `mi355_matmul_launch` needs for this problem
- * (0 for most kernels). */
+/* Bytes of device scratch that `mi355_matmul_launch` uses for this problem:
+ * copies in another layout, column and row sums, packed block scales, and for
+ * a product of few tiles of dst and a long K, which is split over workgroups,
+ * up to 64 MiB of partial sums. */
 int mi355_matmul_scratch_bytes(const mi355_matmul_desc_t *desc, size_t *bytes);
+
+/* The same in two buffers: `own`, which a launch cannot do without, and
+ * `parts`, which it can.  own + parts may exceed mi355_matmul_scratch_bytes by
+ * a little.  With these a caller keeps one buffer for the parts of all its
+ * problems on a stream (the largest of their needs), and scratch per problem
+ * only where it is needed. */
+int mi355_matmul_scratch_parts(const mi355_matmul_desc_t *desc, size_t *own, size_t *parts);
 
 /* Enqueue the matmul on `stream` (a hipStream_t passed as void*, NULL =
  * default stream).  Asynchronous.  `scratch` may be NULL when
@@ -375,6 +386,12 @@ int mi355_matmul_scratch_bytes(const mi355_matmul_desc_t *desc, size_t *bytes);
  * over workgroups (which is then not split: slower). */
 int mi355_matmul_launch(const mi355_matmul_desc_t *desc,
         const mi355_matmul_args_t *args, void *scratch, void *stream);
+
+/* The launch with the buffers of mi355_matmul_scratch_parts.  `parts` may be
+ * NULL whatever the query says: K is then not split.  f32 sums of a split K are
+ * added in another order (the same one at every launch). */
+int mi355_matmul_launch_parts(const mi355_matmul_desc_t *desc,
+        const mi355_matmul_args_t *args, void *own, void *parts, void *stream);
 
 /* The same launch for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): no

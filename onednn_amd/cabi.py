@@ -150,7 +150,7 @@ KERNEL_SYMBOLS = [
     "mi355_event_destroy", "mi355_event_record", "mi355_event_sync", "mi355_event_elapsed_ms",
     "mi355_stream_wait_event", "mi355_mem_store_scalar",
     "mi355_graph_capture_begin", "mi355_graph_capture_end", "mi355_graph_launch", "mi355_graph_destroy",
-    "mi355_capture_mode_exchange",
+    "mi355_capture_mode_exchange", "mi355_stream_capturing", "mi355_event_done", "mi355_matmul_scratch_parts", "mi355_matmul_launch_parts",
     "mi355_last_error", "mi355_matmul_query", "mi355_matmul_impl_name",
     "mi355_matmul_scratch_bytes", "mi355_matmul_launch", "mi355_matmul_launch_noalloc", "mi355_reorder_query",
     "mi355_reorder_launch", "mi355_wei_pack_reorder_dims", "mi355_tuning_set", "mi355_colsum_launch", "mi355_sdpa_softmax_launch",
@@ -207,6 +207,10 @@ def load_kernels():
     lib.mi355_event_sync.argtypes = [vp]
     lib.mi355_event_elapsed_ms.argtypes = [C.POINTER(C.c_float), vp, vp]
     lib.mi355_stream_wait_event.argtypes = [vp, vp]
+    lib.mi355_event_done.argtypes = [vp, C.POINTER(C.c_int)]
+    lib.mi355_stream_capturing.argtypes = [vp, C.POINTER(C.c_int)]
+    lib.mi355_matmul_scratch_parts.argtypes = [C.POINTER(MatmulDesc), C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
+    lib.mi355_matmul_launch_parts.argtypes = [C.POINTER(MatmulDesc), C.POINTER(MatmulArgs), vp, vp, vp]
     lib.mi355_graph_capture_begin.argtypes = [vp]
     lib.mi355_graph_capture_end.argtypes = [vp, C.POINTER(vp)]
     lib.mi355_graph_launch.argtypes = [vp, vp]
@@ -345,6 +349,13 @@ def scratch_bytes(desc):
     n = C.c_size_t(0)
     check(load_kernels().mi355_matmul_scratch_bytes(C.byref(desc), C.byref(n)))
     return n.value
+
+
+def scratch_parts(desc):
+    """(own, parts): the bytes a launch cannot do without, and those of a split K's partial sums."""
+    own, parts = C.c_size_t(0), C.c_size_t(0)
+    check(load_kernels().mi355_matmul_scratch_parts(C.byref(desc), C.byref(own), C.byref(parts)))
+    return own.value, parts.value
 
 
 def tuning_set(name, value=None):

@@ -7,6 +7,7 @@
 
 #include <stdlib.h>
 
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -85,7 +86,12 @@ int ensure_dynamic_lds(const void *kernel, int bytes, const char *who) {
     std::lock_guard<std::mutex> lock(mu);
     auto it = done.find({kernel, dev});
     if (it != done.end() && it->second >= bytes) return MI355_SUCCESS;
-    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+    // (a stream may be under capture: the caller's eager launches may have run another kernel, K in parts for one)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const hipError_t set = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (set != hipSuccess) {
         set_error("%s: cannot reserve %d bytes of LDS", who, bytes);
         return MI355_RUNTIME_ERROR;
     }
@@ -95,6 +101,7 @@ int ensure_dynamic_lds(const void *kernel, int bytes, const char *who) {
 
 static int hip_status(hipError_t e, const char *what) {
     if (e == hipSuccess) return MI355_SUCCESS;
+    (void)hipGetLastError(); // reported here: not by the next launch
     set_error("%s: %s", what, hipGetErrorString(e));
     return e == hipErrorOutOfMemory ? MI355_OUT_OF_MEMORY : MI355_RUNTIME_ERROR;
 }
@@ -472,6 +479,13 @@ int mi355_capture_mode_exchange(int *mode) {
     *mode = (int)m;
     return st;
 }
+int mi355_stream_capturing(void *stream, int *capturing) {
+    if (!capturing) return MI355_INVALID_ARGUMENTS;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    const int st = hip_status(hipStreamIsCapturing((hipStream_t)stream, &status), "hipStreamIsCapturing");
+    *capturing = st || status != hipStreamCaptureStatusNone;
+    return st;
+}
 int mi355_stream_sync(void *stream) {
     return hip_status(hipStreamSynchronize((hipStream_t)stream), "hipStreamSynchronize");
 }
@@ -488,6 +502,16 @@ int mi355_event_destroy(void *event) {
 }
 int mi355_event_record(void *event, void *stream) {
     return hip_status(hipEventRecord((hipEvent_t)event, (hipStream_t)stream), "hipEventRecord");
+}
+int mi355_event_done(void *event, int *done) {
+    if (!done) return MI355_INVALID_ARGUMENTS;
+    const hipError_t e = hipEventQuery((hipEvent_t)event);
+    *done = e == hipSuccess;
+    if (e == hipErrorNotReady) {
+        (void)hipGetLastError(); // the answer, not an error
+        return MI355_SUCCESS;
+    }
+    return hip_status(e, "hipEventQuery");
 }
 int mi355_event_sync(void *event) {
     return hip_status(hipEventSynchronize((hipEvent_t)event), "hipEventSynchronize");
@@ -527,27 +551,42 @@ int mi355_matmul_query(const mi355_matmul_desc_t *desc, int impl, int *chosen_im
     return st;
 }
 
-static int scratch_bytes(const mi355_matmul_desc_t *desc, bool parts, size_t *bytes) {
-    if (!bytes) return MI355_INVALID_ARGUMENTS;
-    *bytes = 0;
+static int scratch_bytes(const mi355_matmul_desc_t *desc, bool parts, size_t *bytes, size_t *fixed) {
+    *bytes = *fixed = 0;
     int st = validate(desc);
     if (st) return st;
     int impl = 0;
     if ((st = choose_impl(*desc, &impl))) return st;
     switch (impl) {
-        case MI355_IMPL_I8_MFMA: *bytes = i8_scratch_bytes(*desc, parts); break;
-        case MI355_IMPL_F8_MFMA: *bytes = f8_scratch_bytes(*desc, parts); break;
-        case MI355_IMPL_H16_MFMA: *bytes = h16_scratch_bytes(*desc, parts); break;
-        case MI355_IMPL_MXF4_MFMA: *bytes = mxf4_scratch_bytes(*desc, parts); break;
-        case MI355_IMPL_WOQ_GEMV: *bytes = woq_scratch_bytes(*desc); break;
+        case MI355_IMPL_I8_MFMA: *bytes = i8_scratch_bytes(*desc, parts, fixed); break;
+        case MI355_IMPL_F8_MFMA: *bytes = f8_scratch_bytes(*desc, parts, fixed); break;
+        case MI355_IMPL_H16_MFMA: *bytes = h16_scratch_bytes(*desc, parts, fixed); break;
+        case MI355_IMPL_MXF4_MFMA: *bytes = mxf4_scratch_bytes(*desc, parts, fixed); break;
+        case MI355_IMPL_WOQ_GEMV: *bytes = *fixed = woq_scratch_bytes(*desc); break;
         default: break;
     }
     return MI355_SUCCESS;
 }
 
-int mi355_matmul_scratch_bytes(const mi355_matmul_desc_t *desc, size_t *bytes) { return scratch_bytes(desc, true, bytes); }
+int mi355_matmul_scratch_bytes(const mi355_matmul_desc_t *desc, size_t *bytes) {
+    size_t fixed;
+    return bytes ? scratch_bytes(desc, true, bytes, &fixed) : MI355_INVALID_ARGUMENTS;
+}
 
-static int launch(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *args, void *scratch, bool parts, void *stream) {
+int mi355_matmul_scratch_parts(const mi355_matmul_desc_t *desc, size_t *own, size_t *parts) {
+    if (!own || !parts) return MI355_INVALID_ARGUMENTS;
+    size_t total, fixed, without, unused;
+    int st = scratch_bytes(desc, true, &total, &fixed);
+    if (!st) st = scratch_bytes(desc, false, &without, &unused);
+    if (st) return st;
+    // a problem that needs none without a split gets by with none of its own: what the split plan wants besides its
+    // sums (int8: column sums, which the small tiles make by themselves) lies with them
+    *own = without == 0 && total > fixed ? 0 : std::max(without, fixed);
+    *parts = total > fixed ? total - (*own ? fixed : 0) : 0;
+    return MI355_SUCCESS;
+}
+
+static int launch(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *args, const scratch_t &S, void *stream) {
     int st = validate(desc);
     if (st) return st;
     if (!args) {
@@ -564,11 +603,11 @@ static int launch(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *ar
     hipStream_t s = (hipStream_t)stream;
     switch (impl) {
         case MI355_IMPL_REF: return ref_launch(P, s);
-        case MI355_IMPL_I8_MFMA: return i8_launch(*desc, P, scratch, parts, s);
-        case MI355_IMPL_F8_MFMA: return f8_launch(*desc, P, scratch, parts, s);
-        case MI355_IMPL_H16_MFMA: return h16_launch(*desc, P, scratch, parts, s);
-        case MI355_IMPL_MXF4_MFMA: return mxf4_launch(*desc, P, scratch, parts, s);
-        case MI355_IMPL_WOQ_GEMV: return woq_launch(*desc, P, scratch, s);
+        case MI355_IMPL_I8_MFMA: return i8_launch(*desc, P, S, s);
+        case MI355_IMPL_F8_MFMA: return f8_launch(*desc, P, S, s);
+        case MI355_IMPL_H16_MFMA: return h16_launch(*desc, P, S, s);
+        case MI355_IMPL_MXF4_MFMA: return mxf4_launch(*desc, P, S, s);
+        case MI355_IMPL_WOQ_GEMV: return woq_launch(*desc, P, S.p, s);
         case MI355_IMPL_WOQ_PACKED: return woqp_launch(*desc, P, s);
         default: return MI355_UNIMPLEMENTED;
     }
@@ -576,14 +615,28 @@ static int launch(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *ar
 
 int mi355_matmul_launch(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *args,
         void *scratch, void *stream) {
-    return launch(desc, args, scratch, scratch != nullptr, stream);
+    return launch(desc, args, scratch_t {scratch, scratch != nullptr, nullptr}, stream);
+}
+
+int mi355_matmul_launch_parts(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *args,
+        void *own, void *parts, void *stream) {
+    if (!parts) return launch(desc, args, scratch_t {own, false, nullptr}, stream);
+    size_t own_bytes = 0, bytes = 0;
+    const int st = mi355_matmul_scratch_parts(desc, &own_bytes, &bytes);
+    if (st) return st;
+    if (own_bytes == 0) return launch(desc, args, scratch_t {parts, true, nullptr}, stream);
+    if (!own) {
+        set_error("mi355_matmul_launch_parts: %zu bytes of scratch required besides the parts", own_bytes);
+        return MI355_INVALID_ARGUMENTS;
+    }
+    return launch(desc, args, scratch_t {own, true, parts}, stream);
 }
 
 // (without parts: problems that need no scratch stay free to overlap on one GPU)
 int mi355_matmul_launch_noalloc(const mi355_matmul_desc_t *desc, const mi355_matmul_args_t *args,
         void *stream) {
-    size_t bytes = 0;
-    int st = scratch_bytes(desc, false, &bytes);
+    size_t bytes = 0, fixed = 0;
+    int st = scratch_bytes(desc, false, &bytes, &fixed);
     if (st) return st;
     int impl = 0;
     if (bytes > (size_t)MI355_NOALLOC_SCRATCH_BYTES && choose_impl(*desc, &impl) == MI355_SUCCESS && impl == MI355_IMPL_I8_MFMA
@@ -601,7 +654,7 @@ int mi355_matmul_launch_noalloc(const mi355_matmul_desc_t *desc, const mi355_mat
     // every kernel family writes the part of its scratch it reads within the same
     // launch (transposed weights, row / column sums, split-K partial sums): nothing
     // has to start at zero
-    return launch(desc, args, scratch, false, stream);
+    return launch(desc, args, scratch_t {scratch, false, nullptr}, stream);
 }
 
 } // extern "C"

@@ -115,12 +115,15 @@ int f8_supported(const mi355_matmul_desc_t &d) {
     return MI355_SUCCESS;
 }
 
-size_t f8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts) {
-    return make_plan(d, parts).total;
+size_t f8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts, size_t *fixed) {
+    const f8_plan_t p = make_plan(d, parts);
+    *fixed = p.off_parts;
+    return p.total;
 }
 
-int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts, hipStream_t stream) {
-    const f8_plan_t plan = make_plan(d, parts);
+int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_t &S, hipStream_t stream) {
+    const f8_plan_t plan = make_plan(d, S.split);
+    void *const scratch = S.p;
     if (plan.total > 0 && !scratch) {
         set_error("mfma_f8: %zu bytes of scratch required", plan.total);
         return MI355_INVALID_ARGUMENTS;
@@ -153,7 +156,7 @@ int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, b
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K;
         C.sc = X.sc;
-        C.parts = (char *)scratch + plan.off_parts;
+        C.parts = S.parts ? (char *)S.parts : (char *)scratch + plan.off_parts;
         C.split = plan.split.split;
         C.part_steps = plan.split.part_steps;
         if (small) {

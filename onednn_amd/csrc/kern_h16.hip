@@ -349,8 +349,9 @@ int h16_supported(const mi355_matmul_desc_t &d) {
     return h16_plan(d, false).ok ? MI355_SUCCESS : MI355_UNIMPLEMENTED;
 }
 
-size_t h16_scratch_bytes(const mi355_matmul_desc_t &d, bool parts) {
+size_t h16_scratch_bytes(const mi355_matmul_desc_t &d, bool parts, size_t *fixed) {
     const h16_plan_t p = h16_plan(d, parts);
+    *fixed = p.ok ? p.off_parts : 0;
     return p.ok ? p.total : 0;
 }
 
@@ -408,8 +409,9 @@ static int h16_across(const mi355_matmul_desc_t &d, const h16_plan_t &p, const p
     return d.src_stride[2] != 1 && lines(P.src, d.src_stride[1], d.src_stride[2], d.src_stride[0], d.M) ? 2 : 0;
 }
 
-int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratch, bool parts, hipStream_t stream) {
-    h16_plan_t plan = h16_plan(d, parts);
+int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, const scratch_t &S, hipStream_t stream) {
+    h16_plan_t plan = h16_plan(d, S.split);
+    void *const scratch = S.p;
     if (!plan.ok) {
         set_error("mfma_h16: the problem is not one this family takes");
         return MI355_UNIMPLEMENTED;
@@ -437,7 +439,7 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, void *scratc
     const bool split_both = across == 2 && plan.split_across.split > 1;
     if (across == 2 && narrow && !split_both) across = d.K % 8 == 0 ? 1 : 0;
     auto split = [&](const chain_split_t &s) {
-        C.parts = (char *)scratch + plan.off_parts;
+        C.parts = S.parts ? (char *)S.parts : (char *)scratch + plan.off_parts;
         C.split = s.split;
         C.part_steps = s.part_steps;
     };

@@ -445,18 +445,20 @@ int i8_supported(const mi355_matmul_desc_t &d) {
 
 bool i8_scratch_optional(const mi355_matmul_desc_t &d) { return d.K % BK != 0 && d.wei_stride[1] == 1; }
 
-size_t i8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts) {
+size_t i8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts, size_t *fixed) {
     problem_t P;
     problem_of_desc(d, P);
     chain_t C;
-    return make_plan(d, i8_chain(P, C), parts).total;
+    const i8_plan_t p = make_plan(d, i8_chain(P, C), parts);
+    *fixed = p.off_parts;
+    return p.total;
 }
 
-int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts,
-        hipStream_t stream) {
+int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_t &S, hipStream_t stream) {
+    void *const scratch = S.p;
     chain_t C {};
     bool chain = i8_chain(P, C);
-    i8_plan_t plan = make_plan(d, chain, parts);
+    i8_plan_t plan = make_plan(d, chain, S.split);
     const uintptr_t at = (uintptr_t)P.src | (plan.need_transpose ? 0 : (uintptr_t)P.wei);
     // K is split on the LDS tiles, whose loads bring whole chunks from 16-byte boundaries straight to LDS: operands off one
     // have the tiles that they have without parts, the small ones where those are the better ones
@@ -509,7 +511,7 @@ int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, b
         C.colsum_bs = plan.Bw > 1 ? d.N : 0;
         C.src_zp = P.src_zp.dt != MI355_DT_UNDEF ? (const int *)P.src_zp.p : nullptr;
         C.off_s = su ? 128 : 0;
-        C.parts = sc + plan.off_parts;
+        C.parts = S.parts ? (char *)S.parts : sc + plan.off_parts;
         C.split = plan.split.split;
         C.part_steps = plan.split.part_steps;
     }

@@ -259,12 +259,15 @@ int mxf4_supported(const mi355_matmul_desc_t &d) {
     return MI355_SUCCESS;
 }
 
-size_t mxf4_scratch_bytes(const mi355_matmul_desc_t &d, bool parts) {
-    return make_plan(d, parts).total;
+size_t mxf4_scratch_bytes(const mi355_matmul_desc_t &d, bool parts, size_t *fixed) {
+    const mxf4_plan_t p = make_plan(d, parts);
+    *fixed = p.off_parts;
+    return p.total;
 }
 
-int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts, hipStream_t stream) {
-    const mxf4_plan_t plan = make_plan(d, parts);
+int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_t &S, hipStream_t stream) {
+    const mxf4_plan_t plan = make_plan(d, S.split);
+    void *const scratch = S.p;
     if (!scratch) {
         set_error("mfma_mxf4: %zu bytes of scratch required", plan.total);
         return MI355_INVALID_ARGUMENTS;
@@ -298,7 +301,7 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch,
         C.bt = X.bt; C.ldb = X.ldb; C.b_bs = X.bt_bstride;
         C.kbytes = P.K / 2;
         C.sc = X.sc;
-        C.parts = sc + plan.off_parts;
+        C.parts = S.parts ? (char *)S.parts : sc + plan.off_parts;
         C.split = plan.split.split;
         C.part_steps = plan.split.part_steps;
         if (small) {

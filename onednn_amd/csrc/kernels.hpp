@@ -12,26 +12,29 @@ namespace mi355 {
 int ref_supported(const mi355_matmul_desc_t &d);
 int ref_launch(const problem_t &P, hipStream_t stream);
 
-// parts: the scratch has room for partial sums of a K split over workgroups (chain_gemm.hpp); false: a launch without them
+// A launch's scratch.  split: with room for the partial sums of a K split over workgroups (chain_gemm.hpp), at `parts` or, where
+// that is null, behind the rest of `p`; false: a launch without them.
+struct scratch_t {
+    void *p;
+    bool split;
+    void *parts;
+};
+// *_scratch_bytes: of either kind of launch; *fixed: of those, what is not for the partial sums
 int i8_supported(const mi355_matmul_desc_t &d);
-size_t i8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts);
+size_t i8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts, size_t *fixed);
 bool i8_scratch_optional(const mi355_matmul_desc_t &d); // i8_launch takes a null scratch all the same
-int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts,
-        hipStream_t stream);
+int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_t &S, hipStream_t stream);
 
 int f8_supported(const mi355_matmul_desc_t &d);
-size_t f8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts);
-int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts,
-        hipStream_t stream);
+size_t f8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts, size_t *fixed);
+int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_t &S, hipStream_t stream);
 int h16_supported(const mi355_matmul_desc_t &d);
-size_t h16_scratch_bytes(const mi355_matmul_desc_t &d, bool parts);
-int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts,
-        hipStream_t stream);
+size_t h16_scratch_bytes(const mi355_matmul_desc_t &d, bool parts, size_t *fixed);
+int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_t &S, hipStream_t stream);
 
 int mxf4_supported(const mi355_matmul_desc_t &d);
-size_t mxf4_scratch_bytes(const mi355_matmul_desc_t &d, bool parts);
-int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, void *scratch, bool parts,
-        hipStream_t stream);
+size_t mxf4_scratch_bytes(const mi355_matmul_desc_t &d, bool parts, size_t *fixed);
+int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_t &S, hipStream_t stream);
 
 int woq_supported(const mi355_matmul_desc_t &d);
 size_t woq_scratch_bytes(const mi355_matmul_desc_t &d);

@@ -86,9 +86,106 @@ const char *dt_name(int dt) {
 } // namespace
 
 // ------------------------------------------------------------------ objects
+// A device event.  Recording one costs a launch some 4 us on the device, so an execution records one for all that it orders.
+struct event_t {
+    void *h = nullptr;
+    event_t() { mi355_event_create(&h); } // the device is current here
+    ~event_t() { mi355_event_destroy(h); }
+    event_t(const event_t &) = delete;
+    bool record(void *stream) { return h && mi355_event_record(h, stream) == MI355_SUCCESS; }
+};
+
+// Buffers for the partial sums of products whose K is split over workgroups.  A launch can do without them
+// (mi355_matmul_launch_parts), so they belong to no primitive: hundreds of layers would hold 32 MiB each, and executions of
+// one primitive on several streams would wait for each other.  A device has up to MOST of them for as long as it has an
+// engine.  An execution takes the one that its stream used last, or one whose last use has ended, or a new one, and
+// where there is none -- no memory, more streams busy at once -- K is not split; nothing ever waits here.  Nor is it split
+// under capture: a graph would keep the buffer.
+struct parts_pool_t {
+    static constexpr size_t BYTES = size_t(64) << 20, MOST = 16; // (256 parts of 256 x 256 tiles)
+    struct buffer_t {
+        void *p;
+        std::shared_ptr<event_t> event; // recorded behind every use
+        void *stream = nullptr;         // of the last one
+        bool used = false;
+    };
+    std::mutex mutex;
+    std::vector<buffer_t> buffers;
+    size_t engines = 0;
+
+    // a new buffer, or null
+    buffer_t *add() {
+        if (buffers.size() >= MOST) return nullptr;
+        buffer_t b {nullptr, std::make_shared<event_t>()};
+        if (!b.event->h || mi355_mem_alloc(&b.p, BYTES) != MI355_SUCCESS) return nullptr;
+        buffers.push_back(b);
+        return &buffers.back();
+    }
+    // the mutex is held from here until the launches that use it and its event are enqueued; the device is current
+    buffer_t *take(void *stream, size_t bytes) {
+        int capturing = 0;
+        if (bytes > BYTES || mi355_stream_capturing(stream, &capturing) != MI355_SUCCESS || capturing) return nullptr;
+        for (buffer_t &b : buffers)
+            if (b.used && b.stream == stream) {
+                // (nothing to wait for, unless the handle is another stream's by now)
+                return mi355_stream_wait_event(stream, b.event->h) == MI355_SUCCESS ? &b : nullptr;
+            }
+        int mode = 2; // (another stream may be under capture, which forbids these calls otherwise)
+        if (mi355_capture_mode_exchange(&mode) != MI355_SUCCESS) return nullptr;
+        buffer_t *found = nullptr;
+        for (buffer_t &b : buffers) {
+            int done = !b.used;
+            if (done || (mi355_event_done(b.event->h, &done) == MI355_SUCCESS && done)) {
+                found = &b;
+                break;
+            }
+        }
+        if (!found) found = add();
+        mi355_capture_mode_exchange(&mode);
+        return found;
+    }
+    void give(buffer_t *b, void *stream) {
+        b->stream = stream;
+        b->used = true;
+        if (!b->event->record(stream)) mi355_stream_sync(stream);
+    }
+    // the device's first buffer, ahead of the first execution; without one that allocates it, or does without
+    void reserve() {
+        std::lock_guard<std::mutex> lock(mutex);
+        if (!buffers.empty()) return;
+        int mode = 2;
+        if (mi355_capture_mode_exchange(&mode) != MI355_SUCCESS) return;
+        add();
+        mi355_capture_mode_exchange(&mode);
+    }
+    void engine_gone(int device) {
+        std::lock_guard<std::mutex> lock(mutex);
+        if (--engines > 0 || buffers.empty()) return;
+        int mode = 2;
+        const bool relaxed = mi355_capture_mode_exchange(&mode) == MI355_SUCCESS;
+        if (mi355_device_set(device) == MI355_SUCCESS) {
+            for (const buffer_t &b : buffers) mi355_mem_free(b.p); // waits for the device
+        }
+        buffers.clear();
+        if (relaxed) mi355_capture_mode_exchange(&mode);
+    }
+    static parts_pool_t &of(size_t device) { // never destroyed: the runtime may be gone before
+        static std::mutex all;
+        static auto *pools = new std::map<size_t, parts_pool_t>;
+        std::lock_guard<std::mutex> lock(all);
+        return (*pools)[device];
+    }
+};
+
 struct dnnl_engine {
     dnnl_engine_kind_t kind;
     size_t index;
+    parts_pool_t *parts;
+    dnnl_engine(dnnl_engine_kind_t k, size_t i) : kind(k), index(i), parts(&parts_pool_t::of(i)) {
+        std::lock_guard<std::mutex> lock(parts->mutex);
+        ++parts->engines;
+    }
+    ~dnnl_engine() { parts->engine_gone((int)index); }
 };
 
 struct dnnl_stream {
@@ -265,7 +362,9 @@ struct dnnl_primitive_desc {
     mi355_grouped_desc_t gdesc;
     std::vector<int> impls;       // kernel families that can run it, best first
     size_t impl_pos = 0;
-    size_t scratch_bytes = 0;
+    size_t scratch_bytes = 0;     // of the scratchpad: the primitive's own, or the user's
+    size_t parts_bytes = 0;       // partial sums of a split K: shared ones (parts_pool_t), or in the user's scratchpad
+    size_t own_bytes = 0;         // of the scratchpad without the parts
     std::string impl_name;
     // some dim or stride is DNNL_RUNTIME_DIM_VAL: the descriptor is validated
     // as far as the known values allow, and lowered and dispatched at each
@@ -305,7 +404,8 @@ struct dnnl_primitive {
     // scratchpad, host-scalar slots, runtime-dims scratch) are ordered on the
     // device as well as on the host: each records `order_event` behind its
     // launches, and the next one on another stream makes its stream wait for it.
-    void *order_event = nullptr;
+    // (its own, or that of the parts' buffer, whose later uses lie behind this one)
+    std::shared_ptr<event_t> own_event, order_event;
     void *last_stream = nullptr;
     bool event_recorded = false;
     ~dnnl_primitive() {
@@ -315,7 +415,6 @@ struct dnnl_primitive {
         if (scratch) mi355_mem_free(scratch);
         for (void *q : rt_scratch) mi355_mem_free(q);
         if (host_scalars) mi355_mem_free(host_scalars);
-        if (order_event) mi355_event_destroy(order_event);
     }
 };
 
@@ -796,9 +895,10 @@ dnnl_status_t select_impl(dnnl_primitive_desc &pd) {
     pd.desc.impl = pd.impls[pd.impl_pos];
     pd.impl_name = mi355_matmul_impl_name(pd.desc.impl);
     size_t bytes = 0;
-    const int st = mi355_matmul_scratch_bytes(&pd.desc, &bytes);
+    int st = mi355_matmul_scratch_parts(&pd.desc, &pd.own_bytes, &pd.parts_bytes);
+    if (st == MI355_SUCCESS) st = mi355_matmul_scratch_bytes(&pd.desc, &bytes);
     if (st != MI355_SUCCESS) return from_mi355(st);
-    pd.scratch_bytes = bytes;
+    pd.scratch_bytes = pd.attr.scratchpad_mode == dnnl_scratchpad_mode_user ? bytes : pd.own_bytes;
     pd.scratchpad = dnnl_memory_desc();
     if (pd.attr.scratchpad_mode == dnnl_scratchpad_mode_user && bytes > 0) {
         pd.scratchpad.ndims = 1;
@@ -887,7 +987,7 @@ dnnl_status_t concretize(dnnl_primitive &prim, const std::map<int, dnnl_memory_t
         if (st) return st;
         prim.rt_pd = std::move(c);
     }
-    const size_t need = prim.rt_pd->scratch_bytes;
+    const size_t need = prim.rt_pd->own_bytes;
     if (need > prim.rt_scratch_bytes) {
         if (mi355_device_set((int)pd0.engine->index) != MI355_SUCCESS) return dnnl_runtime_error;
         void *q = nullptr;
@@ -916,7 +1016,7 @@ DNNL_EXPORT dnnl_status_t dnnl_engine_create(dnnl_engine_t *engine, dnnl_engine_
         if (rc != MI355_SUCCESS) return dnnl_runtime_error;
         CHECK_ARG((int)index < n);
     }
-    *engine = new dnnl_engine {kind, index};
+    *engine = new dnnl_engine(kind, index);
     return dnnl_success;
 }
 DNNL_EXPORT size_t dnnl_engine_get_count(dnnl_engine_kind_t kind) {
@@ -2592,6 +2692,9 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_create(dnnl_primitive_t *primitive, con
         const int st = mi355_mem_alloc(&p->scratch, p->pd.scratch_bytes);
         if (st != MI355_SUCCESS) return from_mi355(st);
     }
+    if (p->pd.attr.scratchpad_mode == dnnl_scratchpad_mode_library && p->pd.parts_bytes > 0) {
+        if (mi355_device_set((int)p->pd.engine->index) == MI355_SUCCESS) p->pd.engine->parts->reserve();
+    }
     if (p->pd.sdpa && !p->pd.sdpa->fused) {
         p->composed = p->scratch;
         const dnnl_status_t st = sdpa_compose(*p);
@@ -2677,9 +2780,16 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
         if (ordered) return;
         ordered = true;
         if (!lock.owns_lock()) lock.lock();
-        if (!prim->order_event) mi355_event_create(&prim->order_event); // the device is current here
-        if (prim->order_event && prim->event_recorded && prim->last_stream != stream->hip_stream)
-            mi355_stream_wait_event(stream->hip_stream, prim->order_event);
+        if (!prim->own_event) prim->own_event = std::make_shared<event_t>(); // the device is current here
+        if (prim->event_recorded && prim->last_stream != stream->hip_stream)
+            mi355_stream_wait_event(stream->hip_stream, prim->order_event->h);
+    };
+    // ... and behind its last use
+    auto record = [&](const std::shared_ptr<event_t> &recorded) {
+        if (!ordered || !(recorded || prim->own_event->record(stream->hip_stream))) return;
+        prim->order_event = recorded ? recorded : prim->own_event;
+        prim->event_recorded = true;
+        prim->last_stream = stream->hip_stream;
     };
     if (pd0.sdpa) {
         const dnnl_primitive_desc::sdpa_t &S = *pd0.sdpa;
@@ -2695,12 +2805,6 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
         if (S.dst.nelems() == 0) return dnnl_success;
         CHECK_ARG(q->handle && k->handle && v->handle && d->handle);
         if (mi355_device_set((int)pd0.engine->index) != MI355_SUCCESS) return dnnl_runtime_error;
-        auto record = [&]() {
-            if (prim->order_event && mi355_event_record(prim->order_event, stream->hip_stream) == MI355_SUCCESS) {
-                prim->event_recorded = true;
-                prim->last_stream = stream->hip_stream;
-            }
-        };
         // The fused kernel takes aligned buffers, and a dst of its own: it stores rows while others are still reading.
         // (The composition has read q, k, the mask and the scale before it stores; q itself is safe as dst where every
         // element stays in its place, since a wavefront holds its queries before it stores their rows.)
@@ -2715,7 +2819,7 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
             if (prim->scratch) order_on_device(); // the parts of a split launch belong to the primitive
             const int rc = mi355_sdpa_launch(&S.fused_desc, q->handle, k->handle, v->handle, d->handle,
                     scale ? scale->handle : nullptr, mask ? mask->handle : nullptr, prim->scratch, stream->hip_stream);
-            if (ordered) record();
+            record(nullptr);
             return from_mi355(rc);
         }
         order_on_device(); // the scores and probabilities belong to the primitive
@@ -2754,7 +2858,7 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
         if (rc != MI355_SUCCESS) return from_mi355(rc);
         const dnnl_exec_arg_t a2[3] = {{DNNL_ARG_SRC, &pr_mem}, {DNNL_ARG_WEIGHTS, v}, {DNNL_ARG_DST, d}};
         st = dnnl_primitive_execute(prim->sdpa_vs, stream, 3, a2);
-        record();
+        record(nullptr);
         return st;
     }
     void *rt_scratch = nullptr;
@@ -2948,8 +3052,7 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
     if (pd0.runtime) {
         scratch = rt_scratch;
     } else if (pd.attr.scratchpad_mode == dnnl_scratchpad_mode_user) {
-        // (the launch refuses a problem that cannot do without)
-        if ((st = handle(DNNL_ARG_SCRATCHPAD, false, &scratch))) return st;
+        if ((st = handle(DNNL_ARG_SCRATCHPAD, pd.own_bytes > 0, &scratch))) return st;
     } else if (scratch) {
         // the library-mode scratchpad belongs to the primitive: executions of
         // one primitive object are serialised on the host while they enqueue
@@ -2958,9 +3061,22 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
     }
     if (mi355_device_set((int)pd.engine->index) != MI355_SUCCESS) return dnnl_runtime_error;
     const auto t0 = std::chrono::steady_clock::now();
+    // (a primitive with runtime dims has scratch of its own in either mode)
+    const bool users = pd.attr.scratchpad_mode == dnnl_scratchpad_mode_user && !pd0.runtime;
+    parts_pool_t &pool = *pd.engine->parts;
+    std::unique_lock<std::mutex> pool_lock(pool.mutex, std::defer_lock);
+    parts_pool_t::buffer_t *parts = nullptr;
+    if (!users && pd.parts_bytes > 0) {
+        pool_lock.lock();
+        parts = pool.take(stream->hip_stream, pd.parts_bytes);
+    }
+    auto launch = [&](const mi355_matmul_args_t &a) {
+        return users ? mi355_matmul_launch(&pd.desc, &a, scratch, stream->hip_stream)
+                     : mi355_matmul_launch_parts(&pd.desc, &a, scratch, parts ? parts->p : nullptr, stream->hip_stream);
+    };
     int rc = MI355_SUCCESS;
     if (pd.outer_n == 0) {
-        rc = mi355_matmul_launch(&pd.desc, &A, scratch, stream->hip_stream);
+        rc = launch(A);
     } else {
         // one launch per index of the batch dims that are walked on the host (in stream order: they share the scratch)
         dim_t count = 1;
@@ -2983,21 +3099,19 @@ DNNL_EXPORT dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t cprimiti
             if (pd.with_bias) B.bias = shifted(A.bias, ob, pd.bias.dt);
             for (int k = 0; k < pd.desc.n_post_ops; ++k)
                 if (pd.desc.post_ops[k].kind == MI355_PO_BINARY) B.po_arg[k] = shifted(A.po_arg[k], op[k], pd.desc.post_ops[k].dt);
-            rc = mi355_matmul_launch(&pd.desc, &B, scratch, stream->hip_stream);
+            rc = launch(B);
         }
     }
     if (rc == MI355_SUCCESS && ip_diff_bias_mem && pd0.ip_diff_bias) {
         // diff_bias[oc] = sum over mb of diff_dst[mb, oc], added in the order of the rows
-        CHECK_ARG(ip_diff_bias_mem->handle && ip_diff_dst_mem->handle);
-        rc = mi355_colsum_launch(ip_diff_dst_mem->handle, (int)pd0.ip_dst.dt, pd0.ip_dst.dims[0], pd0.ip_dst.dims[1],
+        rc = !ip_diff_bias_mem->handle || !ip_diff_dst_mem->handle
+                ? (int)MI355_INVALID_ARGUMENTS
+                : mi355_colsum_launch(ip_diff_dst_mem->handle, (int)pd0.ip_dst.dt, pd0.ip_dst.dims[0], pd0.ip_dst.dims[1],
                 pd0.ip_dst.strides[0], ip_diff_bias_mem->handle, (int)pd0.ip_bias.dt, stream->hip_stream);
     }
-    if (ordered && prim->order_event) {
-        if (mi355_event_record(prim->order_event, stream->hip_stream) == MI355_SUCCESS) {
-            prim->event_recorded = true;
-            prim->last_stream = stream->hip_stream;
-        }
-    }
+    if (parts) pool.give(parts, stream->hip_stream);
+    record(parts ? parts->event : nullptr);
+    if (pool_lock.owns_lock()) pool_lock.unlock();
     if (verbose_level() >= 2) {
         mi355_stream_sync(stream->hip_stream);
         const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
