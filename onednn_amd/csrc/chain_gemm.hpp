@@ -40,6 +40,8 @@ inline chain_split_t chain_split(long batch, long M, long N, long kbytes, bool w
     chain_split_t r {1, (int)steps};
     if (tiles < 1 || tiles > 128) return r;
     long best = steps * step_ns - CHAIN_SPLIT_NS;
+    // (no s does better than the least of steps / s * step_ns + s * tiles * part_ns: most launches leave here)
+    if (best <= 0 || 4. * steps * step_ns * tiles * part_ns >= (double)best * best) return r;
     for (long s = 2; s * tiles <= 256; ++s) {
         const long per = (steps + s - 1) / s;
         if (per < 2) break;
@@ -79,6 +81,11 @@ struct chain_t {
     const void *dsc;
     int dsc_dt, ds_mode; // 0 none, 1 divide, 2 multiply by the reciprocal
     int lo, hi;          // 8-bit dst
+};
+
+// ... and what the kernels of parts of K and of the 32 x 32 tiles of 16-bit, fp8 and block-scaled operands also read; a type of
+// its own, so that the others' arguments are no longer for it (every launch writes them to the device)
+struct chain_more_t : chain_t {
     // split > 1: K in parts of part_steps steps, a workgroup each; their accumulators go to parts and chain_sum_kernel
     // (kern_chain_sum.hip) adds them and does the rest
     char *parts;
@@ -87,6 +94,8 @@ struct chain_t {
     const uint8_t *sa, *sb;
     long sa_bs, sb_bs;
 };
+template <int DST>
+using chain_arg_t = std::conditional_t<DST == CHAIN_PART, chain_more_t, chain_t>; // of chain_gemm_kernel
 
 // A product of few 32 x 32 tiles on chain_small_float_kernel (kern_chain_small.hip): small_tiles_float says whether (mx: 0, or
 // the bits of a block-scaled type).
@@ -94,10 +103,10 @@ enum chain_small_t { CHAIN_SMALL_BF16, CHAIN_SMALL_F16, CHAIN_SMALL_F8, CHAIN_SM
 // small_tiles_fit: whether its 32-bit steps of K and offsets of block scales reach that far.
 bool small_tiles_fit(long M, long N, long kbytes, int mx);
 bool small_tiles_float(long batch, long M, long N, long kbytes, const chain_split_t &split, long step_ns, const chain_t &C, int mx);
-int chain_launch_small(chain_small_t kind, int dst_dt, chain_t &C, unsigned batch, hipStream_t stream);
+int chain_launch_small(chain_small_t kind, int dst_dt, chain_more_t &C, unsigned batch, hipStream_t stream);
 
 // the sums of a problem whose parts lie at C.parts, and its epilogue (integer: they are s32)
-int chain_launch_sum(bool integer, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
+int chain_launch_sum(bool integer, int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream);
 
 // The problem's epilogue as a chain; false: not one of them (the general kernels run it).  What the K loop reads (a,
 // bt, lda, ldb, the batches' strides, kbytes, block scales, colsum) is the family's to fill in.  scaled: src and
@@ -117,15 +126,15 @@ int mx_pack_scales(const mi355_matmul_desc_t &d, const problem_t &P, long Bsa, l
 
 // The families' launchers on the chain kernels, a translation unit each; C as chain_from and the family left it.
 // wide: the 256 x 256 tiles whatever the size.  A 16-bit dst of the operands' other type takes a C of full = false.
-int chain_launch_h16(bool bf16, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
+int chain_launch_h16(bool bf16, int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream);
 // ... with the weights (across = 1), or src and the weights (2, 256 x 256 tiles only), contiguous across K: lda / ldb are the
 // bytes from one k to the next
-int chain_launch_h16_across(bool bf16, int dst_dt, int across, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
-int chain_launch_i8(bool src_u8, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream);
+int chain_launch_h16_across(bool bf16, int dst_dt, int across, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream);
+int chain_launch_i8(bool src_u8, int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream);
 // ... on 32 x 32 tiles that make their own column sums (C.colsum is not read)
 int chain_launch_i8_small(bool src_u8, int dst_dt, chain_t &C, unsigned batch, hipStream_t stream);
-int chain_launch_f8(int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream); // e4m3 x e4m3
-int chain_launch_mx(bool fp4, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream); // e4m3 x e4m3 or fp4
+int chain_launch_f8(int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream); // e4m3 x e4m3
+int chain_launch_mx(bool fp4, int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream); // e4m3 x e4m3 or fp4
 
 #ifdef MI355_CHAIN_KERNELS
 namespace {
@@ -377,15 +386,18 @@ struct chain_part_t {
 extern __shared__ __attribute__((aligned(128))) char chain_smem[];
 
 template <class Mma, int DST>
-__global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu(Mma::G::NW / 4))) chain_gemm_kernel(const chain_t C) {
+__global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu(Mma::G::NW / 4))) chain_gemm_kernel(const chain_arg_t<DST> C) {
     using G = typename Mma::G;
     using V = typename Mma::acc_t;
     static_assert(G::WCOLS == 64, "a wavefront's part is 128 x 64");
     char *smem = chain_smem;
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     constexpr bool PART = DST == CHAIN_PART;
-    const long b = PART ? blockIdx.z / C.split : blockIdx.z;
-    const long step0 = PART ? (long)(blockIdx.z % C.split) * C.part_steps : 0; // the first step of the part
+    long b = blockIdx.z, step0 = 0; // (the first step of the part)
+    if constexpr (PART) {
+        b = blockIdx.z / C.split;
+        step0 = (long)(blockIdx.z % C.split) * C.part_steps;
+    }
     const tile_pos_t tp = tile_position<G>((int)blockIdx.x, C.tiles_m, C.tiles_n);
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem;
     const unsigned tab = lds0 + line_loader_t<Mma>::LDS_BYTES;
@@ -463,13 +475,13 @@ __global__ void __launch_bounds__(Mma::G::NT) __attribute__((amdgpu_waves_per_eu
 }
 
 template <class Mma, int DST>
-int chain_go(chain_t &C, unsigned batch, hipStream_t stream, const char *who) {
+int chain_go(chain_more_t &C, unsigned batch, hipStream_t stream, const char *who) {
     constexpr int smem_bytes = line_loader_t<Mma>::LDS_BYTES + CT_BYTES;
     C.tiles_m = (int)((C.M + BM - 1) / BM);
     C.tiles_n = (int)((C.N + Mma::G::BN - 1) / Mma::G::BN);
     const dim3 grid((unsigned)(C.tiles_m * C.tiles_n), 1, DST == CHAIN_PART ? batch * C.split : batch);
     if (const int st = ensure_dynamic_lds((const void *)chain_gemm_kernel<Mma, DST>, smem_bytes, who)) return st;
-    hipLaunchKernelGGL((chain_gemm_kernel<Mma, DST>), grid, dim3(Mma::G::NT), smem_bytes, stream, C);
+    hipLaunchKernelGGL((chain_gemm_kernel<Mma, DST>), grid, dim3(Mma::G::NT), smem_bytes, stream, static_cast<const chain_arg_t<DST> &>(C));
     return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
 }
 // The chain for four consecutive columns of one row, a thread at a time: what chain_part_t::store does with a tile.
@@ -548,7 +560,7 @@ struct chain_quad_t {
 
 // K in parts (C.split of them), then their sums and the epilogue
 template <class Mma>
-int chain_go_parts(int dst_dt, chain_t &C, unsigned batch, hipStream_t stream, const char *who) {
+int chain_go_parts(int dst_dt, chain_more_t &C, unsigned batch, hipStream_t stream, const char *who) {
     if (const int st = chain_go<Mma, CHAIN_PART>(C, batch, stream, who)) return st;
     return chain_launch_sum(Mma::INTEGER, dst_dt, C, batch, Mma::G::BN == 256, stream);
 }

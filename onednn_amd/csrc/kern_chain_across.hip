@@ -6,7 +6,7 @@
 
 namespace mi355 {
 
-int chain_launch_h16_across(bool bf16, int dst_dt, int across, chain_t &C, unsigned batch, bool wide, hipStream_t stream) {
+int chain_launch_h16_across(bool bf16, int dst_dt, int across, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream) {
     using narrow_t = geo_t<4, 128>;
     using wide_t = geo_t<8, 256>;
     auto go = [&](auto b16, auto dst) -> int {

@@ -5,7 +5,7 @@
 
 namespace mi355 {
 
-int chain_launch_f8(int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream) {
+int chain_launch_f8(int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream) {
     auto go = [&](auto dst) -> int {
         constexpr int D = decltype(dst)::value;
         return wide ? chain_go<f8_mma_t<0, 0, geo_t<8, 256>>, D>(C, batch, stream, "mfma_f8")

@@ -82,7 +82,7 @@ bool chain_from_mx(const problem_t &P, bool mx, bool full, chain_t &C) {
     return chain_from(Q, false, full, C);
 }
 
-int chain_launch_h16(bool bf16, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream) {
+int chain_launch_h16(bool bf16, int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream) {
     using narrow_t = geo_t<4, 128>;
     using wide_t = geo_t<8, 256>;
     auto go = [&](auto b16, auto dst) -> int {

@@ -177,7 +177,7 @@ int chain_launch_i8_small(bool src_u8, int dst_dt, chain_t &C, unsigned batch, h
     return C.src_zp ? by_dst(std::false_type {}, std::true_type {}) : by_dst(std::false_type {}, std::false_type {});
 }
 
-int chain_launch_i8(bool src_u8, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream) {
+int chain_launch_i8(bool src_u8, int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream) {
     auto go = [&](auto u8, auto dst) -> int {
         constexpr bool U = decltype(u8)::value;
         constexpr int D = decltype(dst)::value;

@@ -5,7 +5,7 @@
 
 namespace mi355 {
 
-int chain_launch_mx(bool fp4, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream) {
+int chain_launch_mx(bool fp4, int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream) {
     using wide_t = geo_t<8, 256>;
     using narrow_t = geo_t<4, 128>;
     auto go = [&](auto dst) -> int {

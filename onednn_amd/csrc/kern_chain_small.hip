@@ -27,7 +27,7 @@ using small_mma_t = std::conditional_t<KIND == CHAIN_SMALL_BF16, h16x16_mma_t<tr
 
 // IN_ORDER: a wavefront owns 16 x 16 of the tile and all of K, in the large tiles' order of sums.
 template <int KIND, int DST, bool IN_ORDER>
-__global__ void __launch_bounds__(FSNW * 64, IN_ORDER ? 3 : KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) chain_small_float_kernel(const chain_t C) {
+__global__ void __launch_bounds__(FSNW * 64, IN_ORDER ? 3 : KIND >= CHAIN_SMALL_MXF8 ? 2 : 4) chain_small_float_kernel(const chain_more_t C) {
     using Mma = small_mma_t<KIND>;
     constexpr int NU = Mma::NU, NS = Mma::SCALE_SETS; // instructions a pair; scales a lane, fragment and step
     // steps of a wavefront in flight (four, at half the workgroups a CU, took as long or up to 1.8 times as long: 512 x 2048 x 512
@@ -180,7 +180,7 @@ bool small_tiles_float(long batch, long M, long N, long kbytes, const chain_spli
     return small < 0.95 * rest;
 }
 
-int chain_launch_small(chain_small_t kind, int dst_dt, chain_t &C, unsigned batch, hipStream_t stream) {
+int chain_launch_small(chain_small_t kind, int dst_dt, chain_more_t &C, unsigned batch, hipStream_t stream) {
     const long tm = (C.M + FST - 1) / FST, tn = (C.N + FST - 1) / FST;
     C.tiles_m = (int)tm;
     C.tiles_n = (int)tn;

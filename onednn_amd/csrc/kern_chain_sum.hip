@@ -11,7 +11,7 @@ namespace {
 // timing.  Bound: the parts' bytes (they were written a moment ago and come from the memory-side cache) and, for small
 // problems, the launch.
 template <bool INTEGER, int DST, class G>
-__global__ void __launch_bounds__(256) chain_sum_kernel(const chain_t C) {
+__global__ void __launch_bounds__(256) chain_sum_kernel(const chain_more_t C) {
     using V = std::conditional_t<INTEGER, v4i, v4f>;
     const int t = threadIdx.x, lane = t & 63, k = t >> 6;
     const int i = blockIdx.x % 8, wave = blockIdx.x / 8 % G::NW, id = blockIdx.x / (8 * G::NW);
@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(256) chain_sum_kernel(const chain_t C) {
 
 } // namespace
 
-int chain_launch_sum(bool integer, int dst_dt, chain_t &C, unsigned batch, bool wide, hipStream_t stream) {
+int chain_launch_sum(bool integer, int dst_dt, chain_more_t &C, unsigned batch, bool wide, hipStream_t stream) {
     auto go = [&](auto is_int, auto dst, auto geo) -> int {
         using G = decltype(geo);
         hipLaunchKernelGGL((chain_sum_kernel<decltype(is_int)::value, decltype(dst)::value, G>),

@@ -141,7 +141,7 @@ int f8_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_t 
         X.bt_bstride = d.wei_stride[0];
     }
     const int fa = d.src_dt == MI355_DT_F8_E5M2, fb = d.wei_dt == MI355_DT_F8_E5M2;
-    chain_t C {};
+    chain_more_t C {};
     const bool small = plan.small && f8_chain(P, plan.mx, true, C);
     const bool chain = small || (is_e4m3_pair(d) && f8_chain(P, plan.mx, false, C));
     if (plan.mx && !small) {

@@ -433,7 +433,7 @@ int h16_launch(const mi355_matmul_desc_t &d, const problem_t &P_in, const scratc
         return force == TUNE_NARROW || (line_tiles_narrow(d.batch, d.M, d.N, plan.Kp * EB, chain) && force != TUNE_WIDE);
     };
     bool narrow = narrow_for(true);
-    chain_t C {};
+    chain_more_t C {};
     int across = h16_across(d, plan, P);
     // the 256 x 128 tile takes weights across K only: src is copied there (whole chunks of K)
     const bool split_both = across == 2 && plan.split_across.split > 1;

@@ -456,7 +456,7 @@ size_t i8_scratch_bytes(const mi355_matmul_desc_t &d, bool parts, size_t *fixed)
 
 int i8_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_t &S, hipStream_t stream) {
     void *const scratch = S.p;
-    chain_t C {};
+    chain_more_t C {};
     bool chain = i8_chain(P, C);
     i8_plan_t plan = make_plan(d, chain, S.split);
     const uintptr_t at = (uintptr_t)P.src | (plan.need_transpose ? 0 : (uintptr_t)P.wei);

@@ -291,7 +291,7 @@ int mxf4_launch(const mi355_matmul_desc_t &d, const problem_t &P, const scratch_
     }
     // (MI355_F8_TILES keeps one geometry here as well)
     const int force = tuning(TUNE_F8_TILES);
-    chain_t C {};
+    chain_more_t C {};
     const bool small = plan.small && mxf4_chain(P, true, C), chain = small || mxf4_chain(P, false, C);
     if (!small)
         if (const int st = mx_pack_scales(d, P, plan.Bsa, plan.Bsb, sc + plan.off_sa, sc + plan.off_sb, X.sc, stream)) return st;

@@ -3,6 +3,10 @@ end, every compiled-in epilogue of the kernel that adds them, and the launches t
 
 Exact data (any order of the sum gives the same bits) against the oracle, bit for bit.
 """
+import os
+import re
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -83,6 +87,27 @@ def test_what_the_offsets_of_the_small_tiles_do_not_reach(dt, shape):
             unsplit = cabi.scratch_bytes(d)
         with cabi.tuning("MI355_F8_TILES", "small"):
             assert (cabi.scratch_bytes(d) == unsplit) == fits, k
+
+
+def test_kernels_that_read_no_parts_have_no_arguments_for_them(tmp_path):
+    """the launch of a small int8 product is a few microseconds, and every argument is written to the device for it"""
+    from tests.test_loop_isa import OBJDUMP
+    readelf = OBJDUMP.replace("objdump", "readelf")
+    if not os.path.exists(readelf):
+        pytest.skip("no disassembler")
+    os.symlink(os.path.abspath(cabi.KERNEL_LIB_PATH), tmp_path / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
+    size = {}
+    for f in os.listdir(tmp_path):
+        if "gfx950" in f:
+            notes = subprocess.run([readelf, "--notes", f], cwd=tmp_path, check=True, capture_output=True, text=True).stdout
+            for k in notes.split("- .agpr_count")[1:]:
+                name = re.search(r"\.name: +(\S*chain_\S*kernel\S*)", k)
+                if name:
+                    size[name.group(1)] = int(re.search(r"\.kernarg_segment_size: (\d+)", k).group(1))
+    part = re.compile(r"chain_gemm_kernel.*Li4EE|chain_sum_kernel|chain_small_float")
+    with_parts, without = ({v for k, v in size.items() if bool(part.search(k)) == w} for w in (True, False))
+    assert len(size) > 60 and len(without) == 1 and max(without) <= min(with_parts) - 48, (with_parts, without)
 
 
 # steps of the last part: whole, one chunk, a chunk short of a step
