@@ -145,13 +145,6 @@ __device__ __forceinline__ void decode_zps(int dt, const raw_t<NPL, BITS> &r, fl
     }
 }
 
-// a sum, or where it is NaN that of its terms (woq_ops.hpp)
-template <bool F16>
-__device__ __forceinline__ float woq_checked(const woq_extra_t &X, float v, int m, int n) {
-    if (!F16 || v == v) return v;
-    return woq_term_sum(X, X.G, m, n, [&](int k) { return X.wei[(long)k * X.row_bytes + n / 2] >> (n % 2 * 4); });
-}
-
 // CHD dwords per lane and row; MT 16-row tiles of activations; NWV wavefronts
 // per workgroup share one column chunk and split its K range; SS = 16-row steps
 // of one super-step; SCB / ZPB = bits per scale / zero point (0 = absent).
@@ -281,6 +274,7 @@ __global__ void __launch_bounds__(NWV * 64) woq_gemv_kernel(const problem_t P_, 
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) rows_used[mt] = M - 16 * mt < 4 ? M - 16 * mt : 4;
     bool first_flush = true;
+    float poison = 0.f; // F16: NaN once a sum is not finite
     auto flush_group = [&](const qraw_t &qr) __attribute__((always_inline)) {
         float sc[NPL], zc[NPL];
         decode_scales<NPL, SCB>(X.sc_dt, qr.s, sc);
@@ -308,7 +302,12 @@ __global__ void __launch_bounds__(NWV * 64) woq_gemv_kernel(const problem_t P_, 
                             if (r < rows_used[mt]) // uniform: skips the padding rows of small M
                                 val[r] = sc[i] * __builtin_fmaf(-zc[i], rs[mt][r], acc[p][h][mt][r]);
                         v4f *slot = col + i * 16 * mqt;
-                        *slot = first_flush ? val : *slot + val;
+                        if (!first_flush) val = *slot + val;
+                        *slot = val;
+                        if constexpr (F16) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) poison = __builtin_fmaf(0.f, val[r], poison);
+                        }
                     }
             }
         }
@@ -359,6 +358,27 @@ __global__ void __launch_bounds__(NWV * 64) woq_gemv_kernel(const problem_t P_, 
     if (first_flush) { // empty K range: contribute zeros
         for (int u = lane; u < MQ * NW; u += 64) red4[wave * MQ * NW + u] = v4f {0.f, 0.f, 0.f, 0.f};
     }
+    if constexpr (F16) { // sums that are not finite, from their terms (woq_ops.hpp); cold code
+        if (__builtin_amdgcn_ballot_w64(poison != poison) != 0) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll 1
+            for (int nl = lane; nl < NW; nl += 64) {
+                const int n = min(chunk * NW + nl, N - 1);
+                const bool inside = chunk * NW + nl < N;
+                const bool all = woq_bad_scales(X, X.G, n, kb, ke, inside);
+#pragma unroll 1
+                for (int m = 0; m < M; ++m) {
+                    const int mt = m / 16, mqt = mt ? MQ - MQ0 : MQ0;
+                    float *cell = red + ((wave * MQ + mt * MQ0) * NW + (nl % NPL * 16 + nl / NPL) * mqt + m % 16 / 4) * 4 + m % 4;
+                    const bool need = inside && !__builtin_isfinite(*cell);
+                    if (__builtin_amdgcn_ballot_w64(need) == 0) continue;
+                    const float sum = woq_term_sum(X, X.G, m, n, kb, ke, all, need,
+                            [&](int k8, int i) { return X.wei[(long)(k8 + i) * X.row_bytes + n / 2] >> (n % 2 * 4); });
+                    if (need && !__builtin_isfinite(sum)) *cell = sum;
+                }
+            }
+        }
+    }
     // ---- reduce the wavefronts' LDS slices.  A unit is one 16-byte word: four
     // rows of one column, in the order the flush wrote them; the partial sums
     // in scratch keep that order, [split][chunk][unit].
@@ -393,14 +413,14 @@ __global__ void __launch_bounds__(NWV * 64) woq_gemv_kernel(const problem_t P_, 
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int m = mt * 16 + mq * 4 + r;
-            if (m < M) epilogue_store(P, woq_checked<F16>(X, v[r], m, n), 0, m, n);
+            if (m < M) epilogue_store(P, v[r], 0, m, n);
         }
     }
 }
 
 // Second pass: the partial sums of all splits are added in split order, one
 // thread per row quad and column over the whole device.
-template <int CHD, bool F16>
+template <int CHD>
 __global__ void __launch_bounds__(256) woq_reduce_kernel(const problem_t P_, const woq_extra_t X, int chunks) {
     const auto &P = MI355_KERNARG_PROBLEM();
     constexpr int NPL = CHD * 8, NW = 16 * NPL;
@@ -435,7 +455,7 @@ __global__ void __launch_bounds__(256) woq_reduce_kernel(const problem_t P_, con
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int m = mt * 16 + mq * 4 + r;
-        if (m < M) epilogue_store(P, woq_checked<F16>(X, v[r], m, n), 0, m, n);
+        if (m < M) epilogue_store(P, v[r], 0, m, n);
     }
 }
 
@@ -515,8 +535,8 @@ int launch_variant(int scb, int zpb, dim3 grid, size_t lds, hipStream_t stream, 
         hipLaunchKernelGGL(f16 ? kern_f16 : kern, grid, dim3(NWV * 64), lds, stream, P, X);
         if (X.ksplit > 1) {
             const long total = (long)grid.x * ((X.M + 3) / 4) * (16 * 8 * CHD);
-            hipLaunchKernelGGL(f16 ? (woq_reduce_kernel<CHD, true>) : (woq_reduce_kernel<CHD, false>), dim3((unsigned)((total + 255) / 256)),
-                    dim3(256), 0, stream, P, X, (int)grid.x);
+            hipLaunchKernelGGL(woq_reduce_kernel<CHD>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream,
+                    P, X, (int)grid.x);
         }
         return hipGetLastError() == hipSuccess ? MI355_SUCCESS : MI355_RUNTIME_ERROR;
     };

@@ -557,15 +557,6 @@ __global__ void __launch_bounds__(NWV * 64)
         }
     }
 
-    // an element whose sums came out as NaN, from its terms (woq_ops.hpp); cold code
-    auto term_sum = [&](int m, int n) __attribute__((always_inline)) {
-        const kernarg_woqp_extra_t &Y = *(kernarg_woqp_extra_t *)__builtin_amdgcn_kernarg_segment_ptr();
-        return woq_term_sum(Y, Y.spg == NO_GROUPS ? Y.K : Y.spg * KBLK, m, n, [&](int k) {
-            const unsigned at = (k / 8) * 512 + (n % 16) * 32 + (n % CHUNK) / 16 * 8 + (k % 2) * 4 + (k % 8) / 2; // in nibbles
-            return Y.wei[(long)(n / CHUNK) * Y.K * (CHUNK / 2) + at / 2] >> (at % 2 * 4);
-        });
-    };
-
     // ---- add the wavefronts' sums in wavefront order and store.  LDS holds
     // [wavefront][row][column] floats; a thread then owns four consecutive
     // columns of one row and runs the four-wide epilogue of the GEMM tiles.
@@ -579,6 +570,33 @@ __global__ void __launch_bounds__(NWV * 64)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 red[wave * WSTRIDE + (mt * 16 + 4 * q + r) * CHUNK + tt * 16 + j] = tot[mt][tt][r];
+    if constexpr (F16) { // sums that are not finite, from their terms (woq_ops.hpp); cold code
+        v4f poison = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) poison[r] = __builtin_fmaf(0.f, tot[mt][tt][r], poison[r]);
+        const float any = (poison[0] + poison[1]) + (poison[2] + poison[3]);
+        if (__builtin_amdgcn_ballot_w64(any != any) != 0) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const kernarg_woqp_extra_t &Y = *(kernarg_woqp_extra_t *)__builtin_amdgcn_kernarg_segment_ptr();
+            const int first = wave * Y.kbw * KBLK, last = min(first + Y.kbw * KBLK, Y.K);
+            const uint8_t *col = Y.wei + (long)chunk * Y.K * (CHUNK / 2) + j * 16 + q * 4; // (lane = column)
+            const int group = Y.spg == NO_GROUPS ? Y.K : Y.spg * KBLK;
+            const bool all = woq_bad_scales(Y, group, chunk * CHUNK + lane, first, last, true);
+#pragma unroll 1
+            for (int m = 0; m < Y.M; ++m) {
+                float *cell = red + wave * WSTRIDE + m * CHUNK + lane;
+                const bool need = !__builtin_isfinite(*cell);
+                if (__builtin_amdgcn_ballot_w64(need) == 0) continue;
+                const float sum = woq_term_sum(Y, group, m, chunk * CHUNK + lane, first, last, all, need,
+                        [&](int k8, int i) { return *(const unsigned *)(col + (long)k8 * (CHUNK / 2)) >> (i % 2 * 16 + i / 2 * 4); });
+                if (need && !__builtin_isfinite(sum)) *cell = sum;
+            }
+        }
+    }
     __syncthreads();
     if constexpr (PLAIN) {
         // one element per thread, 64 consecutive columns per wavefront
@@ -589,7 +607,6 @@ __global__ void __launch_bounds__(NWV * 64)
             float v = cell[0];
 #pragma unroll
             for (int wv = 1; wv < NWV; ++wv) v += cell[wv * WSTRIDE];
-            if (F16 && v != v) v = term_sum(m, chunk * CHUNK + nl);
             const unsigned bits = X.dst_dt == MI355_DT_F32 ? f2u(v)
                     : X.dst_dt == MI355_DT_BF16 ? (unsigned)f32_to_bf16(v) : (unsigned)f32_to_f16(v);
             const long off = (long)m * X.dst_ld + chunk * CHUNK + nl;
@@ -611,7 +628,6 @@ __global__ void __launch_bounds__(NWV * 64)
             float v = cell[0];
 #pragma unroll
             for (int wv = 1; wv < NWV; ++wv) v += cell[wv * WSTRIDE];
-            if (F16 && v != v) v = term_sum(m, chunk * CHUNK + nl);
             epilogue_store(P, v, 0, m, chunk * CHUNK + nl);
         }
         return;
@@ -626,11 +642,6 @@ __global__ void __launch_bounds__(NWV * 64)
         for (int wv = 1; wv < NWV; ++wv) sum += cell[wv * (WSTRIDE / 4)];
         float v[4] = {sum[0], sum[1], sum[2], sum[3]};
         const long n = (long)chunk * CHUNK + nq * 4;
-        if constexpr (F16) {
-#pragma unroll 1
-            for (int i = 0; i < 4; ++i)
-                if (v[i] != v[i]) v[i] = term_sum(m, (int)n + i);
-        }
         gemm::apply_epilogue4(P, v, 0, m, n, 4);
         gemm::store4(P, P.ds[2] == 1 && gemm::vec_ok_store(P.dst, P.ds[0], P.ds[1], dt_bits(P.dst_dt)), v, 0, m, n, 4);
     }

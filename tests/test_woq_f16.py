@@ -7,7 +7,7 @@ import pytest
 
 from onednn_amd import cabi, configs
 from onednn_amd import dtypes as dtp
-from onednn_amd.problem import run_gpu
+from onednn_amd.problem import GpuRun, run_gpu
 from tests.helpers import assert_bit_exact, assert_decode_close, decode
 
 IMPLS = {"plain": (cabi.IMPL_WOQ_GEMV, "hip:woq_gemv"), "packed": (cabi.IMPL_WOQ_PACKED, "hip:woq_packed")}
@@ -90,6 +90,72 @@ def test_f16_infinite_activations(gpu, oracle, layout, M, K, wdt, zkind, ddt, re
     want = oracle.run_oracle(p)
     g, w = (decode(p.dst_dt, x, M * 192).astype(np.float64).reshape(M, 192)[:3] for x in (got, want))
     np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", IMPLS)
+@pytest.mark.parametrize("M,K,group,fill", [(2, 8320, 64, "a row"), (32, 1056, 1056, "a row"), (5, 2048, 128, "every 37th"),
+                                            (17, 4096, 512, "scales")])
+def test_f16_sums_that_are_not_finite(gpu, oracle, layout, M, K, group, fill):
+    """rows of infinities and infinite scales; no w is 0, so no term is NaN"""
+    N = 192
+    p = f16_problem(M, N, K, group, layout, sdt="f32", zkind="none", ddt="f32")
+    r = np.random.default_rng(K)
+    p.wei = dtp.pack_nibbles(r.integers(1, 16, size=(K, N), dtype=np.uint8))
+    src = np.asarray(p.src).view(np.float16).reshape(M, K)
+    src[src == 0] = 1
+    bad = M - 1
+    if fill == "a row":
+        src[bad] = np.inf
+    elif fill == "every 37th":
+        src[bad, 5::37] = -np.inf
+    else:
+        src[...] = np.abs(src)
+        p.quant["wei_scale"].data.reshape(-1, N)[-1, ::7] = np.inf
+    p.src = src.view(np.uint16)
+    got, name = run_gpu(p, IMPLS[layout][0])
+    want = oracle.run_oracle(p)
+    g, w = (decode(p.dst_dt, x, M * N).astype(np.float64).reshape(M, N) for x in (got, want))
+    special = ~np.isfinite(w)
+    assert special.any()
+    np.testing.assert_array_equal(g[special], w[special])
+    assert np.isfinite(g[~special]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", IMPLS)
+@pytest.mark.parametrize("M,times", [(1, 8), (32, 32)])
+def test_f16_infinite_activations_take_no_walk_along_k(gpu, layout, M, times):
+    """An infinity in a row is looked up in a pass over the row's activations, a few latencies for a wavefront's part of K and row:
+    at most a launch more where M is 1 (measured 1.2 times the time), and 2.9 and 4.1 times with one in each of 32 rows.  A
+    walk of every element over all of K, a term after the other, took 16384 latencies: 400 to 900 times."""
+    import ctypes as C
+    lib = cabi.load_kernels()
+    p = f16_problem(M, 8192, 16384, 128, layout)
+    clean, src = p.src, np.asarray(p.src).view(np.float16).reshape(M, -1).copy()
+    src[:, 4097] = np.inf
+    ms = {}
+    for what, values in (("finite", clean), ("infinite", src.view(np.uint16))):
+        p.src = values
+        run = GpuRun(p, IMPLS[layout][0])
+        ev = [C.c_void_p(), C.c_void_p()]
+        for e in ev:
+            cabi.check(lib.mi355_event_create(C.byref(e)))
+        try:
+            run.launch()
+            cabi.check(lib.mi355_event_record(ev[0], None))
+            for _ in range(4):
+                run.launch()
+            cabi.check(lib.mi355_event_record(ev[1], None))
+            cabi.check(lib.mi355_event_sync(ev[1]))
+            t = C.c_float()
+            cabi.check(lib.mi355_event_elapsed_ms(C.byref(t), ev[0], ev[1]))
+            ms[what] = t.value / 4
+        finally:
+            run.free()
+            for e in ev:
+                lib.mi355_event_destroy(e)
+    assert ms["infinite"] < times * ms["finite"], ms
 
 
 @pytest.mark.parametrize("dt,M,N,K", [("f16", 1, 14336, 4096), ("f16", 32, 64, 128), ("f16", 4, 1024, 16384), ("bf16", 8, 8128, 4096),
