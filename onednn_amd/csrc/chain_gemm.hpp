@@ -26,10 +26,11 @@ enum chain_act_t { CHAIN_NONE, CHAIN_RELU, CHAIN_GELU, CHAIN_SWISH };
 // (256 x 128, or 256 x 256) a launch takes its K steps one after the other on T of 256 CUs.  S parts make that steps / S, for
 // a second kernel (3 us and more of a launch), the parts' way out and in again (a part of a tile 128 / 256 KB each way) and
 // a workgroup's fixed cost, which is why S is not 256 / T: per step_ns + S T part_ns + CHAIN_SPLIT_NS is what a launch of S
-// parts of `per` steps takes beyond one without, and the S of the least is within 1.05 of the best S measured on 20 shapes of every
-// type.  Unsplit / split, us: fp8 256 x 4352 x 12224 73.7 / 30.4, 64 x 640 x 16384 66.6 / 18.3, 512 x 7168 x 16384 (two parts) 73.0 / 60.0;
-// MXFP4 100 x 1040 x 16352 58.3 / 27.1; bf16 4096 x 960 x 13312 125 / 95.6, f16 300 x 2048 x 4096 38.8 / 23.0; int8 256 x 6272 x
-// 6528 (u8) 53.0 / 36.3; where steps are few the second kernel costs more than it gives (bf16 512 x 3600 x 704 15.0 / 23.2).
+// parts of `per` steps takes beyond one without.  Its S against the best of up to 12 on 22 shapes of every type: within 1.05 on
+// 18, at worst 1.15 (fp8 300 x 2048 x 2048, which it does not split: 17.4 us, two parts 15.1).  Unsplit / split, us, launches after each
+// other on the same operands: fp8 256 x 4352 x 12224 73.8 / 27.8, 64 x 640 x 16384 67.3 / 15.8, 512 x 7168 x 16384 (two parts) 74.5 / 59.0; MXFP4
+// 100 x 1040 x 16352 55.0 / 23.3; bf16 4096 x 960 x 13312 118 / 92.9, f16 300 x 2048 x 4096 39.2 / 19.6; int8 256 x 6272 x 6528 (u8) 50.6 /
+// 34.9; where steps are few the second kernel costs more than it gives (bf16 512 x 3600 x 704 14.8 / 19.2 in two parts).
 constexpr long CHAIN_SPLIT_NS = 5000;
 struct chain_split_t {
     int split, part_steps;

@@ -162,12 +162,13 @@ bool small_tiles_fit(long M, long N, long kbytes, int mx) {
             && (mx == 0 || kbytes * 8 / mx / 32 * N < (1L << 32));
 }
 
-// Both sides in ns, as measured on 64 shapes of every type (small / 256 x 128 tiles, K split where that pays, us): fp8 16 x 2240 x
-// 1024 5.3 / 12.9, 256 x 2048 x 1024 7.2 / 13.4, 64 x 4096 x 4096 10.7 / 19.8, 916 x 512 x 640 with gelu_tanh and a residual 7.7 / 16.7, but 64 x
-// 640 x 16384 30.7 / 19.0; bf16 32 x 1792 x 768 6.2 / 13.9, 512 x 1024 x 1024 10.2 / 16.3, 128 x 1024 x 8192 (f16) 34.0 / 20.1, 512 x 3600 x
-// 704 23.5 / 14.7; MXFP4 128 x 2048 x 2048 9.4 / 23.0 (whose 7 us of pre-pass kernels it does without), MXFP8 300 x 1040 x 1056 9.0 / 25.9.
+// Both sides in ns.  Small / 256 x 128 tiles, K split where that pays, us, launches after each other on the same operands: fp8 16 x
+// 2240 x 1024 4.1 / 12.7, 256 x 2048 x 1024 6.3 / 13.5, 64 x 4096 x 4096 10.3 / 16.2, but 64 x 640 x 16384 30.1 / 15.9; bf16 32 x 1792 x 768
+// 5.1 / 13.8, 512 x 1024 x 1024 9.7 / 16.2, 128 x 1024 x 8192 (f16) 30.4 / 16.1, 512 x 3600 x 704 23.1 / 14.7; MXFP4 128 x 2048 x 2048 5.4 / 18.4
+// (whose 7 us of pre-pass kernels it does without), MXFP8 240 x 1040 x 1056 7.1 / 20.7.  On 25 shapes the side taken is the faster or within 1.03 of
+// it, but for fp8 300 x 1040 x 4096 (17.1 / 14.8).
 // MXFP8 beyond 256 tiles, in the large tiles' order (data that tests/test_mxf8_gemm.py calls exact takes 25 bits there, so that its
-// bits follow the order of the sums): 128 x 3520 x 1408 15.8 / 24.5, 700 x 1024 x 640 12.9 / 21.5.
+// bits follow the order of the sums): 300 x 1040 x 1056 7.7 / 20.6, 128 x 3520 x 1408 13.2 / 20.1, 700 x 1024 x 640 9.8 / 17.1.
 // A workgroup's steps are a chain (1.67 ns a byte of K), its neighbours' traffic comes on top (per tile).
 bool small_tiles_float(long batch, long M, long N, long kbytes, const chain_split_t &split, long step_ns, const chain_t &C, int mx) {
     const double tiles = (double)((M + FST - 1) / FST) * ((N + FST - 1) / FST) * batch;

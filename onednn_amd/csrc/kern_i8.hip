@@ -357,8 +357,9 @@ bool small_tiles_better(const mi355_matmul_desc_t &d, bool chain) {
 }
 
 // The line of small_tiles_better is drawn against LDS tiles that take all of K; with K split (chain_gemm.hpp) they are the better
-// ones from fewer small tiles on where K is long.  Both sides in ns, from a dozen shapes: 128 x 4096 x 4096 17.1 us small, 20.2
-// split, 1024 x 1024 x 4096 31 and 20.3, with sums 64 x 2048 x 16384 31.0 and 33.4; a tenth in favour of the small tiles, one launch.
+// ones from fewer small tiles on where K is long.  Both sides in ns: 128 x 4096 x 4096 17.1 us small, 20.2
+// split, 1024 x 1024 x 4096 31 and 20.3, 300 x 2048 x 8192 45.4 and 20.2, with sums 64 x 2048 x 16384 31.0 and 33.4, 415 x 1664 x 13024
+// 56.1 and 34.2; a tenth in favour of the small tiles, one launch.
 bool split_tiles_better(const mi355_matmul_desc_t &d, const chain_split_t &s) {
     const bool sums = d.src_dt == MI355_DT_U8 || !quant_absent(d.src_zp);
     const double small_tiles = (double)((d.M + ST - 1) / ST) * ((d.N + ST - 1) / ST) * d.batch;
